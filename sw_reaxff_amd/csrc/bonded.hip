@@ -596,26 +596,27 @@ __global__ void __launch_bounds__(BT) k_hb_fold(int N, unsigned long long *__res
 // type h) with |p_val1| > 0.001: the angle, penalty and coalition energies;
 // their coefficients into Cdbo of both bonds and of all of j's bonds
 // (CEval6 BO^7), Cdbopi/Cdbopi2 of j's bonds (CEval5), CdDelta of j, k and
-// h, and the angle derivative into fCdDelta[.][0..2] of k, j and h.  One
-// thread per j writes j's own bond slots and row; the terms of k and h go
+// h, and the angle derivative into fCdDelta[.][0..2] of k, j and h.  A group
+// of lanes per j writes j's own bond slots and row; the terms of k and h go
 // into 64-bit fixed-point accumulators by integer atomics (order-independent
 // sums), folded into fCdDelta by k_va_fold.  The centres with angles are
 // listed by angle count (k_va_count, k_wl_scan, k_va_scatter: a centre with
-// ten bonds has 45 pairs, one with two bonds one) and the threads take them
+// ten bonds has 45 pairs, one with two bonds one) and the groups take them
 // largest first.
 constexpr double DEG2RAD_PI = 3.14159265;   // constPI, reaxc_defs_sunway.h:61 (DEG2RAD :55)
 
 // ---------------------------------------------------------------- work lists
-// The valence and torsion passes give each lane one item (a centre atom, a
-// central bond) and most items have little or no work while a few have
-// dozens of angles: items are counted first, bucketed by count and handed
-// to lanes largest first, so the lanes of a wave do about the same work.
-// Counters: the list length, a histogram of the counts and each bucket's
-// next free position.  Which lane takes which item changes no result: every
+// The valence and torsion passes work on items (a centre atom, a central
+// bond) of which most have little or no work while a few have dozens of
+// angles: items are counted first, bucketed by count and handed out largest
+// first, each to a group of as many lanes as it has evaluations.
+// Counters: the list length, a histogram of the counts, each bucket's next
+// free position and where each group size ends.  Which lane takes which item changes no result: every
 // item writes only its own entries and adds into the others through
 // fixed-point integer atomics.
 constexpr int WL_NB = 128;    // count buckets; counts of WL_NB - 1 and more share the last
-enum { WL_NTASK = 0, WL_HIST = 1, WL_CUR = WL_HIST + WL_NB, WL_CTL_INTS = WL_CUR + WL_NB };
+enum { WL_NTASK = 0, WL_HIST = 1, WL_CUR = WL_HIST + WL_NB, WL_ABOVE = WL_CUR + WL_NB, WL_CTL_INTS = WL_ABOVE + 6 };
+constexpr int WL_NABOVE = 6;   // ctl[WL_ABOVE + q]: items with counts above 32 >> q
 __device__ __forceinline__ int wl_bucket(int c) { return c < WL_NB - 1 ? c : WL_NB - 1; }
 
 // Bucket starts, largest count first; the histogram is left at zero.
@@ -629,6 +630,122 @@ __global__ void __launch_bounds__(WL_NB) k_wl_scan(int *__restrict__ ctl) {
   for (int q = b + 1; q < WL_NB; ++q) start += h[q];
   ctl[WL_CUR + b] = start;
   if (b == 0) ctl[WL_NTASK] = start + h[0];
+  // items with counts above 32, 16, .., 1: where each group size ends
+  for (int q = 0; q < WL_NABOVE; ++q)
+    if (b == (SWR_WAVE >> (q + 1))) ctl[WL_ABOVE + q] = start;
+}
+
+// The waves of a listed pass.  An item of count c gets a group of G lanes, the
+// power of two at or above c (at most 64), so one round of the group evaluates
+// the whole item; items sit in the list in falling count, so the groups of
+// each size are consecutive and a wave holds 64 / G groups of one size.  A
+// group has at least gmin lanes: finding an item's evaluations among the pairs
+// of its bonds is spread over the group too, which is what a short list (few
+// waves, each waiting for its own chain of loads) needs, while a long list
+// fills the chip with narrow groups and would only evaluate with fewer lanes.
+struct WlWave {
+  int G;        // lanes per group
+  int t;        // this lane's item (live: inside the list)
+  int sub;      // lane within the group
+  bool live;
+};
+
+__device__ __forceinline__ bool wl_wave(const int *__restrict__ ctl, int unit, int gmin, WlWave &w) {
+  const int lane = lane_id();
+  int first = 0;   // items of wider groups
+#pragma unroll
+  for (int q = 0; q <= WL_NABOVE; ++q) {
+    const int G = SWR_WAVE >> q;
+    const bool last = G <= gmin;
+    const int end = last || q == WL_NABOVE ? ctl[WL_NTASK] : ctl[WL_ABOVE + q];
+    const int waves = (end - first + (1 << q) - 1) >> q;
+    if (unit < waves) {
+      w.G = G;
+      w.t = first + (unit << q) + lane / G;
+      w.sub = lane % G;
+      w.live = w.t < end;
+      return true;
+    }
+    if (last) return false;
+    unit -= waves;
+    first = end;
+  }
+  return false;
+}
+
+// Sum over the aligned group of G lanes (a power of two), on every lane.
+__device__ __forceinline__ double group_sum(double v, int G) {
+  for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o, SWR_WAVE);
+  return v;
+}
+__device__ __forceinline__ double group_product(double v, int G) {
+  for (int o = 1; o < G; o <<= 1) v *= __shfl_xor(v, o, SWR_WAVE);
+  return v;
+}
+
+// Orders a wave's own LDS accesses (each wave has its own slice).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Each group's pending evaluations: (a, b) positions in two bond ranges as
+// a << 8 | b, in pair order, at most 2 G - 1 of them.
+struct PairQueue {
+  unsigned short *q;   // the group's slice (2 G entries) of the wave's LDS
+  int n;               // pending
+  int r, a, b;         // this lane's next raw pair r = a * mb + b
+  int da, db;          // G / mb, G % mb
+};
+
+// Tests raw pairs (a < ma, b < mb), G at a time, until every group of the
+// wave has G pending or no pairs left; test(a, b) says whether one is an
+// evaluation.  The order of the pending ones is the raw order.
+template <class Test>
+__device__ __forceinline__ void queue_fill(PairQueue &Q, const WlWave &w, int ma, int mb, Test test) {
+  const int lane = lane_id(), g0 = lane - w.sub;
+  const unsigned long long gm = w.G == SWR_WAVE ? ~0ull : ((1ull << w.G) - 1ull);
+  const unsigned long long below = (1ull << w.sub) - 1ull;
+  const int R = w.live ? ma * mb : 0;
+  while (true) {
+    const bool more = Q.n < w.G && Q.r - w.sub < R;   // the same on the group's lanes
+    if (!__any(more)) break;
+    bool pass = false;
+    const int code = Q.a << 8 | Q.b;
+    if (more) {
+      if (Q.r < R) pass = test(Q.a, Q.b);
+      Q.r += w.G;
+      Q.a += Q.da;
+      Q.b += Q.db;
+      if (Q.b >= mb) { Q.b -= mb; Q.a += 1; }
+    }
+    const unsigned long long m = (__ballot(pass) >> g0) & gm;
+    if (pass) Q.q[Q.n + __popcll(m & below)] = (unsigned short)code;
+    Q.n += __popcll(m);
+  }
+  wave_lds_order();
+}
+
+// After a round took the first `took` pending pairs.
+__device__ __forceinline__ void queue_drop(PairQueue &Q, const WlWave &w, int took) {
+  const int rem = Q.n - took;   // at most G - 1
+  const unsigned short v = w.sub < rem ? Q.q[took + w.sub] : (unsigned short)0;
+  wave_lds_order();
+  if (w.sub < rem) Q.q[w.sub] = v;
+  Q.n = rem;
+  wave_lds_order();
+}
+
+__device__ __forceinline__ void queue_init(PairQueue &Q, const WlWave &w, unsigned short *wave_lds, int mb) {
+  const int m = mb > 0 ? mb : 1;
+  Q.q = wave_lds + 2 * (lane_id() - w.sub);
+  Q.n = 0;
+  Q.r = w.sub;
+  Q.a = w.sub / m;
+  Q.b = w.sub - Q.a * m;
+  Q.da = w.G / m;
+  Q.db = w.G - Q.da * m;
 }
 
 // Workgroup histogram of counts c (> 0 adds) into the global one.
@@ -718,28 +835,51 @@ __global__ void __launch_bounds__(BT) k_va_scatter(int n, VaArgs A) {
   if (b >= 0) A.order[base[b] + r] = j;
 }
 
-// One thread per listed centre j (largest angle count first).
-__global__ void __launch_bounds__(BT) k_valence(VaArgs A) {
-  const int t = blockIdx.x * BT + threadIdx.x;
-  if (t >= A.ctl[WL_NTASK]) return;
-  const int j = A.order[t];
-  const DevParams *__restrict__ P = A.P;
-  const int tj = A.atoms[j].type;
-  const int b0 = A.bidx[j], b1 = A.bend[j];
-  double e_ang = 0.0, e_pen = 0.0, e_coa = 0.0;
-  if (tj >= 0 && b1 > b0) {
+// Waves of one-wave workgroups a listed pass starts at most; each wave takes
+// its next set of groups that many on (the first ones hold the largest items).
+constexpr int WL_MAX_WAVES = 4096;
+// Shortest group while a list has few items, as lanes in all: below it the
+// pass is bound by each item's chain of loads and transcendentals, not by
+// lanes.
+__device__ __forceinline__ int wl_gmin(int ntask) { return ntask <= 4096 ? 16 : ntask <= 16384 ? 4 : 1; }
+
+// One group of lanes per listed centre j (largest angle count first): the
+// group's lanes test j's bond pairs and each evaluates one passing pair a
+// round.  What bounds the pass is the latency of one pair's transcendentals
+// (at 1-2 waves a SIMD), so a centre's pairs side by side instead of in turn
+// take the longest centre off the critical path.  Per round the pairs' Cdbo
+// terms go to LDS and the lane that owns a slot adds them in pair order; the
+// centre's sums are group butterflies, so every order is fixed.  One thread
+// per centre took 52 us on a 64-water box and 150 us on the 32,000-water one;
+// this takes 18 and 108 (512 clusters: 1.05 ms either way, all lanes busy).
+__global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
+  __shared__ unsigned short queue[2 * SWR_WAVE];
+  __shared__ double spk[SWR_WAVE], sph[SWR_WAVE];
+  const int lane = lane_id();
+  const int gmin = wl_gmin(A.ctl[WL_NTASK]);
+  WlWave w;
+  for (int unit = blockIdx.x; wl_wave(A.ctl, unit, gmin, w); unit += gridDim.x) {
+    const int j = w.live ? A.order[w.t] : 0;
+    const int G = w.G, g0 = lane - w.sub;
+    const DevParams *__restrict__ P = A.P;
+    const int tj = w.live ? A.atoms[j].type : 0;
+    const int b0 = w.live ? A.bidx[j] : 0, b1 = w.live ? A.bend[j] : 0;
+    const int m = b1 - b0;
+    double e_ang = 0.0, e_pen = 0.0, e_coa = 0.0;
     const double thb_cut = P->thb_cut, thb_cutsq = P->thb_cutsq;
     const double Dboc_j = A.bo_dboc[2 * (size_t)j + 1];
     const double p_val3 = P->p_val3[tj], p_val5 = P->p_val5[tj];
     const double p_val6 = P->p_val6, p_val8 = P->p_val8, p_val9 = P->p_val9, p_val10 = P->p_val10;
     double SBOp = 0.0, prod_SBO = 1.0;
-    for (int t = b0; t < b1; ++t) {
+    for (int t = b0 + w.sub; t < b1; t += G) {
       SBOp += A.BOpi[2 * (size_t)t] + A.BOpi[2 * (size_t)t + 1];
       double b2 = A.BO[t] * A.BO[t];
       b2 *= b2;
       b2 *= b2;
       prod_SBO *= exp(-b2);
     }
+    SBOp = group_sum(SBOp, G);
+    prod_SBO = group_product(prod_SBO, G);
     double vlpadj, dSBO2;
     if (A.vlpex[j] >= 0) {
       vlpadj = 0.0;
@@ -769,26 +909,33 @@ __global__ void __launch_bounds__(BT) k_valence(VaArgs A) {
     const double Cf9j = (-P->p_pen3 * exp_pen3 * trm_pen34 - (2.0 + exp_pen3) * (-P->p_pen3 * exp_pen3 + P->p_pen4 * exp_pen4)) /
                         (trm_pen34 * trm_pen34);
     const double exp_coa2 = exp(P->p_coa2 * A.Delta_val[j]);
-    double ce5 = 0.0, ce6 = 0.0, cdj = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    for (int pk = b0; pk < b1; ++pk) {
-      const double BO_jk = A.BO[pk];
-      if (!(BO_jk > thb_cut)) continue;
-      const swr_bond_t bjk = A.bonds[pk];
-      const int k = bjk.nbr;
-      if (A.bend[k] <= A.bidx[k]) continue;
-      const int tk = A.atoms[k].type;
-      const double BOA_jk = BO_jk - thb_cut;
-      for (int ph = pk + 1; ph < b1; ++ph) {
-        const double BO_hj = A.BO[ph];
-        if (!(BO_hj > thb_cut) || !(BO_jk * BO_hj > thb_cutsq)) continue;
-        const int th = A.atoms[A.bonds[ph].nbr].type;
-        if (tk < 0 || th < 0) continue;
+    double ce5 = 0.0, ce6 = 0.0, cdj = 0.0, g0s = 0.0, g1s = 0.0, g2s = 0.0;
+    PairQueue Q;
+    queue_init(Q, w, queue, m);
+    while (true) {
+      queue_fill(Q, w, m, m, [&](int a, int b) {
+        if (b <= a) return false;
+        const double BO_jk = A.BO[b0 + a], BO_hj = A.BO[b0 + b];
+        const int k = A.bonds[b0 + a].nbr, h = A.bonds[b0 + b].nbr;
+        const int tk = A.atoms[k].type, th = A.atoms[h].type;
+        if (!(BO_jk > thb_cut) || !(BO_hj > thb_cut) || !(BO_jk * BO_hj > thb_cutsq)) return false;
+        if (tk < 0 || th < 0 || A.bend[k] <= A.bidx[k]) return false;
+        return P->thb_n[(tk * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + th] != 0;
+      });
+      const int take = min(Q.n, G);
+      if (!__any(take > 0)) break;
+      const bool ev = w.sub < take;
+      double cdbo_jk = 0.0, cdbo_hj = 0.0;
+      if (ev) {
+        const int code = Q.q[w.sub];
+        const int pk = b0 + (code >> 8), ph = b0 + (code & 255);
+        const double BO_jk = A.BO[pk], BO_hj = A.BO[ph];
+        const swr_bond_t bjk = A.bonds[pk], bhj = A.bonds[ph];
+        const int k = bjk.nbr, h = bhj.nbr;
+        const int tk = A.atoms[k].type, th = A.atoms[h].type;
+        const double BOA_jk = BO_jk - thb_cut, BOA_hj = BO_hj - thb_cut;
         const int tri = (tk * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + th;
         const int nset = P->thb_n[tri];
-        if (nset == 0) continue;
-        const swr_bond_t bhj = A.bonds[ph];
-        const int h = bhj.nbr;
-        const double BOA_hj = BO_hj - thb_cut;
         // Calculate_Theta / Calculate_dCos_Theta (:1510-1547) with the j-k
         // bond first: di belongs to k, dk to h
         const double dot = bjk.dvec[0] * bhj.dvec[0] + bjk.dvec[1] * bhj.dvec[1] + bjk.dvec[2] * bhj.dvec[2];
@@ -815,7 +962,6 @@ __global__ void __launch_bounds__(BT) k_valence(VaArgs A) {
                                          exp(-P->p_coa4 * (BOA_hj - 1.5) * (BOA_hj - 1.5))
                                    : 0.0;
         double ck[4] = {0.0, 0.0, 0.0, 0.0}, chh[4] = {0.0, 0.0, 0.0, 0.0};
-        double cdbo_jk = 0.0, cdbo_hj = 0.0;
         for (int c = 0; c < nset; ++c) {
           const DevThb &q = P->thb[tri][c];
           const double p_val1 = q.p_val1, p_val2 = q.p_val2, p_val4 = q.p_val4, p_val7 = q.p_val7;
@@ -870,13 +1016,11 @@ __global__ void __launch_bounds__(BT) k_valence(VaArgs A) {
             const double dk = bjk.dvec[d] * inv_d - cinv3 * sq_jk * bhj.dvec[d];
             ck[d] += CEval8 * di;
             chh[d] += CEval8 * dk;
-            if (d == 0) g0 += CEval8 * dj;
-            if (d == 1) g1 += CEval8 * dj;
-            if (d == 2) g2 += CEval8 * dj;
+            if (d == 0) g0s += CEval8 * dj;
+            if (d == 1) g1s += CEval8 * dj;
+            if (d == 2) g2s += CEval8 * dj;
           }
         }
-        A.Cdbo[pk] += cdbo_jk;
-        A.Cdbo[ph] += cdbo_hj;
         unsigned long long *ak = A.acc + 4 * (size_t)k, *ah = A.acc + 4 * (size_t)h;
         {
           unsigned long long *const ga[8] = {ak, ak + 1, ak + 2, ak + 3, ah, ah + 1, ah + 2, ah + 3};
@@ -885,23 +1029,50 @@ __global__ void __launch_bounds__(BT) k_valence(VaArgs A) {
           fix_add_group<8>(A.flags, ga, gc, gv);
         }
       }
+      // the round's Cdbo terms onto j's slots, in pair order by each slot's lane
+      spk[lane] = cdbo_jk;
+      sph[lane] = cdbo_hj;
+      wave_lds_order();
+      for (int t0 = 0; t0 < m; t0 += G) {
+        const int t = t0 + w.sub;
+        double add = 0.0;
+        for (int e = 0; e < take; ++e) {
+          const int code = Q.q[e];
+          if ((code >> 8) == t) add += spk[g0 + e];
+          if ((code & 255) == t) add += sph[g0 + e];
+        }
+        if (add != 0.0) A.Cdbo[b0 + t] += add;
+      }
+      wave_lds_order();
+      queue_drop(Q, w, take);
     }
+    ce5 = group_sum(ce5, G);
+    ce6 = group_sum(ce6, G);
     if (ce5 != 0.0 || ce6 != 0.0)
-      for (int t = b0; t < b1; ++t) {
+      for (int t = b0 + w.sub; t < b1; t += G) {
         const double bo = A.BO[t];
         const double bo3 = bo * bo * bo;
         A.Cdbo[t] += ce6 * (bo3 * bo3 * bo);
         A.Cdbopi[t] += ce5;
         A.Cdbopi2[t] += ce5;
       }
-    A.fcd[4 * (size_t)j] += g0;
-    A.fcd[4 * (size_t)j + 1] += g1;
-    A.fcd[4 * (size_t)j + 2] += g2;
-    A.fcd[4 * (size_t)j + 3] += cdj;
+    cdj = group_sum(cdj, G);
+    g0s = group_sum(g0s, G);
+    g1s = group_sum(g1s, G);
+    g2s = group_sum(g2s, G);
+    e_ang = group_sum(e_ang, G);
+    e_pen = group_sum(e_pen, G);
+    e_coa = group_sum(e_coa, G);
+    if (w.live && w.sub == 0) {
+      A.fcd[4 * (size_t)j] += g0s;
+      A.fcd[4 * (size_t)j + 1] += g1s;
+      A.fcd[4 * (size_t)j + 2] += g2s;
+      A.fcd[4 * (size_t)j + 3] += cdj;
+      A.part[j] = e_ang;
+      A.part[A.stride + j] = e_pen;
+      A.part[2 * A.stride + j] = e_coa;
+    }
   }
-  A.part[j] = e_ang;
-  A.part[A.stride + j] = e_pen;
-  A.part[2 * A.stride + j] = e_coa;
 }
 
 // fCdDelta (all four columns) += the fixed-point terms; the accumulators are
@@ -939,8 +1110,8 @@ __global__ void __launch_bounds__(BT) k_va_fold(int N, unsigned long long *__res
 //   k_to_scatter  one thread per local atom: its central bonds with work
 //                 into the list (the order inside a bucket is arbitrary and
 //                 changes no result);
-//   k_torsion     one lane per listed central bond: the slot's Cdbopi and
-//                 Cdbo written directly, j's row terms and energies into
+//   k_torsion     a group of lanes per listed central bond, one quadruple a
+//                 lane: the slot's Cdbopi and Cdbo written directly, j's row terms and energies into
 //                 the slot's row entry, Cdbo of j-i and k-l and the terms of
 //                 i, k, l into 64-bit fixed-point accumulators by integer
 //                 atomics (folded by k_va_fold / k_to_slot_fold);
@@ -993,10 +1164,22 @@ __device__ __forceinline__ double tan_inv(double s, double c) {
   return c / s;
 }
 
-// Quadruples the torsion body evaluates for the bond in slot pk of local
-// atom j (type tj >= 0, slots [b0, b1)): the body's filters in its order;
-// 0 when the bond is no central bond (its BO, the orig_id order, a k without
-// bonds or type) or makes no torsion.
+// Whether bonds ph (j-i) and pw (k-l) make a torsion with the central bond pk
+// (j-k; pj its reverse slot).  All loads are unconditional, so that the tests
+// of consecutive pairs overlap their latencies.
+__device__ __forceinline__ bool to_pass(const ToArgs &A, int tj, int tk, double BO_jk, int pk, int pj, int ph, int pw,
+                                        double thb_cut) {
+  const double BO_ij = A.BO[ph], BO_kl = A.BO[pw];
+  const int i = A.bnbr[ph], l = A.bnbr[pw];
+  const int ti = A.atoms[i].type, tl = A.atoms[l].type;
+  if (ph == pk || pw == pj || i == l || ti < 0 || tl < 0) return false;
+  if (!(BO_ij > thb_cut) || !(BO_kl > thb_cut) || !(BO_ij * BO_jk * BO_kl > thb_cut)) return false;
+  return A.P->tor[((ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + tl].cnt != 0;
+}
+
+// Quadruples of the bond in slot pk of local atom j (type tj >= 0, slots
+// [b0, b1)); 0 when the bond is no central bond (its BO, the orig_id order, a
+// k without bonds or type) or makes no torsion.
 __device__ __forceinline__ int to_count(const ToArgs &A, const swr_atom_pack_t &aj, int tj, int b0, int b1,
                                         int pk, double thb_cut) {
   const double BO_jk = A.BO[pk];
@@ -1011,23 +1194,10 @@ __device__ __forceinline__ int to_count(const ToArgs &A, const swr_atom_pack_t &
   const int pj = A.bonds[pk].sym_index;
   int c = 0;
   for (int ph = b0; ph < b1; ++ph) {
-    if (ph == pk) continue;
     const double BO_ij = A.BO[ph];
-    if (!(BO_ij > thb_cut)) continue;
-    const int i = A.bnbr[ph];
-    const int ti = A.atoms[i].type;
-    if (ti < 0) continue;
-    for (int pw = k0; pw < k1; ++pw) {
-      if (pw == pj) continue;
-      const double BO_kl = A.BO[pw];
-      if (!(BO_kl > thb_cut) || !(BO_ij * BO_jk * BO_kl > thb_cut)) continue;
-      const int l = A.bnbr[pw];
-      if (i == l) continue;
-      const int tl = A.atoms[l].type;
-      if (tl < 0) continue;
-      if (!A.P->tor[((ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + tl].cnt) continue;
-      ++c;
-    }
+    if (ph == pk || !(BO_ij > thb_cut)) continue;
+#pragma unroll 4
+    for (int pw = k0; pw < k1; ++pw) c += to_pass(A, tj, tk, BO_jk, pk, pj, ph, pw, thb_cut) ? 1 : 0;
   }
   return c;
 }
@@ -1081,198 +1251,218 @@ __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
   }
 }
 
-__global__ void __launch_bounds__(BT) k_torsion(ToArgs A) {
-  const int task = blockIdx.x * BT + threadIdx.x;
-  if (task >= A.ctl[WL_NTASK]) return;
-  const int2 jp = A.task[task];
-  const int j = jp.x, pk = jp.y;
+// One group of lanes per listed central bond (most quadruples first): the
+// group's lanes test the pairs of j-i and k-l bonds and each evaluates one
+// quadruple a round.  A quadruple is ~2000 dependent FP64 instructions at one
+// wave per SIMD, so what bounded the pass was the longest bond's chain of
+// quadruples.  i's terms are summed over the round's quadruples of one j-i
+// bond (a segmented scan: they are neighbours in the queue) before their
+// fixed-point add, and j's, k's and the bond's over the group, so the large
+// cotangent terms of a nearly linear angle cancel in FP64 first.  One lane
+// per bond took 87 us on a 64-water box, 133 us on the 32,000-water one and
+// 2.38 ms on 512 clusters; this takes 19, 65 us and 1.34 ms.
+__global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
+  __shared__ unsigned short queue[2 * SWR_WAVE];
+  constexpr double MIN_SINE = 1e-10;
+  const int lane = lane_id();
+  const int gmin = wl_gmin(A.ctl[WL_NTASK]);
   const DevParams *__restrict__ P = A.P;
-  double e_tor = 0.0, e_con = 0.0;
-  double fj[4] = {0.0, 0.0, 0.0, 0.0};
-  const swr_atom_pack_t aj = A.atoms[j];
-  const int tj = aj.type;
-  const int b0 = A.bidx[j], b1 = A.bend[j];
-  {
-    constexpr double MIN_SINE = 1e-10;
+  WlWave w;
+  for (int unit = blockIdx.x; wl_wave(A.ctl, unit, gmin, w); unit += gridDim.x) {
+    const int2 jp = w.live ? A.task[w.t] : A.task[0];
+    const int j = jp.x, pk = jp.y, G = w.G;
+    double e_tor = 0.0, e_con = 0.0;
+    double fj[4] = {0.0, 0.0, 0.0, 0.0};
+    const int tj = A.atoms[j].type;
+    const int b0 = A.bidx[j], b1 = A.bend[j];
     const double thb_cut = P->thb_cut;
     const double p_tor2 = P->p_tor2, p_tor3 = P->p_tor3, p_tor4 = P->p_tor4, p_cot2 = P->p_cot2;
     const double Delta_j = A.bo_dboc[2 * (size_t)j + 1];
-    do {
-      const double BO_jk = A.BO[pk];
-      if (!(BO_jk - thb_cut > 0.0)) break;
-      const swr_bond_t bjk = A.bonds[pk];
-      const int k = bjk.nbr;
-      const int k0 = A.bidx[k], k1 = A.bend[k];
-      if (k1 <= k0) break;
-      const swr_atom_pack_t ak = A.atoms[k];
-      if (aj.orig_id > ak.orig_id) break;
-      if (aj.orig_id == ak.orig_id) {
-        if (ak.x[2] < aj.x[2]) break;
-        if (ak.x[2] == aj.x[2] && ak.x[1] < aj.x[1]) break;
-        if (ak.x[2] == aj.x[2] && ak.x[1] == aj.x[1] && ak.x[0] < aj.x[0]) break;
-      }
-      const int tk = ak.type;
-      if (tk < 0) break;
-      const int pj = bjk.sym_index;
-      const swr_bond_t bkj = A.bonds[pj];
-      const double BOA_jk = BO_jk - thb_cut;
-      const double Delta_k = A.bo_dboc[2 * (size_t)k + 1];
-      const double r_jk = bjk.d;
-      const double exp_tor2_jk = exp(-p_tor2 * BOA_jk);
-      const double exp_cot2_jk = exp(-p_cot2 * (BOA_jk - 1.5) * (BOA_jk - 1.5));
-      const double exp_tor3_DjDk = exp(-p_tor3 * (Delta_j + Delta_k));
-      const double exp_tor4_DjDk = exp(p_tor4 * (Delta_j + Delta_k));
-      const double exp_tor34_inv = 1.0 / (1.0 + exp_tor3_DjDk + exp_tor4_DjDk);
-      const double f11_DjDk = (2.0 + exp_tor3_DjDk) * exp_tor34_inv;
-      const double dfn11 = (-p_tor3 * exp_tor3_DjDk +
-                            (p_tor3 * exp_tor3_DjDk - p_tor4 * exp_tor4_DjDk) * (2.0 + exp_tor3_DjDk) * exp_tor34_inv) *
-                           exp_tor34_inv;
-      const double BOpi_jk = A.BOpi[2 * (size_t)pk];
-      double cdbopi_jk = 0.0, cdbo_jk = 0.0, cd_k = 0.0;
-      double fk[3] = {0.0, 0.0, 0.0};
-      for (int ph = b0; ph < b1; ++ph) {
-        if (ph == pk) continue;
-        const double BO_ij = A.BO[ph];
-        if (!(BO_ij > thb_cut)) continue;
-        const swr_bond_t bij = A.bonds[ph];
-        const int i = bij.nbr;
-        const int ti = A.atoms[i].type;
-        if (ti < 0) continue;
-        // the i-j-k angle terms, evaluated at the first k-l bond that makes
-        // a torsion with this j-i bond (most j-i bonds make none)
-        double ijk_di[3], ijk_dj[3], ijk_dk[3];   // of k, j, i
-        double theta_ijk = 0.0, sin_ijk = 0.0, cos_ijk = 0.0, tan_ijk_i = 0.0, exp_tor2_ij = 0.0, exp_cot2_ij = 0.0;
-        bool have_ijk = false;
+    const double BO_jk = A.BO[pk];
+    const swr_bond_t bjk = A.bonds[pk];
+    const int k = bjk.nbr;
+    const int k0 = A.bidx[k], k1 = A.bend[k];
+    const int tk = A.atoms[k].type;
+    const int pj = bjk.sym_index;
+    const swr_bond_t bkj = A.bonds[pj];
+    const double BOA_jk = BO_jk - thb_cut;
+    const double Delta_k = A.bo_dboc[2 * (size_t)k + 1];
+    const double r_jk = bjk.d;
+    const double exp_tor2_jk = exp(-p_tor2 * BOA_jk);
+    const double exp_cot2_jk = exp(-p_cot2 * (BOA_jk - 1.5) * (BOA_jk - 1.5));
+    const double exp_tor3_DjDk = exp(-p_tor3 * (Delta_j + Delta_k));
+    const double exp_tor4_DjDk = exp(p_tor4 * (Delta_j + Delta_k));
+    const double exp_tor34_inv = 1.0 / (1.0 + exp_tor3_DjDk + exp_tor4_DjDk);
+    const double f11_DjDk = (2.0 + exp_tor3_DjDk) * exp_tor34_inv;
+    const double dfn11 = (-p_tor3 * exp_tor3_DjDk +
+                          (p_tor3 * exp_tor3_DjDk - p_tor4 * exp_tor4_DjDk) * (2.0 + exp_tor3_DjDk) * exp_tor34_inv) *
+                         exp_tor34_inv;
+    const double BOpi_jk = A.BOpi[2 * (size_t)pk];
+    double cdbopi_jk = 0.0, cdbo_jk = 0.0, cd_k = 0.0;
+    double fk[3] = {0.0, 0.0, 0.0};
+    PairQueue Q;
+    queue_init(Q, w, queue, k1 - k0);
+    while (true) {
+      queue_fill(Q, w, b1 - b0, k1 - k0, [&](int a, int b) {
+        return to_pass(A, tj, tk, BO_jk, pk, pj, b0 + a, k0 + b, thb_cut);
+      });
+      const int take = min(Q.n, G);
+      if (!__any(take > 0)) break;
+      const bool ev = w.sub < take;
+      int ph = -1 - lane, i = 0;   // (a key no other lane has)
+      double cdbo_ij = 0.0;
+      double fi[3] = {0.0, 0.0, 0.0};
+      if (ev) {
+        const int code = Q.q[w.sub];
+        const int pw = k0 + (code & 255);
+        ph = b0 + (code >> 8);
+        const double BO_ij = A.BO[ph], BO_kl = A.BO[pw];
+        const swr_bond_t bij = A.bonds[ph], bkl = A.bonds[pw];
+        i = bij.nbr;
+        const int l = bkl.nbr;
+        const swr_atom_pack_t ai = A.atoms[i], al = A.atoms[l];
+        const double xi[3] = {ai.x[0], ai.x[1], ai.x[2]};
+        const DevTor &fb = P->tor[((ai.type * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + al.type];
         const double r_ij = bij.d;
         const double BOA_ij = BO_ij - thb_cut;
-        const double xi[3] = {A.atoms[i].x[0], A.atoms[i].x[1], A.atoms[i].x[2]};
-        double cdbo_ij = 0.0;
-        double fi[3] = {0.0, 0.0, 0.0};
-        for (int pw = k0; pw < k1; ++pw) {
-          if (pw == pj) continue;
-          const double BO_kl = A.BO[pw];
-          if (!(BO_kl > thb_cut) || !(BO_ij * BO_jk * BO_kl > thb_cut)) continue;
-          const swr_bond_t bkl = A.bonds[pw];
-          const int l = bkl.nbr;
-          if (i == l) continue;
-          const swr_atom_pack_t al = A.atoms[l];
-          if (al.type < 0) continue;
-          const DevTor &fb = P->tor[((ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + al.type];
-          if (!fb.cnt) continue;
-          if (!have_ijk) {
-            theta_ijk = theta_dcos(bjk, bij, ijk_di, ijk_dj, ijk_dk);
-            sin_ijk = sin(theta_ijk);
-            cos_ijk = cos(theta_ijk);
-            tan_ijk_i = tan_inv(sin_ijk, cos_ijk);
-            exp_tor2_ij = exp(-p_tor2 * BOA_ij);
-            exp_cot2_ij = exp(-p_cot2 * (BOA_ij - 1.5) * (BOA_ij - 1.5));
-            have_ijk = true;
-          }
-          double jkl_di[3], jkl_dj[3], jkl_dk[3];   // of j, k, l
-          const double theta_jkl = theta_dcos(bkj, bkl, jkl_di, jkl_dj, jkl_dk);
-          const double r_kl = bkl.d;
-          const double BOA_kl = BO_kl - thb_cut;
-          double sin_jkl = sin(theta_jkl);
-          const double cos_jkl = cos(theta_jkl);
-          const double tan_jkl_i = tan_inv(sin_jkl, cos_jkl);
-          const double dvec_li[3] = {xi[0] - al.x[0], xi[1] - al.x[1], xi[2] - al.x[2]};
-          const double r_li = sqrt(dvec_li[0] * dvec_li[0] + dvec_li[1] * dvec_li[1] + dvec_li[2] * dvec_li[2]);
-          // Calculate_Omega
-          const double *dij = bij.dvec, *djk = bjk.dvec, *dkl = bkl.dvec;
-          const double d_ij_jk = dij[0] * djk[0] + dij[1] * djk[1] + dij[2] * djk[2];
-          const double d_jk_kl = djk[0] * dkl[0] + djk[1] * dkl[1] + djk[2] * dkl[2];
-          const double d_ij_kl = dij[0] * dkl[0] + dij[1] * dkl[1] + dij[2] * dkl[2];
-          const double cr[3] = {djk[1] * dkl[2] - djk[2] * dkl[1], djk[2] * dkl[0] - djk[0] * dkl[2],
-                                djk[0] * dkl[1] - djk[1] * dkl[0]};
-          const double uc = -d_ij_jk * d_jk_kl + r_jk * r_jk * d_ij_kl;
-          const double us = -r_jk * (dij[0] * cr[0] + dij[1] * cr[1] + dij[2] * cr[2]);
-          const double omega = atan2(us, uc);
-          const double htra = r_ij + cos_ijk * (r_kl * cos_jkl - r_jk);
-          const double htrb = r_jk - r_ij * cos_ijk - r_kl * cos_jkl;
-          const double htrc = r_kl + cos_jkl * (r_ij * cos_ijk - r_jk);
-          const double hthd = r_ij * sin_ijk * (r_jk - r_kl * cos_jkl);
-          const double hthe = r_kl * sin_jkl * (r_jk - r_ij * cos_ijk);
-          const double hnra = r_kl * sin_ijk * sin_jkl;
-          const double hnrc = r_ij * sin_ijk * sin_jkl;
-          const double hnhd = r_ij * r_kl * cos_ijk * sin_jkl;
-          const double hnhe = r_ij * r_kl * sin_ijk * cos_jkl;
-          double poem = 2.0 * r_ij * r_kl * sin_ijk * sin_jkl;
-          if (poem < 1e-20) poem = 1e-20;
-          const double tel = r_ij * r_ij + r_jk * r_jk + r_kl * r_kl - r_li * r_li -
-                             2.0 * (r_ij * r_jk * cos_ijk - r_ij * r_kl * cos_ijk * cos_jkl + r_jk * r_kl * cos_jkl);
-          double arg = tel / poem;
-          if (arg > 1.0) arg = 1.0;
-          if (arg < -1.0) arg = -1.0;
-          double s_ijk = sin_ijk, s_jkl = sin_jkl;   // clamped copies for the divisions
-          if (s_ijk >= 0 && s_ijk <= MIN_SINE) s_ijk = MIN_SINE;
-          else if (s_ijk <= 0 && s_ijk >= -MIN_SINE) s_ijk = -MIN_SINE;
-          if (s_jkl >= 0 && s_jkl <= MIN_SINE) s_jkl = MIN_SINE;
-          else if (s_jkl <= 0 && s_jkl >= -MIN_SINE) s_jkl = -MIN_SINE;
-          const double sc = 2.0 / poem;
-          const double a_ij = (htra - arg * hnra) / r_ij, a_kl = (htrc - arg * hnrc) / r_kl, a_jk = htrb / r_jk;
-          const double t_d = (hthd - arg * hnhd) / s_ijk, t_e = (hthe - arg * hnhe) / s_jkl;
-          // torsion and conjugation energies
-          const double cos_omega = cos(omega), cos2omega = cos(2. * omega), cos3omega = cos(3. * omega);
-          const double exp_tor1 = exp(fb.p_tor1 * (2.0 - BOpi_jk - f11_DjDk) * (2.0 - BOpi_jk - f11_DjDk));
-          const double exp_tor2_kl = exp(-p_tor2 * BOA_kl);
-          const double exp_cot2_kl = exp(-p_cot2 * (BOA_kl - 1.5) * (BOA_kl - 1.5));
-          const double fn10 = (1.0 - exp_tor2_ij) * (1.0 - exp_tor2_jk) * (1.0 - exp_tor2_kl);
-          const double CV = 0.5 * (fb.V1 * (1.0 + cos_omega) + fb.V2 * exp_tor1 * (1.0 - cos2omega) +
-                                   fb.V3 * (1.0 + cos3omega));
-          e_tor += fn10 * sin_ijk * sin_jkl * CV;
-          const double CEtors1 = sin_ijk * sin_jkl * CV;
-          const double CEtors2 = -fn10 * 2.0 * fb.p_tor1 * fb.V2 * exp_tor1 * (2.0 - BOpi_jk - f11_DjDk) *
-                                 (1.0 - cos_omega * cos_omega) * sin_ijk * sin_jkl;
-          const double CEtors3 = CEtors2 * dfn11;
-          const double CEtors4 = CEtors1 * p_tor2 * exp_tor2_ij * (1.0 - exp_tor2_jk) * (1.0 - exp_tor2_kl);
-          const double CEtors5 = CEtors1 * p_tor2 * (1.0 - exp_tor2_ij) * exp_tor2_jk * (1.0 - exp_tor2_kl);
-          const double CEtors6 = CEtors1 * p_tor2 * (1.0 - exp_tor2_ij) * (1.0 - exp_tor2_jk) * exp_tor2_kl;
-          const double cmn = -fn10 * CV;
-          const double CEtors7 = cmn * sin_jkl * tan_ijk_i;
-          const double CEtors8 = cmn * sin_ijk * tan_jkl_i;
-          const double CEtors9 = fn10 * sin_ijk * sin_jkl *
-                                 (0.5 * fb.V1 - 2.0 * fb.V2 * exp_tor1 * cos_omega +
-                                  1.5 * fb.V3 * (cos2omega + 2.0 * cos_omega * cos_omega));
-          const double fn12 = exp_cot2_ij * exp_cot2_jk * exp_cot2_kl;
-          const double conj = 1.0 + (cos_omega * cos_omega - 1.0) * sin_ijk * sin_jkl;
-          e_con += fb.p_cot1 * fn12 * conj;
-          const double Cconj = -2.0 * fn12 * fb.p_cot1 * p_cot2 * conj;
-          const double CEconj4 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_jkl * tan_ijk_i;
-          const double CEconj5 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_ijk * tan_jkl_i;
-          const double CEconj6 = 2.0 * fb.p_cot1 * fn12 * cos_omega * sin_ijk * sin_jkl;
-          cdbopi_jk += CEtors2;
-          fj[3] += CEtors3;
-          cd_k += CEtors3;
-          cdbo_ij += CEtors4 + Cconj * (BOA_ij - 1.5e0);
-          cdbo_jk += CEtors5 + Cconj * (BOA_jk - 1.5e0);
-          const double cdbo_kl = CEtors6 + Cconj * (BOA_kl - 1.5e0);
-          const double c7 = CEtors7 + CEconj4, c8 = CEtors8 + CEconj5, c9 = CEtors9 + CEconj6;
-          double fl[3];
+        double ijk_di[3], ijk_dj[3], ijk_dk[3];   // of k, j, i
+        const double theta_ijk = theta_dcos(bjk, bij, ijk_di, ijk_dj, ijk_dk);
+        const double sin_ijk = sin(theta_ijk);
+        const double cos_ijk = cos(theta_ijk);
+        const double tan_ijk_i = tan_inv(sin_ijk, cos_ijk);
+        const double exp_tor2_ij = exp(-p_tor2 * BOA_ij);
+        const double exp_cot2_ij = exp(-p_cot2 * (BOA_ij - 1.5) * (BOA_ij - 1.5));
+        double jkl_di[3], jkl_dj[3], jkl_dk[3];   // of j, k, l
+        const double theta_jkl = theta_dcos(bkj, bkl, jkl_di, jkl_dj, jkl_dk);
+        const double r_kl = bkl.d;
+        const double BOA_kl = BO_kl - thb_cut;
+        double sin_jkl = sin(theta_jkl);
+        const double cos_jkl = cos(theta_jkl);
+        const double tan_jkl_i = tan_inv(sin_jkl, cos_jkl);
+        const double dvec_li[3] = {xi[0] - al.x[0], xi[1] - al.x[1], xi[2] - al.x[2]};
+        const double r_li = sqrt(dvec_li[0] * dvec_li[0] + dvec_li[1] * dvec_li[1] + dvec_li[2] * dvec_li[2]);
+        // Calculate_Omega
+        const double *dij = bij.dvec, *djk = bjk.dvec, *dkl = bkl.dvec;
+        const double d_ij_jk = dij[0] * djk[0] + dij[1] * djk[1] + dij[2] * djk[2];
+        const double d_jk_kl = djk[0] * dkl[0] + djk[1] * dkl[1] + djk[2] * dkl[2];
+        const double d_ij_kl = dij[0] * dkl[0] + dij[1] * dkl[1] + dij[2] * dkl[2];
+        const double cr[3] = {djk[1] * dkl[2] - djk[2] * dkl[1], djk[2] * dkl[0] - djk[0] * dkl[2],
+                              djk[0] * dkl[1] - djk[1] * dkl[0]};
+        const double uc = -d_ij_jk * d_jk_kl + r_jk * r_jk * d_ij_kl;
+        const double us = -r_jk * (dij[0] * cr[0] + dij[1] * cr[1] + dij[2] * cr[2]);
+        const double omega = atan2(us, uc);
+        const double htra = r_ij + cos_ijk * (r_kl * cos_jkl - r_jk);
+        const double htrb = r_jk - r_ij * cos_ijk - r_kl * cos_jkl;
+        const double htrc = r_kl + cos_jkl * (r_ij * cos_ijk - r_jk);
+        const double hthd = r_ij * sin_ijk * (r_jk - r_kl * cos_jkl);
+        const double hthe = r_kl * sin_jkl * (r_jk - r_ij * cos_ijk);
+        const double hnra = r_kl * sin_ijk * sin_jkl;
+        const double hnrc = r_ij * sin_ijk * sin_jkl;
+        const double hnhd = r_ij * r_kl * cos_ijk * sin_jkl;
+        const double hnhe = r_ij * r_kl * sin_ijk * cos_jkl;
+        double poem = 2.0 * r_ij * r_kl * sin_ijk * sin_jkl;
+        if (poem < 1e-20) poem = 1e-20;
+        const double tel = r_ij * r_ij + r_jk * r_jk + r_kl * r_kl - r_li * r_li -
+                           2.0 * (r_ij * r_jk * cos_ijk - r_ij * r_kl * cos_ijk * cos_jkl + r_jk * r_kl * cos_jkl);
+        double arg = tel / poem;
+        if (arg > 1.0) arg = 1.0;
+        if (arg < -1.0) arg = -1.0;
+        double s_ijk = sin_ijk, s_jkl = sin_jkl;   // clamped copies for the divisions
+        if (s_ijk >= 0 && s_ijk <= MIN_SINE) s_ijk = MIN_SINE;
+        else if (s_ijk <= 0 && s_ijk >= -MIN_SINE) s_ijk = -MIN_SINE;
+        if (s_jkl >= 0 && s_jkl <= MIN_SINE) s_jkl = MIN_SINE;
+        else if (s_jkl <= 0 && s_jkl >= -MIN_SINE) s_jkl = -MIN_SINE;
+        const double sc = 2.0 / poem;
+        const double a_ij = (htra - arg * hnra) / r_ij, a_kl = (htrc - arg * hnrc) / r_kl, a_jk = htrb / r_jk;
+        const double t_d = (hthd - arg * hnhd) / s_ijk, t_e = (hthe - arg * hnhe) / s_jkl;
+        // torsion and conjugation energies
+        const double cos_omega = cos(omega), cos2omega = cos(2. * omega), cos3omega = cos(3. * omega);
+        const double exp_tor1 = exp(fb.p_tor1 * (2.0 - BOpi_jk - f11_DjDk) * (2.0 - BOpi_jk - f11_DjDk));
+        const double exp_tor2_kl = exp(-p_tor2 * BOA_kl);
+        const double exp_cot2_kl = exp(-p_cot2 * (BOA_kl - 1.5) * (BOA_kl - 1.5));
+        const double fn10 = (1.0 - exp_tor2_ij) * (1.0 - exp_tor2_jk) * (1.0 - exp_tor2_kl);
+        const double CV = 0.5 * (fb.V1 * (1.0 + cos_omega) + fb.V2 * exp_tor1 * (1.0 - cos2omega) +
+                                 fb.V3 * (1.0 + cos3omega));
+        e_tor += fn10 * sin_ijk * sin_jkl * CV;
+        const double CEtors1 = sin_ijk * sin_jkl * CV;
+        const double CEtors2 = -fn10 * 2.0 * fb.p_tor1 * fb.V2 * exp_tor1 * (2.0 - BOpi_jk - f11_DjDk) *
+                               (1.0 - cos_omega * cos_omega) * sin_ijk * sin_jkl;
+        const double CEtors3 = CEtors2 * dfn11;
+        const double CEtors4 = CEtors1 * p_tor2 * exp_tor2_ij * (1.0 - exp_tor2_jk) * (1.0 - exp_tor2_kl);
+        const double CEtors5 = CEtors1 * p_tor2 * (1.0 - exp_tor2_ij) * exp_tor2_jk * (1.0 - exp_tor2_kl);
+        const double CEtors6 = CEtors1 * p_tor2 * (1.0 - exp_tor2_ij) * (1.0 - exp_tor2_jk) * exp_tor2_kl;
+        const double cmn = -fn10 * CV;
+        const double CEtors7 = cmn * sin_jkl * tan_ijk_i;
+        const double CEtors8 = cmn * sin_ijk * tan_jkl_i;
+        const double CEtors9 = fn10 * sin_ijk * sin_jkl *
+                               (0.5 * fb.V1 - 2.0 * fb.V2 * exp_tor1 * cos_omega +
+                                1.5 * fb.V3 * (cos2omega + 2.0 * cos_omega * cos_omega));
+        const double fn12 = exp_cot2_ij * exp_cot2_jk * exp_cot2_kl;
+        const double conj = 1.0 + (cos_omega * cos_omega - 1.0) * sin_ijk * sin_jkl;
+        e_con += fb.p_cot1 * fn12 * conj;
+        const double Cconj = -2.0 * fn12 * fb.p_cot1 * p_cot2 * conj;
+        const double CEconj4 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_jkl * tan_ijk_i;
+        const double CEconj5 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_ijk * tan_jkl_i;
+        const double CEconj6 = 2.0 * fb.p_cot1 * fn12 * cos_omega * sin_ijk * sin_jkl;
+        cdbopi_jk += CEtors2;
+        fj[3] += CEtors3;
+        cd_k += CEtors3;
+        cdbo_ij = CEtors4 + Cconj * (BOA_ij - 1.5e0);
+        cdbo_jk += CEtors5 + Cconj * (BOA_jk - 1.5e0);
+        const double cdbo_kl = CEtors6 + Cconj * (BOA_kl - 1.5e0);
+        const double c7 = CEtors7 + CEconj4, c8 = CEtors8 + CEconj5, c9 = CEtors9 + CEconj6;
+        double fl[3];
 #pragma unroll
-          for (int q = 0; q < 3; q++) {
-            const double w_i = sc * (a_ij * dij[q] - dvec_li[q] - t_d * ijk_dk[q]);
-            const double w_j = sc * (-a_ij * dij[q] - a_jk * djk[q] - t_d * ijk_dj[q] - t_e * jkl_di[q]);
-            const double w_k = sc * (-a_kl * dkl[q] + a_jk * djk[q] - t_d * ijk_di[q] - t_e * jkl_dj[q]);
-            const double w_l = sc * (a_kl * dkl[q] + dvec_li[q] - t_e * jkl_dk[q]);
-            fi[q] += c7 * ijk_dk[q] + c9 * w_i;
-            fj[q] += c7 * ijk_dj[q] + c8 * jkl_di[q] + c9 * w_j;
-            fk[q] += c7 * ijk_di[q] + c8 * jkl_dj[q] + c9 * w_k;
-            fl[q] = c8 * jkl_dk[q] + c9 * w_l;
-          }
-          unsigned long long *al4 = A.acc + 4 * (size_t)l;
-          unsigned long long *const ga[4] = {A.sacc + pw, al4, al4 + 1, al4 + 2};
-          const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
-          const double gv[4] = {cdbo_kl, fl[0], fl[1], fl[2]};
-          fix_add_group<4>(A.flags, ga, gc, gv);
+        for (int q = 0; q < 3; q++) {
+          const double w_i = sc * (a_ij * dij[q] - dvec_li[q] - t_d * ijk_dk[q]);
+          const double w_j = sc * (-a_ij * dij[q] - a_jk * djk[q] - t_d * ijk_dj[q] - t_e * jkl_di[q]);
+          const double w_k = sc * (-a_kl * dkl[q] + a_jk * djk[q] - t_d * ijk_di[q] - t_e * jkl_dj[q]);
+          const double w_l = sc * (a_kl * dkl[q] + dvec_li[q] - t_e * jkl_dk[q]);
+          fi[q] = c7 * ijk_dk[q] + c9 * w_i;
+          fj[q] += c7 * ijk_dj[q] + c8 * jkl_di[q] + c9 * w_j;
+          fk[q] += c7 * ijk_di[q] + c8 * jkl_dj[q] + c9 * w_k;
+          fl[q] = c8 * jkl_dk[q] + c9 * w_l;
         }
-        if (cdbo_ij != 0.0 || fi[0] != 0.0 || fi[1] != 0.0 || fi[2] != 0.0) {
-          unsigned long long *ai4 = A.acc + 4 * (size_t)i;
-          unsigned long long *const ga[4] = {A.sacc + ph, ai4, ai4 + 1, ai4 + 2};
-          const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
-          const double gv[4] = {cdbo_ij, fi[0], fi[1], fi[2]};
-          fix_add_group<4>(A.flags, ga, gc, gv);
+        unsigned long long *al4 = A.acc + 4 * (size_t)l;
+        unsigned long long *const ga[4] = {A.sacc + pw, al4, al4 + 1, al4 + 2};
+        const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
+        const double gv[4] = {cdbo_kl, fl[0], fl[1], fl[2]};
+        fix_add_group<4>(A.flags, ga, gc, gv);
+      }
+      // i's terms: each j-i bond's quadruples are neighbouring lanes; their
+      // sum ends on the first of them
+      const int before = __shfl_up(ph, 1, SWR_WAVE);
+      for (int o = 1; o < G; o <<= 1) {
+        const bool same = __shfl_down(ph, o, SWR_WAVE) == ph && w.sub + o < G;
+        const double v0 = __shfl_down(cdbo_ij, o, SWR_WAVE), v1 = __shfl_down(fi[0], o, SWR_WAVE);
+        const double v2 = __shfl_down(fi[1], o, SWR_WAVE), v3 = __shfl_down(fi[2], o, SWR_WAVE);
+        if (same) {
+          cdbo_ij += v0;
+          fi[0] += v1;
+          fi[1] += v2;
+          fi[2] += v3;
         }
       }
+      if (ev && (w.sub == 0 || before != ph) &&
+          (cdbo_ij != 0.0 || fi[0] != 0.0 || fi[1] != 0.0 || fi[2] != 0.0)) {
+        unsigned long long *ai4 = A.acc + 4 * (size_t)i;
+        unsigned long long *const ga[4] = {A.sacc + ph, ai4, ai4 + 1, ai4 + 2};
+        const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
+        const double gv[4] = {cdbo_ij, fi[0], fi[1], fi[2]};
+        fix_add_group<4>(A.flags, ga, gc, gv);
+      }
+      queue_drop(Q, w, take);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) fj[q] = group_sum(fj[q], G);
+#pragma unroll
+    for (int q = 0; q < 3; q++) fk[q] = group_sum(fk[q], G);
+    cd_k = group_sum(cd_k, G);
+    cdbopi_jk = group_sum(cdbopi_jk, G);
+    cdbo_jk = group_sum(cdbo_jk, G);
+    e_tor = group_sum(e_tor, G);
+    e_con = group_sum(e_con, G);
+    if (w.live && w.sub == 0) {
       if (cdbopi_jk != 0.0) A.Cdbopi[pk] += cdbopi_jk;
       if (cdbo_jk != 0.0) A.Cdbo[pk] += cdbo_jk;
       if (cd_k != 0.0 || fk[0] != 0.0 || fk[1] != 0.0 || fk[2] != 0.0) {
@@ -1282,13 +1472,13 @@ __global__ void __launch_bounds__(BT) k_torsion(ToArgs A) {
         const double gv[4] = {fk[0], fk[1], fk[2], cd_k};
         fix_add_group<4>(A.flags, ga, gc, gv);
       }
-    } while (false);
-  }
-  double *rw = A.row + 6 * (size_t)pk;
+      double *rw = A.row + 6 * (size_t)pk;
 #pragma unroll
-  for (int q = 0; q < 4; q++) rw[q] = fj[q];
-  rw[4] = e_tor;
-  rw[5] = e_con;
+      for (int q = 0; q < 4; q++) rw[q] = fj[q];
+      rw[4] = e_tor;
+      rw[5] = e_con;
+    }
+  }
 }
 
 // j's row and torsion/conjugation energies: its slots' entries in slot order.
@@ -1494,7 +1684,7 @@ int swr_valence_angles_run(swr_system *S) {
     hipLaunchKernelGGL(k_va_count, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_wl_scan, dim3(1), dim3(WL_NB), 0, S->stream, S->va_ctl);
     hipLaunchKernelGGL(k_va_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
-    hipLaunchKernelGGL(k_valence, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, A);
+    hipLaunchKernelGGL(k_valence, dim3(std::min(WL_MAX_WAVES, n)), dim3(SWR_WAVE), 0, S->stream, A);
   }
   hipLaunchKernelGGL(k_va_fold, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, S->va_acc, S->fcd);
   hipLaunchKernelGGL(k_sum_rows, dim3(3), dim3(1024), 0, S->stream, n, (const double *)S->va_part, stride,
@@ -1560,8 +1750,8 @@ int swr_torsion_angles_run(swr_system *S) {
     hipLaunchKernelGGL(k_to_count, dim3(div_up(n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_wl_scan, dim3(1), dim3(WL_NB), 0, S->stream, S->to_ctl);
     hipLaunchKernelGGL(k_to_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
-    // (at most one task per bond slot; lanes past the list's length exit)
-    hipLaunchKernelGGL(k_torsion, dim3(div_up(nslots, BT)), dim3(BT), 0, S->stream, A);
+    const int waves = (int)std::min<long long>(WL_MAX_WAVES, 8LL * n);
+    hipLaunchKernelGGL(k_torsion, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
     hipLaunchKernelGGL(k_to_row, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
   }
   hipLaunchKernelGGL(k_va_fold, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, S->to_acc, S->fcd);
