@@ -673,21 +673,25 @@ __device__ __forceinline__ bool wl_wave(const int *__restrict__ ctl, int unit, i
   return false;
 }
 
-// Sum over the aligned group of G lanes (a power of two), on every lane.
-__device__ __forceinline__ double group_sum(double v, int G) {
-  for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o, SWR_WAVE);
-  return v;
-}
-__device__ __forceinline__ double group_product(double v, int G) {
-  for (int o = 1; o < G; o <<= 1) v *= __shfl_xor(v, o, SWR_WAVE);
-  return v;
-}
-
 // Orders a wave's own LDS accesses (each wave has its own slice).
 __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Running totals of each group, NC components: after a round every lane of the
+// group adds its share of the components over the round's evaluations in their
+// order, so a total is the sum one thread would have made in a loop over them
+// (the trajectory of a run depends on these sums to the last bit, and the
+// solve of the charges turns a last bit into 1e-8).
+template <int NC>
+struct GroupTotals {
+  double t[NC][SWR_WAVE];   // [component][the group's first lane]
+};
+template <int NC>
+__device__ __forceinline__ void totals_init(GroupTotals<NC> &T, const WlWave &w) {
+  for (int c = w.sub; c < NC; c += w.G) T.t[c][lane_id() - w.sub] = 0.0;
 }
 
 // Each group's pending evaluations: (a, b) positions in two bond ranges as
@@ -847,14 +851,17 @@ __device__ __forceinline__ int wl_gmin(int ntask) { return ntask <= 4096 ? 16 : 
 // group's lanes test j's bond pairs and each evaluates one passing pair a
 // round.  What bounds the pass is the latency of one pair's transcendentals
 // (at 1-2 waves a SIMD), so a centre's pairs side by side instead of in turn
-// take the longest centre off the critical path.  Per round the pairs' Cdbo
-// terms go to LDS and the lane that owns a slot adds them in pair order; the
-// centre's sums are group butterflies, so every order is fixed.  One thread
+// take the longest centre off the critical path.  Per round the pairs' terms
+// go to LDS and each slot and total is summed by one lane in pair order.  One thread
 // per centre took 52 us on a 64-water box and 150 us on the 32,000-water one;
-// this takes 18 and 108 (512 clusters: 1.05 ms either way, all lanes busy).
+// this takes 17 and 115 (512 clusters: 1.05 and 1.11 ms, all lanes busy).
 __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
   __shared__ unsigned short queue[2 * SWR_WAVE];
-  __shared__ double spk[SWR_WAVE], sph[SWR_WAVE];
+  // the round's pairs: Cdbo terms, and per parameter set the centre's terms
+  enum { V_ANG = 0, V_PEN, V_COA, V_CE5, V_CE6, V_CDJ, V_G0, V_G1, V_G2, V_NC };
+  __shared__ double spk[SWR_WAVE], sph[SWR_WAVE], term[V_NC][SWR_MAX_THB][SWR_WAVE];
+  __shared__ int sset[SWR_WAVE];
+  __shared__ GroupTotals<V_NC> T;
   const int lane = lane_id();
   const int gmin = wl_gmin(A.ctl[WL_NTASK]);
   WlWave w;
@@ -865,21 +872,27 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
     const int tj = w.live ? A.atoms[j].type : 0;
     const int b0 = w.live ? A.bidx[j] : 0, b1 = w.live ? A.bend[j] : 0;
     const int m = b1 - b0;
-    double e_ang = 0.0, e_pen = 0.0, e_coa = 0.0;
+    totals_init(T, w);
     const double thb_cut = P->thb_cut, thb_cutsq = P->thb_cutsq;
     const double Dboc_j = A.bo_dboc[2 * (size_t)j + 1];
     const double p_val3 = P->p_val3[tj], p_val5 = P->p_val5[tj];
     const double p_val6 = P->p_val6, p_val8 = P->p_val8, p_val9 = P->p_val9, p_val10 = P->p_val10;
+    // SBO: the group's lanes take a bond each for the exponentials
     double SBOp = 0.0, prod_SBO = 1.0;
-    for (int t = b0 + w.sub; t < b1; t += G) {
-      SBOp += A.BOpi[2 * (size_t)t] + A.BOpi[2 * (size_t)t + 1];
-      double b2 = A.BO[t] * A.BO[t];
+    for (int t0 = b0; __any(t0 < b1); t0 += G) {
+      const int t = t0 + w.sub;
+      double b2 = t < b1 ? A.BO[t] * A.BO[t] : 0.0;
       b2 *= b2;
       b2 *= b2;
-      prod_SBO *= exp(-b2);
+      spk[lane] = t < b1 ? A.BOpi[2 * (size_t)t] + A.BOpi[2 * (size_t)t + 1] : 0.0;
+      sph[lane] = exp(-b2);
+      wave_lds_order();
+      for (int e = 0; e < G && t0 + e < b1; ++e) {
+        SBOp += spk[g0 + e];
+        prod_SBO *= sph[g0 + e];
+      }
+      wave_lds_order();
     }
-    SBOp = group_sum(SBOp, G);
-    prod_SBO = group_product(prod_SBO, G);
     double vlpadj, dSBO2;
     if (A.vlpex[j] >= 0) {
       vlpadj = 0.0;
@@ -909,7 +922,6 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
     const double Cf9j = (-P->p_pen3 * exp_pen3 * trm_pen34 - (2.0 + exp_pen3) * (-P->p_pen3 * exp_pen3 + P->p_pen4 * exp_pen4)) /
                         (trm_pen34 * trm_pen34);
     const double exp_coa2 = exp(P->p_coa2 * A.Delta_val[j]);
-    double ce5 = 0.0, ce6 = 0.0, cdj = 0.0, g0s = 0.0, g1s = 0.0, g2s = 0.0;
     PairQueue Q;
     queue_init(Q, w, queue, m);
     while (true) {
@@ -926,6 +938,7 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
       if (!__any(take > 0)) break;
       const bool ev = w.sub < take;
       double cdbo_jk = 0.0, cdbo_hj = 0.0;
+      int nset = 0;
       if (ev) {
         const int code = Q.q[w.sub];
         const int pk = b0 + (code >> 8), ph = b0 + (code & 255);
@@ -935,7 +948,7 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
         const int tk = A.atoms[k].type, th = A.atoms[h].type;
         const double BOA_jk = BO_jk - thb_cut, BOA_hj = BO_hj - thb_cut;
         const int tri = (tk * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + th;
-        const int nset = P->thb_n[tri];
+        nset = P->thb_n[tri];
         // Calculate_Theta / Calculate_dCos_Theta (:1510-1547) with the j-k
         // bond first: di belongs to k, dk to h
         const double dot = bjk.dvec[0] * bhj.dvec[0] + bjk.dvec[1] * bhj.dvec[1] + bjk.dvec[2] * bhj.dvec[2];
@@ -987,16 +1000,16 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
           const double Ctheta_0 = p_val10 * (q.theta_00 * DEG2RAD_PI / 180.0) * exp10;
           const double CEval5 = -CEval4 * Ctheta_0 * CSBO2;
           const double CEval8 = -CEval4 / sin_t;
-          e_ang += f7_jk * f7_hj * f8_Dj * expval12theta;
+          term[V_ANG][c][lane] = f7_jk * f7_hj * f8_Dj * expval12theta;
           // penalty
           const double ep = q.p_pen1 * f9_Dj * pen2;
-          e_pen += ep;
+          term[V_PEN][c][lane] = ep;
           const double CEpen1 = ep * Cf9j / f9_Dj;
           const double tp = -2.0 * P->p_pen2 * ep;
           const double CEpen2 = tp * (BOA_jk - 2.0), CEpen3 = tp * (BOA_hj - 2.0);
           // coalition
           const double ec = q.p_coa1 * coa;
-          e_coa += ec;
+          term[V_COA][c][lane] = ec;
           const double CEcoa1 = -2 * P->p_coa4 * (BOA_jk - 1.5) * ec;
           const double CEcoa2 = -2 * P->p_coa4 * (BOA_hj - 1.5) * ec;
           const double CEcoa3 = -P->p_coa2 * exp_coa2 * ec / (1 + exp_coa2);
@@ -1004,11 +1017,11 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
           const double CEcoa5 = -2 * P->p_coa3 * (bo_h0 - BOA_hj) * ec;
           cdbo_jk += CEval1 + CEpen2 + (CEcoa1 - CEcoa4);
           cdbo_hj += CEval2 + CEpen3 + (CEcoa2 - CEcoa5);
-          cdj += (CEval3 + CEval5 * dSBO2) + CEpen1 + CEcoa3;
+          term[V_CDJ][c][lane] = (CEval3 + CEval5 * dSBO2) + CEpen1 + CEcoa3;
           ck[3] += CEcoa4;
           chh[3] += CEcoa5;
-          ce5 += CEval5;
-          ce6 += CEval5 * dSBO1;
+          term[V_CE5][c][lane] = CEval5;
+          term[V_CE6][c][lane] = CEval5 * dSBO1;
 #pragma unroll
           for (int d = 0; d < 3; ++d) {
             const double di = bhj.dvec[d] * inv_d - cinv3 * sq_hj * bjk.dvec[d];
@@ -1016,9 +1029,7 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
             const double dk = bjk.dvec[d] * inv_d - cinv3 * sq_jk * bhj.dvec[d];
             ck[d] += CEval8 * di;
             chh[d] += CEval8 * dk;
-            if (d == 0) g0s += CEval8 * dj;
-            if (d == 1) g1s += CEval8 * dj;
-            if (d == 2) g2s += CEval8 * dj;
+            term[V_G0 + d][c][lane] = CEval8 * dj;
           }
         }
         unsigned long long *ak = A.acc + 4 * (size_t)k, *ah = A.acc + 4 * (size_t)h;
@@ -1029,25 +1040,38 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
           fix_add_group<8>(A.flags, ga, gc, gv);
         }
       }
-      // the round's Cdbo terms onto j's slots, in pair order by each slot's lane
+      // the round's Cdbo terms onto j's slots, and its other terms onto the
+      // centre's totals: each by one lane, in pair (and set) order
       spk[lane] = cdbo_jk;
       sph[lane] = cdbo_hj;
+      sset[lane] = nset;
       wave_lds_order();
       for (int t0 = 0; t0 < m; t0 += G) {
         const int t = t0 + w.sub;
-        double add = 0.0;
+        double v = 0.0;
+        bool touched = false;
         for (int e = 0; e < take; ++e) {
           const int code = Q.q[e];
-          if ((code >> 8) == t) add += spk[g0 + e];
-          if ((code & 255) == t) add += sph[g0 + e];
+          const bool k = (code >> 8) == t;
+          if (k || (code & 255) == t) {
+            if (!touched) v = A.Cdbo[b0 + t];
+            touched = true;
+            v += k ? spk[g0 + e] : sph[g0 + e];
+          }
         }
-        if (add != 0.0) A.Cdbo[b0 + t] += add;
+        if (touched) A.Cdbo[b0 + t] = v;
+      }
+      for (int c = w.sub; c < V_NC; c += G) {
+        double v = T.t[c][g0];
+        for (int e = 0; e < take; ++e)
+          for (int q = 0; q < sset[g0 + e]; ++q) v += term[c][q][g0 + e];
+        T.t[c][g0] = v;
       }
       wave_lds_order();
       queue_drop(Q, w, take);
     }
-    ce5 = group_sum(ce5, G);
-    ce6 = group_sum(ce6, G);
+    wave_lds_order();
+    const double ce5 = T.t[V_CE5][g0], ce6 = T.t[V_CE6][g0];
     if (ce5 != 0.0 || ce6 != 0.0)
       for (int t = b0 + w.sub; t < b1; t += G) {
         const double bo = A.BO[t];
@@ -1056,22 +1080,15 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
         A.Cdbopi[t] += ce5;
         A.Cdbopi2[t] += ce5;
       }
-    cdj = group_sum(cdj, G);
-    g0s = group_sum(g0s, G);
-    g1s = group_sum(g1s, G);
-    g2s = group_sum(g2s, G);
-    e_ang = group_sum(e_ang, G);
-    e_pen = group_sum(e_pen, G);
-    e_coa = group_sum(e_coa, G);
     if (w.live && w.sub == 0) {
-      A.fcd[4 * (size_t)j] += g0s;
-      A.fcd[4 * (size_t)j + 1] += g1s;
-      A.fcd[4 * (size_t)j + 2] += g2s;
-      A.fcd[4 * (size_t)j + 3] += cdj;
-      A.part[j] = e_ang;
-      A.part[A.stride + j] = e_pen;
-      A.part[2 * A.stride + j] = e_coa;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) A.fcd[4 * (size_t)j + d] += T.t[V_G0 + d][g0];
+      A.fcd[4 * (size_t)j + 3] += T.t[V_CDJ][g0];
+      A.part[j] = T.t[V_ANG][g0];
+      A.part[A.stride + j] = T.t[V_PEN][g0];
+      A.part[2 * A.stride + j] = T.t[V_COA][g0];
     }
+    wave_lds_order();   // (before the next groups' totals start)
   }
 }
 
@@ -1256,13 +1273,18 @@ __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
 // quadruple a round.  A quadruple is ~2000 dependent FP64 instructions at one
 // wave per SIMD, so what bounded the pass was the longest bond's chain of
 // quadruples.  i's terms are summed over the round's quadruples of one j-i
-// bond (a segmented scan: they are neighbours in the queue) before their
-// fixed-point add, and j's, k's and the bond's over the group, so the large
+// bond (they are neighbours in the queue) before their fixed-point add, and
+// j's, k's and the bond's over all, each by one lane in order, so the large
 // cotangent terms of a nearly linear angle cancel in FP64 first.  One lane
 // per bond took 87 us on a 64-water box, 133 us on the 32,000-water one and
-// 2.38 ms on 512 clusters; this takes 19, 65 us and 1.34 ms.
+// 2.38 ms on 512 clusters; this takes 16, 66 us and 1.31 ms.
 __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
+  // the round's quadruples: the bond's and i's terms
+  enum { O_FJ = 0, O_FK = 4, O_CDK = 7, O_PI, O_BO, O_TOR, O_CON, O_NC };
   __shared__ unsigned short queue[2 * SWR_WAVE];
+  __shared__ double term[O_NC][SWR_WAVE], iterm[4][SWR_WAVE];
+  __shared__ int sph[SWR_WAVE];
+  __shared__ GroupTotals<O_NC> T;
   constexpr double MIN_SINE = 1e-10;
   const int lane = lane_id();
   const int gmin = wl_gmin(A.ctl[WL_NTASK]);
@@ -1270,9 +1292,8 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
   WlWave w;
   for (int unit = blockIdx.x; wl_wave(A.ctl, unit, gmin, w); unit += gridDim.x) {
     const int2 jp = w.live ? A.task[w.t] : A.task[0];
-    const int j = jp.x, pk = jp.y, G = w.G;
-    double e_tor = 0.0, e_con = 0.0;
-    double fj[4] = {0.0, 0.0, 0.0, 0.0};
+    const int j = jp.x, pk = jp.y, G = w.G, g0 = lane - w.sub;
+    totals_init(T, w);
     const int tj = A.atoms[j].type;
     const int b0 = A.bidx[j], b1 = A.bend[j];
     const double thb_cut = P->thb_cut;
@@ -1298,8 +1319,6 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
                           (p_tor3 * exp_tor3_DjDk - p_tor4 * exp_tor4_DjDk) * (2.0 + exp_tor3_DjDk) * exp_tor34_inv) *
                          exp_tor34_inv;
     const double BOpi_jk = A.BOpi[2 * (size_t)pk];
-    double cdbopi_jk = 0.0, cdbo_jk = 0.0, cd_k = 0.0;
-    double fk[3] = {0.0, 0.0, 0.0};
     PairQueue Q;
     queue_init(Q, w, queue, k1 - k0);
     while (true) {
@@ -1309,9 +1328,7 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
       const int take = min(Q.n, G);
       if (!__any(take > 0)) break;
       const bool ev = w.sub < take;
-      int ph = -1 - lane, i = 0;   // (a key no other lane has)
-      double cdbo_ij = 0.0;
-      double fi[3] = {0.0, 0.0, 0.0};
+      int ph = -1, i = 0;
       if (ev) {
         const int code = Q.q[w.sub];
         const int pw = k0 + (code & 255);
@@ -1383,7 +1400,7 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
         const double fn10 = (1.0 - exp_tor2_ij) * (1.0 - exp_tor2_jk) * (1.0 - exp_tor2_kl);
         const double CV = 0.5 * (fb.V1 * (1.0 + cos_omega) + fb.V2 * exp_tor1 * (1.0 - cos2omega) +
                                  fb.V3 * (1.0 + cos3omega));
-        e_tor += fn10 * sin_ijk * sin_jkl * CV;
+        term[O_TOR][lane] = fn10 * sin_ijk * sin_jkl * CV;
         const double CEtors1 = sin_ijk * sin_jkl * CV;
         const double CEtors2 = -fn10 * 2.0 * fb.p_tor1 * fb.V2 * exp_tor1 * (2.0 - BOpi_jk - f11_DjDk) *
                                (1.0 - cos_omega * cos_omega) * sin_ijk * sin_jkl;
@@ -1399,16 +1416,16 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
                                 1.5 * fb.V3 * (cos2omega + 2.0 * cos_omega * cos_omega));
         const double fn12 = exp_cot2_ij * exp_cot2_jk * exp_cot2_kl;
         const double conj = 1.0 + (cos_omega * cos_omega - 1.0) * sin_ijk * sin_jkl;
-        e_con += fb.p_cot1 * fn12 * conj;
+        term[O_CON][lane] = fb.p_cot1 * fn12 * conj;
         const double Cconj = -2.0 * fn12 * fb.p_cot1 * p_cot2 * conj;
         const double CEconj4 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_jkl * tan_ijk_i;
         const double CEconj5 = -fb.p_cot1 * fn12 * (cos_omega * cos_omega - 1.0) * sin_ijk * tan_jkl_i;
         const double CEconj6 = 2.0 * fb.p_cot1 * fn12 * cos_omega * sin_ijk * sin_jkl;
-        cdbopi_jk += CEtors2;
-        fj[3] += CEtors3;
-        cd_k += CEtors3;
-        cdbo_ij = CEtors4 + Cconj * (BOA_ij - 1.5e0);
-        cdbo_jk += CEtors5 + Cconj * (BOA_jk - 1.5e0);
+        term[O_PI][lane] = CEtors2;
+        term[O_FJ + 3][lane] = CEtors3;
+        term[O_CDK][lane] = CEtors3;
+        iterm[0][lane] = CEtors4 + Cconj * (BOA_ij - 1.5e0);
+        term[O_BO][lane] = CEtors5 + Cconj * (BOA_jk - 1.5e0);
         const double cdbo_kl = CEtors6 + Cconj * (BOA_kl - 1.5e0);
         const double c7 = CEtors7 + CEconj4, c8 = CEtors8 + CEconj5, c9 = CEtors9 + CEconj6;
         double fl[3];
@@ -1418,9 +1435,9 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
           const double w_j = sc * (-a_ij * dij[q] - a_jk * djk[q] - t_d * ijk_dj[q] - t_e * jkl_di[q]);
           const double w_k = sc * (-a_kl * dkl[q] + a_jk * djk[q] - t_d * ijk_di[q] - t_e * jkl_dj[q]);
           const double w_l = sc * (a_kl * dkl[q] + dvec_li[q] - t_e * jkl_dk[q]);
-          fi[q] = c7 * ijk_dk[q] + c9 * w_i;
-          fj[q] += c7 * ijk_dj[q] + c8 * jkl_di[q] + c9 * w_j;
-          fk[q] += c7 * ijk_di[q] + c8 * jkl_dj[q] + c9 * w_k;
+          iterm[1 + q][lane] = c7 * ijk_dk[q] + c9 * w_i;
+          term[O_FJ + q][lane] = c7 * ijk_dj[q] + c8 * jkl_di[q] + c9 * w_j;
+          term[O_FK + q][lane] = c7 * ijk_di[q] + c8 * jkl_dj[q] + c9 * w_k;
           fl[q] = c8 * jkl_dk[q] + c9 * w_l;
         }
         unsigned long long *al4 = A.acc + 4 * (size_t)l;
@@ -1429,55 +1446,50 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
         const double gv[4] = {cdbo_kl, fl[0], fl[1], fl[2]};
         fix_add_group<4>(A.flags, ga, gc, gv);
       }
-      // i's terms: each j-i bond's quadruples are neighbouring lanes; their
-      // sum ends on the first of them
-      const int before = __shfl_up(ph, 1, SWR_WAVE);
-      for (int o = 1; o < G; o <<= 1) {
-        const bool same = __shfl_down(ph, o, SWR_WAVE) == ph && w.sub + o < G;
-        const double v0 = __shfl_down(cdbo_ij, o, SWR_WAVE), v1 = __shfl_down(fi[0], o, SWR_WAVE);
-        const double v2 = __shfl_down(fi[1], o, SWR_WAVE), v3 = __shfl_down(fi[2], o, SWR_WAVE);
-        if (same) {
-          cdbo_ij += v0;
-          fi[0] += v1;
-          fi[1] += v2;
-          fi[2] += v3;
+      sph[lane] = ph;
+      wave_lds_order();
+      // i's terms: each j-i bond's quadruples are neighbouring lanes; the
+      // first of them sums them
+      if (ev && (w.sub == 0 || sph[lane - 1] != ph)) {
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int e = w.sub; e < take && sph[g0 + e] == ph; ++e)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] += iterm[q][g0 + e];
+        if (v[0] != 0.0 || v[1] != 0.0 || v[2] != 0.0 || v[3] != 0.0) {
+          unsigned long long *ai4 = A.acc + 4 * (size_t)i;
+          unsigned long long *const ga[4] = {A.sacc + ph, ai4, ai4 + 1, ai4 + 2};
+          const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
+          fix_add_group<4>(A.flags, ga, gc, v);
         }
       }
-      if (ev && (w.sub == 0 || before != ph) &&
-          (cdbo_ij != 0.0 || fi[0] != 0.0 || fi[1] != 0.0 || fi[2] != 0.0)) {
-        unsigned long long *ai4 = A.acc + 4 * (size_t)i;
-        unsigned long long *const ga[4] = {A.sacc + ph, ai4, ai4 + 1, ai4 + 2};
-        const size_t gc[4] = {A.scoff, A.coff, A.coff, A.coff};
-        const double gv[4] = {cdbo_ij, fi[0], fi[1], fi[2]};
-        fix_add_group<4>(A.flags, ga, gc, gv);
+      // the bond's totals, in quadruple order
+      for (int c = w.sub; c < O_NC; c += G) {
+        double v = T.t[c][g0];
+        for (int e = 0; e < take; ++e) v += term[c][g0 + e];
+        T.t[c][g0] = v;
       }
+      wave_lds_order();
       queue_drop(Q, w, take);
     }
-#pragma unroll
-    for (int q = 0; q < 4; q++) fj[q] = group_sum(fj[q], G);
-#pragma unroll
-    for (int q = 0; q < 3; q++) fk[q] = group_sum(fk[q], G);
-    cd_k = group_sum(cd_k, G);
-    cdbopi_jk = group_sum(cdbopi_jk, G);
-    cdbo_jk = group_sum(cdbo_jk, G);
-    e_tor = group_sum(e_tor, G);
-    e_con = group_sum(e_con, G);
+    wave_lds_order();
     if (w.live && w.sub == 0) {
+      const double cdbopi_jk = T.t[O_PI][g0], cdbo_jk = T.t[O_BO][g0];
       if (cdbopi_jk != 0.0) A.Cdbopi[pk] += cdbopi_jk;
       if (cdbo_jk != 0.0) A.Cdbo[pk] += cdbo_jk;
-      if (cd_k != 0.0 || fk[0] != 0.0 || fk[1] != 0.0 || fk[2] != 0.0) {
+      const double gv[4] = {T.t[O_FK][g0], T.t[O_FK + 1][g0], T.t[O_FK + 2][g0], T.t[O_CDK][g0]};
+      if (gv[0] != 0.0 || gv[1] != 0.0 || gv[2] != 0.0 || gv[3] != 0.0) {
         unsigned long long *ak4 = A.acc + 4 * (size_t)k;
         unsigned long long *const ga[4] = {ak4, ak4 + 1, ak4 + 2, ak4 + 3};
         const size_t gc[4] = {A.coff, A.coff, A.coff, A.coff};
-        const double gv[4] = {fk[0], fk[1], fk[2], cd_k};
         fix_add_group<4>(A.flags, ga, gc, gv);
       }
       double *rw = A.row + 6 * (size_t)pk;
 #pragma unroll
-      for (int q = 0; q < 4; q++) rw[q] = fj[q];
-      rw[4] = e_tor;
-      rw[5] = e_con;
+      for (int q = 0; q < 4; q++) rw[q] = T.t[O_FJ + q][g0];
+      rw[4] = T.t[O_TOR][g0];
+      rw[5] = T.t[O_CON][g0];
     }
+    wave_lds_order();   // (before the next groups' totals start)
   }
 }
 
