@@ -390,7 +390,7 @@ int swr_destroy(swr_system *S) {
   void *ptrs[] = {S->dp, S->x, S->v, S->q, S->type, S->tag, S->owner, S->img, S->mask, S->packed,
                   S->bin_of, S->bin_count, S->bin_start, S->bin_occ, S->rs_keys, S->rs_vals, S->rs_hist, S->bp_pos, S->bp_id, S->stencil_rows,
                   S->voff, S->vcount, S->vlist, S->far, S->far_index, S->far_end, S->num_bonds, S->num_hbonds,
-                  S->Hindex, S->bond_index, S->bond_end, S->bonds, S->bond_nbr, S->bo_data, S->prow, S->pbeg, S->pcnt, S->pcol, S->pkey, S->jloc, S->sys_panel, S->BO, S->BOpi, S->Cdbo,
+                  S->Hindex, S->bond_index, S->bond_end, S->bonds, S->bond_nbr, S->bo_data, S->prow, S->pbeg, S->pcnt, S->pcol, S->pkey, S->jloc, S->sys_panel, S->small_panel, S->BO, S->BOpi, S->Cdbo,
                   S->Cdbopi,
                   S->Cdbopi2, S->hbond_index, S->hbond_end, S->hbonds, S->bo_dboc, S->dDeltap_self, S->bond_mark,
                   S->fcd, S->nb_partials, S->nb_result, S->nb_eatom, S->be_part, S->be_ce, S->be_bufc, S->be_result, S->hb_part,
@@ -645,7 +645,7 @@ int swr_qeq_cg(swr_system *S, int *iters_s, int *iters_t) {
   if (!S || !S->H_val) return SWR_ERR_STATE;
   int its0 = 0;
   for (size_t k = 0; k < S->h_sys_iters.size(); k += 2) its0 = std::max(its0, S->h_sys_iters[k]);
-  int rc = S->mixed ? swr_qeq_mixed_solve(S) : swr_qeq_cg_run(S, its0 + 2);
+  int rc = S->mixed ? swr_qeq_mixed_solve(S) : swr_qeq_cg_run(S, its0);
   if (rc) return rc;
   if (S->mixed) {  // the FP64 solve's last done check already brought status and counts back
     S->h_sys_iters.resize(2 * (size_t)S->nsys);
@@ -869,6 +869,7 @@ bool lookup(swr_system *S, const std::string &k, View &v) {
   if (k == "H_val") return set(S->H_val, 8 * S->Hcap);
   if (k == "H_val32") return set(S->H_val32, S->H_val32 ? 4 * S->Hcap : 0);
   if (k == "Hdia_inv") return set(S->Hdia_inv, 8 * n);
+  if (k == "panel_count" || k == "panel_columns" || k == "H_jloc") (void)swr_panel_lists(S);
   if (k == "panel_rows") return set(S->prow, S->prow ? 4 * (int64_t)S->prow_n : 0);
   if (k == "panel_begin") return set(S->pbeg, S->pbeg ? 4 * ((int64_t)S->npanel + 1) : 0);
   if (k == "panel_count") return set(S->pcnt, S->pcnt ? 4 * (int64_t)S->npanel : 0);

@@ -12,8 +12,10 @@
 // instead of the 4-byte column.  A panel with more than SWR_PANEL_MAXC
 // columns keeps pcnt = -1 and its rows gather from global memory as before.
 //
-// The row order changes only when the bins or the batch partition change
-// (a neighbour-list build or swr_set_batch); the column lists are rebuilt
+// Small systems (qeq_small.h) keep their rows in atom order instead, and their
+// lists are built only when something else asks for them (the no-allocation
+// solve, the autotuner, a download).  The row order changes only when the bins or the batch partition
+// change (a neighbour-list build or swr_set_batch); the column lists are rebuilt
 // with H every step.  Dense indices follow the hash table's slot order,
 // which can differ between runs, but a row's sum runs over its entries in
 // H order whatever the indices are, so the SpMV results do not depend on it.
@@ -55,6 +57,12 @@ __global__ void k_sys_keys(int n, const int *__restrict__ order, const int *__re
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   key[k] = row_sys[order[k]];
+}
+
+// The row order of small systems (qeq_small.h): atom order.
+__global__ void k_atom_order(int n, int *__restrict__ prow) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) prow[i] = i;
 }
 
 __global__ void k_panels_off(int np, int *__restrict__ pcnt) {
@@ -181,7 +189,7 @@ int swr_panel_build(swr_system *S) {
   int rc;
   if ((rc = swr_qeq_layout(S))) return rc;
   if (n <= 0) return SWR_OK;
-  if (S->prow_n != n || S->prow_nbr_gen != S->nbr_gen || S->prow_layout_gen != S->layout_gen) {
+  if (S->prow_n != n || S->prow_layout_gen != S->layout_gen || (!S->cg_small && S->prow_nbr_gen != S->nbr_gen)) {
     if (!S->bin_of) {
       swr_set_error_msg("SpMV panels need the neighbour list's bins (build the neighbour list first)");
       return SWR_ERR_STATE;
@@ -190,9 +198,12 @@ int swr_panel_build(swr_system *S) {
         (rc = swr_reserve(&S->pkey, S->cap_pkey, 2 * (size_t)n)))
       return rc;
     swr_kt_begin(S, KT_PANEL);
-    hipLaunchKernelGGL(k_morton_keys, dim3(div_up(n, 256)), dim3(256), 0, S->stream, n, (const int *)S->bin_of,
-                       S->nbin[0], S->nbin[1], S->pkey);
-    if (S->nsys <= 1) {
+    if (!S->cg_small)
+      hipLaunchKernelGGL(k_morton_keys, dim3(div_up(n, 256)), dim3(256), 0, S->stream, n, (const int *)S->bin_of,
+                         S->nbin[0], S->nbin[1], S->pkey);
+    if (S->cg_small) {
+      hipLaunchKernelGGL(k_atom_order, dim3(div_up(n, 256)), dim3(256), 0, S->stream, n, S->prow);
+    } else if (S->nsys <= 1) {
       if ((rc = swr_radix_sort_i32(S, S->pkey, nullptr, n, 30, S->prow))) return rc;
     } else {
       // Morton order, then stably by system: each system's rows together, in
@@ -216,6 +227,16 @@ int swr_panel_build(swr_system *S) {
     sys_panel[nsys] = (int)pbeg.size();
     pbeg.push_back(n);
     const int np = (int)pbeg.size() - 1;
+    std::vector<int> place;   // SmallPanel of each panel
+    if (S->cg_small) {
+      for (int s = 0; s < nsys; s++)
+        for (int p = sys_panel[s]; p < sys_panel[s + 1]; p++)
+          place.insert(place.end(), {pbeg[p], p + 1 < sys_panel[s + 1] ? pbeg[p + 1] : S->sys_row[s + 1], S->sys_row[s],
+                                     S->sys_row[s + 1], s, sys_panel[s], sys_panel[s + 1], 0});
+      if ((rc = swr_reserve(&S->small_panel, S->cap_small_panel, place.size()))) return rc;
+      HIP_CHECK(hipMemcpyAsync(S->small_panel, place.data(), sizeof(int) * place.size(), hipMemcpyHostToDevice,
+                               S->stream));
+    }
     if ((rc = swr_reserve(&S->pbeg, S->cap_pbeg, pbeg.size())) || (rc = swr_reserve(&S->pcnt, S->cap_pcnt, (size_t)np)) ||
         (rc = swr_reserve(&S->sys_panel, S->cap_sys_panel, sys_panel.size())))
       return rc;
@@ -228,7 +249,14 @@ int swr_panel_build(swr_system *S) {
     S->prow_nbr_gen = S->nbr_gen;
     S->prow_layout_gen = S->layout_gen;
   }
+  S->panel_lists = false;
+  return S->cg_small ? SWR_OK : swr_panel_lists(S);
+}
+
+int swr_panel_lists(swr_system *S) {
+  if (S->panel_lists || S->npanel <= 0) return SWR_OK;
   const int np = S->npanel;
+  int rc;
   if ((rc = swr_reserve(&S->pcol, S->cap_pcol, (size_t)np * SWR_PANEL_MAXC)) ||
       (rc = swr_reserve(&S->jloc, S->cap_jloc, (size_t)std::max(S->Hcap, 1LL))))
     return rc;
@@ -241,5 +269,6 @@ int swr_panel_build(swr_system *S) {
     hipLaunchKernelGGL(k_panels_off, dim3(div_up(np, 256)), dim3(256), 0, S->stream, np, S->pcnt);
   swr_kt_end(S, KT_PANEL);
   HIP_CHECK(hipGetLastError());
+  S->panel_lists = true;
   return SWR_OK;
 }

@@ -15,8 +15,8 @@
 // x[owner], so the SpMV result is unchanged and x needs only n entries.
 //
 // CG: CG_v2 (fix_qeq_reax_sunway.cpp:983-1167) for s and t at once; the
-// kernels are templates in qeq_cg.h, instantiated here in FP64.
-#include "qeq_cg.h"
+// kernels are in qeq_cg.h (any size) and qeq_small.h (small systems).
+#include "qeq_small.h"
 
 #include <algorithm>
 #include <cmath>
@@ -364,7 +364,7 @@ int swr_qeq_layout(swr_system *S) {
   HIP_CHECK(hipMemsetAsync(S->cgs, 0, sizeof(CgScalars) * 4 * nsys, S->stream));
   const int ps = std::max(std::max(div_up(std::max(n, 1), RPB), nsblk), ntiles);
   if (ps > S->cg_pstride || !S->partials) {
-    if ((rc = swr_alloc(&S->partials, (size_t)ps * 8))) return rc;
+    if ((rc = swr_alloc(&S->partials, (size_t)ps * CG_PART_ROWS))) return rc;
     S->cg_pstride = ps;
   }
   if (!S->done_count && (rc = swr_alloc(&S->done_count, 1))) return rc;
@@ -372,6 +372,7 @@ int swr_qeq_layout(swr_system *S) {
   S->nsys = nsys;
   S->ntiles = ntiles;
   S->nsblk = nsblk;
+  S->cg_small = small_rule(S->sys_row, S->mixed);
   S->h_sys_iters.assign(2 * nsys, 0);
   S->layout_dirty = false;
   S->layout_gen++;
@@ -397,6 +398,7 @@ int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
   int rc = swr_qeq_layout(S);
   if (rc) return rc;
   if (!S->H_val || S->n <= 0) return SWR_ERR_STATE;
+  if ((rc = swr_panel_lists(S))) return rc;
   CgVecsT<double> V = make_vecs(S);
   const int n = S->n;
   const CgScalars *cgs = S->cgs;
@@ -428,9 +430,11 @@ int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
   return SWR_OK;
 }
 
-// Runs the FP64 solves of every system to convergence (first batch of
-// first_batch iteration launches, then batches of 4 between host checks).
-int swr_qeq_cg_run(swr_system *S, int first_batch) {
+// Runs the FP64 solves of every system to convergence; last_iters: the most
+// iterations of the previous solve (0: from zero history), which size the
+// first batch of iteration launches (one more than it took).
+int swr_qeq_cg_run(swr_system *S, int last_iters) {
+  const int first_batch = last_iters > 0 ? last_iters + 1 : CG_COLD_BATCH;
   int rc = swr_qeq_layout(S);
   if (rc) return rc;
   CgRun<double, double> R{};
@@ -451,7 +455,13 @@ int swr_qeq_cg_run(swr_system *S, int first_batch) {
   R.kt_scalars = KT_CG_SCALARS;
   R.partials = S->partials;
   R.pstride = S->cg_pstride;
-  return cg_solve(S, R, first_batch, 0);
+  if (S->cg_small) {
+    const SmallVecs V = small_vecs(R, (double2 *)S->cgv, S->ncap);
+    int all = 0;   // (a system without rows has no workgroup to finish it)
+    for (int s = 0; s < S->nsys; s++) all += S->sys_row[s + 1] > S->sys_row[s];
+    return cg_solve(S, R, first_batch, all, [&](int ph, int k) { return small_step(S, R, V, ph, k); });
+  }
+  return cg_solve(S, R, first_batch, S->nsys, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); });
 }
 
 int swr_qeq_calc_q(swr_system *S) {
@@ -670,7 +680,14 @@ int swr_qeq_cg_noalloc_run(swr_system *S, const double *b, double *x, int *iters
   for (size_t k = 0; k < S->h_sys_iters.size(); k += 2) its0 = std::max(its0, S->h_sys_iters[k]);
   const bool ktime = S->ktime;
   S->ktime = false;
-  const int rc = cg_solve(S, R, its0 + 2, 0);
+  int rc;
+  if (S->cg_small) {   // (its columns have no panel lists)
+    R.pstride = SMALL_ROWS / SWR_PANEL_ROWS;
+    const SmallVecs W = small_vecs(R, vb, NA_MAX_ROWS);
+    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return small_step(S, R, W, ph, k); });
+  } else {
+    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); });
+  }
   S->ktime = ktime;
   if (rc) return rc;
   if (iters_s) *iters_s = its[0];

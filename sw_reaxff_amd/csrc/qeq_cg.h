@@ -32,6 +32,7 @@ constexpr int ROWS_PER_WAVE = 2;           // one row per half-wave
 constexpr int RPB = QW * ROWS_PER_WAVE;    // rows per block (fixed: results do not depend on grid size)
 constexpr int RT = 1024;                   // threads of the one-workgroup reduction kernels
 constexpr int UT = 256;                    // rows (threads) per block of the update kernels
+constexpr int CG_PART_ROWS = 10;           // rows of partial dots (eight here, ten in qeq_small.h)
 
 enum { PH_S1 = 0, PH_S2, PH_S3, PH_A1, PH_K };
 
@@ -117,7 +118,7 @@ __device__ __forceinline__ void block_partials(const double *d, double *__restri
 
 // Scalars after the A step of an iteration reduced dots l0 = u.r, l1 = u.w
 // (fix_qeq_reax_sunway.cpp:1133-1141 and :1152).
-__device__ inline void cg_after_A(CgScalars &c, double l0, double l1, int imax) {
+__device__ __forceinline__ void cg_after_A(CgScalars &c, double l0, double l1, int imax) {
   const double beta = l0 / c.sig_old;
   c.heta = l1 - beta * beta * c.heta;
   c.beta = beta;
@@ -129,6 +130,25 @@ __device__ inline void cg_after_A(CgScalars &c, double l0, double l1, int imax) 
   c.iter += 1;
   c.active_b = 1;
   c.active_a = (c.iter < imax && sqrt(l0) / c.b_norm > c.tol) ? 1 : 0;
+}
+
+// Scalars at the end of the setup (CG_v2 :1020-1087) from the six dots.
+__device__ __forceinline__ unsigned cg_setup_scalars(CgScalars &c, double bb, double ur, double uw, double tol, int imax) {
+  if (tol > 0) c.tol = tol;
+  c.bdot = bb; c.udot_r = ur; c.udot_w = uw;
+  c.b_norm = sqrt(bb);
+  c.sig_old = ur;
+  c.heta = uw;
+  c.alpha_a = c.sig_old / c.heta;
+  c.alpha_x = 0.0;
+  c.beta = 0.0;
+  c.dg0 = c.sig_old;
+  c.dg1 = 0.0;
+  c.iter = 1;
+  c.active_b = 0;
+  c.active_a = (1 < imax && c.tol > 0 && c.b_norm > 0 && sqrt(c.dg0) / c.b_norm > c.tol) ? 1 : 0;
+  c.done = c.active_a ? 0 : 1;
+  return !isfinite(c.alpha_a) && c.active_a ? 1u : 0u;
 }
 
 // Four consecutive stored values of an aligned row as T (two 16-byte loads
@@ -258,7 +278,10 @@ inline PanelArgs panel_args(const swr_system *S) { return PanelArgs{S->prow, S->
 // and the barrier orders LDS only: the values stream from HBM while the
 // list fills.  FU = 2 keeps the default shape within 128 registers (four
 // waves per SIMD).
-template <typename T, typename VT, int NT, int G, int U, class Src, class Row>
+//
+// ZERO: the vector may be the zero vector (a solve from zero history starts
+// from it); a panel whose list holds only zeros then reads no values.
+template <typename T, typename VT, int NT, int G, int U, bool ZERO = false, class Src, class Row>
 __device__ __forceinline__ void panel_rows(int p, const PanelArgs &A, const int *__restrict__ firstnbr,
                                            const int *__restrict__ numnbrs, const int *__restrict__ jlist,
                                            const VT *__restrict__ val, Src src, typename Vec2<T>::type *xl,
@@ -288,11 +311,22 @@ __device__ __forceinline__ void panel_rows(int p, const PanelArgs &A, const int 
     const ushort4 *J = reinterpret_cast<const ushort4 *>(A.jloc + beg);
     RowBatch<T, VT, U, ushort4> b0;
     row_batch0<T, VT, G, U>(cnt, J, val + beg, b0);
+    bool any = false;
+    auto put = [&](int k, const T2 &v) {
+      xl[k] = v;
+      if (ZERO) any |= v.x != (T)0 || v.y != (T)0;
+    };
 #pragma unroll
     for (int u = 0; u < FU; u++)
-      if (threadIdx.x + u * NT < m) xl[threadIdx.x + u * NT] = xk[u];
-    for (int k = threadIdx.x + FU * NT; k < m; k += NT) xl[k] = src(pc[k]);
-    lds_barrier();
+      if (threadIdx.x + u * NT < m) put(threadIdx.x + u * NT, xk[u]);
+    for (int k = threadIdx.x + FU * NT; k < m; k += NT) put(k, src(pc[k]));
+    if (ZERO && !__syncthreads_or(any)) {
+      T2 q;
+      q.x = q.y = (T)0;
+      for (; rb < r1; rb += NT / G) row(rb + grp < r1 ? A.prow[rb + grp] : 0, rb + grp < r1, q);
+      return;
+    }
+    if (!ZERO) lds_barrier();
     const T2 q = row_sum4<T, VT, G, U, true>(cnt, J, val + beg, [&](int k) { return xl[k]; }, &b0);
     row(i, live, q);
     rb += NT / G;
@@ -341,13 +375,12 @@ __device__ __forceinline__ T2 mk2(T a, T b) {
   return r;
 }
 
-// Whether a system's solves still run in phase PH (PH_A1, PH_K read the
-// scalars; c points at the system's s and t scalars).
-__device__ __forceinline__ bool cg_any_active(int PH, const CgScalars *__restrict__ c) {
-  if (PH != PH_A1 && PH != PH_K) return true;
-  // all four flags requested at once (no short-circuit chain of loads)
-  const int ab = c[0].active_b | c[1].active_b, aa = c[0].active_a | c[1].active_a;
-  return ((PH == PH_K ? ab : 0) | aa) != 0;
+// Whether phase PH multiplies (c points at the system's s and t scalars): an
+// iteration in which neither solve goes on to another A step only adds
+// alpha p to x, which needs no product.
+__device__ __forceinline__ bool cg_multiplies(int PH, const CgScalars *__restrict__ c) {
+  if (PH != PH_K) return true;
+  return (c[0].active_a | c[1].active_a) != 0;   // (both requested at once)
 }
 
 // q = eta d + H d (sparse_matvec_C_para, fix_qeq_reax_sw64.c:424-466) of the
@@ -362,16 +395,16 @@ k_cg_spmv(int n, const DevParams *__restrict__ P, const int *__restrict__ type, 
   constexpr int NT = SpmvShape<SH>::NT, G = SpmvShape<SH>::G, U = SpmvShape<SH>::U;
   __shared__ T2 xl[SWR_PANEL_MAXC];
   const int p = blockIdx.x;
-  // skipped once both solves of the panel's system have finished (a panel
-  // holds rows of one system)
-  if (!BATCH && !cg_any_active(PH, cgs)) return;
+  // skipped once neither solve of the panel's system needs a product (a
+  // panel holds rows of one system)
+  if (!BATCH && !cg_multiplies(PH, cgs)) return;
   if (BATCH) {
     const int r0 = A.pbeg[p];
-    if (r0 < A.pbeg[p + 1] && !cg_any_active(PH, cgs + 2 * row_sys[A.prow[r0]])) return;
+    if (r0 < A.pbeg[p + 1] && !cg_multiplies(PH, cgs + 2 * row_sys[A.prow[r0]])) return;
   }
   const T2 *src = PH == PH_S1 ? V.x : PH == PH_S2 ? V.d[0] : PH == PH_S3 ? V.d[1] : (par_in ? V.d[1] : V.d[0]);
-  panel_rows<T, VT, NT, G, U>(p, A, firstnbr, numnbrs, jlist, val, [&](int j) { return src[j]; }, xl,
-                              [&](int i, bool live, T2 q) {
+  panel_rows<T, VT, NT, G, U, PH == PH_S1>(p, A, firstnbr, numnbrs, jlist, val, [&](int j) { return src[j]; }, xl,
+                                           [&](int i, bool live, T2 q) {
     if (lane_id() % G == 0 && live) {
       const T eta = (T)P->eta[type[i]];
       const T2 xi = src[i];
@@ -490,22 +523,8 @@ k_cg_scalars(const double *__restrict__ partials, int pstride, CgScalars *__rest
   int *its = iters_out + 2 * sys;
   if constexpr (PH == PH_S3) {
     auto setup = [&](CgScalars &cc, double bb, double ur, double uw, int s) {
-      if (tol > 0) cc.tol = tol;
-      cc.bdot = bb; cc.udot_r = ur; cc.udot_w = uw;
-      cc.b_norm = sqrt(bb);
-      cc.sig_old = ur;
-      cc.heta = uw;
-      cc.alpha_a = cc.sig_old / cc.heta;
-      cc.alpha_x = 0.0;
-      cc.beta = 0.0;
-      cc.dg0 = cc.sig_old;
-      cc.dg1 = 0.0;
-      cc.iter = 1;
-      cc.active_b = 0;
-      cc.active_a = (1 < imax && cc.tol > 0 && cc.b_norm > 0 && sqrt(cc.dg0) / cc.b_norm > cc.tol) ? 1 : 0;
-      cc.done = cc.active_a ? 0 : 1;
+      bad |= cg_setup_scalars(cc, bb, ur, uw, tol, imax);
       if (cc.done) its[s] = cc.iter;
-      if (!isfinite(cc.alpha_a) && cc.active_a) bad = 1;
     };
     setup(c0, tot[0], tot[1], tot[2], 0);
     setup(c1, tot[3], tot[4], tot[5], 1);
@@ -614,21 +633,26 @@ int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzer
   return SWR_OK;
 }
 
-// Runs the solves of every system of R to convergence.  Iteration kernels
-// are enqueued in batches (the first of first_batch launches); between
-// batches the host reads how many systems have finished.  Launches enqueued
-// after a system finished skip its rows.
-template <typename T, typename VT>
-int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int xzero) {
+// Runs the solves of every system of R to convergence: the setup phases, then
+// iterations in batches (the first of first_batch); between batches the host
+// reads how many systems have finished (`all` of them end the solve).
+// Launches enqueued after a system finished skip its rows.  step(ph, k)
+// enqueues phase ph, k the iteration of PH_K.
+//
+// A solve from zero history has no last count to size its first batch by: 16
+// launches, then 8 at a time (a wait costs ~30 us of idle GPU, a launch
+// that finds nothing to do ~3; cold solves take 14 to 50 iterations).
+constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8;
+
+template <typename T, typename VT, class Step>
+int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Step step) {
   int rc;
-  if ((rc = launch_cg(S, R, PH_S1, 0, xzero)) || (rc = launch_cg(S, R, PH_S2, 0, 0)) ||
-      (rc = launch_cg(S, R, PH_S3, 0, 0)) || (rc = launch_cg(S, R, PH_A1, 0, 0)))
-    return rc;
+  if ((rc = step(PH_S1, 0)) || (rc = step(PH_S2, 0)) || (rc = step(PH_S3, 0)) || (rc = step(PH_A1, 0))) return rc;
   int k = 1;
   int batch = first_batch > 2 ? first_batch : 2;
   while (k < R.imax + 1) {
     for (int b = 0; b < batch && k < R.imax + 1; b++, k++)
-      if ((rc = launch_cg(S, R, PH_K, (k - 1) & 1, 0))) return rc;
+      if ((rc = step(PH_K, k))) return rc;
     // one round trip: done count, status block and iteration counts (into
     // pinned memory when the run has it)
     int done = 0;
@@ -642,8 +666,8 @@ int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int xzero) {
     done = *dh;
     if (R.iters_host && ih != R.iters_host) std::memcpy(R.iters_host, ih, sizeof(int) * 2 * R.L.nsys);
     swr_after_sync(S);
-    if (done >= R.L.nsys) break;
-    batch = 4;
+    if (done >= all) break;
+    batch = CG_NEXT_BATCH;
   }
   return SWR_OK;
 }

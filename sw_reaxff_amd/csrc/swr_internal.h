@@ -318,6 +318,9 @@ struct swr_system {
   unsigned short *jloc = nullptr;
   size_t cap_prow = 0, cap_pbeg = 0, cap_pcnt = 0, cap_pcol = 0, cap_pkey = 0, cap_jloc = 0, cap_sys_panel = 0;
   int npanel = 0, prow_n = -1;
+  int *small_panel = nullptr; // qeq_small.h: eight ints per panel (its rows, its system's rows and panels)
+  size_t cap_small_panel = 0;
+  bool panel_lists = false;   // pcol, pcnt and jloc hold the lists of the current H
   long long nbr_gen = 0, layout_gen = 0, prow_nbr_gen = -1, prow_layout_gen = -1;
   int panel_shape = -1;   // tuning family "panels": 0 (default) lists on, 1 off
   int *H_firstnbr = nullptr, *H_numnbrs = nullptr, *H_jlist = nullptr;
@@ -329,13 +332,15 @@ struct swr_system {
   double *s_hist = nullptr, *t_hist = nullptr;  // [n][5]
   double *cgv = nullptr;           // CG vectors, see CGV_* below
   CgScalars *cgs = nullptr;        // [4 nsys]: s, t per system of the FP64 solve, then of the mixed inner solve
-  double *partials = nullptr;      // per-workgroup partial dots, [8][cg_pstride]
+                                   // (or the small FP64 solve's second buffer)
+  double *partials = nullptr;      // per-workgroup partial dots, [CG_PART_ROWS][cg_pstride]
   int cg_pstride = 0;
   unsigned int *counters = nullptr;
 
   // ---- batch of independent systems (one unless swr_set_batch)
   std::vector<int> sys_row;        // nsys + 1 local-row offsets (host)
   int nsys = 1, ntiles = 0;
+  bool cg_small = false;           // the FP64 solve takes one launch per iteration (qeq_small.h)
   bool layout_dirty = true;
   int *row_sys = nullptr;          // [n] system of each local row
   int *tile_beg = nullptr;         // [ntiles + 1]
@@ -440,7 +445,7 @@ constexpr int MARK_MAX_LAUNCH = 128;  // launches of one relaxation at most
 int swr_bo_run(swr_system *S);
 int swr_qeq_build_H(swr_system *S);
 int swr_qeq_spmv(swr_system *S, const double *xv, double *b);
-int swr_qeq_cg_run(swr_system *S, int first_batch);
+int swr_qeq_cg_run(swr_system *S, int last_iters);
 #define SWR_PIN_MIX 4096
 // Grows the pinned iteration-count buffer to nsys systems (synchronises the
 // stream before replacing it).
@@ -461,6 +466,9 @@ int swr_radix_sort_i32(swr_system *S, const int *keys, const int *vals_in, int n
 // SpMV panels (panel.hip): row order + panel ranges when stale, then the
 // column lists and local indices of the current H
 int swr_panel_build(swr_system *S);
+// the column lists of the current H where swr_panel_build left them out
+// (small systems, whose solve needs none)
+int swr_panel_lists(swr_system *S);
 
 template <class T>
 inline int swr_alloc(T **p, size_t count) {

@@ -39,3 +39,70 @@ def test_gpu_valence_and_torsion_groups(gpu_lib, oracle_lib, ffield, case):
     s = GROUP_SYSTEMS[case]()
     for check in (_gpu_vs_oracle, _gpu_tor_vs_oracle):
         check(oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
+
+
+def waters(m, seed):
+    """A non-periodic cluster of m waters (3 m atoms)."""
+    s = systems.water_box(m, seed=seed)
+    return systems.System(x=s.x, v=s.v, type=s.type, tag=s.tag, elements=s.elements, lo=s.x.min(0) - 12.0,
+                          hi=s.x.max(0) + 12.0, periodic=False)
+
+
+@pytest.mark.gpu
+def test_gpu_small_cg_takes_the_general_solves_bits(gpu_lib, ffield):
+    """1024 panels in all is the most the one-launch-per-iteration solve takes;
+    with one more one-panel system the general solve runs instead.  Systems of
+    1 to 3072 rows around the panel (64) and tile (256) edges: the charges
+    and iteration counts of the common systems are the same bits."""
+    from sw_reaxff_amd.batch import Batch
+    parts = [waters(m, seed=m) for m in (1024, 86, 85, 22, 21)] + [waters(1, seed=100 + k) for k in range(964)]
+    assert sum(-(-s.n // 64) for s in parts) == 1024
+    got = []
+    for extra in ([], [waters(1, seed=2000)]):
+        bt = Batch(ffield, tol=1e-6)
+        bt.load(parts + extra)
+        bt.evaluate()
+        bt.sync()
+        n = int(bt.packed.row_off[len(parts)])
+        got.append((bt.sys.get("q")[:n], bt.iterations()[:len(parts)]))
+    assert got[0][1].max() > 10
+    assert np.array_equal(got[0][0], got[1][0])
+    assert np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 21, 22, 85, 86, 1024, 1025])
+def test_gpu_cg_sizes_against_oracle(gpu_lib, oracle_lib, ffield, m):
+    """One system of 3 m rows, up to the last small and the first general one."""
+    from .parity import atoms_of, make_oracle
+    s = waters(m, seed=m)
+    lmp = harness(s, ffield, tol=1e-10)
+    h = lmp.system
+    h.sync()
+    o = make_oracle(oracle_lib, ffield, s.elements, atoms_of(h), tol=1e-10)
+    o.build_verlet(12.0)
+    o.step()
+    assert np.max(np.abs(h.get("q")[:s.n] - o.get("q")[:s.n])) <= 1e-9
+
+
+@pytest.mark.gpu
+def test_gpu_small_cg_with_an_empty_system(gpu_lib, ffield):
+    """A batch may hold systems without rows: nothing waits for them."""
+    import ctypes as C
+
+    from sw_reaxff_amd import _lib
+    s = waters(30, seed=3)
+    got = []
+    for off in ([0, s.n], [0, 0, s.n, s.n]):
+        h = _lib.System(ffield, s.elements, tol=1e-6)
+        h.set_atoms(s.n, s.x, s.type, s.tag)
+        o = np.array(off, dtype=np.int32)
+        _lib.check(h.L.swr_set_batch(h.h, len(off) - 1, o.ctypes.data_as(C.POINTER(C.c_int))), "swr_set_batch")
+        h.build_neighbors()
+        h.call("qeq_init_matvec")
+        its = h.qeq_cg()
+        h.call("calculate_q")
+        h.sync()
+        got.append((its, h.get("q")[:s.n]))
+    assert got[0][0] == got[1][0] and got[0][0][0] < 100
+    assert np.array_equal(got[0][1], got[1][1])
