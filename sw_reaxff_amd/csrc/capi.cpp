@@ -12,8 +12,6 @@
 
 namespace {
 
-constexpr int MARK_SWEEPS = 1024;
-
 int copy_grow(void **p, size_t old_bytes, size_t new_bytes, hipStream_t s) {
   void *np = nullptr;
   hipError_t e = hipMalloc(&np, new_bytes ? new_bytes : 1);
@@ -400,7 +398,7 @@ int swr_destroy(swr_system *S) {
                   S->Hdia_inv, S->b_s, S->st, S->s_hist, S->t_hist, S->cgv, S->cgs, S->partials, S->counters,
                   S->status, S->scan_tmp, S->tmp_i, S->mixw, S->cand, S->cand_count, S->row_sys, S->tile_beg,
                   S->tile_sys, S->sys_tile, S->sblk_beg, S->sys_sblk, S->sys_iters, S->done_count, S->qsum,
-                  S->mark_chg};
+                  S->mark_chg, S->mark_up};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (S->status_host) (void)hipHostFree(S->status_host);
@@ -591,7 +589,7 @@ int swr_validate_lists(swr_system *S) {
 
 int swr_sort_bonds(swr_system *S) {
   if (!S || !S->bonds) return SWR_ERR_STATE;
-  return swr_lists_mark(S, MARK_SWEEPS);
+  return swr_lists_mark(S);
 }
 
 int swr_bo(swr_system *S) {

@@ -719,44 +719,200 @@ __global__ void k_validate(int n, int N, const int *__restrict__ bond_index, con
 // sort_bonds_C (reaxc_forces_sw64.c:932-971): one in-order pass
 // bond_mark[i] = min(bond_mark[i], bond_mark[j]+1).  Its result for ghost i
 // is min(1000, 1 + min over bonded j < i of the result at j) (locals stay 0,
-// later ghosts still hold 1000); Jacobi sweeps over that recursion reach the
-// same fixed point.  flags[0..2]: sweep k reads flags[(k+2)%3] (changed in
-// sweep k-1), sets flags[k%3], clears flags[(k+1)%3].  flags[3] turns 1 once
-// a sweep finds that the previous one changed nothing; later sweeps skip.
-// In-place relaxation of the marks of ghost atoms (local atoms are 0 and
-// never change).  A ghost g takes min(mark[g], mark[j] + 1) over its bonds to
-// lower-index atoms j, `inner` times per launch, reading neighbours' current
-// values (relaxed atomic loads, so other workgroups' updates are seen as they
-// land).  Every value written is >= the value of the reference's sequential
-// pass and the updates only follow j < g, so the marks settle on exactly that
-// pass's result whatever the update order; a launch in which no mark changed
-// has reached it.  chg[launch] is set when the launch changed a mark; a launch
-// after an unchanged one does nothing.
-__global__ void k_bond_mark(int n, int N, int launch, int inner, const int *__restrict__ bond_index,
-                            const int *__restrict__ bond_end, const int *__restrict__ bond_nbr,
-                            int *__restrict__ mark, int *__restrict__ chg) {
-  if (launch > 0 && __hip_atomic_load(&chg[launch - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
-  const int g = n + blockIdx.x * blockDim.x + threadIdx.x;
+// later ghosts still hold 1000).  A relaxation of that recursion from the
+// initial marks never goes below it and only follows j < i, so it settles on
+// exactly that result whatever the order of the updates.
+//
+// Its length is what bounds it: the chain of hops from the local atoms to the
+// farthest bonded ghost (20 to 30 in water's 12 A shell) of dependent reads.
+//
+// Up to MARK_BFS ghosts: the recursion is a breadth-first search from the
+// local atoms along bonds to higher indices, and only a quarter of the ghosts
+// are ever reached, so one workgroup walks it level by level with the visited
+// set and the queue in LDS (k_mark_bfs), from a compact list of each ghost's
+// higher neighbours (k_mark_up; in LDS too up to BFS_LDS ghosts): exact when
+// it ends.
+//
+// More (k_bond_mark): a workgroup relaxes MARK_T consecutive ghosts to their
+// local fixed point in LDS (each thread keeps its ghost's bonds to lower atoms
+// in registers), reading the marks of the others MARK_ROUNDS times a launch as
+// the other workgroups' updates land (relaxed atomics).  chg[launch] is set
+// when the launch changed a mark; a launch in which none changed has reached
+// the fixed point, and a launch after it does nothing.  Each launch clears the
+// flag of the next (a stale chg[0] only makes the host look one launch
+// further).
+//
+// Relaxing in global memory alone, 1.6 us a hop in 4 to 7 launches, took 49 us
+// on a 64-water box, 76 on 648 waters, 94 on 2,667 and 100 on 32,000.
+constexpr int MARK_BFS = 32512;  // (a ghost's position and two codes in 15 bits)
+constexpr int BFS_LDS = 12288;
+constexpr int BFS_T = 1024;
+constexpr int MARK_FAR = 1000;   // mark of a ghost nothing reaches
+constexpr int UP_NONE = 0x7fff, UP_LIST = 0x7ffe, UP_NEAR = 0x8000;
+
+// Per ghost its bonds to higher ghosts: the positions (after n) of up to four,
+// UP_NONE for none; UP_LIST as the last when there are more (the list is
+// walked instead).  UP_NEAR on the first: the ghost is bonded to a local atom.
+__global__ void __launch_bounds__(256)
+k_mark_up(int n, int N, const int *__restrict__ bond_index, const int *__restrict__ bond_end,
+          const int *__restrict__ bond_nbr, ushort4 *__restrict__ up) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x, g = n + r;
   if (g >= N) return;
   const int p0 = bond_index[g], p1 = bond_end[g];
-  int cur = __hip_atomic_load(&mark[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  bool changed = false;
-  for (int it = 0; it < inner; it++) {
-    int best = cur;
-    for (int p = p0; p < p1; p++) {
-      const int j = bond_nbr[p];
-      if (j < g) {
-        const int v = __hip_atomic_load(&mark[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-        if (v < best) best = v;
-      }
-    }
-    if (best < cur) {
-      cur = best;
-      changed = true;
-      __hip_atomic_store(&mark[g], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int u[4] = {UP_NONE, UP_NONE, UP_NONE, UP_NONE};
+  int cnt = 0;
+  bool near = false;
+#pragma unroll 4
+  for (int p = p0; p < p1; p++) {
+    const int j = bond_nbr[p];
+    near |= j < n;
+    if (j > g) {
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (cnt == k) u[k] = j - n;
+      cnt++;
     }
   }
-  if (changed) atomicOr(&chg[launch], 1);
+  if (cnt > 4) u[3] = UP_LIST;
+  up[r] = make_ushort4((unsigned short)(u[0] | (near ? UP_NEAR : 0)), (unsigned short)u[1], (unsigned short)u[2],
+                       (unsigned short)u[3]);
+}
+
+template <bool LDS>
+__global__ void __launch_bounds__(BFS_T)
+k_mark_bfs(int n, int N, const int *__restrict__ bond_index, const int *__restrict__ bond_end,
+           const int *__restrict__ bond_nbr, const ushort4 *__restrict__ up, int *__restrict__ mark) {
+  constexpr int CAP = LDS ? BFS_LDS : MARK_BFS;
+  __shared__ unsigned int seen[CAP / 32];
+  __shared__ unsigned short queue[CAP];   // every ghost enters at most once
+  __shared__ ushort4 lup[LDS ? BFS_LDS : 1];
+  __shared__ int qend;
+  const int ng = N - n;
+  for (int k = threadIdx.x; k < (ng + 31) / 32; k += BFS_T) seen[k] = 0u;
+  if (threadIdx.x == 0) qend = 0;
+  __syncthreads();
+  auto reach = [&](int h, int level) {
+    const unsigned int bit = 1u << (h & 31);
+    if (atomicOr(&seen[h >> 5], bit) & bit) return;
+    queue[atomicAdd(&qend, 1)] = (unsigned short)h;
+    mark[n + h] = level;
+  };
+#pragma unroll 4
+  for (int r = threadIdx.x; r < ng; r += BFS_T) {
+    const ushort4 v = up[r];
+    if (LDS) lup[r] = v;
+    if (v.x & UP_NEAR) reach(r, 1);
+  }
+  __syncthreads();
+  const unsigned short *ups = LDS ? reinterpret_cast<const unsigned short *>(lup)
+                                  : reinterpret_cast<const unsigned short *>(up);
+  int begin = 0;
+  for (int level = 2; level < MARK_FAR; level++) {
+    const int end = qend;
+    __syncthreads();   // (before anyone appends)
+    if (begin == end) break;
+    // four lanes per atom of the frontier, one of its entries each
+    for (int f = begin + (int)threadIdx.x / 4; f < end; f += BFS_T / 4) {
+      const int r = queue[f], k = threadIdx.x % 4;
+      const int h = ups[4 * r + k] & ~UP_NEAR;
+      if (h == UP_LIST) {
+        for (int p = bond_index[n + r]; p < bond_end[n + r]; p++)
+          if (bond_nbr[p] - n > r) reach(bond_nbr[p] - n, level);
+      } else if (h != UP_NONE) {
+        reach(h, level);
+      }
+    }
+    __syncthreads();
+    begin = end;
+  }
+}
+
+constexpr int MARK_T = 1024;
+constexpr int MARK_NB = 6;       // bonds to lower atoms kept in registers
+constexpr int MARK_ROUNDS = 2;   // reads of the outside marks per launch
+constexpr int MARK_SUB = 4;      // passes over the block's bonds between barriers
+
+__global__ void __launch_bounds__(MARK_T)
+k_bond_mark(int n, int N, int launch, const int *__restrict__ bond_index, const int *__restrict__ bond_end,
+            const int *__restrict__ bond_nbr, int *__restrict__ mark, int *__restrict__ chg) {
+  __shared__ int m[MARK_T];
+  volatile int *vm = m;
+  const bool done = launch > 0 && __hip_atomic_load(&chg[launch - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && launch + 1 < MARK_MAX_LAUNCH)
+    __hip_atomic_store(&chg[launch + 1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (done) return;
+  const int t = threadIdx.x, g0 = n + blockIdx.x * MARK_T, g = g0 + t;
+  const bool live = g < N;
+  const int p0 = live ? bond_index[g] : 0, p1 = live ? bond_end[g] : 0;
+  const int first = live ? __hip_atomic_load(&mark[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+  // bonds to lower atoms inside the block (LDS positions) and outside (ids);
+  // unused ones are the ghost itself, which never lowers it, so that the
+  // passes below read all of them at once
+  int in[MARK_NB], out[MARK_NB];
+#pragma unroll
+  for (int k = 0; k < MARK_NB; k++) {
+    in[k] = t;
+    out[k] = live ? g : n;
+  }
+  int nin = 0, nout = 0;
+  for (int p = p0; p < p1; p++) {
+    const int j = bond_nbr[p];
+    if (j >= g) continue;
+    const bool inside = j >= g0;
+#pragma unroll
+    for (int k = 0; k < MARK_NB; k++) {
+      if (inside && nin == k) in[k] = j - g0;
+      if (!inside && nout == k) out[k] = j;
+    }
+    nin += inside;
+    nout += !inside;
+  }
+  const bool more = nin > MARK_NB || nout > MARK_NB;   // (rare: the rest walked in the list)
+  int cur = first, told = first;
+  vm[t] = cur;
+  __syncthreads();
+  for (int round = 0; round < MARK_ROUNDS; round++) {
+    int v[MARK_NB];
+#pragma unroll
+    for (int k = 0; k < MARK_NB; k++) v[k] = __hip_atomic_load(&mark[out[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int best = cur;
+#pragma unroll
+    for (int k = 0; k < MARK_NB; k++) best = min(best, v[k] + 1);
+    if (more)
+      for (int p = p0; p < p1; p++) {
+        const int j = bond_nbr[p];
+        if (j < g0) best = min(best, __hip_atomic_load(&mark[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
+      }
+    bool lower = live && best < cur;
+    if (lower) vm[t] = cur = best;
+    // the block's own chains: MARK_SUB passes between barriers, each reading
+    // what the other waves hold by then; passes in which no mark fell have
+    // settled them (every other set lowers a mark, so it ends)
+    while (__syncthreads_or(lower)) {
+      lower = false;
+      for (int sub = 0; sub < MARK_SUB; sub++) {
+#pragma unroll
+        for (int k = 0; k < MARK_NB; k++) v[k] = vm[in[k]];
+        best = cur;
+#pragma unroll
+        for (int k = 0; k < MARK_NB; k++) best = min(best, v[k] + 1);
+        if (more)
+          for (int p = p0; p < p1; p++) {
+            const int j = bond_nbr[p];
+            if (j >= g0 && j < g) best = min(best, vm[j - g0] + 1);
+          }
+        if (live && best < cur) {
+          vm[t] = cur = best;
+          lower = true;
+        }
+      }
+    }
+    if (cur < told) {
+      told = cur;
+      __hip_atomic_store(&mark[g], cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (cur < first) atomicOr(&chg[launch], 1);
 }
 __global__ void k_estimate(int n, int N, const int *__restrict__ bond_count, const int *__restrict__ hb_count,
                            const swr_atom_pack_t *__restrict__ atoms, const DevParams *__restrict__ P,
@@ -775,13 +931,8 @@ __global__ void k_estimate(int n, int N, const int *__restrict__ bond_count, con
   }
 }
 
-__global__ void k_mark_init(int *__restrict__ chg, int nchg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nchg) chg[i] = 0;
-}
 __global__ void k_set_flag(DevStatus *st, unsigned int f) { atomicOr(&st->flags, f); }
 
-// Reports whether the sweeps converged and at which sweep (host reads it).
 }  // namespace
 
 // ---------------------------------------------------------------- host side
@@ -944,21 +1095,29 @@ int swr_lists_validate(swr_system *S) {
   return SWR_OK;
 }
 
-// bond_mark of sort_bonds_C (reaxc_forces_sw64.c:932-971): one pass over
-// the atoms in index order, each taking min(mark[i], mark[j] + 1) over its
-// bonds with the values current at that point.  Local atoms start at 0 and
-// ghosts at 1000, so only ghosts change, and ghost i ends at
-//   min(1000, min over bonded j < i of final[j] + 1, min over j > i of init[j] + 1).
-// The sweeps below evaluate that recursion over the j < i graph (Jacobi
-// sweeps: sweep s fixes every ghost whose dependency chain has depth <= s)
-// until no mark changes; the host reads the convergence flag between batches.
-// Enqueues the relaxation (last step's launch count + 2, no host wait) and a
-// copy of the per-launch change flags; swr_mark_settle checks them at the next
-// sync and runs further launches only if the last one still changed a mark.
-int swr_lists_mark(swr_system *S, int max_sweeps) {
+// bond_mark of sort_bonds_C.  Enqueues the relaxation (one launch more than
+// it took last time to find nothing to change, no host wait) and a copy of the
+// per-launch change flags; swr_mark_settle checks them at the next sync and
+// runs further launches only if the last one still changed a mark.
+int swr_lists_mark(swr_system *S) {
   const int n = S->n, N = S->N;
   S->mark_launched = 0;
   if (N <= n) return SWR_OK;
+  if (N - n <= MARK_BFS) {   // exact when it ends: nothing to check
+    if (int rc = swr_reserve(&S->mark_up, S->cap_mark_up, 4 * (size_t)(N - n))) return rc;
+    swr_kt_begin(S, KT_MARK);
+    hipLaunchKernelGGL(k_mark_up, dim3(div_up(N - n, 256)), dim3(256), 0, S->stream, n, N, S->bond_index, S->bond_end,
+                       S->bond_nbr, (ushort4 *)S->mark_up);
+    if (N - n <= BFS_LDS)
+      hipLaunchKernelGGL(k_mark_bfs<true>, dim3(1), dim3(BFS_T), 0, S->stream, n, N, S->bond_index, S->bond_end,
+                         S->bond_nbr, (const ushort4 *)S->mark_up, S->bond_mark);
+    else
+      hipLaunchKernelGGL(k_mark_bfs<false>, dim3(1), dim3(BFS_T), 0, S->stream, n, N, S->bond_index, S->bond_end,
+                         S->bond_nbr, (const ushort4 *)S->mark_up, S->bond_mark);
+    swr_kt_end(S, KT_MARK);
+    HIP_CHECK(hipGetLastError());
+    return SWR_OK;
+  }
   if (!S->mark_chg) {
     int rc = swr_alloc(&S->mark_chg, MARK_MAX_LAUNCH);
     if (rc) return rc;
@@ -967,13 +1126,11 @@ int swr_lists_mark(swr_system *S, int max_sweeps) {
       return SWR_ERR_NOMEM;
     }
   }
-  const int max_launch = std::min(MARK_MAX_LAUNCH, div_up(max_sweeps, MARK_INNER));
-  const int L = std::min(max_launch, std::max(2, div_up(S->mark_depth_hint, MARK_INNER) + 2));
+  const int L = std::min(MARK_MAX_LAUNCH, std::max(2, S->mark_launch_hint + 2));
   swr_kt_begin(S, KT_MARK);
-  hipLaunchKernelGGL(k_mark_init, dim3(1), dim3(MARK_MAX_LAUNCH), 0, S->stream, S->mark_chg, MARK_MAX_LAUNCH);
   for (int k = 0; k < L; k++)
-    hipLaunchKernelGGL(k_bond_mark, dim3(div_up(N - n, 256)), dim3(256), 0, S->stream, n, N, k, MARK_INNER,
-                       S->bond_index, S->bond_end, S->bond_nbr, S->bond_mark, S->mark_chg);
+    hipLaunchKernelGGL(k_bond_mark, dim3(div_up(N - n, MARK_T)), dim3(MARK_T), 0, S->stream, n, N, k, S->bond_index,
+                       S->bond_end, S->bond_nbr, S->bond_mark, S->mark_chg);
   HIP_CHECK(hipMemcpyAsync(S->mark_chg_host, S->mark_chg, sizeof(int) * L, hipMemcpyDeviceToHost, S->stream));
   swr_kt_end(S, KT_MARK);
   HIP_CHECK(hipGetLastError());
@@ -992,20 +1149,20 @@ int swr_mark_settle(swr_system *S) {
   S->mark_launched = 0;
   for (int k = 0; k < launch; k++)
     if (S->mark_chg_host[k] == 0) {
-      S->mark_depth_hint = k * MARK_INNER;
+      S->mark_launch_hint = k;
       return SWR_OK;
     }
   while (launch < MARK_MAX_LAUNCH) {
     const int l0 = launch;
     for (int k = 0; k < 4 && launch < MARK_MAX_LAUNCH; k++, launch++)
-      hipLaunchKernelGGL(k_bond_mark, dim3(div_up(N - n, 256)), dim3(256), 0, S->stream, n, N, launch, MARK_INNER,
+      hipLaunchKernelGGL(k_bond_mark, dim3(div_up(N - n, MARK_T)), dim3(MARK_T), 0, S->stream, n, N, launch,
                          S->bond_index, S->bond_end, S->bond_nbr, S->bond_mark, S->mark_chg);
     HIP_CHECK(hipMemcpyAsync(S->mark_chg_host + l0, S->mark_chg + l0, sizeof(int) * (launch - l0),
                              hipMemcpyDeviceToHost, S->stream));
     HIP_CHECK(hipStreamSynchronize(S->stream));
     for (int k = l0; k < launch; k++)
       if (S->mark_chg_host[k] == 0) {
-        S->mark_depth_hint = k * MARK_INNER;
+        S->mark_launch_hint = k;
         return SWR_OK;
       }
   }

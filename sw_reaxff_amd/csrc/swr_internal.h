@@ -247,6 +247,8 @@ struct swr_system {
   // bond_mark relaxation whose convergence is checked at the next sync
   int *mark_chg = nullptr;         // [MARK_MAX_LAUNCH] device: launch k changed a mark
   int *mark_chg_host = nullptr;    // pinned copy
+  unsigned short *mark_up = nullptr;   // four per ghost: its bonds to higher ghosts (the breadth-first form)
+  size_t cap_mark_up = 0;
   int mark_launched = 0;           // launches of the pending relaxation (0: none pending)
   long long vtotal_local = -1;     // Verlet entries of the local rows (voff[n]), known at each build
 
@@ -301,7 +303,7 @@ struct swr_system {
   double *dDeltap_self = nullptr;  // [N][3]
   int *bond_mark = nullptr, *bond_mark2 = nullptr;
   int *counts = nullptr;           // [2][Ncap]: bonds found per atom, hbonds found per H
-  int mark_depth_hint = 0;         // bond_mark sweeps needed last time
+  int mark_launch_hint = 0;        // bond_mark launches that changed a mark last time
   int *cand = nullptr;             // [Ncap][64]: far slots of bond candidates
   int *cand_count = nullptr;
   size_t cand_cap = 0;
@@ -428,7 +430,7 @@ int swr_lists_reset(swr_system *S);
 int swr_lists_run(swr_system *S, int mode);
 int swr_lists_estimate(swr_system *S);
 int swr_lists_validate(swr_system *S);
-int swr_lists_mark(swr_system *S, int max_sweeps);
+int swr_lists_mark(swr_system *S);
 int swr_mark_settle(swr_system *S);
 int swr_after_sync(swr_system *S);
 int swr_nonbonded_run(swr_system *S);
@@ -440,7 +442,6 @@ int swr_torsion_angles_run(swr_system *S);
 int swr_forces_run(swr_system *S);
 int swr_nve_run(swr_system *S, int stage, double dtv, double dtf);
 int swr_quiesce(swr_system *S);
-constexpr int MARK_INNER = 8;         // bond_mark relaxation sweeps per launch
 constexpr int MARK_MAX_LAUNCH = 128;  // launches of one relaxation at most
 int swr_bo_run(swr_system *S);
 int swr_qeq_build_H(swr_system *S);

@@ -106,3 +106,35 @@ def test_gpu_small_cg_with_an_empty_system(gpu_lib, ffield):
         got.append((its, h.get("q")[:s.n]))
     assert got[0][0] == got[1][0] and got[0][0][0] < 100
     assert np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,a", [(8, 1.7), (10, 1.7), (21, 1.7)])
+def test_gpu_bond_marks_of_crowded_ghosts(gpu_lib, ffield, m, a):
+    """sort_bonds_C's one in-order pass restated over the GPU's own bond lists,
+    where ghosts have a dozen bonds: the search with its neighbour lists in
+    LDS (10,000 ghosts), in memory (13,000) and the relaxation (34,000)."""
+    from sw_reaxff_amd import _lib
+    s = lattice(m, a, seed=m)
+    x = np.mod(s.x - 20.0, m * a)
+    xa, owner = systems.borders(x, np.zeros(3), np.full(3, m * a), 12.0)
+    h = _lib.System(ffield, s.elements)
+    h.set_atoms(s.n, xa, s.type[owner], s.tag[owner], owner=owner)
+    h.build_neighbors()
+    h.set_capacities(np.full(owner.size, 32), np.full(owner.size, 256))
+    for stage in ("write_reax_atoms_and_pack", "reset", "write_reax_lists_init_forces", "validate_lists", "sort_bonds"):
+        h.call(stage)
+    h.sync()
+    n, N = s.n, owner.size
+    bi, be, nbr = h.get("bond_index"), h.get("bond_end"), h.get("bonds")["nbr"]
+    mark = np.full(N, 1000)
+    mark[:n] = 0
+    most = 0
+    for i in range(n, N):
+        j = nbr[bi[i]:be[i]]
+        most = max(most, int((j > i).sum()), int((j < i).sum()))
+        if j.size:
+            mark[i] = min(mark[i], (mark[j] + 1).min())
+    assert most > 6 and (mark[n:] < 1000).any()
+    assert {8: N - n <= 12288, 10: 12288 < N - n <= 32512, 21: N - n > 32512}[m]
+    assert np.array_equal(h.get("bond_mark")[:N], mark)
