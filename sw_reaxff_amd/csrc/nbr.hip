@@ -9,9 +9,9 @@
 //
 // Design (MI355X): atoms are counting-sorted into bins of about cutneigh/2,
 // each bin sorted by atom index so that the list order is deterministic.
-// One wave owns one atom i and walks the stencil as (dy,dz) rows; along x
-// the bins of a row are contiguous in the bin-sorted arrays, so each row is
-// one contiguous segment that the 64 lanes stream through.  Hits are
+// A wave owns a few atoms of one bin and walks their stencil as (dy,dz) rows;
+// along x the bins of a row are contiguous in the bin-sorted arrays, so each
+// row is one contiguous segment that the 64 lanes stream through.  Hits are
 // compacted with a wave ballot.  Pass 1 counts, a scan gives CSR offsets,
 // pass 2 writes.
 #include "swr_internal.h"
@@ -210,29 +210,49 @@ __global__ void __launch_bounds__(RS_T) k_rs_scatter(const int *__restrict__ key
   }
 }
 
-// Atoms per bin from the sorted keys: each run of equal keys writes its
-// length (bins without atoms keep the zero they were cleared to) and
-// appends its bin to the occupied-bin list occ (occ[0] counts them; the
-// Verlet build takes one wave per entry, and the rows it writes do not
-// depend on the entries' order).
-__global__ void k_bin_runs(const int *__restrict__ skeys, int N, int *__restrict__ bin_count, int *__restrict__ occ) {
+// Atoms per bin from the sorted keys (bins without atoms keep the zero they
+// were cleared to): the first lane of each run of equal keys in a wave adds
+// the run's length there.
+__global__ void k_bin_runs(const int *__restrict__ skeys, int N, int *__restrict__ bin_count) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= N) return;
-  const int key = skeys[k];
-  if (k > 0 && skeys[k - 1] == key) return;
-  int e = k + 1;
-  while (e < N && skeys[e] == key) e++;
-  bin_count[key] = e - k;
-  occ[1 + atomicAdd(&occ[0], 1)] = key;   // the occupied bins, in no particular order
+  const int key = k < N ? skeys[k] : -1;
+  const int before = __shfl_up(key, 1, SWR_WAVE);
+  const bool first = key >= 0 && (lane_id() == 0 || before != key);
+  const unsigned long long starts = __ballot(first || key < 0);
+  if (first) {
+    const unsigned long long later = lane_id() == SWR_WAVE - 1 ? 0ull : starts >> (lane_id() + 1);
+    atomicAdd(&bin_count[key], later ? __ffsll((unsigned long long)later) : SWR_WAVE - lane_id());
+  }
 }
 
-// Positions of the sorted atoms (x, y, z, unused).
-__global__ void k_bin_pos(int N, const int *__restrict__ bp_id, const double *__restrict__ x,
-                          double4 *__restrict__ bp_pos) {
+// Positions of the sorted atoms (x, y, z, unused), and the work list of the
+// Verlet build: the sorted position of every A-th atom of a bin (occ[0] counts
+// them; the rows the build writes do not depend on their order).
+constexpr int BP_T = 1024;
+__global__ void __launch_bounds__(BP_T) k_bin_pos(int N, int A, const int *__restrict__ skeys, const int *__restrict__ bin_start,
+                          const int *__restrict__ bp_id, const double *__restrict__ x, double4 *__restrict__ bp_pos,
+                          int *__restrict__ occ) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= N) return;
-  const int j = bp_id[k];
-  bp_pos[k] = make_double4(x[3 * j], x[3 * j + 1], x[3 * j + 2], 0.0);
+  bool head = false;
+  if (k < N) {
+    const int j = bp_id[k];
+    bp_pos[k] = make_double4(x[3 * j], x[3 * j + 1], x[3 * j + 2], 0.0);
+    head = (k - bin_start[skeys[k]]) % A == 0;
+  }
+  // one atomic per workgroup (they serialise on the counter)
+  __shared__ int wcnt[BP_T / SWR_WAVE], at;
+  const unsigned long long m = __ballot(head);
+  if (lane_id() == 0) wcnt[wave_in_block()] = __popcll(m);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int c = 0;
+    for (int w = 0; w < BP_T / SWR_WAVE; w++) c += wcnt[w];
+    at = c ? atomicAdd(&occ[0], c) : 0;
+  }
+  __syncthreads();
+  int slot = 1 + at + ballot_rank(m);
+  for (int w = 0; w < wave_in_block(); w++) slot += wcnt[w];
+  if (head) occ[slot] = k;
 }
 
 // ---------------------------------------------------------------- Verlet
@@ -244,85 +264,122 @@ __device__ __forceinline__ long long readlane_ll(long long v, int l) {
 
 // The full Verlet list, row i = every j != i within cutneigh, in stencil
 // order (stencil rows in order, each row's candidates in bin order: the
-// list one wave per atom walking its stencil would write), built one wave
-// per occupied bin: the atoms of a bin share the bin's stencil, so each candidate is
-// loaded once per bin, one per lane, and tested against every atom of the
-// bin in turn (64 atoms at a time).  The atom's position and id are
-// wave-uniform (scalar loads, one atom ahead), its row start and running
-// count live in lane a % 64 of oa and ca; lanes past a row's last
-// candidate test a point at infinity (no branch).  The candidates' cache
-// traffic is that of one wave per atom divided by the bin occupancy (~20
-// atoms in water at half-cutoff bins).
+// list one wave per atom walking its stencil would write).  A wave takes up
+// to A consecutive atoms of one bin: they share the bin's stencil, so each
+// candidate is loaded once for them, one per lane, and tested against every
+// one in turn.  The atom's position and id are wave-uniform (scalar loads, one
+// atom ahead), its row start and running count live in lane a of oa and ca;
+// lanes past a row's last candidate test a point at infinity (no branch).  The
+// stencil rows' ranges are loaded at once, one per lane, and each chunk of 64
+// candidates while the one before is tested.
+//
+// A follows from what bounds the pass (verlet_atoms): with waves to fill the
+// chip the issue of ~14 VALU instructions per atom and chunk, so a wave takes
+// a whole bin (~20 atoms of water in half-cutoff bins) and candidates are
+// loaded as rarely as possible; with few atoms the chain of ~42 chunks per
+// wave, so they are spread thin.  A whole bin a wave took 245 + 199 us (write
+// and count pass) on the 4,900 atoms of a 64-water box with its ghosts.
 template <bool WRITE>
 __global__ void __launch_bounds__(NB_THREADS)
-k_verlet_bins(const int *__restrict__ occ, const int *__restrict__ bin_start, const double4 *__restrict__ bp_pos,
-              const int *__restrict__ bp_id, const int4 *__restrict__ rows, int nrows, int nx, int ny, int nz,
-              double cutsq, int *__restrict__ vcount, const long long *__restrict__ voff, int *__restrict__ vlist,
-              int nrow) {
-  // the grid is sized for the worst case (every atom in its own bin); the
-  // blocks that hold occupied bins are spread over the XCDs by their own
-  // count, so each XCD takes a contiguous share of them
+k_verlet_bins(const int *__restrict__ occ, int A, const int *__restrict__ skeys, const int *__restrict__ bin_start,
+              const double4 *__restrict__ bp_pos, const int *__restrict__ bp_id, const int4 *__restrict__ rows,
+              int nrows, int nx, int ny, int nz, double cutsq, int *__restrict__ vcount,
+              const long long *__restrict__ voff, int *__restrict__ vlist, int nrow) {
+  // the grid is sized for the worst case (every atom on its own); the blocks
+  // with work are spread over the XCDs by their own count, so each XCD takes a
+  // contiguous share of them
   const int nocc = occ[0];
   const int nact = (nocc + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
   if ((int)blockIdx.x >= nact) return;
   const int t = xcd_block(nact) * WAVES_PER_BLOCK + wave_in_block();
   if (t >= nocc) return;
-  const int b = occ[1 + t];   // an occupied bin (a mostly empty grid, as a batch's, costs nothing)
+  const int g = __builtin_amdgcn_readfirstlane(occ[1 + t]);
+  const int b = __builtin_amdgcn_readfirstlane(skeys[g]);
   const int lane = lane_id();
-  const int a0 = __builtin_amdgcn_readfirstlane(bin_start[b]), a1 = __builtin_amdgcn_readfirstlane(bin_start[b + 1]);
+  const int ma = min(A, __builtin_amdgcn_readfirstlane(bin_start[b + 1]) - g);   // at most 64
   const int bx = b % nx, by = (b / nx) % ny, bz = b / (nx * ny);
-  for (int g = a0; g < a1; g += SWR_WAVE) {
-    const int ma = min(SWR_WAVE, a1 - g);
-    int ca = 0;   // lane a: the running count of atom g + a
-    long long oa = 0;   // lane a: its row start
-    if (WRITE && lane < ma) {
-      const int ia = bp_id[g + lane];
-      if (ia < nrow) oa = voff[ia];
-    }
-    for (int r = 0; r < nrows; r++) {
-      const int4 rw = rows[r];
+  int ca = 0;   // lane a: the running count of atom g + a
+  long long oa = 0;   // lane a: its row start
+  int ia = -1;
+  if (lane < ma) {
+    ia = bp_id[g + lane];
+    if (WRITE && ia < nrow) oa = voff[ia];
+  }
+  for (int r0 = 0; r0 < nrows; r0 += SWR_WAVE) {
+    // lane r: the range of stencil row r0 + r (empty outside the grid)
+    int rs = 0, re = 0;
+    if (r0 + lane < nrows) {
+      const int4 rw = rows[r0 + lane];
       const int cy = by + rw.x, cz = bz + rw.y;
-      if (cy < 0 || cy >= ny || cz < 0 || cz >= nz) continue;
-      const int cx0 = max(bx - rw.z, 0), cx1 = min(bx + rw.z, nx - 1);
-      const int rowbase = (cz * ny + cy) * nx;
-      const int s = bin_start[rowbase + cx0], e = bin_start[rowbase + cx1 + 1];
-      for (int base = s; base < e; base += SWR_WAVE) {
-        const int k = base + lane;
-        int j = -1;
-        double px = HUGE_VAL, py = HUGE_VAL, pz = HUGE_VAL;
-        if (k < e) {
-          j = bp_id[k];
-          const double4 p = bp_pos[k];
-          px = p.x;
-          py = p.y;
-          pz = p.z;
-        }
-        // atom a + 1's id and position are requested while atom a is tested
-        // (uniform: scalar loads)
-        int inx = bp_id[g];
-        double4 pnx = bp_pos[g];
-        for (int a = 0; a < ma; a++) {
-          const int i = inx;
-          const double4 pa = pnx;
-          if (a + 1 < ma) {
-            inx = bp_id[g + a + 1];
-            pnx = bp_pos[g + a + 1];
-          }
-          if (i >= nrow) continue;   // rows past nrow stay empty (the local-atom-only list)
-          const double dx = pa.x - px, dy = pa.y - py, dz = pa.z - pz;
-          const double rsq = dx * dx + dy * dy + dz * dz;
-          const bool hit = (j != i) && (rsq <= cutsq);
-          const unsigned long long m = __ballot(hit);
-          if (WRITE && hit) vlist[readlane_ll(oa, a) + __builtin_amdgcn_readlane(ca, a) + ballot_rank(m)] = j;
-          if (lane == a) ca += __popcll(m);
-        }
+      if (cy >= 0 && cy < ny && cz >= 0 && cz < nz) {
+        const int rowbase = (cz * ny + cy) * nx;
+        rs = bin_start[rowbase + max(bx - rw.z, 0)];
+        re = bin_start[rowbase + min(bx + rw.z, nx - 1) + 1];
       }
     }
-    if (!WRITE && lane < ma) {
-      const int ia = bp_id[g + lane];
-      vcount[ia] = ia < nrow ? ca : 0;
+    unsigned long long left = __ballot(re > rs);
+    if (!left) continue;
+    // chunk (base, e) of row r; the next one is requested before it is tested
+    int r = __ffsll(left) - 1;
+    int base = __builtin_amdgcn_readlane(rs, r), e = __builtin_amdgcn_readlane(re, r);
+    left &= left - 1;
+    int jn = -1;
+    double4 pn = make_double4(HUGE_VAL, HUGE_VAL, HUGE_VAL, 0.0);
+    if (base + lane < e) {
+      jn = bp_id[base + lane];
+      pn = bp_pos[base + lane];
+    }
+    bool last = false;
+    while (!last) {
+      const int j = jn;
+      const double px = pn.x, py = pn.y, pz = pn.z;
+      base += SWR_WAVE;
+      if (base >= e) {
+        last = left == 0;
+        if (!last) {
+          r = __ffsll(left) - 1;
+          left &= left - 1;
+          base = __builtin_amdgcn_readlane(rs, r);
+          e = __builtin_amdgcn_readlane(re, r);
+        }
+      }
+      jn = -1;
+      pn = make_double4(HUGE_VAL, HUGE_VAL, HUGE_VAL, 0.0);
+      if (!last && base + lane < e) {
+        jn = bp_id[base + lane];
+        pn = bp_pos[base + lane];
+      }
+      // atom a + 1's id and position are requested while atom a is tested
+      // (uniform: scalar loads)
+      int inx = bp_id[g];
+      double4 pnx = bp_pos[g];
+      for (int a = 0; a < ma; a++) {
+        const int i = inx;
+        const double4 pa = pnx;
+        if (a + 1 < ma) {
+          inx = bp_id[g + a + 1];
+          pnx = bp_pos[g + a + 1];
+        }
+        if (i >= nrow) continue;   // rows past nrow stay empty (the local-atom-only list)
+        const double dx = pa.x - px, dy = pa.y - py, dz = pa.z - pz;
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        const bool hit = (j != i) && (rsq <= cutsq);
+        const unsigned long long m = __ballot(hit);
+        if (WRITE && hit) vlist[readlane_ll(oa, a) + __builtin_amdgcn_readlane(ca, a) + ballot_rank(m)] = j;
+        if (lane == a) ca += __popcll(m);
+      }
     }
   }
+  if (!WRITE && lane < ma) vcount[ia] = ia < nrow ? ca : 0;
+}
+
+// Atoms per wave: about VERLET_WAVES waves in all, a whole bin once that
+// makes it 16 (splitting the fuller half of the bins, at ~22 atoms a wave on
+// 187,000 atoms, took 0.80 + 0.61 ms against 0.66 + 0.51).
+constexpr int VERLET_WAVES = 8192;
+inline int verlet_atoms(int N) {
+  const int a = std::max(1, N / VERLET_WAVES);
+  return a < 16 ? a : SWR_WAVE;
 }
 
 }  // namespace
@@ -552,6 +609,7 @@ int swr_nbr_build(swr_system *S, int local_only) {
       (rc = swr_reserve(&S->rs_vals, S->cap_rs_vals, (size_t)N)) ||
       (rc = swr_reserve(&S->rs_hist, S->cap_rs_hist, 2 * (size_t)RS_RADIX * rs_nblk + 1)))
     return rc;
+  const int *skeys = nullptr;   // the atoms' bins in sorted order
   swr_kt_begin(S, KT_BINS);
   hipLaunchKernelGGL(k_bin_keys, dim3(div_up(N, 256)), dim3(256), 0, S->stream, S->x, N, S->binlo[0], S->binlo[1],
                      S->binlo[2], S->bininv[0], S->bininv[1], S->bininv[2], S->nbin[0], S->nbin[1], S->nbin[2],
@@ -574,19 +632,21 @@ int swr_nbr_build(swr_system *S, int local_only) {
     }
     HIP_CHECK(hipMemsetAsync(S->bin_count, 0, sizeof(int) * (S->nbins + 1), S->stream));
     HIP_CHECK(hipMemsetAsync(S->bin_occ, 0, sizeof(int), S->stream));
-    hipLaunchKernelGGL(k_bin_runs, dim3(div_up(N, 256)), dim3(256), 0, S->stream, kin, N, S->bin_count, S->bin_occ);
+    hipLaunchKernelGGL(k_bin_runs, dim3(div_up(N, 256)), dim3(256), 0, S->stream, kin, N, S->bin_count);
+    skeys = kin;
   }
   if ((rc = swr_scan_i32(S, S->bin_count, S->bin_start, S->nbins + 1, nullptr))) return rc;
-  hipLaunchKernelGGL(k_bin_pos, dim3(div_up(N, 256)), dim3(256), 0, S->stream, N, (const int *)S->bp_id, S->x,
-                     S->bp_pos);
+  const int A = verlet_atoms(N);
+  hipLaunchKernelGGL(k_bin_pos, dim3(div_up(N, BP_T)), dim3(BP_T), 0, S->stream, N, A, skeys,
+                     (const int *)S->bin_start, (const int *)S->bp_id, S->x, S->bp_pos, S->bin_occ);
   swr_kt_end(S, KT_BINS);
   if ((rc = swr_reserve(&S->vcount, S->cap_vcount, N)) || (rc = swr_reserve(&S->voff, S->cap_voff, (size_t)N + 1)))
     return rc;
   const double cutsq = S->cutneigh * S->cutneigh;
-  // one wave per occupied bin (at most min(nbins, N) of them)
-  const int nblk = div_up(std::min(S->nbins, N), WAVES_PER_BLOCK);
+  // at most one wave per A atoms and one more per occupied bin
+  const int nblk = div_up(std::min<long long>(N, (long long)std::min(S->nbins, N) + N / A), WAVES_PER_BLOCK);
   swr_kt_begin(S, KT_VERLET);
-  hipLaunchKernelGGL(k_verlet_bins<false>, dim3(nblk), dim3(NB_THREADS), 0, S->stream, S->bin_occ, S->bin_start,
+  hipLaunchKernelGGL(k_verlet_bins<false>, dim3(nblk), dim3(NB_THREADS), 0, S->stream, S->bin_occ, A, skeys, S->bin_start,
                      S->bp_pos, S->bp_id, S->stencil_rows, S->nrows, S->nbin[0], S->nbin[1], S->nbin[2], cutsq,
                      S->vcount, (const long long *)nullptr, (int *)nullptr, nrow);
   swr_kt_end(S, KT_VERLET);
@@ -603,7 +663,7 @@ int swr_nbr_build(swr_system *S, int local_only) {
   HIP_CHECK(hipMemcpyAsync(&S->vtotal_local, S->voff + S->n, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
   HIP_CHECK(hipStreamSynchronize(S->stream));
   swr_kt_begin(S, KT_VERLET);
-  hipLaunchKernelGGL(k_verlet_bins<true>, dim3(nblk), dim3(NB_THREADS), 0, S->stream, S->bin_occ, S->bin_start,
+  hipLaunchKernelGGL(k_verlet_bins<true>, dim3(nblk), dim3(NB_THREADS), 0, S->stream, S->bin_occ, A, skeys, S->bin_start,
                      S->bp_pos, S->bp_id, S->stencil_rows, S->nrows, S->nbin[0], S->nbin[1], S->nbin[2], cutsq,
                      S->vcount, (const long long *)S->voff, S->vlist, nrow);
   swr_kt_end(S, KT_VERLET);

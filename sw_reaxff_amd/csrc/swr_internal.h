@@ -204,7 +204,7 @@ struct swr_system {
   int nbins = 0, binscap = 0;
   size_t cap_stencil = 0, cap_bin_of = 0, cap_bp_id = 0, cap_bp_pos = 0, cap_vcount = 0, cap_voff = 0;
   int *bin_of = nullptr, *bin_count = nullptr, *bin_start = nullptr;
-  int *bin_occ = nullptr;        // [0]: number of occupied bins, [1..]: their ids
+  int *bin_occ = nullptr;        // the Verlet build's waves: [0] their number, [1..] each one's first sorted atom
   // pinned host buffers the done checks copy into (device-to-host copies
   // into pageable memory are staged through a bounce buffer)
   int *pin_done = nullptr;        // the CG's count of finished systems
