@@ -40,19 +40,19 @@ __global__ void __launch_bounds__(BT) k_ghost_fill(const int *__restrict__ owner
 }
 
 // The fill order above depends on arrival; sorting each owner's segment
-// makes the summation order of k_forces the ascending ghost order.
-__global__ void __launch_bounds__(BT) k_ghost_sort(int n, const int *__restrict__ start, int *__restrict__ list) {
-  const int o = blockIdx.x * BT + threadIdx.x;
+// makes the summation order of k_forces the ascending ghost order.  One wave
+// per owner, a ghost a lane: its place is the number of smaller ones (an
+// atom of a box as short as the ghost cutoff has 26 images; any number works).
+__global__ void __launch_bounds__(BT) k_ghost_sort(int n, const int *__restrict__ start, const int *__restrict__ list,
+                                                   int *__restrict__ sorted) {
+  const int o = blockIdx.x * (BT / SWR_WAVE) + threadIdx.x / SWR_WAVE, lane = threadIdx.x % SWR_WAVE;
   if (o >= n) return;
   const int b = start[o], e = start[o + 1];
-  for (int p = b + 1; p < e; ++p) {
+  for (int p = b + lane; p < e; p += SWR_WAVE) {
     const int g = list[p];
-    int q = p - 1;
-    while (q >= b && list[q] > g) {
-      list[q + 1] = list[q];
-      --q;
-    }
-    list[q + 1] = g;
+    int place = b;
+    for (int q = b; q < e; ++q) place += list[q] < g ? 1 : 0;
+    sorted[place] = g;
   }
 }
 
@@ -61,7 +61,25 @@ __global__ void __launch_bounds__(BT) k_forces(int n, const double *__restrict__
   const int o = blockIdx.x * BT + threadIdx.x;
   if (o >= n) return;
   double g0 = fcd[4 * (size_t)o], g1 = fcd[4 * (size_t)o + 1], g2 = fcd[4 * (size_t)o + 2];
-  for (int p = start[o]; p < start[o + 1]; ++p) {
+  // four ghosts requested at a time, added in order
+  const int e = start[o + 1];
+  int p = start[o];
+  for (; p + 4 <= e; p += 4) {
+    double v[4][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const size_t g = list[p + k];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[k][c] = fcd[4 * g + c];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      g0 += v[k][0];
+      g1 += v[k][1];
+      g2 += v[k][2];
+    }
+  }
+  for (; p < e; ++p) {
     const size_t g = list[p];
     g0 += fcd[4 * g];
     g1 += fcd[4 * g + 1];
@@ -107,7 +125,7 @@ int ghost_csr(swr_system *S) {
   int rc;
   if ((rc = swr_reserve(&S->gcsr_cnt, S->cap_gcsr_cnt, 2 * (size_t)n + 2)) ||
       (rc = swr_reserve(&S->gcsr_start, S->cap_gcsr_start, (size_t)n + 1)) ||
-      (rc = swr_reserve(&S->gcsr_list, S->cap_gcsr_list, (size_t)std::max(N - n, 1))))
+      (rc = swr_reserve(&S->gcsr_list, S->cap_gcsr_list, 2 * (size_t)std::max(N - n, 1))))
     return rc;
   int *cnt = S->gcsr_cnt, *fill = S->gcsr_cnt + n + 1;
   HIP_CHECK(hipMemsetAsync(cnt, 0, sizeof(int) * (2 * (size_t)n + 2), S->stream));
@@ -117,9 +135,9 @@ int ghost_csr(swr_system *S) {
   if ((rc = swr_scan_i32(S, cnt, S->gcsr_start, n, S->gcsr_start + n))) return rc;
   if (ng > 0) {
     hipLaunchKernelGGL(k_ghost_fill, dim3(div_up(ng, BT)), dim3(BT), 0, S->stream, S->owner, n, N,
-                       (const int *)S->gcsr_start, fill, S->gcsr_list);
-    hipLaunchKernelGGL(k_ghost_sort, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, (const int *)S->gcsr_start,
-                       S->gcsr_list);
+                       (const int *)S->gcsr_start, fill, S->gcsr_list + ng);
+    hipLaunchKernelGGL(k_ghost_sort, dim3(div_up(n, BT / SWR_WAVE)), dim3(BT), 0, S->stream, n,
+                       (const int *)S->gcsr_start, (const int *)(S->gcsr_list + ng), S->gcsr_list);
   }
   HIP_CHECK(hipGetLastError());
   S->gcsr_valid = true;

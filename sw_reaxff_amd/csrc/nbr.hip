@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 namespace {
 
@@ -28,32 +29,102 @@ constexpr int WAVES_PER_BLOCK = NB_THREADS / SWR_WAVE;
 // ---------------------------------------------------------------- borders
 // Comm::borders with one process: for dimension d, atoms [0,nlast) with
 // x <= lo+cut are imaged at +L, then atoms with x >= hi-cut at -L.
-__global__ void k_border_flag(const double *__restrict__ x, int nlast, int d, double thr, int side,
-                              int *__restrict__ flag) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nlast) return;
-  double v = x[3 * i + d];
-  flag[i] = side == 0 ? (v <= thr) : (v >= thr);
+//
+// Six passes (three dimensions, two sides), each over the atoms present when
+// its dimension starts; the atom counts stay on the device (cnt[0] = n, then
+// the count after each pass), so the host waits once, after the last.  A pass
+// is two launches: the flagged atoms of each tile, then each tile's images
+// behind those of the tiles before it.  A count past the arrays' capacity
+// writes nothing beyond it; the host grows them and repeats the passes.
+constexpr int BORDER_T = 256;
+constexpr int BORDER_ITEMS = 4;
+constexpr int BORDER_TILE = BORDER_T * BORDER_ITEMS;
+
+struct BorderPass {
+  int pass, d;            // pass = 2 d + side
+  double thr, shift;
+  int sgn;
+};
+
+__device__ __forceinline__ bool border_flag(const double *__restrict__ x, int i, const BorderPass &B) {
+  const double v = x[3 * i + B.d];
+  return B.sgn > 0 ? v <= B.thr : v >= B.thr;
 }
 
-__global__ void k_border_scatter(double *__restrict__ x, double *__restrict__ q, int *__restrict__ type,
-                                 int *__restrict__ tag, int *__restrict__ owner, signed char *__restrict__ img,
-                                 int *__restrict__ num_bonds, int *__restrict__ num_hbonds,
-                                 const int *__restrict__ flag, const int *__restrict__ pos, int nlast, int ncur,
-                                 int d, double shift, int sgn) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nlast || !flag[i]) return;
-  int g = ncur + pos[i];
-  for (int k = 0; k < 3; k++) x[3 * g + k] = x[3 * i + k];
-  x[3 * g + d] = x[3 * i + d] + shift;
-  q[g] = q[i];   // the charge travels with the border data, as atom style charge's does
-  type[g] = type[i];
-  tag[g] = tag[i];
-  owner[g] = owner[i];
-  for (int k = 0; k < 3; k++) img[3 * g + k] = img[3 * i + k];
-  img[3 * g + d] = (signed char)(img[3 * i + d] + sgn);
-  num_bonds[g] = num_bonds[owner[i]];
-  num_hbonds[g] = num_hbonds[owner[i]];
+// Sum of c over the workgroup (on every thread) and over the threads before.
+__device__ __forceinline__ int border_scan(int c, int *lds, int *total) {
+  const int inc = wave_incl_scan(c);
+  if (lane_id() == SWR_WAVE - 1) lds[wave_in_block()] = inc;
+  __syncthreads();
+  int before = 0, tot = 0;
+  for (int w = 0; w < BORDER_T / SWR_WAVE; w++) {
+    if (w < wave_in_block()) before += lds[w];
+    tot += lds[w];
+  }
+  __syncthreads();
+  *total = tot;
+  return before + inc - c;
+}
+
+__global__ void __launch_bounds__(BORDER_T)
+k_border_count(const double *__restrict__ x, BorderPass B, int cap, const int *__restrict__ cnt,
+               int *__restrict__ tiles) {
+  __shared__ int lds[BORDER_T / SWR_WAVE];
+  const int nlast = min(cnt[B.pass & ~1], cap);
+  const int base = blockIdx.x * BORDER_TILE + threadIdx.x * BORDER_ITEMS;
+  if (blockIdx.x * BORDER_TILE >= nlast) return;
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < BORDER_ITEMS; k++)
+    if (base + k < nlast) c += border_flag(x, base + k, B) ? 1 : 0;
+  int tot;
+  border_scan(c, lds, &tot);
+  if (threadIdx.x == 0) tiles[blockIdx.x] = tot;
+}
+
+__global__ void __launch_bounds__(BORDER_T)
+k_border_scatter(double *__restrict__ x, double *__restrict__ q, int *__restrict__ type, int *__restrict__ tag,
+                 int *__restrict__ owner, signed char *__restrict__ img, int *__restrict__ num_bonds,
+                 int *__restrict__ num_hbonds, BorderPass B, int cap, int *__restrict__ cnt,
+                 const int *__restrict__ tiles) {
+  __shared__ int lds[BORDER_T / SWR_WAVE];
+  const int nlast = min(cnt[B.pass & ~1], cap), ncur = cnt[B.pass];
+  const int ntiles = (nlast + BORDER_TILE - 1) / BORDER_TILE;
+  if ((int)blockIdx.x >= ntiles) return;
+  int before = 0;
+  for (int t = threadIdx.x; t < (int)blockIdx.x; t += BORDER_T) before += tiles[t];
+  int first;
+  border_scan(before, lds, &first);
+  const int base = blockIdx.x * BORDER_TILE + threadIdx.x * BORDER_ITEMS;
+  bool f[BORDER_ITEMS];
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < BORDER_ITEMS; k++) {
+    f[k] = base + k < nlast && border_flag(x, base + k, B);
+    c += f[k] ? 1 : 0;
+  }
+  int tot;
+  long long g = (long long)ncur + first + border_scan(c, lds, &tot);
+  if ((int)blockIdx.x == ntiles - 1 && threadIdx.x == 0) cnt[B.pass + 1] = ncur + first + tot;
+#pragma unroll
+  for (int k = 0; k < BORDER_ITEMS; k++) {
+    if (!f[k]) continue;
+    const int i = base + k;
+    if (g < cap) {
+      for (int e = 0; e < 3; e++) x[3 * g + e] = x[3 * i + e];
+      x[3 * g + B.d] = x[3 * i + B.d] + B.shift;
+      q[g] = q[i];   // the charge travels with the border data, as atom style charge's does
+      type[g] = type[i];
+      tag[g] = tag[i];
+      const int o = owner[i];
+      owner[g] = o;
+      for (int e = 0; e < 3; e++) img[3 * g + e] = img[3 * i + e];
+      img[3 * g + B.d] = (signed char)(img[3 * i + B.d] + B.sgn);
+      num_bonds[g] = num_bonds[o];
+      num_hbonds[g] = num_hbonds[o];
+    }
+    g++;
+  }
 }
 
 // Forward comm of positions: ghost = owner + image shift (pbc add of +-L).
@@ -105,7 +176,8 @@ __global__ void k_pbc(double *__restrict__ x, int n, double lox, double loy, dou
   }
 }
 
-__global__ void k_init_local_maps(int *__restrict__ owner, signed char *__restrict__ img, int n) {
+__global__ void k_init_local_maps(int *__restrict__ owner, signed char *__restrict__ img, int n, int *__restrict__ cnt) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) cnt[0] = n;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   owner[i] = i;
@@ -473,13 +545,18 @@ int swr_nbr_set_grid(swr_system *S, const double lo[3], const double hi[3], doub
     S->binscap = nb + 1;
   }
   S->nbins = nb;
+  // an unchanged stencil (a run's rebuilds in one box) stays on the device
   std::vector<int4> rows = stencil_rows(S->binsize, cutneigh);
-  S->nrows = (int)rows.size();
+  const size_t bytes = rows.size() * sizeof(int4);
+  if (S->stencil_host.size() == rows.size() && std::memcmp(S->stencil_host.data(), rows.data(), bytes) == 0)
+    return SWR_OK;
+  S->stencil_host.clear();
   int rc = swr_reserve(&S->stencil_rows, S->cap_stencil, rows.size());
   if (rc) return rc;
-  HIP_CHECK(hipMemcpyAsync(S->stencil_rows, rows.data(), rows.size() * sizeof(int4), hipMemcpyHostToDevice,
-                           S->stream));
+  HIP_CHECK(hipMemcpyAsync(S->stencil_rows, rows.data(), bytes, hipMemcpyHostToDevice, S->stream));
   HIP_CHECK(hipStreamSynchronize(S->stream));  // rows is a local
+  S->stencil_host.swap(rows);
+  S->nrows = (int)S->stencil_host.size();
   return SWR_OK;
 }
 
@@ -497,36 +574,35 @@ int swr_nbr_borders(swr_system *S, const double lo[3], const double hi[3], doubl
   S->next_totals_known = false;  // new ghosts take their owners' capacities
   S->gcsr_valid = false;
   const int n = S->n;
-  int ncur = n;
-  hipLaunchKernelGGL(k_init_local_maps, dim3(div_up(n, 256)), dim3(256), 0, S->stream, S->owner, S->img, n);
-  for (int d = 0; d < 3; d++) {
-    const int nlast = ncur;
-    for (int side = 0; side < 2; side++) {
-      int rc = swr_ensure_tmp(S, sizeof(int) * (2 * (size_t)nlast + 2));
-      if (rc) return rc;
-      int *flag = S->tmp_i, *pos = S->tmp_i + nlast + 1;
-      double thr = side == 0 ? lo[d] + cutghost : hi[d] - cutghost;
-      hipLaunchKernelGGL(k_border_flag, dim3(div_up(nlast, 256)), dim3(256), 0, S->stream, S->x, nlast, d, thr,
-                         side, flag);
-      rc = swr_scan_i32(S, flag, pos, nlast, pos + nlast);
-      if (rc) return rc;
-      int add = 0;
-      HIP_CHECK(hipMemcpyAsync(&add, pos + nlast, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-      HIP_CHECK(hipStreamSynchronize(S->stream));
-      if (ncur + add > S->Ncap) {
-        if ((rc = swr_nbr_ensure_atoms(S, (int)((ncur + add) * 1.3) + 64))) return rc;
-        flag = S->tmp_i;
-        pos = S->tmp_i + nlast + 1;
-      }
-      double L = hi[d] - lo[d];
-      hipLaunchKernelGGL(k_border_scatter, dim3(div_up(nlast, 256)), dim3(256), 0, S->stream, S->x, S->q,
-                         S->type, S->tag, S->owner, S->img, S->num_bonds, S->num_hbonds, flag, pos, nlast, ncur, d,
-                         side == 0 ? L : -L, side == 0 ? 1 : -1);
-      ncur += add;
+  int *last = S->pin_done + SWR_PIN_BORDERS;
+  for (;;) {
+    const int cap = S->Ncap, ntiles = div_up(cap, BORDER_TILE);
+    int rc = swr_ensure_tmp(S, sizeof(int) * (8 + (size_t)ntiles));
+    if (rc) return rc;
+    int *cnt = S->tmp_i, *tiles = S->tmp_i + 8;
+    hipLaunchKernelGGL(k_init_local_maps, dim3(div_up(n, 256)), dim3(256), 0, S->stream, S->owner, S->img, n, cnt);
+    for (int pass = 0; pass < 6; pass++) {
+      const int d = pass / 2;
+      const double L = hi[d] - lo[d];
+      BorderPass B;
+      B.pass = pass;
+      B.d = d;
+      B.thr = pass % 2 == 0 ? lo[d] + cutghost : hi[d] - cutghost;
+      B.shift = pass % 2 == 0 ? L : -L;
+      B.sgn = pass % 2 == 0 ? 1 : -1;
+      hipLaunchKernelGGL(k_border_count, dim3(ntiles), dim3(BORDER_T), 0, S->stream, S->x, B, cap, (const int *)cnt,
+                         tiles);
+      hipLaunchKernelGGL(k_border_scatter, dim3(ntiles), dim3(BORDER_T), 0, S->stream, S->x, S->q, S->type, S->tag,
+                         S->owner, S->img, S->num_bonds, S->num_hbonds, B, cap, cnt, (const int *)tiles);
     }
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(last, cnt + 1, 6 * sizeof(int), hipMemcpyDeviceToHost, S->stream));
+    HIP_CHECK(hipStreamSynchronize(S->stream));
+    if (last[5] <= cap) break;
+    // (counts after a pass that did not fit are a lower bound: grow and repeat)
+    if ((rc = swr_nbr_ensure_atoms(S, (int)(last[5] * 1.3) + 64))) return rc;
   }
-  S->N = ncur;
-  HIP_CHECK(hipGetLastError());
+  S->N = last[5];
   return SWR_OK;
 }
 
@@ -650,8 +726,13 @@ int swr_nbr_build(swr_system *S, int local_only) {
                      S->bp_pos, S->bp_id, S->stencil_rows, S->nrows, S->nbin[0], S->nbin[1], S->nbin[2], cutsq,
                      S->vcount, (const long long *)nullptr, (int *)nullptr, nrow);
   swr_kt_end(S, KT_VERLET);
-  long long total = 0;
-  if ((rc = swr_scan_i32_to_i64(S, S->vcount, S->voff, N, &total))) return rc;
+  if ((rc = swr_scan_i32_to_i64(S, S->vcount, S->voff, N, nullptr))) return rc;
+  // the total, and the local rows' share (the H matrix capacity)
+  long long *vt = (long long *)(S->pin_done + SWR_PIN_VERLET);
+  HIP_CHECK(hipMemcpyAsync(vt, S->voff + N, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
+  HIP_CHECK(hipMemcpyAsync(vt + 1, S->voff + S->n, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
+  HIP_CHECK(hipStreamSynchronize(S->stream));
+  const long long total = vt[0];
   if (total > S->vcap) {
     long long cap = (long long)(total * 1.15) + 1024;
     if ((rc = swr_alloc(&S->vlist, (size_t)cap))) return rc;
@@ -659,9 +740,7 @@ int swr_nbr_build(swr_system *S, int local_only) {
     S->vcap = cap;
   }
   S->vtotal = total;
-  // local rows' share (the H matrix capacity), read once per build
-  HIP_CHECK(hipMemcpyAsync(&S->vtotal_local, S->voff + S->n, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
-  HIP_CHECK(hipStreamSynchronize(S->stream));
+  S->vtotal_local = vt[1];
   swr_kt_begin(S, KT_VERLET);
   hipLaunchKernelGGL(k_verlet_bins<true>, dim3(nblk), dim3(NB_THREADS), 0, S->stream, S->bin_occ, A, skeys, S->bin_start,
                      S->bp_pos, S->bp_id, S->stencil_rows, S->nrows, S->nbin[0], S->nbin[1], S->nbin[2], cutsq,

@@ -207,7 +207,7 @@ struct swr_system {
   int *bin_occ = nullptr;        // the Verlet build's waves: [0] their number, [1..] each one's first sorted atom
   // pinned host buffers the done checks copy into (device-to-host copies
   // into pageable memory are staged through a bounce buffer)
-  int *pin_done = nullptr;        // the CG's count of finished systems
+  int *pin_done = nullptr;        // [16]: the CG's count of finished systems, and SWR_PIN_* below
   void *pin_mix = nullptr;        // the mixed solve's counters and state (SWR_PIN_MIX bytes)
   int *pin_iters = nullptr;       // iteration counts, 2 per system
   int pin_iters_cap = 0;
@@ -220,6 +220,7 @@ struct swr_system {
   int *bp_id = nullptr;
   int nrows = 0;
   int4 *stencil_rows = nullptr;  // (dy, dz, sx, 0)
+  std::vector<int4> stencil_host;   // what stencil_rows holds
   double cutneigh = 12.0;
   long long *voff = nullptr;     // [N+1]
   int *vcount = nullptr;         // [N]
@@ -448,6 +449,8 @@ int swr_qeq_build_H(swr_system *S);
 int swr_qeq_spmv(swr_system *S, const double *xv, double *b);
 int swr_qeq_cg_run(swr_system *S, int last_iters);
 #define SWR_PIN_MIX 4096
+#define SWR_PIN_VERLET 4    // in pin_done: two 64-bit Verlet totals
+#define SWR_PIN_BORDERS 8   // in pin_done: six atom counts of the border passes
 // Grows the pinned iteration-count buffer to nsys systems (synchronises the
 // stream before replacing it).
 int swr_pin_iters_reserve(swr_system *S, int nsys);
