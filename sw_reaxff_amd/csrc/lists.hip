@@ -970,6 +970,19 @@ int swr_lists_reset(swr_system *S) {
   return SWR_OK;
 }
 
+// The far pass's split: the tuned one, else by the Verlet entries it streams.
+// Four writer waves for four gatherers are best while the far list and the
+// gathered atoms stay in the caches (31,000 water atoms with their ghosts: 157
+// us against 174 with eight gatherers and 191 with
+// two writers; 103,000 atoms of 128 clusters: 328, 355, 408); once the list
+// streams to HBM, eight atoms a workgroup share a phase's writes (187,500
+// atoms, 121M entries: 1418 us against 1490 and 1531; 88,000 atoms, 57M: 613,
+// 636, 681).
+int swr_far_shape(const swr_system *S) {
+  if (S->far_shape >= 0) return S->far_shape;
+  return S->vtotal >= 45000000LL ? SWR_FAR_G8W4 : SWR_FAR_G4W4;
+}
+
 int swr_lists_run(swr_system *S, int mode) {
   {  // k_bonds rewrites bond_mark: finish the last relaxation first
     int rc = swr_quiesce(S);
@@ -1000,7 +1013,7 @@ int swr_lists_run(swr_system *S, int mode) {
   if (mode == 2) {
     FAR_ARGS((k_far<true, false, true, 2>));
   } else {
-    far_dispatch(S->far_shape, [&](auto shc) {
+    far_dispatch(swr_far_shape(S), [&](auto shc) {
       constexpr int FG = FarShape<decltype(shc)::value>::FG, FWR = FarShape<decltype(shc)::value>::FWR;
       const dim3 gb(div_up(N, FG)), tb((FG + FWR) * SWR_WAVE);
 #define FARWS_ARGS(k)                                                                                            \

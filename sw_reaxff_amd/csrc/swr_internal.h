@@ -429,6 +429,7 @@ int swr_nbr_ensure_atoms(swr_system *S, int Ncap);
 int swr_lists_pack(swr_system *S);
 int swr_lists_reset(swr_system *S);
 int swr_lists_run(swr_system *S, int mode);
+int swr_far_shape(const swr_system *S);
 int swr_lists_estimate(swr_system *S);
 int swr_lists_validate(swr_system *S);
 int swr_lists_mark(swr_system *S);

@@ -55,7 +55,7 @@ struct Family {
 const Family kFamilies[] = {{"spmv_fp64", kSpmvNames, kSpmvN, kSpmvDefault, true},
                             {"spmv_fp32", kSpmvNames, kSpmvN, kSpmvDefault, true},
                             {"spmv_resid", kSpmvNames, kSpmvN, kSpmvDefault, true},
-                            {"far", kFarNames, kFarN, SWR_FAR_G4W2, true},
+                            {"far", kFarNames, kFarN, SWR_FAR_G4W4, true},
                             {"panels", kPanelNames, 2, 0, false}};
 constexpr int kNFam = 5;
 
@@ -83,6 +83,7 @@ int shape_index(int fam, const char *name) {
 
 int current(swr_system *S, int fam) {
   const int v = *slot(S, fam);
+  if (v < 0 && kFamilies[fam].shapes == kFarNames) return swr_far_shape(S);   // by size
   return v >= 0 ? v : kFamilies[fam].dflt;
 }
 
