@@ -390,7 +390,7 @@ int swr_destroy(swr_system *S) {
                   S->voff, S->vcount, S->vlist, S->far, S->far_index, S->far_end, S->num_bonds, S->num_hbonds,
                   S->Hindex, S->bond_index, S->bond_end, S->bonds, S->bond_nbr, S->bo_data, S->prow, S->pbeg, S->pcnt, S->pcol, S->pkey, S->jloc, S->sys_panel, S->small_panel, S->BO, S->BOpi, S->Cdbo,
                   S->Cdbopi,
-                  S->Cdbopi2, S->hbond_index, S->hbond_end, S->hbonds, S->bo_dboc, S->dDeltap_self, S->bond_mark,
+                  S->Cdbopi2, S->hbond_index, S->hbond_end, S->hbonds, S->hbslot, S->bo_dboc, S->dDeltap_self, S->bond_mark,
                   S->fcd, S->nb_partials, S->nb_result, S->nb_eatom, S->be_part, S->be_ce, S->be_bufc, S->be_result, S->hb_part,
                   S->hb_result, S->hb_acc, S->va_part, S->va_result, S->va_acc, S->va_cnt, S->va_order, S->va_ctl, S->to_part, S->to_result, S->to_acc,
                   S->to_sacc, S->to_tc, S->to_task, S->to_ctl, S->to_row, S->f, S->gcsr_cnt, S->gcsr_start, S->gcsr_list,
@@ -546,6 +546,7 @@ int swr_reset(swr_system *S) {
     if ((rc = swr_lists_pack(S)) || (rc = swr_lists_estimate(S))) return rc;
     S->capacities_set = true;
     S->next_totals_known = false;
+    S->lists_estimated = true;
   }
   // The previous step's Validate_Lists wrote the capacities and their totals
   // (read back at the host's next sync, normally QEq's); when they fit, Reset runs
@@ -696,9 +697,14 @@ int swr_qeq_pre_force(swr_system *S, int *iters_s, int *iters_t) {
 
 int swr_pair_compute(swr_system *S) {
   int rc;
-  if ((rc = swr_write_reax_atoms_and_pack(S)) || (rc = swr_reset(S)) || (rc = swr_write_reax_lists_init_forces(S)) ||
-      (rc = swr_validate_lists(S)) || (rc = swr_sort_bonds(S)) || (rc = swr_bo(S)))
-    return rc;
+  if ((rc = swr_write_reax_atoms_and_pack(S))) return rc;
+  S->lists_estimated = false;
+  if ((rc = swr_reset(S))) return rc;
+  // new atoms: Reset's capacity estimate has just written these packed atoms'
+  // far list, so only the bonds and hydrogen bonds are left to write
+  const bool far_done = S->lists_estimated && S->bonds;
+  rc = far_done ? swr_lists_run(S, 4) : swr_write_reax_lists_init_forces(S);
+  if (rc || (rc = swr_validate_lists(S)) || (rc = swr_sort_bonds(S)) || (rc = swr_bo(S))) return rc;
   return SWR_OK;
 }
 

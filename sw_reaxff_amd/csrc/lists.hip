@@ -312,7 +312,7 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
          int *__restrict__ far_index, int *__restrict__ far_end, int *__restrict__ cand,
          int *__restrict__ cand_count, const int *__restrict__ Hindex, const int *__restrict__ num_hbonds,
          const int *__restrict__ hbond_index, int *__restrict__ hbond_end, swr_hbond_t *__restrict__ hbonds,
-         int *__restrict__ hb_count, int hbond_cap, DevStatus *st) {
+         int *__restrict__ hb_count, int hbond_cap, int *__restrict__ hbslot, DevStatus *st) {
   __shared__ FarStage<FG, FWR> S;
   const int w = __builtin_amdgcn_readfirstlane(wave_in_block());
   const int lane = lane_id();
@@ -336,9 +336,12 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
   unsigned hmask2 = 0;  // elements with p_hbond == 2 (acceptors)
   for (int e = 0; e < SWR_MAX_ELEM; e++) hmask2 |= (P->p_hbond[e] == 2 ? 1u : 0u) << e;
   const bool doH = HB != 0 && live && i < n && ei >= 0 && P->p_hbond[ei] == 1 && hbond_cut > 0;
+  // HB 3 finds the hydrogen bonds before Reset has laid out their list: their
+  // far slots go to hbslot, at the atom's own Verlet offset (k_hb_place)
   const int H = (doH && HB == 2) ? Hindex[i] : -1;
-  int htop = (doH && HB == 2) ? hbond_end[H] : 0;
-  const int hlim = (doH && HB == 2) ? min(hbond_index[H] + num_hbonds[i], hbond_cap) : 0;
+  int htop = (doH && HB == 2) ? hbond_end[H] : (doH && HB == 3) ? (int)cbeg : 0;
+  const int hlim = (doH && HB == 2) ? min(hbond_index[H] + num_hbonds[i], hbond_cap)
+                   : (doH && HB == 3) ? (int)cend : 0;
   if (gatherer) {
     if (CAND && lane < SWR_MAX_ELEM) S.rbo[g][lane] = P->rbo[(ei >= 0 ? ei : 0) * SWR_MAX_ELEM + lane];
     if (lane == 0) {
@@ -423,7 +426,7 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
       if (doH) {
         const bool ish = infar && d <= hbond_cut && tj >= 0 && ((hmask2 >> tj) & 1u);
         const unsigned long long hm = __ballot(ish);
-        if (HB == 2) {
+        if (HB >= 2) {
           const int hr = ballot_rank(hm);
           if (ish && htop + hr < hlim) S.hb[buf][g][hr] = make_int2(cur.j, (int)slot);
           if (lane == 0) {
@@ -432,7 +435,7 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
           }
         }
         htop += __popcll(hm);
-      } else if (HB == 2 && lane == 0) {
+      } else if (HB >= 2 && lane == 0) {
         S.hcnt[buf][g] = 0;
       }
       nfar += __popcll(m);
@@ -477,6 +480,9 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
             const double2 *src = S.far[pb][gg];
             for (int t = lane; t < 4 * cnt; t += SWR_WAVE) store_nt(dstp + t, src[t]);
           }
+          if (HB == 3) {
+            if (lane < S.hcnt[pb][gg]) hbslot[S.hdst[pb][gg] + lane] = S.hb[pb][gg][lane].y;
+          }
           if (HB == 2) {
             const int hc = S.hcnt[pb][gg];
             if (lane < hc) {
@@ -508,8 +514,8 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
       if (ncand > MCAND) atomicOr(&st->flags, SWR_F_BOND_LDS);
     }
     if (doH) {
-      if (HB == 1) {
-        hb_count[i] = htop;
+      if (HB == 3) {
+        hb_count[i] = htop - (int)cbeg;
       } else {
         if (htop > hlim) {
           atomicOr(&st->flags, SWR_F_HBOND_CAP);
@@ -519,6 +525,39 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
         hb_count[i] = htop - hbond_index[H];
       }
     }
+  }
+}
+
+// The hydrogen bonds that the estimate pass found (HB 3), into the list that
+// Reset has laid out since: HP_L lanes per local H atom, entries in order.
+// Also raises the candidate overflow again, which growing the lists clears.
+constexpr int HP_L = 8;
+__global__ void __launch_bounds__(LT)
+k_hb_place(int n, int N, const int *__restrict__ Hindex, const int *__restrict__ hb_count,
+           const int *__restrict__ num_hbonds, const long long *__restrict__ voff, const int *__restrict__ hbslot,
+           swr_far_neighbor_t *far, const int *__restrict__ hbond_index, int *__restrict__ hbond_end,
+           swr_hbond_t *__restrict__ hbonds, int hbond_cap, const int *__restrict__ cand_count, DevStatus *st) {
+  const int i = (int)(blockIdx.x * LT + threadIdx.x) / HP_L, l = threadIdx.x % HP_L;
+  if (i >= N) return;
+  if (l == 0 && cand_count[i] > MCAND) atomicOr(&st->flags, SWR_F_BOND_LDS);
+  if (i >= n || Hindex[i] < 0) return;
+  const int H = Hindex[i], c = hb_count[i], first = hbond_index[H];
+  const int lim = min(first + num_hbonds[i], hbond_cap);
+  const int *src = hbslot + voff[i];
+  for (int k = l; k < c && first + k < lim; k += HP_L) {
+    const int s = src[k];
+    swr_hbond_t hb;
+    hb.nbr = far[s].nbr;
+    hb.scl = 1;
+    hb.ptr = far + s;
+    hbonds[first + k] = hb;
+  }
+  if (l == 0) {
+    if (first + c > lim) {
+      atomicOr(&st->flags, SWR_F_HBOND_CAP);
+      atomicMax(&st->need_hbond_cap, c);
+    }
+    hbond_end[H] = first + c > lim ? lim : first + c;
   }
 }
 
@@ -983,6 +1022,11 @@ int swr_far_shape(const swr_system *S) {
   return S->vtotal >= 45000000LL ? SWR_FAR_G8W4 : SWR_FAR_G4W4;
 }
 
+// mode 0: the far list; 1: far list, bonds and hydrogen bonds; 2: bonds and
+// hydrogen bonds from the far list; 3: far list and counts, for the capacity
+// estimate; 4: bonds and hydrogen bonds after a 3 on the same packed atoms,
+// which spares new atoms the second far pass (168,000 atoms 850 us of a
+// 9.6 ms first pass).
 int swr_lists_run(swr_system *S, int mode) {
   {  // k_bonds rewrites bond_mark: finish the last relaxation first
     int rc = swr_quiesce(S);
@@ -1009,9 +1053,17 @@ int swr_lists_run(swr_system *S, int mode) {
                      S->Cdbo, S->Cdbopi, S->Cdbopi2, S->bo_dboc, S->dDeltap_self, S->bond_mark,                    \
                      ws + (size_t)WS_DELTAP * S->Ncap, ws + (size_t)WS_DELTAP_BOC * S->Ncap, S->counts,            \
                      S->bond_cap, S->status)
+  if (mode == 3) {
+    const long long need = S->vtotal_local >= 0 ? S->vtotal_local : S->vtotal;
+    if ((rc = swr_reserve(&S->hbslot, S->cap_hbslot, (size_t)std::max(need, 1LL)))) return rc;
+  }
   swr_kt_begin(S, KT_FAR);
   if (mode == 2) {
     FAR_ARGS((k_far<true, false, true, 2>));
+  } else if (mode == 4) {
+    hipLaunchKernelGGL(k_hb_place, dim3(div_up((long long)N * HP_L, LT)), dim3(LT), 0, S->stream, S->n, N, S->Hindex,
+                       hb_count, S->num_hbonds, S->voff, S->hbslot, S->far, S->hbond_index, S->hbond_end, S->hbonds,
+                       S->hbond_cap, S->cand_count, S->status);
   } else {
     far_dispatch(swr_far_shape(S), [&](auto shc) {
       constexpr int FG = FarShape<decltype(shc)::value>::FG, FWR = FarShape<decltype(shc)::value>::FWR;
@@ -1019,10 +1071,10 @@ int swr_lists_run(swr_system *S, int mode) {
 #define FARWS_ARGS(k)                                                                                            \
   hipLaunchKernelGGL(k, gb, tb, 0, S->stream, S->n, N, S->dp, S->packed, S->voff, S->vlist, S->far, S->far_index,    \
                      S->far_end, S->cand, S->cand_count, S->Hindex, S->num_hbonds, S->hbond_index, S->hbond_end,     \
-                     S->hbonds, hb_count, S->hbond_cap, S->status)
+                     S->hbonds, hb_count, S->hbond_cap, S->hbslot, S->status)
       if (mode == 0) FARWS_ARGS((k_far_ws<false, 0, FG, FWR>));
       else if (mode == 1) FARWS_ARGS((k_far_ws<true, 2, FG, FWR>));
-      else FARWS_ARGS((k_far_ws<true, 1, FG, FWR>));
+      else FARWS_ARGS((k_far_ws<true, 3, FG, FWR>));
     });
   }
   swr_kt_end(S, KT_FAR);
@@ -1063,7 +1115,7 @@ int swr_lists_time_far(swr_system *S, int sh, int reps, float *ms) {
       hipLaunchKernelGGL((k_far_ws<true, 2, FG, FWR>), dim3(div_up(N, FG)), dim3((FG + FWR) * SWR_WAVE), 0,
                          S->stream, S->n, N, S->dp, S->packed, S->voff, S->vlist, S->far, S->far_index, S->far_end,
                          S->cand, S->cand_count, S->Hindex, S->num_hbonds, S->hbond_index, S->hbond_end, S->hbonds,
-                         hb_count, S->hbond_cap, S->status);
+                         hb_count, S->hbond_cap, S->hbslot, S->status);
     });
     (void)hipEventRecord(ev[2 * r + 1], S->stream);
   }

@@ -241,6 +241,9 @@ struct swr_system {
   double *BO = nullptr, *BOpi = nullptr, *Cdbo = nullptr, *Cdbopi = nullptr, *Cdbopi2 = nullptr;
   int *hbond_index = nullptr, *hbond_end = nullptr;   // [ncap] by Hindex
   int hbond_cap = 0;
+  int *hbslot = nullptr;           // far slots of the estimate pass's hydrogen bonds, at their rows' Verlet offsets
+  size_t cap_hbslot = 0;
+  bool lists_estimated = false;    // the Reset just done ran the estimate: far list and candidates are current
   swr_hbond_t *hbonds = nullptr;
   bool capacities_set = false;
   bool next_totals_known = false;  // status_host holds the totals of the current capacities

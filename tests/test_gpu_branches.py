@@ -138,3 +138,51 @@ def test_gpu_bond_marks_of_crowded_ghosts(gpu_lib, ffield, m, a):
     assert most > 6 and (mark[n:] < 1000).any()
     assert {8: N - n <= 12288, 10: 12288 < N - n <= 32512, 21: N - n > 32512}[m]
     assert np.array_equal(h.get("bond_mark")[:N], mark)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["water1000", "cluster21", "lattice", "no_hydrogen", "overfull"])
+def test_gpu_first_lists_from_the_estimate_pass(gpu_lib, ffield, case):
+    """New atoms' lists come from the capacity estimate's far pass: the same
+    bits as Reset and the fused pass stage by stage, and the same refusal when
+    an atom has more bond candidates than the pass keeps."""
+    from sw_reaxff_amd import _lib
+    s = {"water1000": lambda: systems.water_box(333, seed=6), "cluster21": lambda: systems.cluster(20, seed=1),
+         "lattice": lattice, "no_hydrogen": lattice, "overfull": lambda: lattice(8, 0.9)}[case]()
+    if case == "no_hydrogen":
+        s.type[:] = np.where(s.type == 1, 2, s.type)
+    got = []
+    for stages in (("pair_compute",), ("write_reax_atoms_and_pack", "reset", "write_reax_lists_init_forces",
+                                       "validate_lists", "sort_bonds", "bo")):
+        h = _lib.System(ffield, s.elements)
+        xa, owner = systems.borders(s.x, s.lo, s.hi, 12.0) if s.periodic else (s.x, np.arange(s.n))
+        h.set_atoms(s.n, xa, s.type[owner], s.tag[owner], owner=owner)
+        h.build_neighbors()
+        try:
+            for stage in stages:
+                h.call(stage)
+            h.sync()
+            out = {k: h.get(k) for k in ("far_index", "far_end", "num_bonds", "num_hbonds", "Hindex", "bond_index",
+                                         "bond_end", "bonds", "BO", "bo_data")}
+            numH = int((out["Hindex"] >= 0).sum())
+            assert (numH == 0) == (case == "no_hydrogen")
+            for k in ("hbond_index", "hbond_end"):
+                out[k] = h.get(k)[:numH]
+            rows = [np.concatenate([np.zeros(0, int)] + [np.arange(a, b) for a, b in zip(out[k + "_index"], out[k + "_end"])])
+                    for k in ("bond", "hbond")]
+            for k in ("bonds", "BO", "bo_data"):
+                out[k] = out[k][rows[0]]
+            rows, hb = rows[1], h.get("hbonds")
+            out["hb"] = (hb["nbr"][rows], hb["scl"][rows], h.get("hbond_far")[rows])
+            assert (rows.size > 0) == (numH > 0)
+            got.append(out)
+        except _lib.SwrError as e:
+            got.append(e.code)
+    a, b = got
+    assert isinstance(a, int) == isinstance(b, int) == (case == "overfull")
+    if case == "overfull":
+        assert a == b
+        return
+    for k in a:
+        for x, y in zip(a[k] if k == "hb" else [a[k]], b[k] if k == "hb" else [b[k]]):
+            assert x.tobytes() == y.tobytes(), k
