@@ -365,6 +365,11 @@ int swr_create(const char *ffield_path, int ntypes, const char *const *elements,
     swr_destroy(S);
     return SWR_ERR_NOMEM;
   }
+  if (hipEventCreateWithFlags(&S->ev_read, hipEventDisableTiming) != hipSuccess) {
+    swr_set_error_msg("hipEventCreate failed");
+    swr_destroy(S);
+    return SWR_ERR_HIP;
+  }
   if ((rc = swr_pin_iters_reserve(S, 64))) {
     swr_destroy(S);
     return rc;
@@ -406,6 +411,7 @@ int swr_destroy(swr_system *S) {
   if (S->pin_mix) (void)hipHostFree(S->pin_mix);
   if (S->pin_iters) (void)hipHostFree(S->pin_iters);
   if (S->mark_chg_host) (void)hipHostFree(S->mark_chg_host);
+  if (S->ev_read) (void)hipEventDestroy(S->ev_read);
   if (S->stream) (void)hipStreamDestroy(S->stream);
   delete S;
   return SWR_OK;
@@ -640,17 +646,20 @@ int swr_sparse_matvec_h(swr_system *S, const double *x_host, double *b_host) {
   return rc;
 }
 
-int swr_qeq_cg(swr_system *S, int *iters_s, int *iters_t) {
+static int qeq_solve(swr_system *S, int *iters_s, int *iters_t, bool then_q, bool *q_done) {
+  *q_done = false;
   if (!S || !S->H_val) return SWR_ERR_STATE;
   int its0 = 0;
   for (size_t k = 0; k < S->h_sys_iters.size(); k += 2) its0 = std::max(its0, S->h_sys_iters[k]);
-  int rc = S->mixed ? swr_qeq_mixed_solve(S) : swr_qeq_cg_run(S, its0);
+  bool read_back = true;   // status and iteration counts are here with the solve's last check
+  int rc = S->mixed ? swr_qeq_mixed_solve(S, then_q, &read_back, q_done) : swr_qeq_cg_run(S, its0, then_q, q_done);
   if (rc) return rc;
-  if (S->mixed) {  // the FP64 solve's last done check already brought status and counts back
+  if (S->mixed) {
     S->h_sys_iters.resize(2 * (size_t)S->nsys);
-    HIP_CHECK(hipMemcpyAsync(S->pin_iters, S->sys_iters, sizeof(int) * 2 * S->nsys, hipMemcpyDeviceToHost,
-                             S->stream));
-    if ((rc = refresh_status(S))) return rc;   // (synchronises)
+    if (!read_back)
+      HIP_CHECK(hipMemcpyAsync(S->pin_iters, S->sys_iters, sizeof(int) * 2 * S->nsys, hipMemcpyDeviceToHost,
+                               S->stream));
+    if ((!read_back || swr_after_sync(S)) && (rc = refresh_status(S))) return rc;   // (synchronises)
     std::memcpy(S->h_sys_iters.data(), S->pin_iters, sizeof(int) * 2 * S->nsys);
   }
   int ms = 0, mt = 0;
@@ -661,6 +670,17 @@ int swr_qeq_cg(swr_system *S, int *iters_s, int *iters_t) {
   if (iters_s) *iters_s = ms;
   if (iters_t) *iters_t = mt;
   return status_to_rc(S->status_host->flags);
+}
+
+int swr_qeq_cg(swr_system *S, int *iters_s, int *iters_t) {
+  bool q_done;
+  return qeq_solve(S, iters_s, iters_t, false, &q_done);
+}
+
+int swr_qeq_charges(swr_system *S, int *iters_s, int *iters_t) {
+  bool q_done;
+  const int rc = qeq_solve(S, iters_s, iters_t, true, &q_done);
+  return rc || q_done ? rc : swr_calculate_q(S);
 }
 
 int swr_qeq_cg_noalloc(swr_system *S, const double *b, double *x, int *iters_s, int *iters_t) {
@@ -685,14 +705,13 @@ int swr_set_batch(swr_system *S, int nsys, const int *row_offsets) {
 
 int swr_calculate_q(swr_system *S) {
   if (!S || S->n <= 0) return SWR_ERR_STATE;
-  return swr_qeq_calc_q(S);
+  return swr_qeq_calc_q(S, SwrQGate());
 }
 
 int swr_qeq_pre_force(swr_system *S, int *iters_s, int *iters_t) {
   int rc;
   if ((rc = swr_qeq_init_matvec(S))) return rc;
-  if ((rc = swr_qeq_cg(S, iters_s, iters_t))) return rc;
-  return swr_calculate_q(S);
+  return swr_qeq_charges(S, iters_s, iters_t);
 }
 
 int swr_pair_compute(swr_system *S) {

@@ -198,12 +198,12 @@ struct swr_lmp {
       mark(3);
       if ((rc = swr_qeq_init_matvec(sys))) return rc;
       mark(4);
-      if ((rc = swr_qeq_cg(sys, &iters_s, &iters_t))) return rc;
+      if ((rc = profile ? swr_qeq_cg(sys, &iters_s, &iters_t) : swr_qeq_charges(sys, &iters_s, &iters_t))) return rc;
       total_iters_s += iters_s;
       total_iters_t += iters_t;
       cg_work_launches += std::max(0, std::max(iters_s, iters_t) - 1);
       mark(5);
-      if ((rc = swr_calculate_q(sys))) return rc;
+      if (profile && (rc = swr_calculate_q(sys))) return rc;
     } else {
       mark(3); mark(4); mark(5);
     }

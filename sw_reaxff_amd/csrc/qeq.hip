@@ -205,10 +205,15 @@ k_spmv1(int n, const DevParams *__restrict__ P, const int *__restrict__ type, co
 }
 
 // ---------------------------------------------------------------- calculate_Q
+// The three kernels may be queued before the solve is known to have finished
+// (swr_qeq_charges); the gate then lets them pass or not, all three alike.
+__device__ __forceinline__ bool q_open(const SwrQGate &g) { return !g.done || (*g.done >= g.all && *g.flags == 0); }
+
 // Tile partial sums of s and t over the local atoms (calculate_Q,
 // fix_qeq_reax_sunway.cpp:1733-1734: the two parallel_vector_acc calls).
 __global__ void __launch_bounds__(UT)
-k_q_sums(const double2 *__restrict__ st, CgLayout L, double *__restrict__ partials, int pstride) {
+k_q_sums(const double2 *__restrict__ st, CgLayout L, double *__restrict__ partials, int pstride, SwrQGate gate) {
+  if (!q_open(gate)) return;
   const int tile = blockIdx.x;
   const int i = L.tile_beg[tile] + threadIdx.x;
   double d[2] = {0.0, 0.0};
@@ -218,7 +223,8 @@ k_q_sums(const double2 *__restrict__ st, CgLayout L, double *__restrict__ partia
 
 // Per system: sum s, sum t and u = sum s / sum t (one workgroup each).
 __global__ void __launch_bounds__(RT)
-k_q_total(const double *__restrict__ partials, int pstride, CgLayout L, double *__restrict__ qsum) {
+k_q_total(const double *__restrict__ partials, int pstride, CgLayout L, double *__restrict__ qsum, SwrQGate gate) {
+  if (!q_open(gate)) return;
   const int sys = blockIdx.x;
   double tot[2];
   reduce_partials<2>(partials, pstride, L.sys_tile[sys], L.sys_tile[sys + 1], tot);
@@ -232,9 +238,9 @@ k_q_total(const double *__restrict__ partials, int pstride, CgLayout L, double *
 // the ghost q refresh (calculate_Q :1736-1754).
 __global__ void k_q_apply(int n, int N, const double2 *__restrict__ st, const double *__restrict__ qsum,
                           const int *__restrict__ owner, const int *__restrict__ row_sys, double *__restrict__ q,
-                          double *__restrict__ s_hist, double *__restrict__ t_hist) {
+                          double *__restrict__ s_hist, double *__restrict__ t_hist, SwrQGate gate) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
+  if (i >= N || !q_open(gate)) return;
   const int o = i < n ? i : owner[i];
   const double u = qsum[3 * row_sys[o] + 2];
   const double2 v = st[o];
@@ -433,7 +439,24 @@ int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
 // Runs the FP64 solves of every system to convergence; last_iters: the most
 // iterations of the previous solve (0: from zero history), which size the
 // first batch of iteration launches (one more than it took).
-int swr_qeq_cg_run(swr_system *S, int last_iters) {
+// Copies up to three runs of words into pinned host memory (one launch; a
+// copy each took ~3 us and a ~5 us gap).
+namespace {
+__global__ void __launch_bounds__(256)
+k_publish(SwrPublish P) {
+  for (int r = 0; r < 3; r++)
+    for (int k = threadIdx.x; k < P.words[r]; k += 256) P.dst[r][k] = P.src[r][k];
+  __threadfence_system();
+}
+}  // namespace
+
+int swr_publish(swr_system *S, const SwrPublish &P) {
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(256), 0, S->stream, P);
+  HIP_CHECK(hipGetLastError());
+  return SWR_OK;
+}
+
+int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
   const int first_batch = last_iters > 0 ? last_iters + 1 : CG_COLD_BATCH;
   int rc = swr_qeq_layout(S);
   if (rc) return rc;
@@ -455,26 +478,39 @@ int swr_qeq_cg_run(swr_system *S, int last_iters) {
   R.kt_scalars = KT_CG_SCALARS;
   R.partials = S->partials;
   R.pstride = S->cg_pstride;
+  int all = S->nsys;
+  if (S->cg_small) {   // (a system without rows has no workgroup to finish it)
+    all = 0;
+    for (int s = 0; s < S->nsys; s++) all += S->sys_row[s + 1] > S->sys_row[s];
+  }
+  SwrQGate gate;
+  gate.done = S->done_count;
+  gate.all = all;
+  gate.flags = &S->status->flags;
+  auto behind = [&] { return then_q ? swr_qeq_calc_q(S, gate) : SWR_OK; };
+  bool finished = false;
   if (S->cg_small) {
     const SmallVecs V = small_vecs(R, (double2 *)S->cgv, S->ncap);
-    int all = 0;   // (a system without rows has no workgroup to finish it)
-    for (int s = 0; s < S->nsys; s++) all += S->sys_row[s + 1] > S->sys_row[s];
-    return cg_solve(S, R, first_batch, all, [&](int ph, int k) { return small_step(S, R, V, ph, k); });
+    rc = cg_solve(S, R, first_batch, all, [&](int ph, int k) { return small_step(S, R, V, ph, k); }, behind, &finished);
+  } else {
+    rc = cg_solve(S, R, first_batch, all, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); }, behind,
+                  &finished);
   }
-  return cg_solve(S, R, first_batch, S->nsys, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); });
+  *q_done = then_q && finished && S->status_host->flags == 0;
+  return rc;
 }
 
-int swr_qeq_calc_q(swr_system *S) {
+int swr_qeq_calc_q(swr_system *S, SwrQGate gate) {
   int rc = swr_qeq_layout(S);
   if (rc) return rc;
   const int n = S->n;
   const int ps = S->cg_pstride;
   const CgLayout L = swr_qeq_cg_layout(S);
   swr_kt_begin(S, KT_QEQ_Q);
-  hipLaunchKernelGGL(k_q_sums, dim3(L.ntiles), dim3(UT), 0, S->stream, (const double2 *)S->st, L, S->partials, ps);
-  hipLaunchKernelGGL(k_q_total, dim3(L.nsys), dim3(RT), 0, S->stream, S->partials, ps, L, S->qsum);
+  hipLaunchKernelGGL(k_q_sums, dim3(L.ntiles), dim3(UT), 0, S->stream, (const double2 *)S->st, L, S->partials, ps, gate);
+  hipLaunchKernelGGL(k_q_total, dim3(L.nsys), dim3(RT), 0, S->stream, S->partials, ps, L, S->qsum, gate);
   hipLaunchKernelGGL(k_q_apply, dim3(div_up(S->N, 256)), dim3(256), 0, S->stream, n, S->N, (const double2 *)S->st,
-                     S->qsum, S->owner, S->row_sys, S->q, S->s_hist, S->t_hist);
+                     S->qsum, S->owner, S->row_sys, S->q, S->s_hist, S->t_hist, gate);
   swr_kt_end(S, KT_QEQ_Q);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -681,12 +717,15 @@ int swr_qeq_cg_noalloc_run(swr_system *S, const double *b, double *x, int *iters
   const bool ktime = S->ktime;
   S->ktime = false;
   int rc;
+  bool finished = false;
+  auto nothing = [] { return (int)SWR_OK; };
   if (S->cg_small) {   // (its columns have no panel lists)
     R.pstride = SMALL_ROWS / SWR_PANEL_ROWS;
     const SmallVecs W = small_vecs(R, vb, NA_MAX_ROWS);
-    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return small_step(S, R, W, ph, k); });
+    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return small_step(S, R, W, ph, k); }, nothing, &finished);
   } else {
-    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); });
+    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); }, nothing,
+                  &finished);
   }
   S->ktime = ktime;
   if (rc) return rc;

@@ -566,6 +566,16 @@ struct CgRun {
   int pstride;
 };
 
+// Queues behind()'s work, then waits for what was queued before it.
+template <class Behind>
+int swr_wait_behind(swr_system *S, Behind behind) {
+  HIP_CHECK(hipEventRecord(S->ev_read, S->stream));
+  const int rc = behind();
+  if (rc != SWR_OK) return rc;
+  HIP_CHECK(hipEventSynchronize(S->ev_read));
+  return SWR_OK;
+}
+
 template <typename T, typename VT>
 int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzero) {
   const int n = S->n;
@@ -644,8 +654,13 @@ int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzer
 // that finds nothing to do ~3; cold solves take 14 to 50 iterations).
 constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8;
 
-template <typename T, typename VT, class Step>
-int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Step step) {
+//
+// A run with pinned memory reads everything back in one small launch, and
+// behind() may queue work that is to follow a finished solve: it then fills
+// the ~25 us the GPU otherwise waits for the host.  *finished: the last check found all systems done.
+template <typename T, typename VT, class Step, class Behind>
+int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Step step, Behind behind,
+             bool *finished) {
   int rc;
   if ((rc = step(PH_S1, 0)) || (rc = step(PH_S2, 0)) || (rc = step(PH_S3, 0)) || (rc = step(PH_A1, 0))) return rc;
   int k = 1;
@@ -658,15 +673,24 @@ int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Ste
     int done = 0;
     int *dh = R.pin_done ? R.pin_done : &done;
     int *ih = R.pin_iters ? R.pin_iters : R.iters_host;
-    HIP_CHECK(hipMemcpyAsync(dh, R.L.done_count, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-    HIP_CHECK(hipMemcpyAsync(S->status_host, S->status, sizeof(DevStatus), hipMemcpyDeviceToHost, S->stream));
-    if (ih)
-      HIP_CHECK(hipMemcpyAsync(ih, R.iters_out, sizeof(int) * 2 * R.L.nsys, hipMemcpyDeviceToHost, S->stream));
-    HIP_CHECK(hipStreamSynchronize(S->stream));
+    if (R.pin_done && R.pin_iters) {
+      SwrPublish P;
+      P.src[0] = R.L.done_count; P.dst[0] = dh; P.words[0] = 1;
+      P.src[1] = (const int *)S->status; P.dst[1] = (int *)S->status_host; P.words[1] = sizeof(DevStatus) / 4;
+      P.src[2] = R.iters_out; P.dst[2] = ih; P.words[2] = 2 * R.L.nsys;
+      if ((rc = swr_publish(S, P))) return rc;
+    } else {
+      HIP_CHECK(hipMemcpyAsync(dh, R.L.done_count, sizeof(int), hipMemcpyDeviceToHost, S->stream));
+      HIP_CHECK(hipMemcpyAsync(S->status_host, S->status, sizeof(DevStatus), hipMemcpyDeviceToHost, S->stream));
+      if (ih)
+        HIP_CHECK(hipMemcpyAsync(ih, R.iters_out, sizeof(int) * 2 * R.L.nsys, hipMemcpyDeviceToHost, S->stream));
+    }
+    if ((rc = swr_wait_behind(S, behind))) return rc;
     done = *dh;
     if (R.iters_host && ih != R.iters_host) std::memcpy(R.iters_host, ih, sizeof(int) * 2 * R.L.nsys);
     swr_after_sync(S);
-    if (done >= all) break;
+    *finished = done >= all;
+    if (*finished) break;
     batch = CG_NEXT_BATCH;
   }
   return SWR_OK;

@@ -63,6 +63,7 @@ struct MixState {
   int converged[2];
   int matvecs[2];      // FP64 residual SpMVs + FP32 inner iterations, per rhs
   double rho[2];       // sqrt(u.r)/|b| of the latest residual
+  double rho0[2];      // and of the solve's first
   int inc;             // the next residual may be formed incrementally
 };
 
@@ -78,7 +79,18 @@ struct MixCtl {
   int outer_ndone;     // systems whose refinement has finished
   int inner_ndone;     // systems whose inner s and t solves have both finished
   int inner_itmax;     // most inner iterations of a system in the current inner solve
-  int pad;
+  int first_ndone;     // systems that met the test on the first residual
+};
+
+// The launches between an inner solve and the next one are queued before the
+// host knows that the inner solve has finished: they do nothing unless its
+// `need` systems have stopped and the refinement goes on.
+struct MixGate {
+  const MixCtl *ctl;
+  int need, nsys;
+  __device__ __forceinline__ bool open() const {
+    return ctl->inner_ndone >= need && ctl->outer_ndone < nsys;
+  }
 };
 
 // Workspace layout: MixCtl at 0, MixState[nsys] from byte 64, two buffers of
@@ -106,7 +118,8 @@ k_resid(int n, const DevParams *__restrict__ P, const int *__restrict__ type, co
         const float *__restrict__ val32, const double2 *__restrict__ x, const float2 *__restrict__ dinc,
         const double2 *__restrict__ b, const double *__restrict__ Hd, double2 *__restrict__ r64,
         float2 *__restrict__ r32, double *__restrict__ partials, int pstride, PanelArgs A,
-        const int *__restrict__ row_sys, const MixState *__restrict__ ms, int first) {
+        const int *__restrict__ row_sys, const MixState *__restrict__ ms, int first, MixGate gate) {
+  if (!first && !gate.open()) return;
   constexpr int NT = SpmvShape<SH>::NT, G = SpmvShape<SH>::G, U = SpmvShape<SH>::U;
   __shared__ double2 xl[SWR_PANEL_MAXC];
   const int p = blockIdx.x;
@@ -157,8 +170,9 @@ template <int NT>
 __global__ void __launch_bounds__(NT)
 k_resid_scalars(const double *__restrict__ partials, int pstride, const int *__restrict__ sys_panel,
                 MixCtl *__restrict__ ctl, MixState *__restrict__ msa, CgScalars *__restrict__ inner_all, double tol,
-                int first, DevStatus *st, int *__restrict__ iters_all) {
+                int first, DevStatus *st, int *__restrict__ iters_all, int need) {
   const int sys = blockIdx.x;
+  if (!first && ctl->inner_ndone < need) return;   // (its own counts stop no system: m.done does)
   MixState m = msa[sys];
   if (!first && m.done) return;
   double tot[6];
@@ -183,6 +197,7 @@ k_resid_scalars(const double *__restrict__ partials, int pstride, const int *__r
     const double bn = sqrt(tot[4 + s]), ur = tot[s], rn = sqrt(tot[2 + s]);
     const double rho = bn > 0 ? sqrt(fmax(ur, 0.0)) / bn : 0.0;
     m.rho[s] = rho;
+    if (first) m.rho0[s] = rho;
     if (!(rho > tol)) {  // meets the test (a NaN does not: it is flagged below)
       m.converged[s] = isnan(rho) ? 0 : 1;
       inner[s].tol = -1.0;
@@ -210,14 +225,15 @@ k_resid_scalars(const double *__restrict__ partials, int pstride, const int *__r
     iters_all[2 * sys] = m.matvecs[0];
     iters_all[2 * sys + 1] = m.matvecs[1];
     atomicAdd(&ctl->outer_ndone, 1);
+    if (first) atomicAdd(&ctl->first_ndone, 1);
   }
   msa[sys] = m;
 }
 
 // x += d over all rows (d is 0 in systems whose inner solve did not run).
-__global__ void k_mixed_update(int n, double2 *__restrict__ x, const float2 *__restrict__ d) {
+__global__ void k_mixed_update(int n, double2 *__restrict__ x, const float2 *__restrict__ d, MixGate gate) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || !gate.open()) return;
   const float2 v = d[i];
   double2 xx = x[i];
   xx.x += (double)v.x;
@@ -247,8 +263,9 @@ __global__ void k_mixed_update(int n, double2 *__restrict__ x, const float2 *__r
 __global__ void __launch_bounds__(UT)
 k_pcg_init(CgLayout L, const float2 *__restrict__ rhs, const double *__restrict__ Hd, float2 *__restrict__ d,
            float2 *__restrict__ r, float2 *__restrict__ z, float2 *__restrict__ p, double *__restrict__ partials,
-           int pstride) {
+           int pstride, MixCtl *__restrict__ ctl) {
   const int tile = blockIdx.x;
+  if (tile == 0 && threadIdx.x == 0) ctl->inner_ndone = ctl->inner_itmax = 0;
   const int i = L.tile_beg[tile] + threadIdx.x;
   double dd[4] = {0, 0, 0, 0};
   if (i < L.tile_beg[tile + 1]) {
@@ -413,7 +430,8 @@ k_pcg_p(CgLayout L, const float2 *__restrict__ z, float2 *__restrict__ p, const 
 // accounting reads; the status block gets the largest.
 __global__ void __launch_bounds__(256)
 k_pcg_finish(int nsys, const PcgState *__restrict__ pst, CgScalars *__restrict__ inner_all,
-             int *__restrict__ status_iters) {
+             int *__restrict__ status_iters, MixGate gate) {
+  if (!gate.open()) return;
   __shared__ int mx[2][256];
   int m0 = 0, m1 = 0;
   for (int s = threadIdx.x; s < nsys; s += 256) {
@@ -463,8 +481,9 @@ int ensure_mixw(swr_system *S) {
 
 }  // namespace
 
-int swr_qeq_mixed_solve(swr_system *S) {
+int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_done) {
   int rc;
+  *read_back = *q_done = false;
   if (!S->H_val32) {
     swr_set_error_msg("mixed-precision QEq needs the FP32 H (fix qeq/reax ... mixed at setup)");
     return SWR_ERR_STATE;
@@ -492,47 +511,53 @@ int swr_qeq_mixed_solve(swr_system *S) {
   double2 *x = (double2 *)S->st;
   const double2 *b = (const double2 *)S->b_s;
   if (nblk < 1 || L.ntiles < 1) return SWR_OK;
-  HIP_CHECK(hipMemsetAsync(ctl, 0, sizeof(MixCtl), S->stream));
   struct Head { MixCtl c; char pad[MS_OFF - sizeof(MixCtl)]; MixState m0; };
   static_assert(offsetof(Head, m0) == MS_OFF, "host copy mirrors the workspace");
-  static_assert(sizeof(Head) + sizeof(MixCtl) <= SWR_PIN_MIX, "the pinned copy holds both reads");
-  Head &h = *(Head *)S->pin_mix;                          // pinned: the copies are plain DMA
-  MixCtl &hc = *(MixCtl *)((char *)S->pin_mix + sizeof(Head));
-  int outer = 0;
-  for (;; outer++) {
+  static_assert(sizeof(Head) <= SWR_PIN_MIX && sizeof(Head) % 4 == 0, "the pinned copy holds it");
+  Head &h = *(Head *)S->pin_mix;
+  SwrPublish pub;
+  pub.src[0] = (const int *)ctl; pub.dst[0] = (int *)&h; pub.words[0] = sizeof(Head) / 4;
+  pub.src[1] = (const int *)S->status; pub.dst[1] = (int *)S->status_host; pub.words[1] = sizeof(DevStatus) / 4;
+  pub.src[2] = S->sys_iters; pub.dst[2] = S->pin_iters; pub.words[2] = 2 * nsys;
+  SwrQGate qgate;
+  qgate.done = &ctl->outer_ndone;
+  qgate.all = nsys;
+  qgate.flags = &S->status->flags;
+  auto behind = [&] { return then_q ? swr_qeq_calc_q(S, qgate) : (int)SWR_OK; };
+  // the outer residual and test; only after an inner solve that need systems
+  // have finished, unless it is the first
+  auto residual = [&](int first, int need) {
+    const MixGate gate = {ctl, need, nsys};
     swr_kt_begin(S, KT_MIXED_OUTER);
     spmv_dispatch(S->spmv_shape[2], [&](auto shc) {
       constexpr int SH = decltype(shc)::value;
       const dim3 tb(SpmvShape<SH>::NT);
-      if (batch)
-        hipLaunchKernelGGL((k_resid<true, SH>), dim3(nblk), tb, 0, S->stream, n, S->dp, S->type, S->H_firstnbr,
-                           S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32, (const double2 *)x, (const float2 *)dv, b,
-                           S->Hdia_inv, r64, rhs, S->partials,
-                           ps, panel_args(S), S->row_sys, ms, outer == 0 ? 1 : 0);
-      else
-        hipLaunchKernelGGL((k_resid<false, SH>), dim3(nblk), tb, 0, S->stream, n, S->dp, S->type, S->H_firstnbr,
-                           S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32, (const double2 *)x, (const float2 *)dv, b,
-                           S->Hdia_inv, r64, rhs, S->partials,
-                           ps, panel_args(S), S->row_sys, ms, outer == 0 ? 1 : 0);
+#define RESID_ARGS n, S->dp, S->type, S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32, (const double2 *)x, \
+                   (const float2 *)dv, b, S->Hdia_inv, r64, rhs, S->partials, ps, panel_args(S), S->row_sys, ms, first, gate
+      if (batch) hipLaunchKernelGGL((k_resid<true, SH>), dim3(nblk), tb, 0, S->stream, RESID_ARGS);
+      else hipLaunchKernelGGL((k_resid<false, SH>), dim3(nblk), tb, 0, S->stream, RESID_ARGS);
+#undef RESID_ARGS
     });
     if (batch)
       hipLaunchKernelGGL(k_resid_scalars<BT>, dim3(nsys), dim3(BT), 0, S->stream, S->partials, ps, S->sys_panel, ctl,
-                         ms, inner, S->ctl.tol * OUTER_TOL_FACTOR, outer == 0 ? 1 : 0, S->status, S->sys_iters);
+                         ms, inner, S->ctl.tol * OUTER_TOL_FACTOR, first, S->status, S->sys_iters, need);
     else
       hipLaunchKernelGGL(k_resid_scalars<RT>, dim3(nsys), dim3(RT), 0, S->stream, S->partials, ps, S->sys_panel, ctl,
-                         ms, inner, S->ctl.tol * OUTER_TOL_FACTOR, outer == 0 ? 1 : 0, S->status, S->sys_iters);
+                         ms, inner, S->ctl.tol * OUTER_TOL_FACTOR, first, S->status, S->sys_iters, need);
     swr_kt_end(S, KT_MIXED_OUTER);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(&h, ctl, sizeof(h), hipMemcpyDeviceToHost, S->stream));
-    HIP_CHECK(hipStreamSynchronize(S->stream));
-    if (outer == 0) { S->mixed_rho0[0] = h.m0.rho[0]; S->mixed_rho0[1] = h.m0.rho[1]; }
-    if (h.c.outer_ndone >= nsys || outer + 1 >= MAX_OUTER) break;
-    // inner FP32 PCG from d = 0; iterations launched in batches sized from
-    // the last solve, the host checking the done count between batches
+  };
+  HIP_CHECK(hipMemsetAsync(ctl, 0, sizeof(MixCtl), S->stream));
+  residual(1, 0);
+  // A pass: the inner FP32 PCG from d = 0, x += d, the next residual.  The
+  // first residual hardly ever meets the test, so its inner solve is queued
+  // without a look at it (every launch skips systems that are done).  The
+  // iterations go in batches sized from the last solve, each followed by the
+  // rest of the pass behind a gate, so a pass usually takes one wait.
+  int outer = 1;
+  for (;; outer++) {
     swr_kt_begin(S, KT_MIXED_INNER);
-    HIP_CHECK(hipMemsetAsync(&ctl->inner_ndone, 0, 2 * sizeof(int), S->stream));
     hipLaunchKernelGGL(k_pcg_init, dim3(L.ntiles), dim3(UT), 0, S->stream, L, rhs, S->Hdia_inv, dv, rv, zv, pv,
-                       S->partials, ps);
+                       S->partials, ps, ctl);
     if (batch)
       hipLaunchKernelGGL(k_pcg_init_scalars<BT>, dim3(nsys), dim3(BT), 0, S->stream, S->partials, ps, L, inner, pst,
                          ctl);
@@ -541,7 +566,7 @@ int swr_qeq_mixed_solve(swr_system *S) {
                          ctl);
     int it = 0;
     int nb = std::max(2, S->mixed_last_inner + 1);
-    while (it < INNER_IMAX) {
+    for (;;) {
       for (int k = 0; k < nb && it < INNER_IMAX; k++, it++) {
         PcgState *cur = pst + (it & 1) * 2 * nsys, *nxt = pst + ((it + 1) & 1) * 2 * nsys;
         spmv_dispatch(S->spmv_shape[1], [&](auto shc) {
@@ -562,23 +587,34 @@ int swr_qeq_mixed_solve(swr_system *S) {
         hipLaunchKernelGGL(k_pcg_p, dim3(L.ntiles), dim3(UT), 0, S->stream, L, (const float2 *)zv, pv, cur, nxt,
                            (const double *)S->partials, ps, ctl, INNER_IMAX);
       }
+      swr_kt_end(S, KT_MIXED_INNER);
+      // (every system has stopped by INNER_IMAX iterations)
+      const int need = it < INNER_IMAX ? nsys : 0;
+      const MixGate gate = {ctl, need, nsys};
+      // (the state after `it` iterations; stopped systems were carried into it)
+      hipLaunchKernelGGL(k_pcg_finish, dim3(1), dim3(256), 0, S->stream, nsys, pst + (it & 1) * 2 * nsys, inner,
+                         S->status->inner_iters, gate);
+      hipLaunchKernelGGL(k_mixed_update, dim3(div_up(n, 256)), dim3(256), 0, S->stream, n, x, (const float2 *)dv,
+                         gate);
+      residual(0, need);
       HIP_CHECK(hipGetLastError());
-      HIP_CHECK(hipMemcpyAsync(&hc, ctl, sizeof(hc), hipMemcpyDeviceToHost, S->stream));
-      HIP_CHECK(hipStreamSynchronize(S->stream));
-      if (hc.inner_ndone >= nsys) {
-        S->mixed_last_inner = hc.inner_itmax;
-        break;
-      }
+      if ((rc = swr_publish(S, pub)) || (rc = swr_wait_behind(S, behind))) return rc;
+      if (h.c.inner_ndone >= need || h.c.first_ndone >= nsys) break;
+      swr_kt_begin(S, KT_MIXED_INNER);
       nb = 4;
     }
-    // (the state after `it` iterations; stopped systems were carried into it)
-    hipLaunchKernelGGL(k_pcg_finish, dim3(1), dim3(256), 0, S->stream, nsys, pst + (it & 1) * 2 * nsys, inner,
-                       S->status->inner_iters);
-    swr_kt_end(S, KT_MIXED_INNER);
-    hipLaunchKernelGGL(k_mixed_update, dim3(div_up(n, 256)), dim3(256), 0, S->stream, n, x, (const float2 *)dv);
-    HIP_CHECK(hipGetLastError());
+    if (h.c.first_ndone >= nsys) {   // nothing was left to refine
+      outer = 0;
+      break;
+    }
+    S->mixed_last_inner = h.c.inner_itmax;
+    if (h.c.outer_ndone >= nsys || outer + 1 >= MAX_OUTER) break;
   }
+  S->mixed_rho0[0] = h.m0.rho0[0];
+  S->mixed_rho0[1] = h.m0.rho0[1];
   S->mixed_outer = outer + 1;
+  *read_back = true;
+  *q_done = then_q && h.c.outer_ndone >= nsys && S->status_host->flags == 0;
   return SWR_OK;
 }
 
@@ -615,12 +651,12 @@ int swr_qeq_time_mixed(swr_system *S, int which, int sh, int reps, float *ms) {
           hipLaunchKernelGGL((k_resid<true, SH>), dim3(nblk), tb, 0, S->stream, n, S->dp, S->type, S->H_firstnbr,
                              S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32, x, (const float2 *)dv, b, S->Hdia_inv, r64,
                              rhs, S->partials, ps, panel_args(S),
-                             S->row_sys, mst, 1);
+                             S->row_sys, mst, 1, MixGate());
         else
           hipLaunchKernelGGL((k_resid<false, SH>), dim3(nblk), tb, 0, S->stream, n, S->dp, S->type, S->H_firstnbr,
                              S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32, x, (const float2 *)dv, b, S->Hdia_inv, r64,
                              rhs, S->partials, ps, panel_args(S),
-                             S->row_sys, mst, 1);
+                             S->row_sys, mst, 1, MixGate());
       } else {
         if (batch)
           hipLaunchKernelGGL((k_pcg_spmv<true, SH>), dim3(nblk), tb, 0, S->stream, n, nsys, S->dp, S->type,

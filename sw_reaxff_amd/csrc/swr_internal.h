@@ -382,6 +382,7 @@ struct swr_system {
 
   // ---- status
   DevStatus *status = nullptr;     // device
+  hipEvent_t ev_read = nullptr;      // after the last swr_publish that something was queued behind
   DevStatus *status_host = nullptr;  // pinned
   unsigned int sticky_flags = 0;
 
@@ -451,16 +452,32 @@ constexpr int MARK_MAX_LAUNCH = 128;  // launches of one relaxation at most
 int swr_bo_run(swr_system *S);
 int swr_qeq_build_H(swr_system *S);
 int swr_qeq_spmv(swr_system *S, const double *xv, double *b);
-int swr_qeq_cg_run(swr_system *S, int last_iters);
+int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done);
 #define SWR_PIN_MIX 4096
 #define SWR_PIN_VERLET 4    // in pin_done: two 64-bit Verlet totals
 #define SWR_PIN_BORDERS 8   // in pin_done: six atom counts of the border passes
 // Grows the pinned iteration-count buffer to nsys systems (synchronises the
 // stream before replacing it).
 int swr_pin_iters_reserve(swr_system *S, int nsys);
-int swr_qeq_calc_q(swr_system *S);
 int swr_qeq_layout(swr_system *S);
-int swr_qeq_mixed_solve(swr_system *S);
+int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_done);
+// Solve and charges together (swr_qeq_cg, then swr_calculate_q): the charge
+// kernels are queued before the host waits for the solve.
+extern "C" int swr_qeq_charges(swr_system *S, int *iters_s, int *iters_t);
+// The charge kernels run when *done >= all and *flags == 0 (done null: always).
+struct SwrQGate {
+  const int *done = nullptr;
+  int all = 0;
+  const unsigned int *flags = nullptr;
+};
+int swr_qeq_calc_q(swr_system *S, SwrQGate gate);
+// Device words to copy into pinned host memory.
+struct SwrPublish {
+  const int *src[3] = {};
+  int *dst[3] = {};
+  int words[3] = {};
+};
+int swr_publish(swr_system *S, const SwrPublish &P);
 // autotuner timing hooks (qeq.hip, qeq_mixed.hip, lists.hip)
 int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms);
 int swr_qeq_time_mixed(swr_system *S, int which, int sh, int reps, float *ms);

@@ -186,3 +186,45 @@ def test_gpu_first_lists_from_the_estimate_pass(gpu_lib, ffield, case):
     for k in a:
         for x, y in zip(a[k] if k == "hb" else [a[k]], b[k] if k == "hb" else [b[k]]):
             assert x.tobytes() == y.tobytes(), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("m", [216, 1400])
+def test_gpu_charges_queued_behind_the_solve(gpu_lib, ffield, m, mixed):
+    """swr_qeq_pre_force queues the charges before it knows that the solve has
+    finished: the same bits as solve and charges one after the other, cold
+    (several batches of iterations), warm, and when the extrapolated start
+    already meets the test (648 atoms: the small solve; 4,200: the general)."""
+    from sw_reaxff_amd import _lib
+    s = systems.water_box(m, seed=m)
+    xa, owner = systems.borders(s.x, s.lo, s.hi, 12.0)
+    hs = []
+    for _ in range(2):
+        h = _lib.System(ffield, s.elements, qeq_mixed=mixed)
+        h.set_atoms(s.n, xa, s.type[owner], s.tag[owner], owner=owner)
+        h.build_neighbors()
+        hs.append(h)
+    iters = []
+    for rep in range(8):
+        out = []
+        for k, h in enumerate(hs):
+            if rep == 7:   # a start that is the last solution
+                for name in ("s_hist", "t_hist"):
+                    a = h.get(name).reshape(-1, 5)
+                    h.put(name, np.repeat(a[:, :1], 5, axis=1))
+            if k == 0:
+                its = [_lib.C.c_int(), _lib.C.c_int()]
+                h.call("qeq_pre_force", *map(_lib.C.byref, its))
+                its = tuple(i.value for i in its)
+            else:
+                h.call("qeq_init_matvec")
+                its = tuple(h.qeq_cg())
+                h.call("calculate_q")
+            out.append((its, h.scalar("mixed_outer"), h.get("q").tobytes(), h.get("s_hist").tobytes(),
+                        h.get("t_hist").tobytes()))
+        assert out[0] == out[1]
+        iters.append(out[0][:2])
+    assert max(iters[0][0]) > (3 if mixed else 16) and max(iters[-1][0]) < max(iters[0][0])
+    if mixed:
+        assert iters[0][1] > 1 and iters[-1][1] == 1
