@@ -683,19 +683,19 @@ def main():
     sysh.ktimer_enable(False)
     be_b = algorithmic_bytes("bonded", c)
     be_avg = (ae_ms + db_ms) / max(1, ae_cnt)
-    bonded = {"kernels": "k_atom_energy, k_atom_energy_nbr, k_sum_rows, k_dbond_own, k_dbond_nbr",
+    bonded = {"kernels": "k_atom_energy, k_atom_energy_nbr, k_dbond_own, k_dbond_nbr",
               "avg_us": round(be_avg * 1e3, 2), "atom_energy_us": round(ae_ms * 1e3 / max(1, ae_cnt), 2),
               "dbond_us": round(db_ms * 1e3 / max(1, db_cnt), 2), "launches": ae_cnt, "bytes_per_pass": be_b,
               "achieved_gbs": round(be_b / (be_avg * 1e-3) / 1e9, 1),
               # event spans from the first to the last launch of each pass,
               # which read longer than the kernels' own durations (rocprof)
-              "valence": {"kernels": "k_valence, k_va_fold, k_sum_rows",
+              "valence": {"kernels": "k_valence, k_va_fold",
                           "event_span_us": round(va_ms * 1e3 / max(1, va_cnt), 2),
                           "energies_kcal_mol": [float(v) for v in sysh.get("valence_energy")]},
-              "torsion": {"kernels": "k_torsion, k_va_fold, k_to_slot_fold, k_sum_rows",
+              "torsion": {"kernels": "k_torsion, k_to_fold, k_to_sum",
                           "event_span_us": round(to_ms * 1e3 / max(1, to_cnt), 2),
                           "energies_kcal_mol": [float(v) for v in sysh.get("torsion_energy")]},
-              "hbonds": {"kernels": "k_hb, k_hb_fold, k_sum_rows",
+              "hbonds": {"kernels": "k_hb, k_hb_fold",
                          "event_span_us": round(hb_ms * 1e3 / max(1, hb_cnt), 2),
                          "e_hb_kcal_mol": float(sysh.get("hbond_energy")[0])},
               "energies_kcal_mol": dict(zip(("e_bond", "e_lp", "e_ov", "e_un", "e_pol"),

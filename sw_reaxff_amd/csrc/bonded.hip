@@ -18,7 +18,7 @@
 // floating-point atomics are needed and results are the same on every run:
 //
 //   k_atom_energy     one thread per local atom: energies (per-atom rows,
-//                     summed in a fixed order by k_sum_rows), its own bond
+//                     summed in a fixed order by sum_row), its own bond
 //                     slots' coefficients, its own CdDelta, and the two
 //                     per-atom factors (CEover4, CEunder4) its neighbours need;
 //   k_atom_energy_nbr one thread per atom (local and ghost): the CdDelta terms
@@ -77,6 +77,44 @@ __device__ __forceinline__ bool triple_bond(const DevParams *__restrict__ P, int
   dua = -gp10 * exphu * hulpov * (gp3 * exphua1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1));
   dub = -gp10 * exphu * hulpov * (gp3 * exphub1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1));
   return true;
+}
+
+// One workgroup's fixed-order sum of a per-atom energy row: 1024 running sums
+// over every 1024th entry, then a tree over them.  Each thread keeps four of
+// the sums and U entries of each in flight (one entry at a time left the row
+// waiting for memory: 147 us on 200,000 atoms).  Run by the first workgroups
+// of the launch that follows the row's producer.
+template <int U>
+__device__ __forceinline__ void sum_row(int n, const double *__restrict__ row, double *__restrict__ out) {
+  __shared__ double s[BT];
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  const int t = threadIdx.x;
+  int base = 0;
+  for (; base + 1024 * U <= n; base += 1024 * U) {
+    double v[U][4];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[u][q] = row[base + 1024 * u + BT * q + t];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) acc[q] += v[u][q];
+  }
+  for (; base < n; base += 1024) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int i = base + BT * q + t;
+      if (i < n) acc[q] += row[i];
+    }
+  }
+  s[t] = (acc[0] + acc[2]) + (acc[1] + acc[3]);
+  __syncthreads();
+  for (int o = BT / 2; o > 0; o >>= 1) {
+    if (t < o) s[t] += s[t + o];
+    __syncthreads();
+  }
+  if (t == 0) *out = s[0];
 }
 
 struct BeArgs {
@@ -232,9 +270,14 @@ __global__ void __launch_bounds__(BT) k_atom_energy(int n, BeArgs A) {
 }
 
 // CdDelta terms of atom j from each bonded local atom i (:270-279 and the
-// triple-bond term :305), read through i's slot toward j.
-__global__ void __launch_bounds__(BT) k_atom_energy_nbr(int n, int N, BeArgs A) {
-  const int j = blockIdx.x * BT + threadIdx.x;
+// triple-bond term :305), read through i's slot toward j; the first five
+// workgroups sum k_atom_energy's rows.
+__global__ void __launch_bounds__(BT) k_atom_energy_nbr(int n, int N, BeArgs A, double *__restrict__ sums) {
+  if (blockIdx.x < 5) {
+    sum_row<8>(n, A.part + blockIdx.x * A.stride, sums + blockIdx.x);
+    return;
+  }
+  const int j = (blockIdx.x - 5) * BT + threadIdx.x;
   if (j >= N) return;
   const DevParams *__restrict__ P = A.P;
   const swr_atom_pack_t aj = A.atoms[j];
@@ -264,22 +307,6 @@ __global__ void __launch_bounds__(BT) k_atom_energy_nbr(int n, int N, BeArgs A) 
     }
   }
   A.fcd[4 * (size_t)j + 3] = cdd;
-}
-
-// Fixed-order sums of the per-atom energy rows: block r sums row r.
-__global__ void __launch_bounds__(1024) k_sum_rows(int n, const double *__restrict__ part, size_t stride,
-                                                   double *__restrict__ out) {
-  __shared__ double s[1024];
-  const double *row = part + blockIdx.x * stride;
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) acc += row[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 512; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
 struct DbArgs {
@@ -571,10 +598,16 @@ __global__ void __launch_bounds__(BT) k_hb(int n, HbArgs A) {
   }
 }
 
-// fCdDelta += the fixed-point terms; the accumulators are left at zero.
-__global__ void __launch_bounds__(BT) k_hb_fold(int N, unsigned long long *__restrict__ acc,
-                                                double *__restrict__ fcd) {
-  const int a = blockIdx.x * BT + threadIdx.x;
+// fCdDelta += the fixed-point terms; the accumulators are left at zero.  The
+// first workgroup sums the energies.
+__global__ void __launch_bounds__(BT) k_hb_fold(int n, int N, unsigned long long *__restrict__ acc,
+                                                double *__restrict__ fcd, const double *__restrict__ part,
+                                                double *__restrict__ sum) {
+  if (blockIdx.x == 0) {
+    sum_row<16>(n, part, sum);
+    return;
+  }
+  const int a = (blockIdx.x - 1) * BT + threadIdx.x;
   if (a >= N) return;
   const size_t coff = 3 * (size_t)N;
 #pragma unroll
@@ -600,7 +633,7 @@ __global__ void __launch_bounds__(BT) k_hb_fold(int N, unsigned long long *__res
 // of lanes per j writes j's own bond slots and row; the terms of k and h go
 // into 64-bit fixed-point accumulators by integer atomics (order-independent
 // sums), folded into fCdDelta by k_va_fold.  The centres with angles are
-// listed by angle count (k_va_count, k_wl_scan, k_va_scatter: a centre with
+// listed by angle count (k_va_count, k_va_scatter: a centre with
 // ten bonds has 45 pairs, one with two bonds one) and the groups take them
 // largest first.
 constexpr double DEG2RAD_PI = 3.14159265;   // constPI, reaxc_defs_sunway.h:61 (DEG2RAD :55)
@@ -619,21 +652,36 @@ enum { WL_NTASK = 0, WL_HIST = 1, WL_CUR = WL_HIST + WL_NB, WL_ABOVE = WL_CUR + 
 constexpr int WL_NABOVE = 6;   // ctl[WL_ABOVE + q]: items with counts above 32 >> q
 __device__ __forceinline__ int wl_bucket(int c) { return c < WL_NB - 1 ? c : WL_NB - 1; }
 
-// Bucket starts, largest count first; the histogram is left at zero.
-__global__ void __launch_bounds__(WL_NB) k_wl_scan(int *__restrict__ ctl) {
-  __shared__ int h[WL_NB];
-  const int b = threadIdx.x;
-  h[b] = ctl[WL_HIST + b];
-  ctl[WL_HIST + b] = 0;
+// Bucket starts, largest count first, into start[0, WL_NB) (every workgroup of
+// a scatter pass computes them from the finished histogram); the first
+// workgroup also stores what the pass over the list reads.
+__device__ __forceinline__ void wl_starts(int *__restrict__ ctl, int *start) {
+  if (threadIdx.x < SWR_WAVE) {
+    const int l = threadIdx.x;
+    // lane l holds buckets b1 = WL_NB - 1 - 2 l and b1 - 1
+    const int b1 = WL_NB - 1 - 2 * l;
+    const int h1 = ctl[WL_HIST + b1], h0 = ctl[WL_HIST + b1 - 1];
+    int incl = h1 + h0;
+#pragma unroll
+    for (int o = 1; o < SWR_WAVE; o <<= 1) {
+      const int up = __shfl_up(incl, o, SWR_WAVE);
+      if (l >= o) incl += up;
+    }
+    start[b1] = incl - h1 - h0;
+    start[b1 - 1] = incl - h0;
+    if (blockIdx.x == 0 && l == SWR_WAVE - 1) ctl[WL_NTASK] = incl;
+  }
   __syncthreads();
-  int start = 0;
-  for (int q = b + 1; q < WL_NB; ++q) start += h[q];
-  ctl[WL_CUR + b] = start;
-  if (b == 0) ctl[WL_NTASK] = start + h[0];
   // items with counts above 32, 16, .., 1: where each group size ends
-  for (int q = 0; q < WL_NABOVE; ++q)
-    if (b == (SWR_WAVE >> (q + 1))) ctl[WL_ABOVE + q] = start;
+  if (blockIdx.x == 0 && threadIdx.x < WL_NABOVE) ctl[WL_ABOVE + threadIdx.x] = start[SWR_WAVE >> (threadIdx.x + 1)];
 }
+static_assert(WL_NB == 2 * SWR_WAVE, "a lane of wl_starts holds two buckets");
+
+// Histogram and bucket cursors back to zero, once the list is made.
+__device__ __forceinline__ void wl_clear(int *__restrict__ ctl) {
+  for (int b = threadIdx.x; b < 2 * WL_NB; b += BT) ctl[WL_HIST + b] = 0;
+}
+static_assert(WL_CUR == WL_HIST + WL_NB, "wl_clear clears both at once");
 
 // The waves of a listed pass.  An item of count c gets a group of G lanes, the
 // power of two at or above c (at most 64), so one round of the group evaluates
@@ -824,9 +872,9 @@ __global__ void __launch_bounds__(BT) k_va_count(int n, VaArgs A) {
 }
 
 __global__ void __launch_bounds__(BT) k_va_scatter(int n, VaArgs A) {
-  __shared__ int cnt[WL_NB], base[WL_NB];
+  __shared__ int cnt[WL_NB], base[WL_NB], start[WL_NB];
   for (int b = threadIdx.x; b < WL_NB; b += BT) cnt[b] = 0;
-  __syncthreads();
+  wl_starts(A.ctl, start);
   const int j = blockIdx.x * BT + threadIdx.x;
   int b = -1, r = 0;
   if (j < n && A.cnt[j] > 0) {
@@ -834,7 +882,7 @@ __global__ void __launch_bounds__(BT) k_va_scatter(int n, VaArgs A) {
     r = atomicAdd(&cnt[b], 1);
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < WL_NB; q += BT) base[q] = cnt[q] ? atomicAdd(&A.ctl[WL_CUR + q], cnt[q]) : 0;
+  for (int q = threadIdx.x; q < WL_NB; q += BT) base[q] = cnt[q] ? start[q] + atomicAdd(&A.ctl[WL_CUR + q], cnt[q]) : 0;
   __syncthreads();
   if (b >= 0) A.order[base[b] + r] = j;
 }
@@ -1092,22 +1140,49 @@ __global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
   }
 }
 
-// fCdDelta (all four columns) += the fixed-point terms; the accumulators are
-// left at zero.
-__global__ void __launch_bounds__(BT) k_va_fold(int N, unsigned long long *__restrict__ acc,
-                                                double *__restrict__ fcd) {
-  const int a = blockIdx.x * BT + threadIdx.x;
-  if (a >= N) return;
+// fCdDelta's row a (f, in registers) += the fixed-point terms; the accumulators
+// are left at zero.  Whether there were any.
+__device__ __forceinline__ bool fold4(int N, int a, unsigned long long *__restrict__ acc, double *f) {
   const size_t coff = 4 * (size_t)N;
+  unsigned long long fine[4], coarse[4];
+  unsigned long long *w = acc + 4 * (size_t)a;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    unsigned long long *w = acc + 4 * (size_t)a + c;
-    if (w[0] != 0ull || w[coff] != 0ull) {
-      fcd[4 * (size_t)a + c] += fix_value(w, coff);
-      w[0] = 0ull;
-      w[coff] = 0ull;
-    }
+    fine[c] = w[c];
+    coarse[c] = w[coff + c];
   }
+  bool any = false;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if (fine[c] == 0ull && coarse[c] == 0ull) continue;
+    const unsigned long long pair[2] = {fine[c], coarse[c]};
+    f[c] += fix_value(pair, 1);
+    w[c] = 0ull;
+    w[coff + c] = 0ull;
+    any = true;
+  }
+  return any;
+}
+
+// The end of the valence pass: the first three workgroups sum the energy rows,
+// the next clears the work list's counters, the others fold the terms of k
+// and h into fCdDelta.
+__global__ void __launch_bounds__(BT) k_va_fold(int n, int N, VaArgs A, double *__restrict__ sums) {
+  if (blockIdx.x < 3) {
+    sum_row<16>(n, A.part + blockIdx.x * A.stride, sums + blockIdx.x);
+    return;
+  }
+  if (blockIdx.x == 3) {
+    wl_clear(A.ctl);
+    return;
+  }
+  const int a = (blockIdx.x - 4) * BT + threadIdx.x;
+  if (a >= N) return;
+  double *fcd = A.fcd + 4 * (size_t)a;
+  double f[4] = {fcd[0], fcd[1], fcd[2], fcd[3]};
+  if (fold4(N, a, A.acc, f))
+#pragma unroll
+    for (int c = 0; c < 4; c++) fcd[c] = f[c];
 }
 
 // ---------------------------------------------------------------- torsions
@@ -1123,17 +1198,17 @@ __global__ void __launch_bounds__(BT) k_va_fold(int N, unsigned long long *__res
 //   k_to_count    four lanes per local atom: per bond slot the number of
 //                 quadruples the torsion body evaluates (the same filters),
 //                 a histogram of the counts;
-//   k_wl_scan     start of each count bucket in the list (largest first);
 //   k_to_scatter  one thread per local atom: its central bonds with work
-//                 into the list (the order inside a bucket is arbitrary and
-//                 changes no result);
+//                 into the list, largest counts first (the order inside a
+//                 bucket is arbitrary and changes no result);
 //   k_torsion     a group of lanes per listed central bond, one quadruple a
 //                 lane: the slot's Cdbopi and Cdbo written directly, j's row terms and energies into
 //                 the slot's row entry, Cdbo of j-i and k-l and the terms of
 //                 i, k, l into 64-bit fixed-point accumulators by integer
-//                 atomics (folded by k_va_fold / k_to_slot_fold);
-//   k_to_row      one thread per local atom: its slots' row entries summed
-//                 in slot order into its row and energies.
+//                 atomics;
+//   k_to_fold     one thread per atom: its slots' row entries summed in slot
+//                 order into its row and energies, and the accumulators
+//                 folded into its row and its slots' Cdbo.
 struct ToArgs {
   unsigned int *flags;   // DevStatus::flags
   const DevParams *P;
@@ -1247,9 +1322,9 @@ __global__ void __launch_bounds__(BT) k_to_count(int n, ToArgs A) {
 }
 
 __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
-  __shared__ int cnt[WL_NB], base[WL_NB];
+  __shared__ int cnt[WL_NB], base[WL_NB], start[WL_NB];
   for (int b = threadIdx.x; b < WL_NB; b += BT) cnt[b] = 0;
-  __syncthreads();
+  wl_starts(A.ctl, start);
   const int j = blockIdx.x * BT + threadIdx.x;
   const int b0 = j < n ? A.bidx[j] : 0, b1 = j < n ? A.bend[j] : 0;
   for (int pk = b0; pk < b1; ++pk) {   // rank in the workgroup's share of the bucket
@@ -1260,7 +1335,7 @@ __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
     }
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < WL_NB; b += BT) base[b] = cnt[b] ? atomicAdd(&A.ctl[WL_CUR + b], cnt[b]) : 0;
+  for (int b = threadIdx.x; b < WL_NB; b += BT) base[b] = cnt[b] ? start[b] + atomicAdd(&A.ctl[WL_CUR + b], cnt[b]) : 0;
   __syncthreads();
   for (int pk = b0; pk < b1; ++pk) {
     const int v = A.tc[pk];
@@ -1493,36 +1568,53 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
   }
 }
 
-// j's row and torsion/conjugation energies: its slots' entries in slot order.
-__global__ void __launch_bounds__(BT) k_to_row(int n, ToArgs A) {
-  const int j = blockIdx.x * BT + threadIdx.x;
-  if (j >= n) return;
+// The end of the torsion pass, one thread per atom: j's row and energies from
+// its slots' entries in slot order (local atoms), then the fixed-point terms
+// into its fCdDelta row and into Cdbo of its bond slots; accumulators are left
+// at zero.  The first workgroup clears the work list's counters.
+__global__ void __launch_bounds__(BT) k_to_fold(int n, int N, ToArgs A) {
+  if (blockIdx.x == 0) {
+    wl_clear(A.ctl);
+    return;
+  }
+  const int j = (blockIdx.x - 1) * BT + threadIdx.x;
+  if (j >= N) return;
   const int b0 = A.bidx[j], b1 = A.bend[j];
-  double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double *fcd = A.fcd + 4 * (size_t)j;
+  double f[4] = {fcd[0], fcd[1], fcd[2], fcd[3]};
+  bool any = false;
+  if (j < n) {
+    double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int pk = b0; pk < b1; ++pk) {
+      const double *rw = A.row + 6 * (size_t)pk;
+#pragma unroll
+      for (int q = 0; q < 6; q++) s[q] += rw[q];
+    }
+    if (A.atoms[j].type >= 0) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) f[q] += s[q];
+      any = true;
+    }
+    A.part[j] = s[4];
+    A.part[A.stride + j] = s[5];
+  }
+  any |= fold4(N, j, A.acc, f);
+  if (any)
+#pragma unroll
+    for (int c = 0; c < 4; c++) fcd[c] = f[c];
   for (int pk = b0; pk < b1; ++pk) {
-    const double *rw = A.row + 6 * (size_t)pk;
-#pragma unroll
-    for (int q = 0; q < 6; q++) s[q] += rw[q];
+    unsigned long long *w = A.sacc + pk;
+    if (w[0] != 0ull || w[A.scoff] != 0ull) {
+      A.Cdbo[pk] += fix_value(w, A.scoff);
+      w[0] = 0ull;
+      w[A.scoff] = 0ull;
+    }
   }
-  if (A.atoms[j].type >= 0) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) A.fcd[4 * (size_t)j + q] += s[q];
-  }
-  A.part[j] = s[4];
-  A.part[A.stride + j] = s[5];
 }
 
-// Cdbo of the bond slots += their fixed-point terms; accumulators left at zero.
-__global__ void __launch_bounds__(BT) k_to_slot_fold(int nslots, unsigned long long *__restrict__ sacc,
-                                                     double *__restrict__ Cdbo) {
-  const int s = blockIdx.x * BT + threadIdx.x;
-  if (s >= nslots) return;
-  unsigned long long *w = sacc + s;
-  if (w[0] != 0ull || w[nslots] != 0ull) {
-    Cdbo[s] += fix_value(w, (size_t)nslots);
-    w[0] = 0ull;
-    w[nslots] = 0ull;
-  }
+__global__ void __launch_bounds__(BT) k_to_sum(int n, const double *__restrict__ part, size_t stride,
+                                               double *__restrict__ sums) {
+  sum_row<16>(n, part + blockIdx.x * stride, sums + blockIdx.x);
 }
 
 }  // namespace
@@ -1564,9 +1656,7 @@ int swr_atom_energy_run(swr_system *S) {
   A.stride = stride;
   swr_kt_begin(S, KT_ATOM_ENERGY);
   if (n > 0) hipLaunchKernelGGL(k_atom_energy, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
-  hipLaunchKernelGGL(k_atom_energy_nbr, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A);
-  hipLaunchKernelGGL(k_sum_rows, dim3(5), dim3(1024), 0, S->stream, n, (const double *)S->be_part, stride,
-                     S->be_result);
+  hipLaunchKernelGGL(k_atom_energy_nbr, dim3(5 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A, S->be_result);
   swr_kt_end(S, KT_ATOM_ENERGY);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -1634,9 +1724,8 @@ int swr_hydrogen_bonds_run(swr_system *S) {
   constexpr int WPB = BT / SWR_WAVE;
   swr_kt_begin(S, KT_HBONDS);
   if (n > 0) hipLaunchKernelGGL(k_hb, dim3(div_up(n, WPB)), dim3(BT), 0, S->stream, n, A);
-  hipLaunchKernelGGL(k_hb_fold, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, S->hb_acc, S->fcd);
-  hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(1024), 0, S->stream, n, (const double *)S->hb_part, (size_t)0,
-                     S->hb_result);
+  hipLaunchKernelGGL(k_hb_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, S->hb_acc, S->fcd,
+                     (const double *)S->hb_part, S->hb_result);
   swr_kt_end(S, KT_HBONDS);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -1661,7 +1750,7 @@ int swr_valence_angles_run(swr_system *S) {
     return rc;
   if (S->cap_va_acc != old_acc)
     HIP_CHECK(hipMemsetAsync(S->va_acc, 0, sizeof(unsigned long long) * S->cap_va_acc, S->stream));
-  // the histogram starts at zero; k_wl_scan leaves it so
+  // the counters start at zero; k_va_fold leaves them so
   if (S->cap_va_ctl != old_ctl) HIP_CHECK(hipMemsetAsync(S->va_ctl, 0, sizeof(int) * S->cap_va_ctl, S->stream));
   S->va_stride = stride;
   VaArgs A;
@@ -1694,13 +1783,10 @@ int swr_valence_angles_run(swr_system *S) {
   swr_kt_begin(S, KT_VALENCE);
   if (n > 0) {
     hipLaunchKernelGGL(k_va_count, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
-    hipLaunchKernelGGL(k_wl_scan, dim3(1), dim3(WL_NB), 0, S->stream, S->va_ctl);
     hipLaunchKernelGGL(k_va_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_valence, dim3(std::min(WL_MAX_WAVES, n)), dim3(SWR_WAVE), 0, S->stream, A);
   }
-  hipLaunchKernelGGL(k_va_fold, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, S->va_acc, S->fcd);
-  hipLaunchKernelGGL(k_sum_rows, dim3(3), dim3(1024), 0, S->stream, n, (const double *)S->va_part, stride,
-                     S->va_result);
+  hipLaunchKernelGGL(k_va_fold, dim3(4 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A, S->va_result);
   swr_kt_end(S, KT_VALENCE);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -1730,7 +1816,7 @@ int swr_torsion_angles_run(swr_system *S) {
     HIP_CHECK(hipMemsetAsync(S->to_acc, 0, sizeof(unsigned long long) * S->cap_to_acc, S->stream));
   if (S->cap_to_sacc != old_sacc)
     HIP_CHECK(hipMemsetAsync(S->to_sacc, 0, sizeof(unsigned long long) * S->cap_to_sacc, S->stream));
-  // the histogram starts at zero; k_wl_scan leaves it so
+  // the counters start at zero; k_to_fold leaves them so
   if (S->cap_to_ctl != old_ctl) HIP_CHECK(hipMemsetAsync(S->to_ctl, 0, sizeof(int) * S->cap_to_ctl, S->stream));
   S->to_stride = stride;
   ToArgs A;
@@ -1760,17 +1846,12 @@ int swr_torsion_angles_run(swr_system *S) {
   swr_kt_begin(S, KT_TORSION);
   if (n > 0) {
     hipLaunchKernelGGL(k_to_count, dim3(div_up(n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
-    hipLaunchKernelGGL(k_wl_scan, dim3(1), dim3(WL_NB), 0, S->stream, S->to_ctl);
     hipLaunchKernelGGL(k_to_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     const int waves = (int)std::min<long long>(WL_MAX_WAVES, 8LL * n);
     hipLaunchKernelGGL(k_torsion, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
-    hipLaunchKernelGGL(k_to_row, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
   }
-  hipLaunchKernelGGL(k_va_fold, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, S->to_acc, S->fcd);
-  if (nslots > 0)
-    hipLaunchKernelGGL(k_to_slot_fold, dim3(div_up(nslots, BT)), dim3(BT), 0, S->stream, nslots, S->to_sacc, S->Cdbo);
-  hipLaunchKernelGGL(k_sum_rows, dim3(2), dim3(1024), 0, S->stream, n, (const double *)S->to_part, stride,
-                     S->to_result);
+  hipLaunchKernelGGL(k_to_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A);
+  hipLaunchKernelGGL(k_to_sum, dim3(2), dim3(BT), 0, S->stream, n, (const double *)S->to_part, stride, S->to_result);
   swr_kt_end(S, KT_TORSION);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
