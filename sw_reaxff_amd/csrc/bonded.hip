@@ -17,7 +17,7 @@
 // goes.  Here every kernel writes only entries of its own atom, so no
 // floating-point atomics are needed and results are the same on every run:
 //
-//   k_atom_energy     one thread per local atom: energies (per-atom rows,
+//   k_atom_energy     four lanes per local atom: energies (per-atom rows,
 //                     summed in a fixed order by sum_row), its own bond
 //                     slots' coefficients, its own CdDelta, and the two
 //                     per-atom factors (CEover4, CEunder4) its neighbours need;
@@ -25,7 +25,7 @@
 //                     the reference adds to atom j from each bonded local atom
 //                     i, read through the bond's reverse slot (sym_index), so
 //                     the values are those i's own slot holds;
-//   k_dbond_own       one thread per atom: its own chain-rule terms and the
+//   k_dbond_own       four lanes per atom: its own chain-rule terms and the
 //                     factor buf_c it passes to its neighbours;
 //   k_dbond_nbr       one thread per atom: sum over its bonds of the
 //                     neighbour's buf_c times the neighbour's dBOp toward it.
@@ -58,11 +58,16 @@ __device__ __forceinline__ bool owns_bond(const swr_atom_pack_t &a, const swr_at
 }
 
 // Terminal triple-bond stabilisation of bond (i, j) owned by i (:283-308):
-// returns whether it applies; dbo, dua, dub are the terms for Cdbo of i's
-// slot, CdDelta of i and CdDelta of j; e the energy.
+// the energy and, as pairs of factors, the terms for Cdbo of i's slot
+// (dbo_x dbo_y), CdDelta of i (x ua) and CdDelta of j (x ub).
+struct TripleBond {
+  double e, dbo_x, dbo_y, x, ua, ub;
+};
+
+// Whether it applies; t is only then set.
 __device__ __forceinline__ bool triple_bond(const DevParams *__restrict__ P, int ti, int tj, double BOij,
-                                            double dboc_i, double dboc_j, double Delta_i, double Delta_j, double &e,
-                                            double &dbo, double &dua, double &dub) {
+                                            double dboc_i, double dboc_j, double Delta_i, double Delta_j,
+                                            TripleBond &t) {
   const double mi = P->mass[ti], mj = P->mass[tj];
   if (!(BOij >= 1.00 && (P->gp37 == 2 || (mi == 12.0000 && mj == 15.9990) || (mj == 12.0000 && mi == 15.9990))))
     return false;
@@ -72,11 +77,26 @@ __device__ __forceinline__ bool triple_bond(const DevParams *__restrict__ P, int
   const double exphub1 = exp(-gp3 * (dboc_j - BOij));
   const double exphuov = exp(gp4 * (Delta_i + Delta_j));
   const double hulpov = 1.0 / (1.0 + 25.0 * exphuov);
-  e = gp10 * exphu * hulpov * (exphua1 + exphub1);
-  dbo = gp10 * exphu * hulpov * (exphua1 + exphub1) * (gp3 - 2.0 * gp7 * (BOij - 2.50));
-  dua = -gp10 * exphu * hulpov * (gp3 * exphua1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1));
-  dub = -gp10 * exphu * hulpov * (gp3 * exphub1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1));
+  t.e = gp10 * exphu * hulpov * (exphua1 + exphub1);
+  t.dbo_x = t.e;
+  t.dbo_y = gp3 - 2.0 * gp7 * (BOij - 2.50);
+  t.x = -gp10 * exphu * hulpov;
+  t.ua = gp3 * exphua1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1);
+  t.ub = gp3 * exphub1 + 25.0 * gp4 * exphuov * hulpov * (exphua1 + exphub1);
   return true;
+}
+
+// Lanes of an atom in the passes that spread its bonds, and the atoms of a
+// workgroup there.  Most atoms have two to four bonds.
+constexpr int BG = 4;
+constexpr int AE_ATOMS = BT / BG;
+
+// The largest v of a wave whose groups of G lanes each hold one value.
+template <int G>
+__device__ __forceinline__ int wave_max_groups(int v) {
+#pragma unroll
+  for (int o = G; o < SWR_WAVE; o <<= 1) v = max(v, __shfl_xor(v, o, SWR_WAVE));
+  return v;
 }
 
 // One workgroup's fixed-order sum of a per-atom energy row: 1024 running sums
@@ -133,140 +153,225 @@ struct BeArgs {
   size_t stride;
 };
 
+// What a workgroup's lanes hand from one part of k_atom_energy to the next.
+struct BeAtoms {
+  double ovun1[AE_ATOMS], ovun2[AE_ATOMS], cdd[AE_ATOMS], e_lp[AE_ATOMS];   // sums over the bonds
+  double over1[AE_ATOMS], over4[AE_ATOMS], under4[AE_ATOMS];                // CEover1, CEover4, CEunder4
+};
+
+// A chain of loads and transcendentals per bond and one per atom, at one to
+// two waves a SIMD: one thread per atom left it waiting (19 us on 21 atoms, 27
+// on 1,944, 464 on 200,000).  Here BG lanes take an atom's bonds, one lane
+// per atom the part between the bond loops, and sums over bonds are made in
+// bond order, with the operands of each term exchanged, so they round as one
+// thread's loop does.
 __global__ void __launch_bounds__(BT) k_atom_energy(int n, BeArgs A) {
-  const int i = blockIdx.x * BT + threadIdx.x;
-  if (i >= n) return;
+  __shared__ BeAtoms S;
   const DevParams *__restrict__ P = A.P;
-  const swr_atom_pack_t ai = A.atoms[i];
+  const int a = threadIdx.x / BG, sl = threadIdx.x % BG;
+  const int i = blockIdx.x * AE_ATOMS + a;
+  swr_atom_pack_t ai = {};
+  ai.type = -1;
+  if (i < n) ai = A.atoms[i];
   const int ti = ai.type;
-  double e_bond = 0, e_lp = 0, e_ov = 0, e_un = 0, e_pol = 0;
-  double ceo4 = 0, ceu4 = 0;
-  if (ti >= 0) {
-    const double q = ai.q;
-    e_pol = KCALpMOL_to_EV * (P->chi_e[ti] * q + (P->eta_e[ti] / 2.) * sqr(q));
-    const int b0 = A.bidx[i], b1 = A.bend[i];
-    // lone pair
-    const double p_lp2 = P->p_lp2[ti];
-    const double Dlp = A.Delta_lp[i];
-    const double expvd2 = exp(-75 * Dlp);
-    const double inv_expvd2 = 1. / (1. + expvd2);
-    const double p_ovun2 = P->p_ovun2[ti];
-    const double dfvl = P->mass[ti] > 21.0 ? 0.0 : 1.0;   // 1st-row elements only
-    int numbonds = 0;
-    double sum_ovun1 = 0, sum_ovun2 = 0;
-    for (int pj = b0; pj < b1; ++pj) {
-      numbonds++;
-      const int j = A.bonds[pj].nbr;
-      const int tj = A.atoms[j].type;
-      if (tj < 0) continue;
-      const DevBe &tw = P->be[ti * SWR_MAX_ELEM + tj];
-      sum_ovun1 += tw.p_ovun1 * tw.De_s * A.BO[pj];
-      sum_ovun2 += (A.Delta[j] - dfvl * A.Delta_lp_temp[j]) * (A.BOpi[2 * (size_t)pj] + A.BOpi[2 * (size_t)pj + 1]);
-    }
-    const double dElp = p_lp2 * inv_expvd2 + 75 * p_lp2 * Dlp * expvd2 * sqr(inv_expvd2);
-    const double CElp = dElp * A.dDelta_lp[i];
-    double cdd = A.fcd[4 * (size_t)i + 3];
-    const double Di = A.Delta[i];
-    if (P->p_lp3 > 0.001 && P->is_carbon[ti]) {
-      for (int pj = b0; pj < b1; ++pj) {
+  const bool live = ti >= 0;
+  const int b0 = live ? A.bidx[i] : 0, b1 = live ? A.bend[i] : 0;
+  const int nbmax = wave_max_groups<BG>(b1 - b0);
+  const double Di = live ? A.Delta[i] : 0.0;
+  const double dfvl = live && P->mass[ti] > 21.0 ? 0.0 : 1.0;   // 1st-row elements only
+  const bool carbon = live && P->p_lp3 > 0.001 && P->is_carbon[ti];
+  {
+    double sum_ovun1 = 0, sum_ovun2 = 0, e_lp = 0;
+    double cdd = live ? A.fcd[4 * (size_t)i + 3] : 0.0;
+    for (int m0 = 0; m0 < nbmax; m0 += BG) {
+      const int pj = b0 + m0 + sl;
+      double x1 = 0, y1 = 0, x2 = 0, y2 = 0;   // terms x1 y1 of sum_ovun1, x2 y2 of sum_ovun2
+      double xc = 0, yc = 0, xl = 0, yl = 0;   // carbon: of CdDelta and of e_lp
+      bool lp3 = false;
+      if (pj < b1) {
         const int j = A.bonds[pj].nbr;
         const int tj = A.atoms[j].type;
-        if (tj < 0 || !P->is_carbon[tj]) continue;
-        const double vov3 = A.BO[pj] - Di - 0.040 * pow(Di, 4.);
-        if (vov3 > 3.) {
-          e_lp += P->p_lp3 * sqr(vov3 - 3.0);
-          const double deahu2dbo = 2. * P->p_lp3 * (vov3 - 3.);
-          const double deahu2dsbo = 2. * P->p_lp3 * (vov3 - 3.) * (-1. - 0.16 * pow(Di, 3.));
-          A.Cdbo[pj] += deahu2dbo;
-          cdd += deahu2dsbo;
+        if (tj >= 0) {
+          const DevBe &tw = P->be[ti * SWR_MAX_ELEM + tj];
+          x1 = tw.p_ovun1 * tw.De_s;
+          y1 = A.BO[pj];
+          x2 = A.Delta[j] - dfvl * A.Delta_lp_temp[j];
+          y2 = A.BOpi[2 * (size_t)pj] + A.BOpi[2 * (size_t)pj + 1];
+          if (carbon && P->is_carbon[tj]) {
+            const double vov3 = y1 - Di - 0.040 * pow(Di, 4.);
+            if (vov3 > 3.) {
+              lp3 = true;
+              xl = P->p_lp3;
+              yl = sqr(vov3 - 3.0);
+              xc = 2. * P->p_lp3 * (vov3 - 3.);
+              yc = -1. - 0.16 * pow(Di, 3.);
+              A.Cdbo[pj] += xc;
+            }
+          }
+        }
+      }
+      const bool any_lp3 = __ballot(lp3) != 0ull;
+#pragma unroll
+      for (int q = 0; q < BG; q++) {
+        sum_ovun1 += __shfl(x1, q, BG) * __shfl(y1, q, BG);
+        sum_ovun2 += __shfl(x2, q, BG) * __shfl(y2, q, BG);
+      }
+      if (any_lp3) {
+#pragma unroll
+        for (int q = 0; q < BG; q++) {
+          const double c = __shfl(xc, q, BG), d = __shfl(yc, q, BG), e = __shfl(xl, q, BG), f = __shfl(yl, q, BG);
+          if (e != 0.0) {
+            e_lp += e * f;
+            cdd += c * d;
+          }
         }
       }
     }
-    // over-coordination
-    const double p_ovun4 = P->p_ovun4;
-    const double exp_ovun1 = P->p_ovun3 * exp(p_ovun4 * sum_ovun2);
-    const double inv_exp_ovun1 = 1.0 / (1 + exp_ovun1);
-    const double Dlpt = A.Delta_lp_temp[i];
-    const double Delta_lpcorr = Di - (dfvl * Dlpt) * inv_exp_ovun1;
-    const double exp_ovun2 = exp(p_ovun2 * Delta_lpcorr);
-    const double inv_exp_ovun2 = 1.0 / (1.0 + exp_ovun2);
-    const double DlpVi = 1.0 / (Delta_lpcorr + P->valency[ti] + 1e-8);
-    const double CEover1 = Delta_lpcorr * DlpVi * inv_exp_ovun2;
-    e_ov = sum_ovun1 * CEover1;
-    const double CEover2 =
-        sum_ovun1 * DlpVi * inv_exp_ovun2 * (1.0 - Delta_lpcorr * (DlpVi + p_ovun2 * exp_ovun2 * inv_exp_ovun2));
-    const double dDlp = A.dDelta_lp[i];
-    const double CEover3 = CEover2 * (1.0 - dfvl * dDlp * inv_exp_ovun1);
-    ceo4 = CEover2 * (dfvl * Dlpt) * p_ovun4 * exp_ovun1 * sqr(inv_exp_ovun1);
-    // under-coordination
-    const double p_ovun5 = P->p_ovun5[ti];
-    const double exp_ovun2n = 1.0 / exp_ovun2;
-    const double exp_ovun6 = exp(P->p_ovun6 * Delta_lpcorr);
-    const double exp_ovun8 = P->p_ovun7 * exp(P->p_ovun8 * sum_ovun2);
-    const double inv_exp_ovun2n = 1.0 / (1.0 + exp_ovun2n);
-    const double inv_exp_ovun8 = 1.0 / (1.0 + exp_ovun8);
-    cdd += CEover3;
-    const bool under = numbonds > 0 || P->enobonds;
-    double eu = 0.0;
-    if (under) eu = -p_ovun5 * (1.0 - exp_ovun6) * inv_exp_ovun2n * inv_exp_ovun8;
-    const double CEunder1 =
-        inv_exp_ovun2n * (p_ovun5 * P->p_ovun6 * exp_ovun6 * inv_exp_ovun8 + p_ovun2 * eu * exp_ovun2n);
-    const double CEunder2 = -eu * P->p_ovun8 * exp_ovun8 * inv_exp_ovun8;
-    const double CEunder3 = CEunder1 * (1.0 - dfvl * dDlp * inv_exp_ovun1);
-    ceu4 = CEunder1 * (dfvl * Dlpt) * p_ovun4 * exp_ovun1 * sqr(inv_exp_ovun1) + CEunder2;
-    if (under) {
-      e_un = eu;
-      cdd += CEunder3;
-      cdd += CElp;
-      e_lp += p_lp2 * Dlp * inv_expvd2;
+    if (sl == 0) {
+      S.ovun1[a] = sum_ovun1;
+      S.ovun2[a] = sum_ovun2;
+      S.e_lp[a] = e_lp;
+      S.cdd[a] = cdd;
     }
-    // per bond: over/under-coordination coefficients of this slot, bond
-    // energy and triple-bond stabilisation of the bonds this atom owns
-    for (int pj = b0; pj < b1; ++pj) {
+  }
+  __syncthreads();
+  // ---- one lane per atom: the terms of the whole atom
+  if (threadIdx.x < AE_ATOMS) {
+    const int t = threadIdx.x, i = blockIdx.x * AE_ATOMS + t;
+    double e_lp = 0, e_ov = 0, e_un = 0, e_pol = 0, ceo4 = 0, ceu4 = 0;
+    swr_atom_pack_t ai = {};
+    ai.type = -1;
+    if (i < n) ai = A.atoms[i];
+    const int ti = ai.type;
+    if (ti >= 0) {
+      const double q = ai.q;
+      e_pol = KCALpMOL_to_EV * (P->chi_e[ti] * q + (P->eta_e[ti] / 2.) * sqr(q));
+      const int numbonds = A.bend[i] - A.bidx[i];
+      const double sum_ovun1 = S.ovun1[t], sum_ovun2 = S.ovun2[t];
+      e_lp = S.e_lp[t];
+      double cdd = S.cdd[t];
+      // lone pair
+      const double p_lp2 = P->p_lp2[ti];
+      const double Dlp = A.Delta_lp[i];
+      const double expvd2 = exp(-75 * Dlp);
+      const double inv_expvd2 = 1. / (1. + expvd2);
+      const double p_ovun2 = P->p_ovun2[ti];
+      const double dfvl = P->mass[ti] > 21.0 ? 0.0 : 1.0;
+      const double dElp = p_lp2 * inv_expvd2 + 75 * p_lp2 * Dlp * expvd2 * sqr(inv_expvd2);
+      const double CElp = dElp * A.dDelta_lp[i];
+      const double Di = A.Delta[i];
+      // over-coordination
+      const double p_ovun4 = P->p_ovun4;
+      const double exp_ovun1 = P->p_ovun3 * exp(p_ovun4 * sum_ovun2);
+      const double inv_exp_ovun1 = 1.0 / (1 + exp_ovun1);
+      const double Dlpt = A.Delta_lp_temp[i];
+      const double Delta_lpcorr = Di - (dfvl * Dlpt) * inv_exp_ovun1;
+      const double exp_ovun2 = exp(p_ovun2 * Delta_lpcorr);
+      const double inv_exp_ovun2 = 1.0 / (1.0 + exp_ovun2);
+      const double DlpVi = 1.0 / (Delta_lpcorr + P->valency[ti] + 1e-8);
+      const double CEover1 = Delta_lpcorr * DlpVi * inv_exp_ovun2;
+      e_ov = sum_ovun1 * CEover1;
+      const double CEover2 =
+          sum_ovun1 * DlpVi * inv_exp_ovun2 * (1.0 - Delta_lpcorr * (DlpVi + p_ovun2 * exp_ovun2 * inv_exp_ovun2));
+      const double dDlp = A.dDelta_lp[i];
+      const double CEover3 = CEover2 * (1.0 - dfvl * dDlp * inv_exp_ovun1);
+      ceo4 = CEover2 * (dfvl * Dlpt) * p_ovun4 * exp_ovun1 * sqr(inv_exp_ovun1);
+      // under-coordination
+      const double p_ovun5 = P->p_ovun5[ti];
+      const double exp_ovun2n = 1.0 / exp_ovun2;
+      const double exp_ovun6 = exp(P->p_ovun6 * Delta_lpcorr);
+      const double exp_ovun8 = P->p_ovun7 * exp(P->p_ovun8 * sum_ovun2);
+      const double inv_exp_ovun2n = 1.0 / (1.0 + exp_ovun2n);
+      const double inv_exp_ovun8 = 1.0 / (1.0 + exp_ovun8);
+      cdd += CEover3;
+      const bool under = numbonds > 0 || P->enobonds;
+      double eu = 0.0;
+      if (under) eu = -p_ovun5 * (1.0 - exp_ovun6) * inv_exp_ovun2n * inv_exp_ovun8;
+      const double CEunder1 =
+          inv_exp_ovun2n * (p_ovun5 * P->p_ovun6 * exp_ovun6 * inv_exp_ovun8 + p_ovun2 * eu * exp_ovun2n);
+      const double CEunder2 = -eu * P->p_ovun8 * exp_ovun8 * inv_exp_ovun8;
+      const double CEunder3 = CEunder1 * (1.0 - dfvl * dDlp * inv_exp_ovun1);
+      ceu4 = CEunder1 * (dfvl * Dlpt) * p_ovun4 * exp_ovun1 * sqr(inv_exp_ovun1) + CEunder2;
+      if (under) {
+        e_un = eu;
+        cdd += CEunder3;
+        cdd += CElp;
+        e_lp += p_lp2 * Dlp * inv_expvd2;
+      }
+      S.over1[t] = CEover1;
+      S.over4[t] = ceo4;
+      S.under4[t] = ceu4;
+      S.cdd[t] = cdd;
+    }
+    if (i < n) {
+      A.ce[i] = ceo4;
+      A.ce[A.stride + i] = ceu4;
+      A.part[A.stride + i] = e_lp;
+      A.part[2 * A.stride + i] = e_ov;
+      A.part[3 * A.stride + i] = e_un;
+      A.part[4 * A.stride + i] = e_pol;
+    }
+  }
+  __syncthreads();
+  // ---- per bond: over/under-coordination coefficients of this slot, bond
+  // energy and triple-bond stabilisation of the bonds this atom owns
+  double e_bond = 0.0, cdd = S.cdd[a];
+  const double CEover1 = S.over1[a], ceo4 = S.over4[a], ceu4 = S.under4[a];
+  for (int m0 = 0; m0 < nbmax; m0 += BG) {
+    const int pj = b0 + m0 + sl;
+    double eb = 0, e3 = 0;                 // bond energy, triple-bond energy
+    TripleBond tb = {};
+    bool triple = false;
+    if (pj < b1) {
       const int j = A.bonds[pj].nbr;
       const swr_atom_pack_t aj = A.atoms[j];
       const int tj = aj.type;
-      if (tj < 0) continue;
-      const DevBe &tw = P->be[ti * SWR_MAX_ELEM + tj];
-      double cdbo = A.Cdbo[pj], cdbopi = A.Cdbopi[pj], cdbopi2 = A.Cdbopi2[pj];
-      cdbo += CEover1 * tw.p_ovun1 * tw.De_s;
-      const double dj = A.Delta[j] - dfvl * A.Delta_lp_temp[j];
-      const double ftmp = ceo4 * dj;
-      cdbopi += ftmp;
-      cdbopi2 += ftmp;
-      const double fu = ceu4 * dj;
-      cdbopi += fu;
-      cdbopi2 += fu;
-      if (owns_bond(ai, aj)) {
-        const double BO_s = A.bo[pj].BO_s;
-        const double pow_BOs_be2 = BO_s == 0.0 ? 0.0 : pow(BO_s, tw.p_be2);
-        const double exp_be12 = exp(tw.p_be1 * (1.0 - pow_BOs_be2));
-        const double CEbo = -tw.De_s * exp_be12 * (1.0 - tw.p_be1 * tw.p_be2 * pow_BOs_be2);
-        e_bond += -tw.De_s * BO_s * exp_be12 - tw.De_p * A.BOpi[2 * (size_t)pj] - tw.De_pp * A.BOpi[2 * (size_t)pj + 1];
-        cdbo += CEbo;
-        cdbopi -= (CEbo + tw.De_p);
-        cdbopi2 -= (CEbo + tw.De_pp);
-        double e3, dbo, dua, dub;
-        if (triple_bond(P, ti, tj, A.BO[pj], A.bo_dboc[2 * (size_t)i], A.bo_dboc[2 * (size_t)j], Di, A.Delta[j], e3,
-                        dbo, dua, dub)) {
-          e_bond += e3;
-          cdbo += dbo;
-          cdd += dua;
+      if (tj >= 0) {
+        const DevBe &tw = P->be[ti * SWR_MAX_ELEM + tj];
+        double cdbo = A.Cdbo[pj], cdbopi = A.Cdbopi[pj], cdbopi2 = A.Cdbopi2[pj];
+        cdbo += CEover1 * tw.p_ovun1 * tw.De_s;
+        const double dj = A.Delta[j] - dfvl * A.Delta_lp_temp[j];
+        const double ftmp = ceo4 * dj;
+        cdbopi += ftmp;
+        cdbopi2 += ftmp;
+        const double fu = ceu4 * dj;
+        cdbopi += fu;
+        cdbopi2 += fu;
+        if (owns_bond(ai, aj)) {
+          const double BO_s = A.bo[pj].BO_s;
+          const double pow_BOs_be2 = BO_s == 0.0 ? 0.0 : pow(BO_s, tw.p_be2);
+          const double exp_be12 = exp(tw.p_be1 * (1.0 - pow_BOs_be2));
+          const double CEbo = -tw.De_s * exp_be12 * (1.0 - tw.p_be1 * tw.p_be2 * pow_BOs_be2);
+          eb = -tw.De_s * BO_s * exp_be12 - tw.De_p * A.BOpi[2 * (size_t)pj] - tw.De_pp * A.BOpi[2 * (size_t)pj + 1];
+          cdbo += CEbo;
+          cdbopi -= (CEbo + tw.De_p);
+          cdbopi2 -= (CEbo + tw.De_pp);
+          triple = triple_bond(P, ti, tj, A.BO[pj], A.bo_dboc[2 * (size_t)i], A.bo_dboc[2 * (size_t)j], Di, A.Delta[j],
+                               tb);
+          if (triple) {
+            e3 = tb.e;
+            cdbo += tb.dbo_x * tb.dbo_y;
+          }
         }
+        A.Cdbo[pj] = cdbo;
+        A.Cdbopi[pj] = cdbopi;
+        A.Cdbopi2[pj] = cdbopi2;
       }
-      A.Cdbo[pj] = cdbo;
-      A.Cdbopi[pj] = cdbopi;
-      A.Cdbopi2[pj] = cdbopi2;
     }
-    A.fcd[4 * (size_t)i + 3] = cdd;
+    const bool any_triple = __ballot(triple) != 0ull;
+#pragma unroll
+    for (int q = 0; q < BG; q++) {
+      e_bond += __shfl(eb, q, BG);
+      if (any_triple) {
+        e_bond += __shfl(e3, q, BG);
+        cdd += __shfl(tb.x, q, BG) * __shfl(tb.ua, q, BG);
+      }
+    }
   }
-  A.ce[i] = ceo4;
-  A.ce[A.stride + i] = ceu4;
-  A.part[i] = e_bond;
-  A.part[A.stride + i] = e_lp;
-  A.part[2 * A.stride + i] = e_ov;
-  A.part[3 * A.stride + i] = e_un;
-  A.part[4 * A.stride + i] = e_pol;
+  if (sl == 0 && i < n) {
+    A.part[i] = e_bond;
+    if (live) A.fcd[4 * (size_t)i + 3] = cdd;
+  }
 }
 
 // CdDelta terms of atom j from each bonded local atom i (:270-279 and the
@@ -300,10 +405,10 @@ __global__ void __launch_bounds__(BT) k_atom_energy_nbr(int n, int N, BeArgs A, 
     cdd += A.ce[i] * ftmp2;
     cdd += A.ce[A.stride + i] * ftmp2;
     if (owns_bond(ai, aj)) {
-      double e3, dbo, dua, dub;
+      TripleBond t;
       if (triple_bond(P, ti, tj, A.BO[pj], A.bo_dboc[2 * (size_t)i], A.bo_dboc[2 * (size_t)j], A.Delta[i],
-                      A.Delta[j], e3, dbo, dua, dub))
-        cdd += dub;
+                      A.Delta[j], t))
+        cdd += t.x * t.ub;
     }
   }
   A.fcd[4 * (size_t)j + 3] = cdd;
@@ -319,18 +424,30 @@ struct DbArgs {
   double *bufc;                  // [N]
 };
 
-// The atom's own terms (the reference's forces on i, :532-548) and buf_c.
+// The atom's own terms (the reference's forces on i, :532-548) and buf_c: BG
+// lanes per atom over its bonds, whose terms are added in bond order (one
+// thread per atom waited bond by bond for four gathers: 16 us on 192 atoms
+// with their ghosts, 17 on 1,944, 340 on 200,000).
 __global__ void __launch_bounds__(BT) k_dbond_own(int N, DbArgs A) {
-  const int i = blockIdx.x * BT + threadIdx.x;
-  if (i >= N) return;
-  const int b0 = A.bidx[i], b1 = A.bend[i];
-  double buf_c = 0.0;
+  const int tid = blockIdx.x * BT + threadIdx.x;
+  const int i = tid / BG, sl = tid % BG;
+  const int b0 = i < N ? A.bidx[i] : 0, b1 = i < N ? A.bend[i] : 0;
+  const int nbmax = wave_max_groups<BG>(b1 - b0);
+  double buf_c = 0.0, f0 = 0.0, f1 = 0.0, f2 = 0.0;
+  double ds0 = 0.0, ds1 = 0.0, ds2 = 0.0, cd_i = 0.0;
   if (b0 < b1) {
-    const double ds0 = A.dDeltap_self[3 * (size_t)i], ds1 = A.dDeltap_self[3 * (size_t)i + 1],
-                 ds2 = A.dDeltap_self[3 * (size_t)i + 2];
-    const double cd_i = A.fcd[4 * (size_t)i + 3];
-    double f0 = A.fcd[4 * (size_t)i], f1 = A.fcd[4 * (size_t)i + 1], f2 = A.fcd[4 * (size_t)i + 2];
-    for (int pj = b0; pj < b1; ++pj) {
+    ds0 = A.dDeltap_self[3 * (size_t)i];
+    ds1 = A.dDeltap_self[3 * (size_t)i + 1];
+    ds2 = A.dDeltap_self[3 * (size_t)i + 2];
+    f0 = A.fcd[4 * (size_t)i];
+    f1 = A.fcd[4 * (size_t)i + 1];
+    f2 = A.fcd[4 * (size_t)i + 2];
+    cd_i = A.fcd[4 * (size_t)i + 3];
+  }
+  for (int m0 = 0; m0 < nbmax; m0 += BG) {
+    const int pj = b0 + m0 + sl;
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0, tc = 0.0;
+    if (pj < b1) {
       const swr_bond_t b = A.bonds[pj];
       const int j = b.nbr, sym = b.sym_index;
       const swr_bond_order_t &bo = A.bo[pj];
@@ -344,7 +461,7 @@ __global__ void __launch_bounds__(BT) k_dbond_own(int N, DbArgs A) {
       const double cdd = cd_i + A.fcd[4 * (size_t)j + 3];
       const double C1dDelta = bo.C1dbo * cdd, C2dDelta = bo.C2dbo * cdd;
       const double dbx = bo.dBOp[0], dby = bo.dBOp[1], dbz = bo.dBOp[2];
-      double t0 = C1dbo * dbx, t1 = C1dbo * dby, t2 = C1dbo * dbz;
+      t0 = C1dbo * dbx; t1 = C1dbo * dby; t2 = C1dbo * dbz;
       t0 += C2dbo * ds0; t1 += C2dbo * ds1; t2 += C2dbo * ds2;
       t0 += C1dDelta * dbx; t1 += C1dDelta * dby; t2 += C1dDelta * dbz;
       t0 += C2dDelta * ds0; t1 += C2dDelta * ds1; t2 += C2dDelta * ds2;
@@ -354,15 +471,24 @@ __global__ void __launch_bounds__(BT) k_dbond_own(int N, DbArgs A) {
       t0 += C1dbopi2 * bo.dln_BOp_pi2[0]; t1 += C1dbopi2 * bo.dln_BOp_pi2[1]; t2 += C1dbopi2 * bo.dln_BOp_pi2[2];
       t0 += C2dbopi2 * dbx; t1 += C2dbopi2 * dby; t2 += C2dbopi2 * dbz;
       t0 += C3dbopi2 * ds0; t1 += C3dbopi2 * ds1; t2 += C3dbopi2 * ds2;
-      f0 += t0; f1 += t1; f2 += t2;
-      buf_c += (-C2dbo - C2dDelta - C3dbopi - C3dbopi2);
+      tc = -C2dbo - C2dDelta - C3dbopi - C3dbopi2;
     }
-    A.fcd[4 * (size_t)i] = f0;
-    A.fcd[4 * (size_t)i + 1] = f1;
-    A.fcd[4 * (size_t)i + 2] = f2;
+#pragma unroll
+    for (int q = 0; q < BG; q++) {
+      const double g0 = __shfl(t0, q, BG), g1 = __shfl(t1, q, BG), g2 = __shfl(t2, q, BG), gc = __shfl(tc, q, BG);
+      if (b0 + m0 + q < b1) {
+        f0 += g0;
+        f1 += g1;
+        f2 += g2;
+        buf_c += gc;
+      }
+    }
   }
-  A.bufc[i] = buf_c;
+  if (i >= N) return;
+  if (sl == 3) A.bufc[i] = buf_c;
+  else if (b0 < b1) A.fcd[4 * (size_t)i + sl] = sl == 0 ? f0 : sl == 1 ? f1 : f2;
 }
+static_assert(BG == 4, "a lane of k_dbond_own writes one column");
 
 // The terms the reference adds to k from each bonded atom i (forces on k,
 // :580-584): buf_c of i times i's dBOp toward k.
@@ -824,52 +950,52 @@ struct VaArgs {
   int *ctl;                  // WL_CTL_INTS counters
 };
 
-// Angle evaluations of local centre j: the pairs of its bonds that pass the
-// body's filters, times their parameter sets.
-__device__ __forceinline__ int va_count(const VaArgs &A, int j) {
+// Angle evaluations of local centre j (slots [b0, b1), type tj >= 0) whose
+// first bond is in slot pk: the pairs that pass the body's filters, times
+// their parameter sets.
+__device__ __forceinline__ int va_count(const VaArgs &A, int tj, int pk, int b1) {
   const DevParams *__restrict__ P = A.P;
-  const int tj = A.atoms[j].type;
-  const int b0 = A.bidx[j], b1 = A.bend[j];
-  if (tj < 0 || b1 <= b0) return 0;
   const double thb_cut = P->thb_cut, thb_cutsq = P->thb_cutsq;
+  const double BO_jk = A.BO[pk];
+  const int k = A.bonds[pk].nbr;
+  const int tk = A.atoms[k].type;
+  if (!(BO_jk > thb_cut) || A.bend[k] <= A.bidx[k] || tk < 0) return 0;
   int c = 0;
-  for (int pk = b0; pk < b1; ++pk) {
-    const double BO_jk = A.BO[pk];
-    if (!(BO_jk > thb_cut)) continue;
-    const int k = A.bonds[pk].nbr;
-    if (A.bend[k] <= A.bidx[k]) continue;
-    const int tk = A.atoms[k].type;
-    for (int ph = pk + 1; ph < b1; ++ph) {
-      const double BO_hj = A.BO[ph];
-      if (!(BO_hj > thb_cut) || !(BO_jk * BO_hj > thb_cutsq)) continue;
-      const int th = A.atoms[A.bonds[ph].nbr].type;
-      if (tk < 0 || th < 0) continue;
-      c += P->thb_n[(tk * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + th];
-    }
+#pragma unroll 4
+  for (int ph = pk + 1; ph < b1; ++ph) {
+    const double BO_hj = A.BO[ph];
+    const int th = A.atoms[A.bonds[ph].nbr].type;
+    if (!(BO_hj > thb_cut) || !(BO_jk * BO_hj > thb_cutsq) || th < 0) continue;
+    c += P->thb_n[(tk * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + th];
   }
   return c;
 }
 
-// One thread per local atom: its count and the histogram; a centre without
+// BG lanes per local atom: its count and the histogram; a centre without
 // angles gets its zero energy rows here (the valence kernel skips it).
 __global__ void __launch_bounds__(BT) k_va_count(int n, VaArgs A) {
   __shared__ int hist[WL_NB];
   for (int b = threadIdx.x; b < WL_NB; b += BT) hist[b] = 0;
   __syncthreads();
-  const int j = blockIdx.x * BT + threadIdx.x;
+  const int tid = blockIdx.x * BT + threadIdx.x;
+  const int j = tid / BG, sl = tid % BG;
+  const int tj = j < n ? A.atoms[j].type : -1;
+  const int b0 = tj >= 0 ? A.bidx[j] : 0, b1 = tj >= 0 ? A.bend[j] : 0;
+  int c = 0;
+  for (int pk = b0 + sl; pk < b1; pk += BG) c += va_count(A, tj, pk, b1);
+#pragma unroll
+  for (int o = 1; o < BG; o <<= 1) c += __shfl_xor(c, o, SWR_WAVE);
   if (j < n) {
-    const int c = va_count(A, j);
-    A.cnt[j] = c;
-    if (c > 0) {
-      atomicAdd(&hist[wl_bucket(c)], 1);
-    } else {
-      A.part[j] = 0.0;
-      A.part[A.stride + j] = 0.0;
-      A.part[2 * A.stride + j] = 0.0;
+    if (sl == 0) {
+      A.cnt[j] = c;
+      if (c > 0) atomicAdd(&hist[wl_bucket(c)], 1);
+    } else if (c == 0) {
+      A.part[(sl - 1) * A.stride + j] = 0.0;
     }
   }
   wl_hist_flush(hist, A.ctl);
 }
+static_assert(BG == 4, "a lane of k_va_count clears one energy row");
 
 __global__ void __launch_bounds__(BT) k_va_scatter(int n, VaArgs A) {
   __shared__ int cnt[WL_NB], base[WL_NB], start[WL_NB];
@@ -1195,7 +1321,7 @@ __global__ void __launch_bounds__(BT) k_va_fold(int n, int N, VaArgs A, double *
 // so the tasks are listed with their exact quadruple counts and handed to
 // lanes in decreasing count (a wave's lanes then do about the same work):
 //
-//   k_to_count    four lanes per local atom: per bond slot the number of
+//   k_to_count    sixteen lanes per local atom: per bond slot the number of
 //                 quadruples the torsion body evaluates (the same filters),
 //                 a histogram of the counts;
 //   k_to_scatter  one thread per local atom: its central bonds with work
@@ -1270,52 +1396,58 @@ __device__ __forceinline__ bool to_pass(const ToArgs &A, int tj, int tk, double 
 }
 
 // Quadruples of the bond in slot pk of local atom j (type tj >= 0, slots
-// [b0, b1)); 0 when the bond is no central bond (its BO, the orig_id order, a
-// k without bonds or type) or makes no torsion.
+// [b0, b1)) whose k-l bond is every TO_PAIR_LANES-th from lane pl on; 0 when
+// the bond is no central bond (its BO, the orig_id order, a k without bonds
+// or type).
+constexpr int TO_SLOT_LANES = 4;   // lanes of an atom over its slots, in k_to_count,
+constexpr int TO_PAIR_LANES = 4;   // and of a slot over k's bonds
+constexpr int TO_CNT_LANES = TO_SLOT_LANES * TO_PAIR_LANES;
 __device__ __forceinline__ int to_count(const ToArgs &A, const swr_atom_pack_t &aj, int tj, int b0, int b1,
-                                        int pk, double thb_cut) {
+                                        int pk, int pl, double thb_cut) {
   const double BO_jk = A.BO[pk];
   if (!(BO_jk - thb_cut > 0.0)) return 0;
   const int k = A.bnbr[pk];
   const int k0 = A.bidx[k], k1 = A.bend[k];
-  if (k1 <= k0) return 0;
   const swr_atom_pack_t ak = A.atoms[k];
-  if (!owns_bond(aj, ak)) return 0;
-  const int tk = ak.type;
-  if (tk < 0) return 0;
   const int pj = A.bonds[pk].sym_index;
+  const int tk = ak.type;
+  if (k1 <= k0 || tk < 0 || !owns_bond(aj, ak)) return 0;
   int c = 0;
-  for (int ph = b0; ph < b1; ++ph) {
-    const double BO_ij = A.BO[ph];
-    if (ph == pk || !(BO_ij > thb_cut)) continue;
+  for (int pw = k0 + pl; pw < k1; pw += TO_PAIR_LANES) {
 #pragma unroll 4
-    for (int pw = k0; pw < k1; ++pw) c += to_pass(A, tj, tk, BO_jk, pk, pj, ph, pw, thb_cut) ? 1 : 0;
+    for (int ph = b0; ph < b1; ++ph) c += to_pass(A, tj, tk, BO_jk, pk, pj, ph, pw, thb_cut) ? 1 : 0;
   }
   return c;
 }
 
-constexpr int TO_CNT_LANES = 4;   // lanes per atom in k_to_count, each over every 4th slot
-
+// Sixteen lanes per local atom: with four (each a slot's whole count) the
+// pass waited pair by pair for its gathers, 23 us on 1,944 atoms and 543 on
+// 200,000.
 __global__ void __launch_bounds__(BT) k_to_count(int n, ToArgs A) {
   __shared__ int hist[WL_NB];
   for (int b = threadIdx.x; b < WL_NB; b += BT) hist[b] = 0;
   __syncthreads();
   const int tid = blockIdx.x * BT + threadIdx.x;
   const int j = tid / TO_CNT_LANES;
-  if (j < n) {
-    const swr_atom_pack_t aj = A.atoms[j];
-    const int b0 = A.bidx[j], b1 = A.bend[j];
-    const double thb_cut = A.P->thb_cut;
-    for (int pk = b0 + tid % TO_CNT_LANES; pk < b1; pk += TO_CNT_LANES) {
-      const int c = aj.type >= 0 ? to_count(A, aj, aj.type, b0, b1, pk, thb_cut) : 0;
-      A.tc[pk] = c;
-      if (c > 0) {
-        atomicAdd(&hist[wl_bucket(c)], 1);
-      } else {
-        double *rw = A.row + 6 * (size_t)pk;
+  const int pl = tid % TO_PAIR_LANES;
+  swr_atom_pack_t aj = {};
+  aj.type = -1;
+  if (j < n) aj = A.atoms[j];
+  const int b0 = j < n ? A.bidx[j] : 0, b1 = j < n ? A.bend[j] : 0;
+  const int nbmax = wave_max_groups<TO_CNT_LANES>(b1 - b0);
+  const double thb_cut = A.P->thb_cut;
+  for (int m0 = 0; m0 < nbmax; m0 += TO_SLOT_LANES) {
+    const int pk = b0 + m0 + (tid % TO_CNT_LANES) / TO_PAIR_LANES;
+    int c = pk < b1 && aj.type >= 0 ? to_count(A, aj, aj.type, b0, b1, pk, pl, thb_cut) : 0;
 #pragma unroll
-        for (int q = 0; q < 6; q++) rw[q] = 0.0;
-      }
+    for (int o = 1; o < TO_PAIR_LANES; o <<= 1) c += __shfl_xor(c, o, SWR_WAVE);
+    if (pk >= b1) continue;
+    if (c == 0) {
+      for (int q = pl; q < 6; q += TO_PAIR_LANES) A.row[6 * (size_t)pk + q] = 0.0;
+    }
+    if (pl == 0) {
+      A.tc[pk] = c;
+      if (c > 0) atomicAdd(&hist[wl_bucket(c)], 1);
     }
   }
   wl_hist_flush(hist, A.ctl);
@@ -1655,7 +1787,7 @@ int swr_atom_energy_run(swr_system *S) {
   A.part = S->be_part;
   A.stride = stride;
   swr_kt_begin(S, KT_ATOM_ENERGY);
-  if (n > 0) hipLaunchKernelGGL(k_atom_energy, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
+  if (n > 0) hipLaunchKernelGGL(k_atom_energy, dim3(div_up(n, AE_ATOMS)), dim3(BT), 0, S->stream, n, A);
   hipLaunchKernelGGL(k_atom_energy_nbr, dim3(5 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A, S->be_result);
   swr_kt_end(S, KT_ATOM_ENERGY);
   HIP_CHECK(hipGetLastError());
@@ -1682,7 +1814,7 @@ int swr_dbond_forces_run(swr_system *S) {
   A.fcd = S->fcd;
   A.bufc = S->be_bufc;
   swr_kt_begin(S, KT_DBOND);
-  hipLaunchKernelGGL(k_dbond_own, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, A);
+  hipLaunchKernelGGL(k_dbond_own, dim3(div_up((long long)N * BG, BT)), dim3(BT), 0, S->stream, N, A);
   hipLaunchKernelGGL(k_dbond_nbr, dim3(div_up(N, BT)), dim3(BT), 0, S->stream, N, A);
   swr_kt_end(S, KT_DBOND);
   HIP_CHECK(hipGetLastError());
@@ -1782,7 +1914,7 @@ int swr_valence_angles_run(swr_system *S) {
   A.ctl = S->va_ctl;
   swr_kt_begin(S, KT_VALENCE);
   if (n > 0) {
-    hipLaunchKernelGGL(k_va_count, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
+    hipLaunchKernelGGL(k_va_count, dim3(div_up((long long)n * BG, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_va_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_valence, dim3(std::min(WL_MAX_WAVES, n)), dim3(SWR_WAVE), 0, S->stream, A);
   }
@@ -1845,7 +1977,7 @@ int swr_torsion_angles_run(swr_system *S) {
   A.row = S->to_row;
   swr_kt_begin(S, KT_TORSION);
   if (n > 0) {
-    hipLaunchKernelGGL(k_to_count, dim3(div_up(n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
+    hipLaunchKernelGGL(k_to_count, dim3(div_up((long long)n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_to_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     const int waves = (int)std::min<long long>(WL_MAX_WAVES, 8LL * n);
     hipLaunchKernelGGL(k_torsion, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
