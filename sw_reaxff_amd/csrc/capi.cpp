@@ -343,7 +343,7 @@ int swr_create(const char *ffield_path, int ntypes, const char *const *elements,
     return SWR_ERR_HIP;
   }
   int rc;
-  if ((rc = swr_alloc(&S->dp, 1)) || (rc = swr_alloc(&S->status, 1)) || (rc = swr_alloc(&S->counters, 4))) {
+  if ((rc = swr_alloc(&S->dp, 1)) || (rc = swr_alloc(&S->status, 1)) || (rc = swr_alloc(&S->next_totals, 2))) {
     swr_destroy(S);
     return rc;
   }
@@ -377,7 +377,7 @@ int swr_create(const char *ffield_path, int ntypes, const char *const *elements,
   // the system's stream does not wait for the null stream: everything goes on it
   if (hipMemcpyAsync(S->dp, &S->hp, sizeof(DevParams), hipMemcpyHostToDevice, S->stream) != hipSuccess ||
       hipMemsetAsync(S->status, 0, sizeof(DevStatus), S->stream) != hipSuccess ||
-      hipMemsetAsync(S->counters, 0, 4 * sizeof(unsigned int), S->stream) != hipSuccess ||
+      hipMemsetAsync(S->next_totals, 0, 2 * sizeof(int), S->stream) != hipSuccess ||
       hipStreamSynchronize(S->stream) != hipSuccess) {
     swr_set_error_msg("HIP init: parameter upload failed");
     swr_destroy(S);
@@ -400,7 +400,7 @@ int swr_destroy(swr_system *S) {
                   S->hb_result, S->hb_acc, S->va_part, S->va_result, S->va_acc, S->va_cnt, S->va_order, S->va_ctl, S->to_part, S->to_result, S->to_acc,
                   S->to_sacc, S->to_tc, S->to_task, S->to_ctl, S->to_row, S->f, S->gcsr_cnt, S->gcsr_start, S->gcsr_list,
                   S->bond_mark2, S->counts, S->ws, S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32,
-                  S->Hdia_inv, S->b_s, S->st, S->s_hist, S->t_hist, S->cgv, S->cgs, S->partials, S->counters,
+                  S->Hdia_inv, S->b_s, S->st, S->s_hist, S->t_hist, S->cgv, S->cgs, S->partials, S->next_totals,
                   S->status, S->scan_tmp, S->tmp_i, S->mixw, S->cand, S->cand_count, S->row_sys, S->tile_beg,
                   S->tile_sys, S->sys_tile, S->sblk_beg, S->sys_sblk, S->sys_iters, S->done_count, S->qsum,
                   S->mark_chg, S->mark_up};

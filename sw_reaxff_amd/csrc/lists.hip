@@ -46,33 +46,100 @@ __global__ void k_pack(const int *__restrict__ tag, const int *__restrict__ type
   out[i] = a;
 }
 
-// Reset_Atoms flags / Reset_Neighbor_Lists inputs.
-__global__ void k_reset_flags(const swr_atom_pack_t *__restrict__ P_atoms, const DevParams *__restrict__ P, int n,
-                              int N, double hbond_cut, const int *__restrict__ num_hbonds, int *__restrict__ hflag,
-                              int *__restrict__ hcap) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  int t = P_atoms[i].type;
-  int h = (i < n && hbond_cut > 0 && t >= 0 && P->p_hbond[t] == 1) ? 1 : 0;
-  hflag[i] = h;
-  hcap[i] = h ? num_hbonds[i] : 0;
+// Reset_Atoms / Reset_Neighbor_Lists in two launches: k_reset_sums adds up
+// each tile of RS_TILE atoms (local H atoms, their hydrogen-bond capacities,
+// bond capacities) and zeroes fCdDelta; k_reset_apply adds the tiles before
+// its own and scans its tile.  (Flags, a three-launch scan of the three arrays,
+// their use and a fill were six launches of ~4 us each with their gaps, more
+// than half of it waiting between them, on all but the largest systems.)
+constexpr int RS_T = 256, RS_ITEMS = 4, RS_TILE = RS_T * RS_ITEMS;
+
+struct ResetArgs {
+  const swr_atom_pack_t *atoms;
+  const DevParams *P;
+  int n, N;
+  double hbond_cut;
+  const int *num_hbonds, *num_bonds;
+  int *sums;   // [tiles][3]
+};
+
+// (H atoms, hydrogen-bond capacity, bond capacity) of atom i.
+__device__ __forceinline__ int3 reset_item(const ResetArgs &A, int i) {
+  if (i >= A.N) return make_int3(0, 0, 0);
+  const int t = A.atoms[i].type;
+  const int h = (i < A.n && A.hbond_cut > 0 && t >= 0 && A.P->p_hbond[t] == 1) ? 1 : 0;
+  return make_int3(h, h ? A.num_hbonds[i] : 0, A.num_bonds[i]);
 }
 
-__global__ void k_reset_apply(int n, int N, const int *__restrict__ hflag, const int *__restrict__ hpos,
-                              const int *__restrict__ hstart, int *__restrict__ Hindex,
-                              const int *__restrict__ bond_index, int *__restrict__ bond_end,
-                              int *__restrict__ hbond_index, int *__restrict__ hbond_end, DevStatus *st,
-                              int bond_cap, int hbond_cap) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) {
-    if (st->total_bonds > bond_cap) atomicOr(&st->flags, SWR_F_BOND_TOTAL);
-    if (st->total_hbonds > hbond_cap) atomicOr(&st->flags, SWR_F_HBOND_TOTAL);
+__device__ __forceinline__ int3 add3(int3 a, int3 b) { return make_int3(a.x + b.x, a.y + b.y, a.z + b.z); }
+
+// The workgroup's sum of v; excl: the sum of the threads before this one.
+__device__ __forceinline__ int3 reset_block_scan(int3 v, int3 *lds, int3 *excl) {
+  const int w = wave_in_block(), l = lane_id();
+  const int3 inc = make_int3(wave_incl_scan(v.x), wave_incl_scan(v.y), wave_incl_scan(v.z));
+  __syncthreads();
+  if (l == SWR_WAVE - 1) lds[w] = inc;
+  __syncthreads();
+  int3 off = make_int3(0, 0, 0), tot = off;
+  for (int k = 0; k < RS_T / SWR_WAVE; k++) {
+    if (k < w) off = add3(off, lds[k]);
+    tot = add3(tot, lds[k]);
   }
-  if (i >= N) return;
-  bond_end[i] = bond_index[i];
-  int H = hflag[i] ? hpos[i] : -1;
-  Hindex[i] = H;
-  if (H >= 0) hbond_index[H] = hbond_end[H] = hstart[i];
+  *excl = make_int3(off.x + inc.x - v.x, off.y + inc.y - v.y, off.z + inc.z - v.z);
+  return tot;
+}
+
+__global__ void __launch_bounds__(RS_T) k_reset_sums(ResetArgs A, double *__restrict__ fcd) {
+  __shared__ int3 lds[RS_T / SWR_WAVE];
+  const int base = blockIdx.x * RS_TILE;
+  int3 v = make_int3(0, 0, 0), ex;
+#pragma unroll
+  for (int k = 0; k < RS_ITEMS; k++) v = add3(v, reset_item(A, base + k * RS_T + (int)threadIdx.x));
+  const int3 tot = reset_block_scan(v, lds, &ex);
+  if (threadIdx.x < 3) A.sums[3 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? tot.x : threadIdx.x == 1 ? tot.y : tot.z;
+  double2 *f = reinterpret_cast<double2 *>(fcd);
+#pragma unroll
+  for (int k = 0; k < 2 * RS_ITEMS; k++) {
+    const long long e = 2LL * base + k * RS_T + threadIdx.x;
+    if (e < 2LL * A.N) f[e] = make_double2(0.0, 0.0);
+  }
+}
+
+__global__ void __launch_bounds__(RS_T)
+k_reset_apply(ResetArgs A, int *__restrict__ Hindex, int *__restrict__ bond_index, int *__restrict__ bond_end,
+              int *__restrict__ hbond_index, int *__restrict__ hbond_end, DevStatus *st, int bond_cap,
+              int hbond_cap) {
+  __shared__ int3 lds[RS_T / SWR_WAVE];
+  int3 before = make_int3(0, 0, 0), ex;
+  for (int k = threadIdx.x; k < (int)blockIdx.x; k += RS_T)
+    before = add3(before, make_int3(A.sums[3 * k], A.sums[3 * k + 1], A.sums[3 * k + 2]));
+  const int3 off = reset_block_scan(before, lds, &ex);
+  const int i0 = blockIdx.x * RS_TILE + threadIdx.x * RS_ITEMS;
+  int3 v[RS_ITEMS], sum = make_int3(0, 0, 0);
+#pragma unroll
+  for (int k = 0; k < RS_ITEMS; k++) {
+    v[k] = reset_item(A, i0 + k);
+    sum = add3(sum, v[k]);
+  }
+  const int3 tot = reset_block_scan(sum, lds, &ex);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    const int3 all = add3(off, tot);
+    st->numH = all.x;
+    st->total_hbonds = all.y;
+    st->total_bonds = all.z;
+    if (all.z > bond_cap) atomicOr(&st->flags, SWR_F_BOND_TOTAL);
+    if (all.y > hbond_cap) atomicOr(&st->flags, SWR_F_HBOND_TOTAL);
+  }
+  int3 at = add3(off, ex);
+#pragma unroll
+  for (int k = 0; k < RS_ITEMS; k++) {
+    if (i0 + k < A.N) {
+      bond_index[i0 + k] = bond_end[i0 + k] = at.z;
+      Hindex[i0 + k] = v[k].x ? at.x : -1;
+      if (v[k].x) hbond_index[at.x] = hbond_end[at.x] = at.y;
+    }
+    at = add3(at, v[k]);
+  }
 }
 
 // Per atom, the far-list slots of its bond candidates (d <= bond_cut and
@@ -722,7 +789,7 @@ k_bonds(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__
 __global__ void k_validate(int n, int N, const int *__restrict__ bond_index, const int *__restrict__ bond_count,
                            int *__restrict__ num_bonds, const int *__restrict__ Hindex,
                            const int *__restrict__ hb_count, int *__restrict__ num_hbonds, double saferzone,
-                           int bond_total, DevStatus *st) {
+                           int bond_total, DevStatus *st, int *__restrict__ next_totals) {
   __shared__ int sb[8], sh[8];
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   int tb = 0, th = 0;
@@ -750,9 +817,28 @@ __global__ void k_validate(int n, int N, const int *__restrict__ bond_index, con
   if (threadIdx.x == 0) {
     int a = 0, b = 0;
     for (int w = 0; w < (int)blockDim.x / SWR_WAVE; w++) { a += sb[w]; b += sh[w]; }
-    atomicAdd(&st->next_total_bonds, a);
-    atomicAdd(&st->next_total_hbonds, b);
+    atomicAdd(&next_totals[0], a);
+    atomicAdd(&next_totals[1], b);
   }
+}
+
+// The totals into the status block, left at zero for the next pass, and the
+// block into the host's copy (one launch instead of a fill and a copy).
+static_assert(sizeof(DevStatus) / 4 <= SWR_WAVE && sizeof(DevStatus) % 4 == 0, "a lane of k_validate_end takes one word");
+__global__ void __launch_bounds__(SWR_WAVE) k_validate_end(DevStatus *st, int *__restrict__ next_totals, int *host) {
+  constexpr int W = sizeof(DevStatus) / 4, AT = offsetof(DevStatus, next_total_bonds) / 4;
+  static_assert(offsetof(DevStatus, next_total_hbonds) == 4 * (AT + 1), "the two totals are neighbours");
+  const int l = threadIdx.x;
+  if (l >= W) return;
+  int *words = reinterpret_cast<int *>(st);
+  int v = words[l];
+  if (l == AT || l == AT + 1) {
+    v = next_totals[l - AT];
+    next_totals[l - AT] = 0;
+    words[l] = v;
+  }
+  host[l] = v;
+  __threadfence_system();
 }
 
 // sort_bonds_C (reaxc_forces_sw64.c:932-971): one in-order pass
@@ -986,24 +1072,16 @@ int swr_lists_alloc_bonds(swr_system *S, int bond_cap, int hbond_cap);
 
 int swr_lists_reset(swr_system *S) {
   const int n = S->n, N = S->N;
-  int rc = swr_ensure_tmp(S, sizeof(int) * (4 * (size_t)N + 8));
+  const int ntiles = div_up(N, RS_TILE);
+  int rc = swr_ensure_tmp(S, sizeof(int) * 3 * (size_t)ntiles);
   if (rc) return rc;
-  int *hflag = S->tmp_i, *hcap = hflag + N + 1, *hpos = hcap + N + 1, *hstart = hpos + N + 1;
+  const ResetArgs A = {S->packed, S->dp, n, N, S->ctl.hbond_cut, S->num_hbonds, S->num_bonds, S->tmp_i};
   swr_kt_begin(S, KT_RESET);
   // Reset_Workspace (reaxc_reset_tools_sunway.cpp:122-131) zeroes fCdDelta,
   // which the non-bonded pass accumulates into
-  HIP_CHECK(hipMemsetAsync(S->fcd, 0, sizeof(double) * 4 * (size_t)N, S->stream));
-  hipLaunchKernelGGL(k_reset_flags, dim3(div_up(N, 256)), dim3(256), 0, S->stream, S->packed, S->dp, n, N,
-                     S->ctl.hbond_cut, S->num_hbonds, hflag, hcap);
-  {  // the three prefix sums of Reset in one set of launches
-    const int *in[3] = {hflag, hcap, S->num_bonds};
-    int *out[3] = {hpos, hstart, S->bond_index};
-    int *tot[3] = {&S->status->numH, &S->status->total_hbonds, &S->status->total_bonds};
-    if ((rc = swr_scan3_i32(S, in, out, N, tot))) return rc;
-  }
-  hipLaunchKernelGGL(k_reset_apply, dim3(div_up(N, 256)), dim3(256), 0, S->stream, n, N, hflag, hpos, hstart,
-                     S->Hindex, S->bond_index, S->bond_end, S->hbond_index, S->hbond_end, S->status, S->bond_cap,
-                     S->hbond_cap);
+  hipLaunchKernelGGL(k_reset_sums, dim3(ntiles), dim3(RS_T), 0, S->stream, A, S->fcd);
+  hipLaunchKernelGGL(k_reset_apply, dim3(ntiles), dim3(RS_T), 0, S->stream, A, S->Hindex, S->bond_index, S->bond_end,
+                     S->hbond_index, S->hbond_end, S->status, S->bond_cap, S->hbond_cap);
   swr_kt_end(S, KT_RESET);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -1147,12 +1225,12 @@ int swr_lists_estimate(swr_system *S) {
 int swr_lists_validate(swr_system *S) {
   const int n = S->n, N = S->N;
   swr_kt_begin(S, KT_VALIDATE);
-  HIP_CHECK(hipMemsetAsync(&S->status->next_total_bonds, 0, 2 * sizeof(int), S->stream));
   hipLaunchKernelGGL(k_validate, dim3(div_up(N, 256)), dim3(256), 0, S->stream, n, N, S->bond_index, S->counts,
                      S->num_bonds, S->Hindex, S->counts + S->Ncap, S->num_hbonds, S->ctl.saferzone, S->bond_cap,
-                     S->status);
+                     S->status, S->next_totals);
   // the capacity totals travel back with the next sync (next step's Reset)
-  HIP_CHECK(hipMemcpyAsync(S->status_host, S->status, sizeof(DevStatus), hipMemcpyDeviceToHost, S->stream));
+  hipLaunchKernelGGL(k_validate_end, dim3(1), dim3(SWR_WAVE), 0, S->stream, S->status, S->next_totals,
+                     (int *)S->status_host);
   S->status_copy_queued = true;
   S->next_totals_known = false;
   swr_kt_end(S, KT_VALIDATE);

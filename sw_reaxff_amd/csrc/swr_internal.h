@@ -341,7 +341,7 @@ struct swr_system {
                                    // (or the small FP64 solve's second buffer)
   double *partials = nullptr;      // per-workgroup partial dots, [CG_PART_ROWS][cg_pstride]
   int cg_pstride = 0;
-  unsigned int *counters = nullptr;
+  int *next_totals = nullptr;      // Validate_Lists' sums of the new capacities, until they are in status
 
   // ---- batch of independent systems (one unless swr_set_batch)
   std::vector<int> sys_row;        // nsys + 1 local-row offsets (host)
@@ -418,7 +418,6 @@ enum { CGV_R = 0, CGV_U, CGV_W, CGV_Z, CGV_SS, CGV_V, CGV_P, CGV_D0, CGV_D1, CGV
 // ---- helpers implemented in the .hip files
 int swr_scan_i32_to_i64(swr_system *S, const int *in, long long *out, int n, long long *total_host);
 int swr_scan_i32(swr_system *S, const int *in, int *out, int n, int *total_dev);
-int swr_scan3_i32(swr_system *S, const int *const in[3], int *const out[3], int n, int *const total[3]);
 int swr_ensure_tmp(swr_system *S, size_t bytes);
 
 // Stage implementations (nbr.hip, lists.hip, bo.hip, qeq.hip, qeq_mixed.hip).

@@ -228,3 +228,41 @@ def test_gpu_charges_queued_behind_the_solve(gpu_lib, ffield, m, mixed):
     assert max(iters[0][0]) > (3 if mixed else 16) and max(iters[-1][0]) < max(iters[0][0])
     if mixed:
         assert iters[0][1] > 1 and iters[-1][1] == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 1023, 1024, 1025, 16384, 16385])
+def test_gpu_reset_and_scans_at_tile_edges(gpu_lib, ffield, n):
+    """Reset's positions and the Verlet offsets are the exclusive sums of their
+    counts, around one tile of 1,024 atoms and around the 16 tiles that a scan
+    takes in one launch; ragged capacities."""
+    from sw_reaxff_amd import _lib
+    s = systems.water_box(5462, seed=2)
+    x, t, tag = s.x[:n], s.type[:n], s.tag[:n]
+    rng = np.random.default_rng(n)
+    nb, nh = (rng.integers(25, 70, size=n).astype(np.int32) for _ in range(2))
+    h = _lib.System(ffield, s.elements)
+    h.set_atoms(n, x, t, tag, owner=np.arange(n))
+    h.build_neighbors(9.0)
+    off = h.get("verlet_offsets")
+    assert off.size == n + 1 and off[0] == 0 and h.get("verlet_list").size == off[-1]
+    rows, counts = [], []
+    for i in {0, n // 2, n - 1}:
+        d = ((x - x[i]) ** 2).sum(1)
+        rows.append(i)
+        counts.append(int((d <= 9.0 ** 2).sum()) - 1)
+    assert [int(off[i + 1] - off[i]) for i in rows] == counts
+    h.set_capacities(nb, nh)
+    for _ in range(2):   # the second one finds the lists sized
+        h.call("write_reax_atoms_and_pack")
+        h.call("reset")
+    h.sync()
+    is_h = t == 1 + s.elements.index("H")
+    excl = lambda c: np.concatenate([[0], np.cumsum(c)])
+    assert h.scalar("numH") == is_h.sum() and h.scalar("total_bonds") == nb.sum()
+    assert np.array_equal(h.get("bond_index")[:n], excl(nb)[:-1])
+    assert np.array_equal(h.get("bond_end")[:n], excl(nb)[:-1])
+    assert np.array_equal(h.get("Hindex")[:n], np.where(is_h, excl(is_h)[:-1], -1))
+    assert np.array_equal(h.get("hbond_index"), excl(nh[is_h])[:-1])
+    assert np.array_equal(h.get("hbond_end"), excl(nh[is_h])[:-1])
+    assert not h.get("fCdDelta")[:n].any()
