@@ -383,6 +383,16 @@ __device__ __forceinline__ bool cg_multiplies(int PH, const CgScalars *__restric
   return (c[0].active_a | c[1].active_a) != 0;   // (both requested at once)
 }
 
+// The panel of this workgroup: every product walks the panels the other way
+// round than the one before it.  Read in one direction each time, an H larger
+// than the 256 MB memory-side cache finds nothing of itself there; turned
+// round, a product starts with what the last one read last.
+template <int PH>
+__device__ __forceinline__ int spmv_panel(int par_in) {
+  const bool back = PH == PH_K ? par_in != 0 : PH != PH_S2;
+  return back ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
+}
+
 // q = eta d + H d (sparse_matvec_C_para, fix_qeq_reax_sw64.c:424-466) of the
 // vector phase PH multiplies: x (PH_S1), d0 (PH_S2), d1 (PH_S3) or the
 // current d (PH_K).  One workgroup per SpMV panel (shape SH).
@@ -394,7 +404,7 @@ k_cg_spmv(int n, const DevParams *__restrict__ P, const int *__restrict__ type, 
   typedef typename Vec2<T>::type T2;
   constexpr int NT = SpmvShape<SH>::NT, G = SpmvShape<SH>::G, U = SpmvShape<SH>::U;
   __shared__ T2 xl[SWR_PANEL_MAXC];
-  const int p = blockIdx.x;
+  const int p = spmv_panel<PH>(par_in);
   // skipped once neither solve of the panel's system needs a product (a
   // panel holds rows of one system)
   if (!BATCH && !cg_multiplies(PH, cgs)) return;
