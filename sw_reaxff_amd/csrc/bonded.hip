@@ -91,6 +91,14 @@ __device__ __forceinline__ bool triple_bond(const DevParams *__restrict__ P, int
 constexpr int BG = 4;
 constexpr int AE_ATOMS = BT / BG;
 
+// Butterfly sum of a group of G lanes, on all of them.
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, SWR_WAVE);
+  return v;
+}
+
 // The largest v of a wave whose groups of G lanes each hold one value.
 template <int G>
 __device__ __forceinline__ int wave_max_groups(int v) {
@@ -517,12 +525,12 @@ __global__ void __launch_bounds__(BT) k_dbond_nbr(int N, DbArgs A) {
 // (p_hbond 2) with BO >= 0.01, and a hydrogen-bond partner k of j with
 // orig_id(k) != orig_id(i) and r0_hb(i, j, k) > 0.  Its energy and CEhb1
 // (into Cdbo of j's slot) and the angle/distance terms into fCdDelta of i,
-// j and k.  k_hb computes each triple once, a wave per H atom with its lanes
-// over the atom's hydrogen-bond entries: the energy, CEhb1 and j's own
+// j and k.  k_hb computes each triple once, half a wave per H atom with its
+// lanes over the atom's hydrogen-bond entries: the energy, CEhb1 and j's own
 // terms are summed by a fixed butterfly; the terms of i (summed over the
 // entries, one set per bond) and of k (summed over the bonds, one set per
 // entry) go into fixed-point accumulators (fix_add: 2^-40 resolution for
-// every term, sums up to 2^43) by integer atomics, whose sums do not depend
+// every term, sums up to 2^43) by integer adds, whose sums do not depend
 // on the order they arrive in; k_hb_fold adds them to fCdDelta and clears them.
 // The results are the same on every run.
 constexpr double HB_THRESHOLD = 1e-2;   // reaxc_defs_sunway.h:91
@@ -594,10 +602,14 @@ __device__ __forceinline__ void hb_triple(const DevHb &hbp, double BOij, const d
 constexpr double FIX_COARSE = 1048576.0;   // 2^20: coarse units
 constexpr double FIX_SPLIT = 1024.0;       // terms at least this large are split
 
+// Whether adding d to the word that held old wrapped it.
+__device__ __forceinline__ bool fix_wrapped(unsigned long long old, long long d) {
+  const long long o = (long long)old, sum = (long long)(old + (unsigned long long)d);
+  return ((o ^ sum) & (d ^ sum)) < 0;
+}
+
 __device__ __forceinline__ void fix_word_add(unsigned int *flags, unsigned long long *a, long long d) {
-  const long long old = (long long)atomicAdd(a, (unsigned long long)d);
-  const long long sum = (long long)((unsigned long long)old + (unsigned long long)d);
-  if (((old ^ sum) & (d ^ sum)) < 0) atomicOr(flags, SWR_F_FIXED_RANGE);   // signed wrap
+  if (fix_wrapped(atomicAdd(a, (unsigned long long)d), d)) atomicOr(flags, SWR_F_FIXED_RANGE);
 }
 
 __device__ __forceinline__ void fix_add(unsigned int *flags, unsigned long long *a, size_t coff, double v) {
@@ -635,11 +647,7 @@ __device__ __forceinline__ void fix_add_group(unsigned int *flags, unsigned long
   }
   bool wrap = false;
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const long long o = (long long)old[k];
-    const long long sum = (long long)(old[k] + (unsigned long long)d[k]);
-    wrap |= ((o ^ sum) & (d[k] ^ sum)) < 0;
-  }
+  for (int k = 0; k < K; ++k) wrap |= fix_wrapped(old[k], d[k]);
   if (wrap) atomicOr(flags, SWR_F_FIXED_RANGE);
 }
 
@@ -648,79 +656,168 @@ __device__ __forceinline__ double fix_value(const unsigned long long *a, size_t 
   return (double)(long long)a[0] * (1.0 / HB_FIX) + (double)(long long)a[coff] * (1.0 / FIX_COARSE);
 }
 
-__global__ void __launch_bounds__(BT) k_hb(int n, HbArgs A) {
-  const int j = blockIdx.x * (BT / SWR_WAVE) + wave_in_block();
-  if (j >= n) return;
-  const int lane = lane_id();
-  const DevParams *__restrict__ P = A.P;
-  const swr_atom_pack_t aj = A.atoms[j];
-  const int tj = aj.type;
-  const int H = (tj >= 0 && P->p_hbond[tj] == 1) ? A.Hindex[j] : -1;
-  if (H < 0) {
-    if (lane == 0) A.part[j] = 0.0;
+// A workgroup's sums of the fixed-point terms by atom: neighbouring H atoms
+// have mostly the same partners, and a device-wide atomic costs a trip past
+// the L2s (which eight XCDs do not share), an LDS one does not.  Words of
+// terms below FIX_SPLIT; a workgroup makes at most HB_ATOMS times the bonds of
+// an atom adds per atom, so an LDS word cannot wrap.
+constexpr int HB_SLOTS = 1024;
+struct HbTable {
+  int key[HB_SLOTS];
+  unsigned long long sum[3][HB_SLOTS];
+};
+
+// The slot of atom a, or -1 when it is not there and no slot is free nearby.
+__device__ __forceinline__ int hb_slot(HbTable &T, int a) {
+  int s = (int)(((unsigned)a * 2654435761u) >> 22);
+  for (int q = 0; q < 16; q++) {
+    int key = T.key[s];
+    if (key != a && key < 0) key = atomicCAS(&T.key[s], -1, a);
+    if (key == a || key < 0) return s;
+    s = (s + 1) & (HB_SLOTS - 1);
+  }
+  return -1;
+}
+static_assert(HB_SLOTS == 1 << (32 - 22), "hb_slot's shift leaves a slot number");
+
+// Component c of atom a += v.
+__device__ __forceinline__ void hb_add(const HbArgs &A, HbTable &T, int slot, int a, int c, double v) {
+  if (slot < 0 || !(fabs(v) < FIX_SPLIT)) {
+    fix_add(A.flags, A.acc + 3 * (size_t)a + c, A.coff, v);
     return;
   }
-  const int h0 = A.hidx[H], h1 = A.hend[H];
-  double e = 0.0, f0 = 0.0, f1 = 0.0, f2 = 0.0;
-  for (int pi = A.bidx[j]; pi < A.bend[j]; ++pi) {
-    const swr_bond_t bij = A.bonds[pi];
-    const int i = bij.nbr;
-    const int ti = A.atoms[i].type;
-    const double BOij = A.BO[pi];
-    if (ti < 0 || P->p_hbond[ti] != 2 || !(BOij >= HB_THRESHOLD)) continue;
-    const int oi = A.atoms[i].orig_id;
-    double ce1 = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    for (int pk = h0 + lane; pk < h1; pk += SWR_WAVE) {
-      const swr_hbond_t hb = A.hbonds[pk];
-      const int k = hb.nbr;
-      const swr_atom_pack_t ak = A.atoms[k];
-      if (ak.type < 0 || ak.orig_id == oi) continue;
-      const DevHb &hbp = P->hb[(ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + ak.type];
-      if (hbp.r0_hb <= 0.0) continue;
-      const swr_far_neighbor_t *fe = hb.ptr;
-      const double r_jk = fe->d;
-      const double dvec_jk[3] = {hb.scl * fe->dvec[0], hb.scl * fe->dvec[1], hb.scl * fe->dvec[2]};
-      HbTriple t;
-      hb_triple(hbp, BOij, bij.dvec, bij.d, dvec_jk, r_jk, t);
-      e += t.e;
-      ce1 += t.ce1;
-      f0 += t.ce2 * t.dj[0] - t.ce3 / r_jk * dvec_jk[0];
-      f1 += t.ce2 * t.dj[1] - t.ce3 / r_jk * dvec_jk[1];
-      f2 += t.ce2 * t.dj[2] - t.ce3 / r_jk * dvec_jk[2];
-      g0 += t.ce2 * t.di[0];
-      g1 += t.ce2 * t.di[1];
-      g2 += t.ce2 * t.di[2];
-      unsigned long long *ak3 = A.acc + 3 * (size_t)k;
-      {
-        unsigned long long *const ga[3] = {ak3, ak3 + 1, ak3 + 2};
-        const size_t gc[3] = {A.coff, A.coff, A.coff};
-        const double gv[3] = {t.ce2 * t.dk[0] + t.ce3 / r_jk * dvec_jk[0], t.ce2 * t.dk[1] + t.ce3 / r_jk * dvec_jk[1],
-                              t.ce2 * t.dk[2] + t.ce3 / r_jk * dvec_jk[2]};
-        fix_add_group<3>(A.flags, ga, gc, gv);
+  const long long d = llrint(v * HB_FIX);
+  if (d != 0) atomicAdd(&T.sum[c][slot], (unsigned long long)d);
+}
+
+// One hydrogen-bond entry of a lane (k < 0: none).
+struct HbEntry {
+  int k, type, orig;
+  double d, v[3];
+};
+
+// Two halves of a wave take an H atom each, of the H atoms among `per`
+// consecutive atoms of the workgroup; the lanes take a half's entries, the
+// next 32 of them requested ahead.  The chain of
+// loads to a first triple (atom, list, entry, far entry) bounds a small pass
+// and the atomics a large one (a wave per atom with an atomic per term took
+// 28 us on 1,944 atoms, 13 of them without the atomics; 590 on 96,000).  Sums
+// over the entries are kept for even and odd sets of 32 apart, which makes
+// them the sums of a 64-lane butterfly.
+constexpr int HB_G = 32;
+constexpr int HB_ATOMS = 64;   // at most, of a workgroup
+__global__ void __launch_bounds__(BT) k_hb(int n, int per, HbArgs A) {
+  __shared__ HbTable T;
+  __shared__ int list[HB_ATOMS], count;
+  for (int q = threadIdx.x; q < HB_SLOTS; q += BT) {
+    T.key[q] = -1;
+    T.sum[0][q] = T.sum[1][q] = T.sum[2][q] = 0ull;
+  }
+  if (threadIdx.x < SWR_WAVE) {
+    const int t = threadIdx.x, j = blockIdx.x * per + t;
+    const bool in = t < per && j < n;
+    const bool is_h = in && A.Hindex[j] >= 0;
+    if (in && !is_h) A.part[j] = 0.0;
+    const unsigned long long m = __ballot(is_h);
+    if (is_h) list[ballot_rank(m)] = j;
+    if (t == 0) count = __popcll(m);
+  }
+  __syncthreads();
+  const DevParams *__restrict__ P = A.P;
+  const int sl = threadIdx.x % HB_G, half = (threadIdx.x / HB_G) & 1;
+  for (int it = threadIdx.x / HB_G; it < count; it += BT / HB_G) {
+    const int j = list[it];
+    const int H = A.Hindex[j], tj = A.atoms[j].type;
+    const int b0 = A.bidx[j], b1 = A.bend[j];
+    const int h0 = A.hidx[H], h1 = A.hend[H];
+    auto load = [&](int pk) {
+      HbEntry x;
+      x.k = -1;
+      if (pk < h1) {
+        const swr_hbond_t hb = A.hbonds[pk];
+        x.k = hb.nbr;
+        x.type = A.atoms[hb.nbr].type;
+        x.orig = A.atoms[hb.nbr].orig_id;
+        x.d = hb.ptr->d;
+#pragma unroll
+        for (int c = 0; c < 3; c++) x.v[c] = hb.scl * hb.ptr->dvec[c];
+        if (x.type < 0) x.k = -1;
+      }
+      return x;
+    };
+    const HbEntry first = load(h0 + sl);   // (requested together with the bonds)
+    double e[2] = {0.0, 0.0}, f[3][2] = {};
+    for (int p0 = b0; p0 < b1; p0 += HB_G) {
+      // the acceptors among the atom's bonds
+      const int pl = p0 + sl;
+      bool acc = false;
+      if (pl < b1) {
+        const int ti = A.atoms[A.bonds[pl].nbr].type;
+        acc = ti >= 0 && P->p_hbond[ti] == 2 && A.BO[pl] >= HB_THRESHOLD;
+      }
+      unsigned todo = (unsigned)(__ballot(acc) >> (HB_G * half));
+      while (todo) {
+        const int pi = p0 + __ffs((int)todo) - 1;
+        todo &= todo - 1;
+        const swr_bond_t bij = A.bonds[pi];
+        const int i = bij.nbr;
+        const int ti = A.atoms[i].type, oi = A.atoms[i].orig_id;
+        const double BOij = A.BO[pi];
+        double ce1[2] = {0.0, 0.0}, g[3][2] = {};
+        HbEntry next = first;
+        // set: even and odd sets of 32 entries in turn
+        auto into = [](double (&acc)[2], int set, double v) {
+          acc[0] += set ? 0.0 : v;
+          acc[1] += set ? v : 0.0;
+        };
+        int set = 0;
+#pragma unroll 1
+        for (int pk = h0 + sl; pk - sl < h1; pk += HB_G, set ^= 1) {
+          const HbEntry x = next;
+          next = load(pk + HB_G);
+          if (x.k < 0 || x.orig == oi) continue;
+          const DevHb &hbp = P->hb[(ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + x.type];
+          if (hbp.r0_hb <= 0.0) continue;
+          HbTriple t;
+          hb_triple(hbp, BOij, bij.dvec, bij.d, x.v, x.d, t);
+          into(e, set, t.e);
+          into(ce1, set, t.ce1);
+          const int slot = hb_slot(T, x.k);
+#pragma unroll
+          for (int c = 0; c < 3; c++) {
+            into(f[c], set, t.ce2 * t.dj[c] - t.ce3 / x.d * x.v[c]);
+            into(g[c], set, t.ce2 * t.di[c]);
+            hb_add(A, T, slot, x.k, c, t.ce2 * t.dk[c] + t.ce3 / x.d * x.v[c]);
+          }
+        }
+        const double c1 = group_sum<HB_G>(ce1[0] + ce1[1]);
+        const double g0 = group_sum<HB_G>(g[0][0] + g[0][1]), g1 = group_sum<HB_G>(g[1][0] + g[1][1]),
+                     g2 = group_sum<HB_G>(g[2][0] + g[2][1]);
+        if (sl < 3) hb_add(A, T, hb_slot(T, i), i, sl, sl == 0 ? g0 : sl == 1 ? g1 : g2);
+        if (sl == 0) A.Cdbo[pi] += c1;
       }
     }
-    ce1 = wave_sum(ce1);
-    g0 = wave_sum(g0);
-    g1 = wave_sum(g1);
-    g2 = wave_sum(g2);
-    if (lane == 0) {
-      A.Cdbo[pi] += ce1;
-      unsigned long long *ai3 = A.acc + 3 * (size_t)i;
-      unsigned long long *const ga[3] = {ai3, ai3 + 1, ai3 + 2};
-      const size_t gc[3] = {A.coff, A.coff, A.coff};
-      const double gv[3] = {g0, g1, g2};
-      fix_add_group<3>(A.flags, ga, gc, gv);
-    }
+    const double es = group_sum<HB_G>(e[0] + e[1]);
+    const double f0 = group_sum<HB_G>(f[0][0] + f[0][1]), f1 = group_sum<HB_G>(f[1][0] + f[1][1]),
+                 f2 = group_sum<HB_G>(f[2][0] + f[2][1]);
+    if (sl == 0) A.part[j] = es;
+    if (sl < 3) A.fcd[4 * (size_t)j + sl] += sl == 0 ? f0 : sl == 1 ? f1 : f2;
   }
-  e = wave_sum(e);
-  f0 = wave_sum(f0);
-  f1 = wave_sum(f1);
-  f2 = wave_sum(f2);
-  if (lane == 0) {
-    A.part[j] = e;
-    A.fcd[4 * (size_t)j] += f0;
-    A.fcd[4 * (size_t)j + 1] += f1;
-    A.fcd[4 * (size_t)j + 2] += f2;
+  __syncthreads();
+  for (int q = threadIdx.x; q < HB_SLOTS; q += BT) {
+    const int a = T.key[q];
+    if (a < 0) continue;
+    long long d[3];
+    unsigned long long old[3] = {0ull, 0ull, 0ull};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      d[c] = (long long)T.sum[c][q];
+      if (d[c] != 0) old[c] = atomicAdd(A.acc + 3 * (size_t)a + c, (unsigned long long)d[c]);
+    }
+    bool wrap = false;
+#pragma unroll
+    for (int c = 0; c < 3; c++) wrap |= fix_wrapped(old[c], d[c]);
+    if (wrap) atomicOr(A.flags, SWR_F_FIXED_RANGE);
   }
 }
 
@@ -1853,9 +1950,11 @@ int swr_hydrogen_bonds_run(swr_system *S) {
   A.acc = S->hb_acc;
   A.coff = 3 * (size_t)N;
   A.flags = &S->status->flags;
-  constexpr int WPB = BT / SWR_WAVE;
+  // atoms per workgroup: few while that fills the chip, more share their
+  // partners' sums
+  const int per = n <= 8192 ? 8 : n <= 32768 ? 16 : HB_ATOMS;
   swr_kt_begin(S, KT_HBONDS);
-  if (n > 0) hipLaunchKernelGGL(k_hb, dim3(div_up(n, WPB)), dim3(BT), 0, S->stream, n, A);
+  if (n > 0) hipLaunchKernelGGL(k_hb, dim3(div_up(n, per)), dim3(BT), 0, S->stream, n, per, A);
   hipLaunchKernelGGL(k_hb_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, S->hb_acc, S->fcd,
                      (const double *)S->hb_part, S->hb_result);
   swr_kt_end(S, KT_HBONDS);
