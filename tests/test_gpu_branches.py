@@ -10,6 +10,7 @@ import pytest
 from sw_reaxff_amd import systems
 
 from .parity import harness
+from .test_bonded import _gpu_vs_oracle as _gpu_bonded_vs_oracle
 from .test_valence import _gpu_tor_vs_oracle, _gpu_vs_oracle
 
 
@@ -39,6 +40,24 @@ def test_gpu_valence_and_torsion_groups(gpu_lib, oracle_lib, ffield, case):
     s = GROUP_SYSTEMS[case]()
     for check in (_gpu_vs_oracle, _gpu_tor_vs_oracle):
         check(oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
+
+
+def shuffled(s, seed):
+    """s with its atoms in random order: a workgroup's atoms share no partners."""
+    k = np.random.default_rng(seed).permutation(s.n)
+    return systems.System(x=s.x[k], v=s.v[k], type=s.type[k], tag=np.arange(1, s.n + 1, dtype=np.int32),
+                          elements=s.elements, lo=s.lo, hi=s.hi, periodic=s.periodic)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["lattice", "cluster21", "water4200", "water30k", "shuffled36k"])
+def test_gpu_bonded_groups(gpu_lib, oracle_lib, ffield, case):
+    """Atom energies, hydrogen bonds and dBond forces: atoms with more bonds
+    than their four lanes and more than 64 hydrogen-bond entries (lattice),
+    workgroups of 8, 16 and 64 atoms in the hydrogen-bond pass, and one whose
+    partners overfill its LDS table (shuffled)."""
+    s = shuffled(systems.water_box(12000, seed=7), 8) if case == "shuffled36k" else GROUP_SYSTEMS[case]()
+    _gpu_bonded_vs_oracle(gpu_lib, oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
 
 
 def waters(m, seed):
