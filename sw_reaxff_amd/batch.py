@@ -60,6 +60,22 @@ def _buffer(bufs, name, shape, dtype):
     return b[:shape[0]]
 
 
+def _map_types(batch, elements, out):
+    """out = every atom's 1-based position in `elements`."""
+    kinds, which = {}, []
+    for s in batch:
+        which.append(kinds.setdefault(tuple(s.elements), len(kinds)))
+    tables = [np.array([elements.index(e) + 1 for e in k], dtype=np.int32) for k in kinds]
+    types = np.concatenate([s.type for s in batch])
+    if len(tables) == 1 and types.dtype.kind in "iu" and types.min() >= 1 and types.max() <= len(tables[0]):
+        np.take(tables[0], types - 1, out=out, mode="clip")
+        return
+    a = 0
+    for s, k in zip(batch, which):
+        out[a:a + s.n] = tables[k][s.type - 1]
+        a += s.n
+
+
 def pack(batch: list[systems.System], elements=ELEMENTS, cutghost: float = CUTGHOST, bufs=None) -> Packed:
     """Places the systems in disjoint regions of one box (see module doc);
     ghosts, translation and numbering by swr_batch_pack (host C++).  `bufs`
@@ -69,35 +85,45 @@ def pack(batch: list[systems.System], elements=ELEMENTS, cutghost: float = CUTGH
     K = len(batch)
     nat = np.array([s.n for s in batch], dtype=np.int32)
     n = int(nat.sum())
-    x = np.ascontiguousarray(np.concatenate([s.x for s in batch]) if n else np.zeros((0, 3)), dtype=np.float64)
-    typ = np.empty(n, np.int32)
-    tag = np.empty(n, np.int32)
-    a = 0
-    for s in batch:
-        tmap = np.array([elements.index(e) + 1 for e in s.elements], dtype=np.int32)
-        typ[a:a + s.n] = tmap[s.type - 1]
-        tag[a:a + s.n] = s.tag
-        a += s.n
+    if K == 1:
+        s = batch[0]
+        x = np.ascontiguousarray(s.x, dtype=np.float64)
+        tag = np.ascontiguousarray(s.tag, dtype=np.int32)
+        typ = np.array([elements.index(e) + 1 for e in s.elements], dtype=np.int32)[s.type - 1]
+    else:
+        x = _buffer(bufs, "x_in", (n, 3), np.float64)
+        typ = _buffer(bufs, "type_in", (n,), np.int32)
+        tag = _buffer(bufs, "tag_in", (n,), np.int32)
+        if n:
+            np.concatenate([s.x for s in batch], out=x, casting="unsafe")
+            np.concatenate([s.tag for s in batch], out=tag, casting="unsafe")
+            _map_types(batch, elements, typ)
     lo = np.ascontiguousarray([s.lo for s in batch], dtype=np.float64)
     hi = np.ascontiguousarray([s.hi for s in batch], dtype=np.float64)
     per = np.array([1 if s.periodic else 0 for s in batch], dtype=np.int32)
     N = C.c_longlong(0)
-    args = (K, nat.ctypes.data, x.ctypes.data, typ.ctypes.data, tag.ctypes.data, lo.ctypes.data, hi.ctypes.data,
-            per.ctypes.data, C.c_double(cutghost))
-    _lib.check(L.swr_batch_pack(*args, 0, None, None, None, None, None, None, None, None, C.byref(N)),
-               "swr_batch_pack")
-    Nv = N.value
-    xo = _buffer(bufs, "x", (Nv, 3), np.float64)
-    to = _buffer(bufs, "type", (Nv,), np.int32)
-    go = _buffer(bufs, "tag", (Nv,), np.int32)
-    oo = _buffer(bufs, "owner", (Nv,), np.int32)
-    io = _buffer(bufs, "img", (Nv, 3), np.int8)
     row_off = np.empty(K + 1, np.int32)
     ghost_off = np.empty(K + 1, np.int32)
     shift = np.empty((K, 3), np.float64)
-    _lib.check(L.swr_batch_pack(*args, Nv, xo.ctypes.data, to.ctypes.data, go.ctypes.data, oo.ctypes.data,
-                                io.ctypes.data, row_off.ctypes.data, ghost_off.ctypes.data, shift.ctypes.data,
-                                C.byref(N)), "swr_batch_pack")
+    args = (K, nat.ctypes.data, x.ctypes.data, typ.ctypes.data, tag.ctypes.data, lo.ctypes.data, hi.ctypes.data,
+            per.ctypes.data, C.c_double(cutghost))
+    # into the room the last pack left, when the images fit it; else counted first
+    room = len(bufs["img"]) if bufs and "img" in bufs else 0
+    if room < max(n, 1):
+        _lib.check(L.swr_batch_pack(*args, 0, None, None, None, None, None, None, None, None, C.byref(N)),
+                   "swr_batch_pack")
+        room = N.value
+    while True:
+        out = [_buffer(bufs, k, (room,) + w, t) for k, w, t in (
+            ("x", (3,), np.float64), ("type", (), np.int32), ("tag", (), np.int32), ("owner", (), np.int32),
+            ("img", (3,), np.int8))]
+        rc = L.swr_batch_pack(*args, room, *[a.ctypes.data for a in out], row_off.ctypes.data,
+                              ghost_off.ctypes.data, shift.ctypes.data, C.byref(N))
+        if not rc or N.value <= room:
+            break
+        room = N.value
+    _lib.check(rc, "swr_batch_pack")
+    xo, to, go, oo, io = (a[:N.value] for a in out)
     return Packed(x=xo, type=to, tag=go, owner=oo, img=io, n=n, row_off=row_off, ghost_off=ghost_off, shift=shift)
 
 

@@ -1,8 +1,12 @@
 // Host-side packing of independent systems into one batch (swr_batch_pack).
 // Ghost images follow LAMMPS Comm::borders for an orthogonal periodic box:
 // per dimension, two swaps over the atoms present when the dimension starts.
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
+#include <thread>
 #include <vector>
 
 #include "swr_internal.h"
@@ -57,6 +61,37 @@ void borders(int n, const double *x, const Slabs &B, Scratch &S) {
   }
 }
 
+// Runs part(k) for every system, of `atoms` atoms in all, on up to
+// PACK_THREADS threads that take the next system in turn: a batch of 100,000
+// atoms is half a millisecond of copying for one, and the GPU waits for it.
+// Few atoms stay on the caller's thread (starting one costs the copying of ~10,000
+// atoms).  False when a part ran out of memory.
+constexpr int PACK_THREADS = 8;
+constexpr long long PACK_GRAIN = 32768;   // atoms a thread is worth
+template <class Part>
+bool over_systems(int nsys, long long atoms, Part part) {
+  const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
+  const int T = (int)std::min<long long>({atoms / PACK_GRAIN + 1, PACK_THREADS, hw, nsys});
+  std::atomic<int> next{0};
+  std::atomic<bool> ok{true};
+  auto run = [&] {
+    try {
+      for (int k = next++; k < nsys; k = next++) part(k);
+    } catch (const std::exception &) {
+      ok = false;
+    }
+  };
+  std::vector<std::thread> th;
+  try {
+    th.reserve(T);
+    while ((int)th.size() + 1 < T) th.emplace_back(run);
+  } catch (const std::exception &) {   // no more threads: those there are do it
+  }
+  run();
+  for (auto &t : th) t.join();
+  return ok;
+}
+
 }  // namespace
 
 extern "C" int swr_batch_pack(int nsys, const int *nat, const double *x, const int *type, const int *tag,
@@ -74,25 +109,27 @@ extern "C" int swr_batch_pack(int nsys, const int *nat, const double *x, const i
     first[k + 1] = first[k] + nat[k];
   }
   if (first[nsys] > 0 && (!x || !type || !tag)) { swr_set_error_msg("swr_batch_pack: missing atoms"); return SWR_ERR_ARG; }
+  for (int k = 0; k < nsys; k++) {
+    const double *lk = lo + 3 * k, *hk = hi + 3 * k;
+    if (!periodic[k]) continue;
+    for (int d = 0; d < 3; d++)
+      if (!(hk[d] > lk[d])) { swr_set_error_msg("swr_batch_pack: empty periodic box"); return SWR_ERR_ARG; }
+    // one image per side and dimension covers the ghost shell only when
+    // the box is at least cutghost long (LAMMPS then needs several swaps)
+    for (int d = 0; d < 3; d++)
+      if (hk[d] - lk[d] < cutghost) {
+        swr_set_error_msg("swr_batch_pack: periodic box shorter than the ghost cutoff");
+        return SWR_ERR_ARG;
+      }
+  }
   // pass 1: ghost counts and extents (atoms, their images and the box)
   std::vector<double> elo(3 * (size_t)nsys), ehi(3 * (size_t)nsys);
-  double size = 0;
-  long long n = first[nsys], ng = 0;
-  for (int k = 0; k < nsys; k++) {
+  const bool counted = over_systems(nsys, first[nsys], [&](int k) {
     const double *xk = x ? x + 3 * first[k] : nullptr;
     const double *lk = lo + 3 * k, *hk = hi + 3 * k;
     double mn[3], mx[3];
     for (int d = 0; d < 3; d++) { mn[d] = lk[d]; mx[d] = hk[d]; }
     if (periodic[k]) {
-      for (int d = 0; d < 3; d++)
-        if (!(hk[d] > lk[d])) { swr_set_error_msg("swr_batch_pack: empty periodic box"); return SWR_ERR_ARG; }
-      // one image per side and dimension covers the ghost shell only when
-      // the box is at least cutghost long (LAMMPS then needs several swaps)
-      for (int d = 0; d < 3; d++)
-        if (hk[d] - lk[d] < cutghost) {
-          swr_set_error_msg("swr_batch_pack: periodic box shorter than the ghost cutoff");
-          return SWR_ERR_ARG;
-        }
       const Slabs B(lk, hk, cutghost);
       for (int i = 0; i < nat[k]; i++) {
         long long copies = 1;
@@ -118,8 +155,14 @@ extern "C" int swr_batch_pack(int nsys, const int *nat, const double *x, const i
     for (int d = 0; d < 3; d++) {
       elo[3 * k + d] = mn[d];
       ehi[3 * k + d] = mx[d];
-      size = std::fmax(size, mx[d] - mn[d]);
     }
+  });
+  if (!counted) { swr_set_error_msg("swr_batch_pack: out of memory"); return SWR_ERR_NOMEM; }
+  double size = 0;
+  const long long n = first[nsys];
+  long long ng = 0;
+  for (int k = 0; k < nsys; k++) {
+    for (int d = 0; d < 3; d++) size = std::fmax(size, ehi[3 * k + d] - elo[3 * k + d]);
     ng += nghost[k];
   }
   *N_out = n + ng;
@@ -141,32 +184,41 @@ extern "C" int swr_batch_pack(int nsys, const int *nat, const double *x, const i
     for (int d = 0; d < 3; d++) shift[3 * k + d] = cell[d] * size - elo[3 * k + d];
   }
   // pass 2: images (borders order) and the translated, renumbered output
-  Scratch S;
-  for (int k = 0; k < nsys; k++) {
+  const bool placed = over_systems(nsys, n + ng, [&](int k) {
     const int nk = nat[k];
     const size_t tot = (size_t)nk + (size_t)nghost[k];
     const double *xk = x + 3 * first[k];
     const double *sk = shift + 3 * k;
     const int a = row_off[k];
-    const long long g0 = n + ghost_off[k];
-    if (periodic[k]) {
-      S.x.resize(3 * tot);
-      S.owner.resize(tot);
-      S.img.resize(3 * tot);
-      borders(nk, xk, Slabs(lo + 3 * k, hi + 3 * k, cutghost), S);
+    if (!periodic[k]) {
+      for (size_t i = 0; i < tot; i++) {
+        const size_t r = (size_t)a + i;
+        for (int d = 0; d < 3; d++) x_out[3 * r + d] = xk[3 * i + d] + sk[d];
+        type_out[r] = type[first[k] + i];
+        tag_out[r] = tag[first[k] + i] + a;
+        owner_out[r] = (int)r;
+      }
+      std::memset(img_out + 3 * (size_t)a, 0, 3 * tot);
+      return;
     }
+    Scratch S;
+    const long long g0 = n + ghost_off[k];
+    S.x.resize(3 * tot);
+    S.owner.resize(tot);
+    S.img.resize(3 * tot);
+    borders(nk, xk, Slabs(lo + 3 * k, hi + 3 * k, cutghost), S);
     for (size_t i = 0; i < tot; i++) {
       const long long r = (long long)i < nk ? a + (long long)i : g0 + ((long long)i - nk);
-      const int own = periodic[k] ? S.owner[i] : (int)i;
-      const double *xi = periodic[k] ? &S.x[3 * i] : xk + 3 * i;
+      const int own = S.owner[i];
       for (int d = 0; d < 3; d++) {
-        x_out[3 * r + d] = xi[d] + sk[d];
-        img_out[3 * r + d] = periodic[k] ? S.img[3 * i + d] : 0;
+        x_out[3 * r + d] = S.x[3 * i + d] + sk[d];
+        img_out[3 * r + d] = S.img[3 * i + d];
       }
       type_out[r] = type[first[k] + own];
       tag_out[r] = tag[first[k] + own] + a;
       owner_out[r] = own + a;
     }
-  }
+  });
+  if (!placed) { swr_set_error_msg("swr_batch_pack: out of memory"); return SWR_ERR_NOMEM; }
   return SWR_OK;
 }

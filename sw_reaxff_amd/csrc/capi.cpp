@@ -353,26 +353,30 @@ int swr_create(const char *ffield_path, int ntypes, const char *const *elements,
     swr_destroy(S);
     return rc;
   }
-  if (hipHostMalloc((void **)&S->status_host, sizeof(DevStatus), 0) != hipSuccess) {
+  // one pinned block for the status copy, the counters the host reads back
+  // and the first uploads (each allocation of its own takes ~60 us)
+  constexpr size_t O_DONE = 256, O_MIX = 512, O_ITERS = O_MIX + SWR_PIN_MIX, O_STAGE = O_ITERS + 512;
+  static_assert(sizeof(DevStatus) <= O_DONE && O_ITERS + sizeof(int) * 2 * 64 <= O_STAGE, "the parts fit");
+  if (hipHostMalloc(&S->pin_base, O_STAGE + SWR_STAGES * SWR_STAGE_FIRST, 0) != hipSuccess) {
     swr_set_error_msg("hipHostMalloc failed");
     swr_destroy(S);
     return SWR_ERR_NOMEM;
+  }
+  char *pin = (char *)S->pin_base;
+  S->status_host = (DevStatus *)pin;
+  S->pin_done = (int *)(pin + O_DONE);
+  S->pin_mix = pin + O_MIX;
+  S->pin_iters = (int *)(pin + O_ITERS);
+  S->pin_iters_cap = 2 * 64;
+  for (int k = 0; k < SWR_STAGES; k++) {
+    S->stage[k].pin = pin + O_STAGE + k * SWR_STAGE_FIRST;
+    S->stage[k].cap = SWR_STAGE_FIRST;
   }
   std::memset(S->status_host, 0, sizeof(DevStatus));
-  if (hipHostMalloc((void **)&S->pin_done, 64, 0) != hipSuccess ||
-      hipHostMalloc(&S->pin_mix, SWR_PIN_MIX, 0) != hipSuccess) {
-    swr_set_error_msg("hipHostMalloc failed");
-    swr_destroy(S);
-    return SWR_ERR_NOMEM;
-  }
   if (hipEventCreateWithFlags(&S->ev_read, hipEventDisableTiming) != hipSuccess) {
     swr_set_error_msg("hipEventCreate failed");
     swr_destroy(S);
     return SWR_ERR_HIP;
-  }
-  if ((rc = swr_pin_iters_reserve(S, 64))) {
-    swr_destroy(S);
-    return rc;
   }
   // the system's stream does not wait for the null stream: everything goes on it
   if (hipMemcpyAsync(S->dp, &S->hp, sizeof(DevParams), hipMemcpyHostToDevice, S->stream) != hipSuccess ||
@@ -393,7 +397,7 @@ int swr_destroy(swr_system *S) {
   void *ptrs[] = {S->dp, S->x, S->v, S->q, S->type, S->tag, S->owner, S->img, S->mask, S->packed,
                   S->bin_of, S->bin_count, S->bin_start, S->bin_occ, S->rs_keys, S->rs_vals, S->rs_hist, S->bp_pos, S->bp_id, S->stencil_rows,
                   S->voff, S->vcount, S->vlist, S->far, S->far_index, S->far_end, S->num_bonds, S->num_hbonds,
-                  S->Hindex, S->bond_index, S->bond_end, S->bonds, S->bond_nbr, S->bo_data, S->prow, S->pbeg, S->pcnt, S->pcol, S->pkey, S->jloc, S->sys_panel, S->small_panel, S->BO, S->BOpi, S->Cdbo,
+                  S->Hindex, S->bond_index, S->bond_end, S->bonds, S->bond_nbr, S->bo_data, S->prow, S->panel_all, S->pcnt, S->pcol, S->pkey, S->jloc, S->BO, S->BOpi, S->Cdbo,
                   S->Cdbopi,
                   S->Cdbopi2, S->hbond_index, S->hbond_end, S->hbonds, S->hbslot, S->bo_dboc, S->dDeltap_self, S->bond_mark,
                   S->fcd, S->nb_partials, S->nb_result, S->nb_eatom, S->be_part, S->be_ce, S->be_bufc, S->be_result, S->hb_part,
@@ -401,17 +405,19 @@ int swr_destroy(swr_system *S) {
                   S->to_sacc, S->to_tc, S->to_task, S->to_ctl, S->to_row, S->f, S->gcsr_cnt, S->gcsr_start, S->gcsr_list,
                   S->bond_mark2, S->counts, S->ws, S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32,
                   S->Hdia_inv, S->b_s, S->st, S->s_hist, S->t_hist, S->cgv, S->cgs, S->partials, S->next_totals,
-                  S->status, S->scan_tmp, S->tmp_i, S->mixw, S->cand, S->cand_count, S->row_sys, S->tile_beg,
-                  S->tile_sys, S->sys_tile, S->sblk_beg, S->sys_sblk, S->sys_iters, S->done_count, S->qsum,
+                  S->status, S->scan_tmp, S->tmp_i, S->mixw, S->cand, S->cand_count, S->layout_all, S->atoms_in,
+                  S->done_count, S->qsum,
                   S->mark_chg, S->mark_up};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  if (S->status_host) (void)hipHostFree(S->status_host);
-  if (S->pin_done) (void)hipHostFree(S->pin_done);
-  if (S->pin_mix) (void)hipHostFree(S->pin_mix);
-  if (S->pin_iters) (void)hipHostFree(S->pin_iters);
+  if (S->pin_base) (void)hipHostFree(S->pin_base);
+  if (S->pin_iters_own) (void)hipHostFree(S->pin_iters);
   if (S->mark_chg_host) (void)hipHostFree(S->mark_chg_host);
   if (S->ev_read) (void)hipEventDestroy(S->ev_read);
+  for (SwrStage &g : S->stage) {
+    if (g.own) (void)hipHostFree(g.pin);
+    if (g.ev) (void)hipEventDestroy(g.ev);
+  }
   if (S->stream) (void)hipStreamDestroy(S->stream);
   delete S;
   return SWR_OK;
@@ -442,22 +448,30 @@ int swr_set_atoms(swr_system *S, int n, int N, const int *tag, const int *type, 
   S->have_f = false;
   S->n = n;
   S->N = N;
+  if (N <= SWR_ATOMS_STAGED) {   // few atoms: the copies' own cost counts
+    for (int i = n; i < N; i++)
+      if ((owner ? owner[i] : i) < 0 || (owner ? owner[i] : i) >= n) {
+        swr_set_error_msg("swr_set_atoms: ghost owner out of range");
+        return SWR_ERR_ARG;
+      }
+    return swr_stage_atoms(S, tag, type, x, q, owner, img);
+  }
   HIP_CHECK(hipMemcpyAsync(S->x, x, sizeof(double) * 3 * N, hipMemcpyHostToDevice, S->stream));
   HIP_CHECK(hipMemcpyAsync(S->tag, tag, sizeof(int) * N, hipMemcpyHostToDevice, S->stream));
   HIP_CHECK(hipMemcpyAsync(S->type, type, sizeof(int) * N, hipMemcpyHostToDevice, S->stream));
   if (q) HIP_CHECK(hipMemcpyAsync(S->q, q, sizeof(double) * N, hipMemcpyHostToDevice, S->stream));
   else HIP_CHECK(hipMemsetAsync(S->q, 0, sizeof(double) * N, S->stream));
-  std::vector<int> own(N);
-  std::vector<signed char> im(3 * (size_t)N, 0);
-  for (int i = 0; i < N; i++) own[i] = owner ? owner[i] : i;
-  if (img) std::memcpy(im.data(), img, 3 * (size_t)N);
+  std::vector<int> own(owner ? 0 : N);
+  for (int i = 0; i < (int)own.size(); i++) own[i] = i;
+  if (!owner) owner = own.data();
   for (int i = n; i < N; i++)
-    if (own[i] < 0 || own[i] >= n) {
+    if (owner[i] < 0 || owner[i] >= n) {
       swr_set_error_msg("swr_set_atoms: ghost owner out of range");
       return SWR_ERR_ARG;
     }
-  HIP_CHECK(hipMemcpyAsync(S->owner, own.data(), sizeof(int) * N, hipMemcpyHostToDevice, S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->img, im.data(), 3 * (size_t)N, hipMemcpyHostToDevice, S->stream));
+  HIP_CHECK(hipMemcpyAsync(S->owner, owner, sizeof(int) * N, hipMemcpyHostToDevice, S->stream));
+  if (img) HIP_CHECK(hipMemcpyAsync(S->img, img, 3 * (size_t)N, hipMemcpyHostToDevice, S->stream));
+  else HIP_CHECK(hipMemsetAsync(S->img, 0, 3 * (size_t)N, S->stream));
   HIP_CHECK(hipStreamSynchronize(S->stream));
   return SWR_OK;
 }

@@ -13,6 +13,7 @@
 // Far slots of atom i are [voff[i], voff[i+1]) — bounded by its Verlet
 // count — so no separate counting pass is needed (the reference uses
 // i*maxfar, pair_reaxc_sw64.c:256).
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -44,6 +45,27 @@ __global__ void k_pack(const int *__restrict__ tag, const int *__restrict__ type
   a.x[0] = x[3 * i]; a.x[1] = x[3 * i + 1]; a.x[2] = x[3 * i + 2];
   a.q = q[i];
   out[i] = a;
+}
+
+// An upload of swr_set_atoms ([N] x, y, z, then q if has_q, tag, type, owner if
+// has_owner and img in bytes if has_img) into the atom arrays; without owners
+// each atom owns itself, without q or img these are zero.
+__global__ void k_unpack_atoms(int N, const int *__restrict__ in, int has_q, int has_owner, int has_img,
+                               double *__restrict__ x, double *__restrict__ q, int *__restrict__ tag,
+                               int *__restrict__ type, int *__restrict__ owner, signed char *__restrict__ img) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  const double *d = reinterpret_cast<const double *>(in);
+  for (int c = 0; c < 3; c++) x[3 * (size_t)i + c] = d[3 * (size_t)i + c];
+  d += 3 * (size_t)N;
+  q[i] = has_q ? d[i] : 0.0;
+  const int *w = reinterpret_cast<const int *>(d + (has_q ? N : 0));
+  tag[i] = w[i];
+  type[i] = w[N + i];
+  w += 2 * (size_t)N;
+  owner[i] = has_owner ? w[i] : i;
+  const signed char *b = reinterpret_cast<const signed char *>(w + (has_owner ? N : 0));
+  for (int c = 0; c < 3; c++) img[3 * (size_t)i + c] = has_img ? b[3 * (size_t)i + c] : (signed char)0;
 }
 
 // Reset_Atoms / Reset_Neighbor_Lists in two launches: k_reset_sums adds up
@@ -1069,6 +1091,37 @@ int swr_lists_pack(swr_system *S) {
 }
 
 int swr_lists_alloc_bonds(swr_system *S, int bond_cap, int hbond_cap);
+
+// The atoms in one upload and one launch: five to seven copies and a fill took
+// ~45 us of a 60-atom evaluation's 600.
+int swr_stage_atoms(swr_system *S, const int *tag, const int *type, const double *x, const double *q, const int *owner,
+                    const signed char *img) {
+  const int N = S->N;
+  if (N <= 0) return SWR_OK;
+  const size_t bytes = (size_t)N * (24 + (q ? 8 : 0) + 8 + (owner ? 4 : 0) + (img ? 3 : 0));
+  int rc;
+  if ((rc = swr_reserve(&S->atoms_in, S->cap_atoms_in, (bytes + 3) / 4)) ||
+      (rc = swr_stage_ready(S, SWR_STAGE_ATOMS, bytes)))
+    return rc;
+  char *p = (char *)S->stage[SWR_STAGE_ATOMS].pin;
+  auto put = [&](const void *src, size_t each) {
+    if (!src) return;
+    std::memcpy(p, src, each * N);
+    p += each * N;
+  };
+  put(x, 24);
+  put(q, 8);
+  put(tag, 4);
+  put(type, 4);
+  put(owner, 4);
+  put(img, 3);
+  if ((rc = swr_stage_send(S, SWR_STAGE_ATOMS, S->atoms_in, bytes))) return rc;
+  hipLaunchKernelGGL(k_unpack_atoms, dim3(div_up(N, 256)), dim3(256), 0, S->stream, N, (const int *)S->atoms_in,
+                     q ? 1 : 0, owner ? 1 : 0, img ? 1 : 0, S->x, S->q, S->tag, S->type, S->owner, S->img);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(S->stream));
+  return SWR_OK;
+}
 
 int swr_lists_reset(swr_system *S) {
   const int n = S->n, N = S->N;

@@ -217,33 +217,35 @@ int swr_panel_build(swr_system *S) {
       if ((rc = swr_radix_sort_i32(S, S->pkey, tmp, n, bits, S->prow))) return rc;
     }
     swr_kt_end(S, KT_PANEL);
-    std::vector<int> pbeg;
+    // one upload: the SmallPanel of each panel (small systems; 16-byte
+    // aligned), pbeg[np + 1], sys_panel[nsys + 1]
     const int nsys = (int)S->sys_row.size() - 1;
-    std::vector<int> sys_panel(nsys + 1);
+    int np = 0;
+    for (int s = 0; s < nsys; s++) np += div_up(S->sys_row[s + 1] - S->sys_row[s], SWR_PANEL_ROWS);
+    const size_t o_pb = S->cg_small ? 8 * (size_t)np : 0, o_sp = o_pb + np + 1;
+    std::vector<int> all(o_sp + nsys + 1);
+    int *pbeg = all.data() + o_pb, *sys_panel = all.data() + o_sp;
+    int p = 0;
     for (int s = 0; s < nsys; s++) {
-      sys_panel[s] = (int)pbeg.size();
-      for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r += SWR_PANEL_ROWS) pbeg.push_back(r);
+      sys_panel[s] = p;
+      for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r += SWR_PANEL_ROWS) pbeg[p++] = r;
     }
-    sys_panel[nsys] = (int)pbeg.size();
-    pbeg.push_back(n);
-    const int np = (int)pbeg.size() - 1;
-    std::vector<int> place;   // SmallPanel of each panel
-    if (S->cg_small) {
+    sys_panel[nsys] = p;
+    pbeg[p] = n;
+    if (S->cg_small)
       for (int s = 0; s < nsys; s++)
-        for (int p = sys_panel[s]; p < sys_panel[s + 1]; p++)
-          place.insert(place.end(), {pbeg[p], p + 1 < sys_panel[s + 1] ? pbeg[p + 1] : S->sys_row[s + 1], S->sys_row[s],
-                                     S->sys_row[s + 1], s, sys_panel[s], sys_panel[s + 1], 0});
-      if ((rc = swr_reserve(&S->small_panel, S->cap_small_panel, place.size()))) return rc;
-      HIP_CHECK(hipMemcpyAsync(S->small_panel, place.data(), sizeof(int) * place.size(), hipMemcpyHostToDevice,
-                               S->stream));
-    }
-    if ((rc = swr_reserve(&S->pbeg, S->cap_pbeg, pbeg.size())) || (rc = swr_reserve(&S->pcnt, S->cap_pcnt, (size_t)np)) ||
-        (rc = swr_reserve(&S->sys_panel, S->cap_sys_panel, sys_panel.size())))
+        for (int q = sys_panel[s]; q < sys_panel[s + 1]; q++) {
+          const int place[8] = {pbeg[q], q + 1 < sys_panel[s + 1] ? pbeg[q + 1] : S->sys_row[s + 1], S->sys_row[s],
+                                S->sys_row[s + 1], s, sys_panel[s], sys_panel[s + 1], 0};
+          std::copy(place, place + 8, all.data() + 8 * (size_t)q);
+        }
+    if ((rc = swr_reserve(&S->panel_all, S->cap_panel_all, all.size())) ||
+        (rc = swr_reserve(&S->pcnt, S->cap_pcnt, (size_t)np)))
       return rc;
-    HIP_CHECK(hipMemcpyAsync(S->pbeg, pbeg.data(), sizeof(int) * pbeg.size(), hipMemcpyHostToDevice, S->stream));
-    HIP_CHECK(hipMemcpyAsync(S->sys_panel, sys_panel.data(), sizeof(int) * sys_panel.size(), hipMemcpyHostToDevice,
-                             S->stream));
-    HIP_CHECK(hipStreamSynchronize(S->stream));   // host temporaries
+    S->small_panel = S->panel_all;
+    S->pbeg = S->panel_all + o_pb;
+    S->sys_panel = S->panel_all + o_sp;
+    if ((rc = swr_upload(S, SWR_STAGE_PANEL, S->panel_all, all.data(), sizeof(int) * all.size()))) return rc;
     S->npanel = np;
     S->prow_n = n;
     S->prow_nbr_gen = S->nbr_gen;

@@ -295,6 +295,39 @@ int swr_qeq_spmv(swr_system *S, const double *xv, double *b) {
   return SWR_OK;
 }
 
+int swr_stage_ready(swr_system *S, int which, size_t bytes) {
+  SwrStage &g = S->stage[which];
+  if (!g.ev) HIP_CHECK(hipEventCreateWithFlags(&g.ev, hipEventDisableTiming));
+  else HIP_CHECK(hipEventSynchronize(g.ev));   // the last upload from here
+  if (bytes > g.cap) {
+    if (g.own) HIP_CHECK(hipHostFree(g.pin));
+    g.own = false;
+    g.pin = nullptr;
+    g.cap = 0;
+    const size_t cap = bytes + bytes / 4 + 4096;
+    if (hipHostMalloc(&g.pin, cap, 0) != hipSuccess) {
+      swr_set_error_msg("hipHostMalloc failed");
+      return SWR_ERR_NOMEM;
+    }
+    g.own = true;
+    g.cap = cap;
+  }
+  return SWR_OK;
+}
+
+int swr_stage_send(swr_system *S, int which, void *dst, size_t bytes) {
+  SwrStage &g = S->stage[which];
+  HIP_CHECK(hipMemcpyAsync(dst, g.pin, bytes, hipMemcpyHostToDevice, S->stream));
+  HIP_CHECK(hipEventRecord(g.ev, S->stream));
+  return SWR_OK;
+}
+
+int swr_upload(swr_system *S, int which, void *dst, const void *src, size_t bytes) {
+  if (int rc = swr_stage_ready(S, which, bytes)) return rc;
+  std::memcpy(S->stage[which].pin, src, bytes);
+  return swr_stage_send(S, which, dst, bytes);
+}
+
 // Row/tile layout of the (batch of) systems and the buffers sized by it.
 // Rebuilt when the atoms or the batch partition changed.
 int swr_pin_iters_reserve(swr_system *S, int nsys) {
@@ -303,7 +336,8 @@ int swr_pin_iters_reserve(swr_system *S, int nsys) {
   const int cap = std::max(need, 2 * S->pin_iters_cap);
   if (S->pin_iters) {
     HIP_CHECK(hipStreamSynchronize(S->stream));
-    HIP_CHECK(hipHostFree(S->pin_iters));
+    if (S->pin_iters_own) HIP_CHECK(hipHostFree(S->pin_iters));
+    S->pin_iters_own = false;
     S->pin_iters = nullptr;
     S->pin_iters_cap = 0;
   }
@@ -311,6 +345,7 @@ int swr_pin_iters_reserve(swr_system *S, int nsys) {
     swr_set_error_msg("hipHostMalloc failed");
     return SWR_ERR_NOMEM;
   }
+  S->pin_iters_own = true;
   S->pin_iters_cap = cap;
   return SWR_OK;
 }
@@ -321,52 +356,45 @@ int swr_qeq_layout(swr_system *S) {
   if (S->sys_row.size() < 2 || S->sys_row.back() != n) S->sys_row = {0, n};
   const int nsys = (int)S->sys_row.size() - 1;
   if (int rc = swr_pin_iters_reserve(S, nsys)) return rc;
-  std::vector<int> row_sys(std::max(n, 1)), tile_beg, tile_sys, sys_tile(nsys + 1), sblk_beg, sys_sblk(nsys + 1);
+  int nsblk = 0, ntiles = 0;
   for (int s = 0; s < nsys; s++) {
-    sys_tile[s] = (int)tile_sys.size();
-    for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r += UT) {
-      tile_beg.push_back(r);
-      tile_sys.push_back(s);
+    const int rows = S->sys_row[s + 1] - S->sys_row[s];
+    ntiles += div_up(rows, UT);
+    nsblk += div_up(rows, RPB);
+  }
+  const bool none = ntiles == 0;   // no rows: one empty tile keeps every grid non-empty
+  if (none) ntiles = 1;
+  // all arrays in one upload: row_sys[n], tile_beg[ntiles + 1],
+  // tile_sys[ntiles], sys_tile[nsys + 1], then sys_iters[2 nsys] at zero
+  const size_t o_tb = std::max(n, 1), o_ts = o_tb + ntiles + 1, o_st = o_ts + ntiles, o_it = o_st + nsys + 1;
+  std::vector<int> all(o_it + 2 * (size_t)nsys, 0);
+  int *row_sys = all.data(), *tile_beg = row_sys + o_tb, *tile_sys = row_sys + o_ts, *sys_tile = row_sys + o_st;
+  int t = 0;
+  for (int s = 0; s < nsys; s++) {
+    sys_tile[s] = t;
+    for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r += UT, t++) {
+      tile_beg[t] = r;
+      tile_sys[t] = s;
     }
-    sys_sblk[s] = (int)sblk_beg.size();
-    for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r += RPB) sblk_beg.push_back(r);
-    for (int r = S->sys_row[s]; r < S->sys_row[s + 1]; r++) row_sys[r] = s;
+    std::fill(row_sys + S->sys_row[s], row_sys + S->sys_row[s + 1], s);
   }
-  sys_tile[nsys] = (int)tile_sys.size();
-  tile_beg.push_back(n);
-  const int nsblk = (int)sblk_beg.size();
-  sys_sblk[nsys] = nsblk;
-  sblk_beg.push_back(n);
-  if (tile_sys.empty()) {  // no rows: one empty tile keeps every grid non-empty
-    tile_beg = {0, 0};
-    tile_sys = {0};
-    sys_tile.assign(nsys + 1, 1);
-    sys_tile[0] = 0;
+  sys_tile[nsys] = t;
+  tile_beg[t] = n;
+  if (none) {
+    tile_beg[0] = tile_beg[1] = 0;
+    std::fill(sys_tile + 1, sys_tile + nsys + 1, 1);
   }
-  const int ntiles = (int)tile_sys.size();
   int rc;
-  if ((rc = swr_reserve(&S->row_sys, S->cap_row_sys, row_sys.size())) ||
-      (rc = swr_reserve(&S->tile_beg, S->cap_tile_beg, tile_beg.size())) ||
-      (rc = swr_reserve(&S->tile_sys, S->cap_tile_sys, tile_sys.size())) ||
-      (rc = swr_reserve(&S->sys_tile, S->cap_sys_tile, sys_tile.size())) ||
-      (rc = swr_reserve(&S->sblk_beg, S->cap_sblk_beg, sblk_beg.size())) ||
-      (rc = swr_reserve(&S->sys_sblk, S->cap_sys_sblk, sys_sblk.size())) ||
-      (rc = swr_reserve(&S->sys_iters, S->cap_sys_iters, 2 * (size_t)nsys)) ||
+  if ((rc = swr_reserve(&S->layout_all, S->cap_layout_all, all.size())) ||
       (rc = swr_reserve(&S->cgs, S->cap_cgs, 4 * (size_t)nsys)) ||
       (rc = swr_reserve(&S->qsum, S->cap_qsum, 3 * (size_t)nsys)))
     return rc;
-  HIP_CHECK(hipMemcpyAsync(S->row_sys, row_sys.data(), sizeof(int) * row_sys.size(), hipMemcpyHostToDevice, S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->tile_beg, tile_beg.data(), sizeof(int) * tile_beg.size(), hipMemcpyHostToDevice,
-                           S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->tile_sys, tile_sys.data(), sizeof(int) * tile_sys.size(), hipMemcpyHostToDevice,
-                           S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->sys_tile, sys_tile.data(), sizeof(int) * sys_tile.size(), hipMemcpyHostToDevice,
-                           S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->sblk_beg, sblk_beg.data(), sizeof(int) * sblk_beg.size(), hipMemcpyHostToDevice,
-                           S->stream));
-  HIP_CHECK(hipMemcpyAsync(S->sys_sblk, sys_sblk.data(), sizeof(int) * sys_sblk.size(), hipMemcpyHostToDevice,
-                           S->stream));
-  HIP_CHECK(hipMemsetAsync(S->sys_iters, 0, sizeof(int) * 2 * nsys, S->stream));
+  S->row_sys = S->layout_all;
+  S->tile_beg = S->layout_all + o_tb;
+  S->tile_sys = S->layout_all + o_ts;
+  S->sys_tile = S->layout_all + o_st;
+  S->sys_iters = S->layout_all + o_it;
+  if ((rc = swr_upload(S, SWR_STAGE_LAYOUT, S->layout_all, all.data(), sizeof(int) * all.size()))) return rc;
   HIP_CHECK(hipMemsetAsync(S->cgs, 0, sizeof(CgScalars) * 4 * nsys, S->stream));
   const int ps = std::max(std::max(div_up(std::max(n, 1), RPB), nsblk), ntiles);
   if (ps > S->cg_pstride || !S->partials) {
@@ -374,10 +402,8 @@ int swr_qeq_layout(swr_system *S) {
     S->cg_pstride = ps;
   }
   if (!S->done_count && (rc = swr_alloc(&S->done_count, 1))) return rc;
-  HIP_CHECK(hipStreamSynchronize(S->stream));
   S->nsys = nsys;
   S->ntiles = ntiles;
-  S->nsblk = nsblk;
   S->cg_small = small_rule(S->sys_row, S->mixed);
   S->h_sys_iters.assign(2 * nsys, 0);
   S->layout_dirty = false;

@@ -179,6 +179,17 @@ enum { KT_VERLET = 0, KT_FAR, KT_BUILD_H, KT_CG_ITER, KT_CG_SETUP, KT_BO, KT_VAL
        KT_QEQ_Q, KT_BINS, KT_MIXED_INNER, KT_MIXED_OUTER, KT_BONDS, KT_CG_SCALARS, KT_MARK, KT_CG_UPDATE, KT_NONBONDED, KT_ATOM_ENERGY,
        KT_DBOND, KT_HBONDS, KT_VALENCE, KT_TORSION, KT_PANEL, KT_COUNT };
 
+// Pinned memory of one kind of upload; ev has passed when it may be written again.
+struct SwrStage {
+  void *pin = nullptr;
+  size_t cap = 0;
+  bool own = false;       // an allocation of its own, not part of pin_base
+  hipEvent_t ev = nullptr;
+};
+enum { SWR_STAGE_LAYOUT = 0, SWR_STAGE_PANEL, SWR_STAGE_ATOMS, SWR_STAGES };
+constexpr size_t SWR_STAGE_FIRST = 8192;
+constexpr int SWR_ATOMS_STAGED = 16384;   // swr_set_atoms: one upload up to here
+
 struct swr_system {
   // ---- host-side configuration
   int device = 0;
@@ -209,8 +220,11 @@ struct swr_system {
   // into pageable memory are staged through a bounce buffer)
   int *pin_done = nullptr;        // [16]: the CG's count of finished systems, and SWR_PIN_* below
   void *pin_mix = nullptr;        // the mixed solve's counters and state (SWR_PIN_MIX bytes)
+  SwrStage stage[SWR_STAGES];
   int *pin_iters = nullptr;       // iteration counts, 2 per system
   int pin_iters_cap = 0;
+  bool pin_iters_own = false;     // an allocation of its own, not part of pin_base
+  void *pin_base = nullptr;       // the one pinned allocation of swr_create
   size_t cap_bin_occ = 0;
   // counting sort by bin (radix passes staged in LDS): key/value ping-pong
   // buffers and the per-(digit, block) counts and starts
@@ -322,10 +336,10 @@ struct swr_system {
   int *prow = nullptr, *pbeg = nullptr, *pcnt = nullptr, *pcol = nullptr, *pkey = nullptr;
   int *sys_panel = nullptr;   // [nsys + 1] system s owns panels [sys_panel[s], sys_panel[s+1])
   unsigned short *jloc = nullptr;
-  size_t cap_prow = 0, cap_pbeg = 0, cap_pcnt = 0, cap_pcol = 0, cap_pkey = 0, cap_jloc = 0, cap_sys_panel = 0;
+  int *panel_all = nullptr;   // small_panel, pbeg and sys_panel in one allocation
+  size_t cap_prow = 0, cap_panel_all = 0, cap_pcnt = 0, cap_pcol = 0, cap_pkey = 0, cap_jloc = 0;
   int npanel = 0, prow_n = -1;
   int *small_panel = nullptr; // qeq_small.h: eight ints per panel (its rows, its system's rows and panels)
-  size_t cap_small_panel = 0;
   bool panel_lists = false;   // pcol, pcnt and jloc hold the lists of the current H
   long long nbr_gen = 0, layout_gen = 0, prow_nbr_gen = -1, prow_layout_gen = -1;
   int panel_shape = -1;   // tuning family "panels": 0 (default) lists on, 1 off
@@ -348,19 +362,15 @@ struct swr_system {
   int nsys = 1, ntiles = 0;
   bool cg_small = false;           // the FP64 solve takes one launch per iteration (qeq_small.h)
   bool layout_dirty = true;
+  int *atoms_in = nullptr;         // an upload of swr_set_atoms, before k_unpack_atoms spreads it
+  size_t cap_atoms_in = 0;
+  int *layout_all = nullptr;       // the arrays below up to sys_tile, and sys_iters, in one allocation
   int *row_sys = nullptr;          // [n] system of each local row
   int *tile_beg = nullptr;         // [ntiles + 1]
   int *tile_sys = nullptr;         // [ntiles]
   int *sys_tile = nullptr;         // [nsys + 1]
-  // half-wave-per-row kernels over a batch: block b runs rows
-  // [sblk_beg[b], sblk_beg[b+1]) (at most 8, one system), system s owns
-  // blocks [sys_sblk[s], sys_sblk[s+1])
-  int *sblk_beg = nullptr;         // [nsblk + 1]
-  int *sys_sblk = nullptr;         // [nsys + 1]
-  int nsblk = 0;
   // capacities of the layout arrays (grown, never shrunk)
-  size_t cap_row_sys = 0, cap_tile_beg = 0, cap_tile_sys = 0, cap_sys_tile = 0, cap_sblk_beg = 0,
-         cap_sys_sblk = 0, cap_sys_iters = 0, cap_cgs = 0, cap_qsum = 0;
+  size_t cap_layout_all = 0, cap_cgs = 0, cap_qsum = 0;
   int *sys_iters = nullptr;        // [2 nsys] iterations of s, t per system (device)
   std::vector<int> h_sys_iters;    // host copy after each solve
   int *done_count = nullptr;       // systems finished in the running solve
@@ -470,6 +480,15 @@ struct SwrQGate {
   const unsigned int *flags = nullptr;
 };
 int swr_qeq_calc_q(swr_system *S, SwrQGate gate);
+// Copies bytes of host memory that the caller may change at once to dst, by way
+// of the system's own pinned memory `which` (grown, never shrunk).
+int swr_upload(swr_system *S, int which, void *dst, const void *src, size_t bytes);
+// The two halves of it, for a source that is written into the pinned memory.
+int swr_stage_ready(swr_system *S, int which, size_t bytes);
+int swr_stage_send(swr_system *S, int which, void *dst, size_t bytes);
+// n, N and the arrays' room are set; q, owner and img may be null.
+int swr_stage_atoms(swr_system *S, const int *tag, const int *type, const double *x, const double *q, const int *owner,
+                    const signed char *img);
 // Device words to copy into pinned host memory.
 struct SwrPublish {
   const int *src[3] = {};

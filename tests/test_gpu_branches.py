@@ -285,3 +285,32 @@ def test_gpu_reset_and_scans_at_tile_edges(gpu_lib, ffield, n):
     assert np.array_equal(h.get("hbond_index"), excl(nh[is_h])[:-1])
     assert np.array_equal(h.get("hbond_end"), excl(nh[is_h])[:-1])
     assert not h.get("fCdDelta")[:n].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 16384, 16385])
+def test_gpu_set_atoms_uploads(gpu_lib, ffield, n):
+    """The one-upload path (16,384 atoms at most) and the one beyond it put the
+    same arrays, with and without charges, owners and images, after a larger
+    and after a smaller set."""
+    from sw_reaxff_amd import _lib
+    rng = np.random.default_rng(n)
+    h = _lib.System(ffield, ["H", "O", "C"])
+    for m in (n, max(1, n // 3), n):
+        nloc = (m + 1) // 2
+        x = rng.normal(size=(m, 3)) * 20.0
+        t = rng.integers(1, 4, size=m).astype(np.int32)
+        tag = rng.permutation(m).astype(np.int32) + 1
+        for q, owner, img in ((None, True, None), (rng.normal(size=m), True, True), (None, False, True)):
+            k = nloc if owner else m
+            own = np.concatenate([np.arange(k), rng.integers(0, k, size=m - k)]).astype(np.int32)
+            im = rng.integers(-1, 2, size=(m, 3)).astype(np.int8) if img else None
+            h.set_atoms(k, x, t, tag, owner=own if owner else None, img=im, q=q)
+            assert np.array_equal(h.get("x")[:3 * m].reshape(-1, 3), x)
+            for name, want in (("type", t), ("tag", tag), ("owner", own), ("q", np.zeros(m) if q is None else q),
+                               ("img", np.zeros(3 * m, np.int8) if im is None else im.ravel())):
+                assert np.array_equal(h.get(name)[:want.size], want), name
+    bad = np.full(n, n, np.int32)
+    if n > 1:
+        with pytest.raises(_lib.SwrError, match="owner out of range"):
+            h.set_atoms(n // 2, x, t, tag, owner=bad)
