@@ -176,15 +176,23 @@ __device__ __forceinline__ void store_nt(double2 *dst, double2 v) {
   __builtin_nontemporal_store(t, reinterpret_cast<nd2 *>(dst));
 }
 
-// One far entry as four 16-byte pieces at dst (rel_box stays 0).
-__device__ __forceinline__ void stage_far(double2 *dst, int j, int tj, int tagj, double d, double qj, double dx,
-                                          double dy, double dz) {
+// The r-th far entry of a chunk as four 16-byte pieces in the chunk's LDS
+// (rel_box stays 0), turned by r / 4: pieces of one column in their plain
+// places would be 64 bytes apart, sixteen entries on four banks of 16 bytes
+// (two thirds of the far pass's LDS cycles: 1585 -> 1415 us on 512 clusters,
+// 625 -> 549 on 36,000 water atoms, 69 -> 63 on 1,944).
+__device__ __forceinline__ void stage_far(double2 *chunk, int r, int j, int tj, int tagj, double d, double qj,
+                                          double dx, double dy, double dz) {
+  double2 *dst = chunk + 4 * r;
   int4 *p = reinterpret_cast<int4 *>(dst);
-  p[0] = make_int4(j, tj, tagj, 0);
-  p[1] = make_int4(0, 0, __double2loint(d), __double2hiint(d));
-  dst[2] = make_double2(qj, dx);
-  dst[3] = make_double2(dy, dz);
+  const int t = r >> 2;
+  p[t & 3] = make_int4(j, tj, tagj, 0);
+  p[(t + 1) & 3] = make_int4(0, 0, __double2loint(d), __double2hiint(d));
+  dst[(t + 2) & 3] = make_double2(qj, dx);
+  dst[(t + 3) & 3] = make_double2(dy, dz);
 }
+// Where piece t (counted through the chunk's entries) is.
+__device__ __forceinline__ int staged_piece(int t) { return (t & ~3) + ((t + (t >> 4)) & 3); }
 
 // Uncorrected bond order of one pair (BOp_single, reaxc_forces_sunway.cpp:695-717).
 struct BOpTerms { double BO, BO_s, pi, pi2, C12, C34, C56; };
@@ -283,11 +291,11 @@ k_far(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__re
         // 16-byte pieces (lane t writes piece t, t+64, ...): full-line
         // stores instead of one 64-byte entry per lane.
         double2 *sw = sfar[w];
-        if (infar) stage_far(sw + 4 * r, j, tj, tagj, d, qj, dx, dy, dz);
+        if (infar) stage_far(sw, r, j, tj, tagj, d, qj, dx, dy, dz);
         wave_lds_sync();
         double2 *dst = reinterpret_cast<double2 *>(far + far0 + nfar);
         const int pieces = 4 * __popcll(m);
-        for (int t = lane; t < pieces; t += SWR_WAVE) store_nt(dst + t, sw[t]);
+        for (int t = lane; t < pieces; t += SWR_WAVE) store_nt(dst + t, sw[staged_piece(t)]);
         wave_lds_sync();
       }
       nfar += __popcll(m);
@@ -498,7 +506,7 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
       const unsigned long long m = __ballot(infar);
       const int r = ballot_rank(m);
       const long long slot = far0 + nfar + r;
-      if (infar) stage_far(S.far[buf][g] + 4 * r, cur.j, tj, cur.a.orig_id, d, cur.a.q, dx, dy, dz);
+      if (infar) stage_far(S.far[buf][g], r, cur.j, tj, cur.a.orig_id, d, cur.a.q, dx, dy, dz);
       if (lane == 0) {
         S.dst[buf][g] = far0 + nfar;
         S.cnt[buf][g] = __popcll(m);
@@ -567,7 +575,7 @@ k_far_ws(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *_
           if (cnt > 0) {
             double2 *dstp = reinterpret_cast<double2 *>(far + S.dst[pb][gg]);
             const double2 *src = S.far[pb][gg];
-            for (int t = lane; t < 4 * cnt; t += SWR_WAVE) store_nt(dstp + t, src[t]);
+            for (int t = lane; t < 4 * cnt; t += SWR_WAVE) store_nt(dstp + t, src[staged_piece(t)]);
           }
           if (HB == 3) {
             if (lane < S.hcnt[pb][gg]) hbslot[S.hdst[pb][gg] + lane] = S.hb[pb][gg][lane].y;
@@ -1140,17 +1148,16 @@ int swr_lists_reset(swr_system *S) {
   return SWR_OK;
 }
 
-// The far pass's split: the tuned one, else by the Verlet entries it streams.
-// Four writer waves for four gatherers are best while the far list and the
-// gathered atoms stay in the caches (31,000 water atoms with their ghosts: 157
-// us against 174 with eight gatherers and 191 with
-// two writers; 103,000 atoms of 128 clusters: 328, 355, 408); once the list
-// streams to HBM, eight atoms a workgroup share a phase's writes (187,500
-// atoms, 121M entries: 1418 us against 1490 and 1531; 88,000 atoms, 57M: 613,
-// 636, 681).
+// The far pass's split: the tuned one, else by the workgroups there are.  Four
+// writer waves for four gatherers while eight atoms a workgroup would leave
+// the last round of 512 of them much of the time (13,000 atoms with their
+// ghosts 63 us against 72 with eight gatherers and 72 with two writers; 31,000:
+// 141, 154, 160; 47,000 of 64 clusters: 135, 143, 163); beyond, eight atoms
+// share a phase's barrier and writes (52,000: 246, 240, 297; 103,000 of 128
+// clusters: 295, 277, 347; 187,500: 1452, 1370, 1496).
 int swr_far_shape(const swr_system *S) {
   if (S->far_shape >= 0) return S->far_shape;
-  return S->vtotal >= 45000000LL ? SWR_FAR_G8W4 : SWR_FAR_G4W4;
+  return S->N >= 49152 ? SWR_FAR_G8W4 : SWR_FAR_G4W4;
 }
 
 // mode 0: the far list; 1: far list, bonds and hydrogen bonds; 2: bonds and
