@@ -1492,59 +1492,94 @@ __device__ __forceinline__ bool to_pass(const ToArgs &A, int tj, int tk, double 
   return A.P->tor[((ti * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + tl].cnt != 0;
 }
 
-// Quadruples of the bond in slot pk of local atom j (type tj >= 0, slots
-// [b0, b1)) whose k-l bond is every TO_PAIR_LANES-th from lane pl on; 0 when
-// the bond is no central bond (its BO, the orig_id order, a k without bonds
-// or type).
-constexpr int TO_SLOT_LANES = 4;   // lanes of an atom over its slots, in k_to_count,
-constexpr int TO_PAIR_LANES = 4;   // and of a slot over k's bonds
-constexpr int TO_CNT_LANES = TO_SLOT_LANES * TO_PAIR_LANES;
-__device__ __forceinline__ int to_count(const ToArgs &A, const swr_atom_pack_t &aj, int tj, int b0, int b1,
-                                        int pk, int pl, double thb_cut) {
-  const double BO_jk = A.BO[pk];
-  if (!(BO_jk - thb_cut > 0.0)) return 0;
-  const int k = A.bnbr[pk];
-  const int k0 = A.bidx[k], k1 = A.bend[k];
-  const swr_atom_pack_t ak = A.atoms[k];
-  const int pj = A.bonds[pk].sym_index;
-  const int tk = ak.type;
-  if (k1 <= k0 || tk < 0 || !owns_bond(aj, ak)) return 0;
-  int c = 0;
-  for (int pw = k0 + pl; pw < k1; pw += TO_PAIR_LANES) {
-#pragma unroll 4
-    for (int ph = b0; ph < b1; ++ph) c += to_pass(A, tj, tk, BO_jk, pk, pj, ph, pw, thb_cut) ? 1 : 0;
-  }
-  return c;
-}
-
-// Sixteen lanes per local atom: with four (each a slot's whole count) the
-// pass waited pair by pair for its gathers, 23 us on 1,944 atoms and 543 on
-// 200,000.
+// Sixteen lanes per local atom.  They hold its bonds, a bond each, and find
+// the central ones together; for each of those they hold k's bonds, and the
+// atom's strong bonds go round by lane exchange, so the quadruples are tested
+// without a load but the parameter table's.  (With each pair's bonds gathered
+// again the pass waited for them: 10 us on 60 atoms, 80 on 96,000, 500 on 512
+// clusters; with four lanes an atom 23 on 1,944.)
+constexpr int TO_CNT_LANES = 16;
 __global__ void __launch_bounds__(BT) k_to_count(int n, ToArgs A) {
+  constexpr int L = TO_CNT_LANES;
   __shared__ int hist[WL_NB];
   for (int b = threadIdx.x; b < WL_NB; b += BT) hist[b] = 0;
   __syncthreads();
+  const DevParams *__restrict__ P = A.P;
   const int tid = blockIdx.x * BT + threadIdx.x;
-  const int j = tid / TO_CNT_LANES;
-  const int pl = tid % TO_PAIR_LANES;
+  const int j = tid / L, sl = tid % L, shift = lane_id() & ~(L - 1);
+  const double thb_cut = P->thb_cut;
+  auto group = [&](bool x) { return (unsigned)(__ballot(x) >> shift) & ((1u << L) - 1u); };
   swr_atom_pack_t aj = {};
   aj.type = -1;
   if (j < n) aj = A.atoms[j];
+  const int tj = aj.type;
   const int b0 = j < n ? A.bidx[j] : 0, b1 = j < n ? A.bend[j] : 0;
-  const int nbmax = wave_max_groups<TO_CNT_LANES>(b1 - b0);
-  const double thb_cut = A.P->thb_cut;
-  for (int m0 = 0; m0 < nbmax; m0 += TO_SLOT_LANES) {
-    const int pk = b0 + m0 + (tid % TO_CNT_LANES) / TO_PAIR_LANES;
-    int c = pk < b1 && aj.type >= 0 ? to_count(A, aj, aj.type, b0, b1, pk, pl, thb_cut) : 0;
-#pragma unroll
-    for (int o = 1; o < TO_PAIR_LANES; o <<= 1) c += __shfl_xor(c, o, SWR_WAVE);
-    if (pk >= b1) continue;
-    if (c == 0) {
-      for (int q = pl; q < 6; q += TO_PAIR_LANES) A.row[6 * (size_t)pk + q] = 0.0;
+  for (int c0 = b0; c0 < b1; c0 += L) {
+    // this lane's bond as the central one: k, its bonds, the reverse slot
+    const int pc = c0 + sl;
+    const bool mine = pc < b1;
+    double BO = 0.0;
+    int k = 0, k0 = 0, k1 = 0, tk = -1, pj = 0;
+    bool central = false;
+    if (mine && tj >= 0) {
+      BO = A.BO[pc];
+      k = A.bnbr[pc];
+      k0 = A.bidx[k];
+      k1 = A.bend[k];
+      const swr_atom_pack_t ak = A.atoms[k];
+      tk = ak.type;
+      pj = A.bonds[pc].sym_index;
+      central = BO - thb_cut > 0.0 && k1 > k0 && tk >= 0 && owns_bond(aj, ak);
     }
-    if (pl == 0) {
-      A.tc[pk] = c;
-      if (c > 0) atomicAdd(&hist[wl_bucket(c)], 1);
+    if (mine && !central) {
+      A.tc[pc] = 0;
+#pragma unroll
+      for (int q = 0; q < 6; q++) A.row[6 * (size_t)pc + q] = 0.0;
+    }
+    for (unsigned todo = group(central); todo; todo &= todo - 1) {
+      const int e = __ffs((int)todo) - 1, pk = c0 + e;
+      const double BO_jk = __shfl(BO, e, L);
+      const int w0 = __shfl(k0, e, L), w1 = __shfl(k1, e, L), tc = __shfl(tk, e, L), pr = __shfl(pj, e, L);
+      int c = 0;
+      for (int ww = w0; ww < w1; ww += L) {
+        const int pw = ww + sl;
+        double BO_kl = 0.0;
+        int l = 0, tl = -1;
+        if (pw < w1) {
+          BO_kl = A.BO[pw];
+          l = A.bnbr[pw];
+          tl = A.atoms[l].type;
+        }
+        const bool far_end = pw < w1 && pw != pr && tl >= 0 && BO_kl > thb_cut;
+        for (int h0 = b0; h0 < b1; h0 += L) {
+          // the atom's bonds as j-i, a lane each (those of the outer round as they are)
+          double BO_ij = BO;
+          int i = k, ti = tk;
+          if (h0 != c0) {
+            const int ph = h0 + sl;
+            BO_ij = ph < b1 ? A.BO[ph] : 0.0;
+            i = ph < b1 ? A.bnbr[ph] : 0;
+            ti = ph < b1 ? A.atoms[i].type : -1;
+          }
+          unsigned strong = group(ti >= 0 && BO_ij > thb_cut);
+          if (h0 == c0) strong &= ~(1u << e);
+          for (; strong; strong &= strong - 1) {
+            const int q = __ffs((int)strong) - 1;
+            const double bij = __shfl(BO_ij, q, L);
+            const int ii = __shfl(i, q, L), t4 = __shfl(ti, q, L);
+            if (far_end && ii != l && bij * BO_jk * BO_kl > thb_cut &&
+                P->tor[((t4 * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tc) * SWR_MAX_ELEM + tl].cnt != 0)
+              c++;
+          }
+        }
+      }
+#pragma unroll
+      for (int o = 1; o < L; o <<= 1) c += __shfl_xor(c, o, SWR_WAVE);
+      if (c == 0 && sl < 6) A.row[6 * (size_t)pk + sl] = 0.0;
+      if (sl == 0) {
+        A.tc[pk] = c;
+        if (c > 0) atomicAdd(&hist[wl_bucket(c)], 1);
+      }
     }
   }
   wl_hist_flush(hist, A.ctl);
