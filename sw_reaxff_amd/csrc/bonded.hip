@@ -1126,11 +1126,17 @@ __device__ __forceinline__ int wl_gmin(int ntask) { return ntask <= 4096 ? 16 : 
 // go to LDS and each slot and total is summed by one lane in pair order.  One thread
 // per centre took 52 us on a 64-water box and 150 us on the 32,000-water one;
 // this takes 17 and 115 (512 clusters: 1.05 and 1.11 ms, all lanes busy).
-__global__ void __launch_bounds__(SWR_WAVE) k_valence(VaArgs A) {
+//
+// SETS: parameter sets per angle type that the round's terms have room for; two
+// (15 KB instead of 29) let eight waves a CU be resident, and the registers are
+// held to that (eight spilled): 512 clusters 1138 -> 804 us, 96,000 water atoms
+// 117 -> 92, 1,944 19 either way.
+template <int SETS>
+__global__ void __launch_bounds__(SWR_WAVE) __attribute__((amdgpu_waves_per_eu(2))) k_valence(VaArgs A) {
   __shared__ unsigned short queue[2 * SWR_WAVE];
   // the round's pairs: Cdbo terms, and per parameter set the centre's terms
   enum { V_ANG = 0, V_PEN, V_COA, V_CE5, V_CE6, V_CDJ, V_G0, V_G1, V_G2, V_NC };
-  __shared__ double spk[SWR_WAVE], sph[SWR_WAVE], term[V_NC][SWR_MAX_THB][SWR_WAVE];
+  __shared__ double spk[SWR_WAVE], sph[SWR_WAVE], term[V_NC][SETS][SWR_WAVE];
   __shared__ int sset[SWR_WAVE];
   __shared__ GroupTotals<V_NC> T;
   const int lane = lane_id();
@@ -1452,25 +1458,34 @@ struct ToArgs {
 };
 
 
-// Calculate_Theta + Calculate_dCos_Theta of bonds a (first) and b from one
-// centre: di belongs to a's far atom, dj to the centre, dk to b's.
-__device__ __forceinline__ double theta_dcos(const swr_bond_t &a, const swr_bond_t &b, double *di, double *dj,
-                                             double *dk) {
-  const double dot = a.dvec[0] * b.dvec[0] + a.dvec[1] * b.dvec[1] + a.dvec[2] * b.dvec[2];
+// Calculate_Theta of bonds a (first) and b from one centre; dot: their dot
+// product.
+__device__ __forceinline__ double theta_of(const swr_bond_t &a, const swr_bond_t &b, double &dot) {
+  dot = a.dvec[0] * b.dvec[0] + a.dvec[1] * b.dvec[1] + a.dvec[2] * b.dvec[2];
   double c = dot / (a.d * b.d);
   if (c > 1.0) c = 1.0;
   if (c < -1.0) c = -1.0;
-  const double sa = a.d * a.d, sb = b.d * b.d;
-  const double inv = 1.0 / (a.d * b.d);
-  const double ci3 = dot * (inv * inv * inv);
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    di[q] = b.dvec[q] * inv - ci3 * sb * a.dvec[q];
-    dj[q] = -(b.dvec[q] + a.dvec[q]) * inv + ci3 * (sb * a.dvec[q] + sa * b.dvec[q]);
-    dk[q] = a.dvec[q] * inv - ci3 * sa * b.dvec[q];
-  }
   return acos(c);
 }
+
+// Calculate_dCos_Theta of the same: component q of di (a's far atom), dj (the
+// centre) and dk (b's far atom).  Apart from the angle, so that the nine
+// numbers are not held in registers through the energies between.
+struct DCos {
+  double inv, ci3, sa, sb;
+  __device__ __forceinline__ DCos(const swr_bond_t &a, const swr_bond_t &b, double dot) {
+    inv = 1.0 / (a.d * b.d);
+    ci3 = dot * (inv * inv * inv);
+    sa = a.d * a.d;
+    sb = b.d * b.d;
+  }
+  __device__ __forceinline__ void get(const swr_bond_t &a, const swr_bond_t &b, int q, double &di, double &dj,
+                                      double &dk) const {
+    di = b.dvec[q] * inv - ci3 * sb * a.dvec[q];
+    dj = -(b.dvec[q] + a.dvec[q]) * inv + ci3 * (sb * a.dvec[q] + sa * b.dvec[q]);
+    dk = a.dvec[q] * inv - ci3 * sa * b.dvec[q];
+  }
+};
 
 __device__ __forceinline__ double tan_inv(double s, double c) {
   constexpr double MIN_SINE = 1e-10;   // reaxc_torsion_angles_sw64.c:12
@@ -1617,7 +1632,12 @@ __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
 // cotangent terms of a nearly linear angle cancel in FP64 first.  One lane
 // per bond took 87 us on a 64-water box, 133 us on the 32,000-water one and
 // 2.38 ms on 512 clusters; this takes 16, 66 us and 1.31 ms.
-__global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
+//
+// WAVES: waves per SIMD the registers are held to.  Two (ten of 266 spilled)
+// pay once a list keeps every SIMD busy with quadruples: 512 clusters 1333 ->
+// 1016 us; 64 clusters 183 -> 188, 96,000 water atoms 64 -> 70, 1,944 17 -> 19.
+template <int WAVES>
+__global__ void __launch_bounds__(SWR_WAVE) __attribute__((amdgpu_waves_per_eu(WAVES))) k_torsion(ToArgs A) {
   // the round's quadruples: the bond's and i's terms
   enum { O_FJ = 0, O_FK = 4, O_CDK = 7, O_PI, O_BO, O_TOR, O_CON, O_NC };
   __shared__ unsigned short queue[2 * SWR_WAVE];
@@ -1681,15 +1701,14 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
         const DevTor &fb = P->tor[((ai.type * SWR_MAX_ELEM + tj) * SWR_MAX_ELEM + tk) * SWR_MAX_ELEM + al.type];
         const double r_ij = bij.d;
         const double BOA_ij = BO_ij - thb_cut;
-        double ijk_di[3], ijk_dj[3], ijk_dk[3];   // of k, j, i
-        const double theta_ijk = theta_dcos(bjk, bij, ijk_di, ijk_dj, ijk_dk);
+        double dot_ijk, dot_jkl;
+        const double theta_ijk = theta_of(bjk, bij, dot_ijk);
         const double sin_ijk = sin(theta_ijk);
         const double cos_ijk = cos(theta_ijk);
         const double tan_ijk_i = tan_inv(sin_ijk, cos_ijk);
         const double exp_tor2_ij = exp(-p_tor2 * BOA_ij);
         const double exp_cot2_ij = exp(-p_cot2 * (BOA_ij - 1.5) * (BOA_ij - 1.5));
-        double jkl_di[3], jkl_dj[3], jkl_dk[3];   // of j, k, l
-        const double theta_jkl = theta_dcos(bkj, bkl, jkl_di, jkl_dj, jkl_dk);
+        const double theta_jkl = theta_of(bkj, bkl, dot_jkl);
         const double r_kl = bkl.d;
         const double BOA_kl = BO_kl - thb_cut;
         double sin_jkl = sin(theta_jkl);
@@ -1768,16 +1787,20 @@ __global__ void __launch_bounds__(SWR_WAVE) k_torsion(ToArgs A) {
         const double cdbo_kl = CEtors6 + Cconj * (BOA_kl - 1.5e0);
         const double c7 = CEtors7 + CEconj4, c8 = CEtors8 + CEconj5, c9 = CEtors9 + CEconj6;
         double fl[3];
+        const DCos ijk(bjk, bij, dot_ijk), jkl(bkj, bkl, dot_jkl);
 #pragma unroll
         for (int q = 0; q < 3; q++) {
-          const double w_i = sc * (a_ij * dij[q] - dvec_li[q] - t_d * ijk_dk[q]);
-          const double w_j = sc * (-a_ij * dij[q] - a_jk * djk[q] - t_d * ijk_dj[q] - t_e * jkl_di[q]);
-          const double w_k = sc * (-a_kl * dkl[q] + a_jk * djk[q] - t_d * ijk_di[q] - t_e * jkl_dj[q]);
-          const double w_l = sc * (a_kl * dkl[q] + dvec_li[q] - t_e * jkl_dk[q]);
-          iterm[1 + q][lane] = c7 * ijk_dk[q] + c9 * w_i;
-          term[O_FJ + q][lane] = c7 * ijk_dj[q] + c8 * jkl_di[q] + c9 * w_j;
-          term[O_FK + q][lane] = c7 * ijk_di[q] + c8 * jkl_dj[q] + c9 * w_k;
-          fl[q] = c8 * jkl_dk[q] + c9 * w_l;
+          double ijk_di, ijk_dj, ijk_dk, jkl_di, jkl_dj, jkl_dk;   // of k, j, i; of j, k, l
+          ijk.get(bjk, bij, q, ijk_di, ijk_dj, ijk_dk);
+          jkl.get(bkj, bkl, q, jkl_di, jkl_dj, jkl_dk);
+          const double w_i = sc * (a_ij * dij[q] - dvec_li[q] - t_d * ijk_dk);
+          const double w_j = sc * (-a_ij * dij[q] - a_jk * djk[q] - t_d * ijk_dj - t_e * jkl_di);
+          const double w_k = sc * (-a_kl * dkl[q] + a_jk * djk[q] - t_d * ijk_di - t_e * jkl_dj);
+          const double w_l = sc * (a_kl * dkl[q] + dvec_li[q] - t_e * jkl_dk);
+          iterm[1 + q][lane] = c7 * ijk_dk + c9 * w_i;
+          term[O_FJ + q][lane] = c7 * ijk_dj + c8 * jkl_di + c9 * w_j;
+          term[O_FK + q][lane] = c7 * ijk_di + c8 * jkl_dj + c9 * w_k;
+          fl[q] = c8 * jkl_dk + c9 * w_l;
         }
         unsigned long long *al4 = A.acc + 4 * (size_t)l;
         unsigned long long *const ga[4] = {A.sacc + pw, al4, al4 + 1, al4 + 2};
@@ -2050,7 +2073,11 @@ int swr_valence_angles_run(swr_system *S) {
   if (n > 0) {
     hipLaunchKernelGGL(k_va_count, dim3(div_up((long long)n * BG, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_va_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
-    hipLaunchKernelGGL(k_valence, dim3(std::min(WL_MAX_WAVES, n)), dim3(SWR_WAVE), 0, S->stream, A);
+    int sets = 0;   // most parameter sets of one angle type
+    for (int q = 0; q < SWR_MAX_ELEM * SWR_MAX_ELEM * SWR_MAX_ELEM; q++) sets = std::max(sets, (int)S->hp.thb_n[q]);
+    const dim3 waves(std::min(WL_MAX_WAVES, n)), wave(SWR_WAVE);
+    if (sets <= 2) hipLaunchKernelGGL(k_valence<2>, waves, wave, 0, S->stream, A);
+    else hipLaunchKernelGGL(k_valence<SWR_MAX_THB>, waves, wave, 0, S->stream, A);
   }
   hipLaunchKernelGGL(k_va_fold, dim3(4 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A, S->va_result);
   swr_kt_end(S, KT_VALENCE);
@@ -2114,7 +2141,8 @@ int swr_torsion_angles_run(swr_system *S) {
     hipLaunchKernelGGL(k_to_count, dim3(div_up((long long)n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_to_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     const int waves = (int)std::min<long long>(WL_MAX_WAVES, 8LL * n);
-    hipLaunchKernelGGL(k_torsion, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
+    if (n >= 131072) hipLaunchKernelGGL(k_torsion<2>, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
+    else hipLaunchKernelGGL(k_torsion<1>, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
   }
   hipLaunchKernelGGL(k_to_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A);
   hipLaunchKernelGGL(k_to_sum, dim3(2), dim3(BT), 0, S->stream, n, (const double *)S->to_part, stride, S->to_result);

@@ -314,3 +314,53 @@ def test_gpu_set_atoms_uploads(gpu_lib, ffield, n):
     if n > 1:
         with pytest.raises(_lib.SwrError, match="owner out of range"):
             h.set_atoms(n // 2, x, t, tag, owner=bad)
+
+
+@pytest.mark.gpu
+def test_gpu_valence_with_many_parameter_sets(gpu_lib, oracle_lib, ffield, tmp_path):
+    """Three parameter sets for H-O-H and H-C-H and five for H-C-O, more than the usual two that the
+    valence pass's smaller form has room for."""
+    lines = open(ffield).read().splitlines()
+    k = next(i for i, l in enumerate(lines) if "Nr of angles" in l)
+    n = int(lines[k].split()[0])
+    extra = []
+    for l in lines[k + 1:k + 1 + n]:
+        t = l.split()
+        sets = {"232": 3, "212": 3, "213": 5, "312": 5}.get("".join(t[:3]), 1)   # (at most 3 where both ends are alike)
+        for m in range(1, sets):
+            extra.append("  ".join(t[:3] + [f"{float(t[3]) + 4.0 * m:.4f}", f"{float(t[4]) * (1.0 - 0.15 * m):.4f}"] + t[5:]))
+    assert len(extra) == 8
+    lines[k] = lines[k].replace(str(n), str(n + len(extra)), 1)
+    path = str(tmp_path / "ffield.sets")
+    with open(path, "w") as f:
+        f.write("\n".join(lines[:k + 1 + n] + extra + lines[k + 1 + n:]) + "\n")
+    s = systems.cluster(700, seed=9)
+    h = harness(s, path, tol=1e-10)
+    _gpu_vs_oracle(oracle_lib, path, h, s.elements, s.type, s.tag)
+    plain = harness(s, ffield, tol=1e-10)
+    plain.system.call("valence_angles")
+    plain.system.sync()
+    assert plain.system.get("valence_energy")[0] != h.system.get("valence_energy")[0]
+
+
+@pytest.mark.gpu
+def test_gpu_torsions_of_a_large_batch(gpu_lib, ffield):
+    """131,072 atoms and more take the torsion pass's form with two waves a SIMD:
+    each member's energies are those of a batch of three (whose other members
+    put it elsewhere in the box: coordinates of ~1e3 A round at 1e-13)."""
+    from sw_reaxff_amd.batch import Batch
+    kinds = [systems.cluster(m, seed=m) for m in (60, 75, 90)]
+    got = []
+    for reps in (1, 131072 // sum(k.n for k in kinds) + 1):
+        bt = Batch(tol=1e-6)
+        parts = kinds * reps
+        bt.load(parts)
+        bt.evaluate(nonbonded=False, bonded=True)
+        n = bt.sys.scalar("n")
+        assert (n >= 131072) == (reps > 1)
+        got.append([bt.sys.get(k).reshape(-1, n) for k in ("torsion_eatom", "valence_eatom")])
+    per = sum(k.n for k in kinds)
+    for a, b in zip(*got):
+        assert np.abs(a).max() > 1e-3
+        for r in (0, 1, b.shape[1] // per - 1):
+            assert np.max(np.abs(b[:, r * per:(r + 1) * per] - a)) <= 1e-8 * np.abs(a).max()
