@@ -480,9 +480,7 @@ int swr_new_atoms(swr_system *S) {
   if (!S) return SWR_ERR_ARG;
   if (int rc = swr_quiesce(S)) return rc;
   if (S->ncap > 0) {
-    HIP_CHECK(hipMemsetAsync(S->s_hist, 0, sizeof(double) * 5 * S->ncap, S->stream));
-    HIP_CHECK(hipMemsetAsync(S->t_hist, 0, sizeof(double) * 5 * S->ncap, S->stream));
-    HIP_CHECK(hipMemsetAsync(S->st, 0, sizeof(double) * 2 * S->ncap, S->stream));
+    if (int rc = swr_qeq_clear(S)) return rc;
   }
   S->capacities_set = false;
   S->next_totals_known = false;
@@ -563,7 +561,7 @@ int swr_reset(swr_system *S) {
   if ((rc = swr_quiesce(S))) return rc;  // Reset rewrites the bond ranges a pending relaxation reads
   if (!S->capacities_set) {
     // setup-time estimate (Estimate_Storages) from a counting pass
-    if ((rc = swr_lists_pack(S)) || (rc = swr_lists_estimate(S))) return rc;
+    if ((!S->just_packed && (rc = swr_lists_pack(S))) || (rc = swr_lists_estimate(S))) return rc;
     S->capacities_set = true;
     S->next_totals_known = false;
     S->lists_estimated = true;
@@ -732,7 +730,10 @@ int swr_pair_compute(swr_system *S) {
   int rc;
   if ((rc = swr_write_reax_atoms_and_pack(S))) return rc;
   S->lists_estimated = false;
-  if ((rc = swr_reset(S))) return rc;
+  S->just_packed = true;
+  rc = swr_reset(S);
+  S->just_packed = false;
+  if (rc) return rc;
   // new atoms: Reset's capacity estimate has just written these packed atoms'
   // far list, so only the bonds and hydrogen bonds are left to write
   const bool far_done = S->lists_estimated && S->bonds;

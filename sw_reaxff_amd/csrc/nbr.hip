@@ -285,8 +285,9 @@ __global__ void __launch_bounds__(RS_T) k_rs_scatter(const int *__restrict__ key
 // Atoms per bin from the sorted keys (bins without atoms keep the zero they
 // were cleared to): the first lane of each run of equal keys in a wave adds
 // the run's length there.
-__global__ void k_bin_runs(const int *__restrict__ skeys, int N, int *__restrict__ bin_count) {
+__global__ void k_bin_runs(const int *__restrict__ skeys, int N, int *__restrict__ bin_count, int *__restrict__ occ) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) occ[0] = 0;   // k_bin_pos counts from here
   const int key = k < N ? skeys[k] : -1;
   const int before = __shfl_up(key, 1, SWR_WAVE);
   const bool first = key >= 0 && (lane_id() == 0 || before != key);
@@ -498,18 +499,16 @@ __global__ void __launch_bounds__(256) k_bbox(const double *__restrict__ x, int 
     __syncthreads();
   }
   if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
+  __threadfence_system();   // (part is the host's memory)
 }
 }  // namespace
 
 // Bounding box of all N atoms (lo, hi on the host).
 int swr_nbr_bbox(swr_system *S, double lo[3], double hi[3]) {
-  int rc = swr_ensure_tmp(S, sizeof(double) * 6 * BBOX_BLOCKS);
-  if (rc) return rc;
-  double *part = (double *)S->tmp_i;
-  double h[6 * BBOX_BLOCKS];
-  hipLaunchKernelGGL(k_bbox, dim3(BBOX_BLOCKS), dim3(256), 0, S->stream, S->x, S->N, part);
+  static_assert(sizeof(double) * 6 * BBOX_BLOCKS <= SWR_PIN_MIX, "the partial boxes fit");
+  double *h = (double *)S->pin_mix;   // (no mixed solve runs meanwhile)
+  hipLaunchKernelGGL(k_bbox, dim3(BBOX_BLOCKS), dim3(256), 0, S->stream, S->x, S->N, h);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(h, part, sizeof(h), hipMemcpyDeviceToHost, S->stream));
   HIP_CHECK(hipStreamSynchronize(S->stream));
   for (int d = 0; d < 3; d++) { lo[d] = 1e300; hi[d] = -1e300; }
   for (int b = 0; b < BBOX_BLOCKS; b++)
@@ -707,8 +706,7 @@ int swr_nbr_build(swr_system *S, int local_only) {
       vin = vout;
     }
     HIP_CHECK(hipMemsetAsync(S->bin_count, 0, sizeof(int) * (S->nbins + 1), S->stream));
-    HIP_CHECK(hipMemsetAsync(S->bin_occ, 0, sizeof(int), S->stream));
-    hipLaunchKernelGGL(k_bin_runs, dim3(div_up(N, 256)), dim3(256), 0, S->stream, kin, N, S->bin_count);
+    hipLaunchKernelGGL(k_bin_runs, dim3(div_up(N, 256)), dim3(256), 0, S->stream, kin, N, S->bin_count, S->bin_occ);
     skeys = kin;
   }
   if ((rc = swr_scan_i32(S, S->bin_count, S->bin_start, S->nbins + 1, nullptr))) return rc;
@@ -729,8 +727,10 @@ int swr_nbr_build(swr_system *S, int local_only) {
   if ((rc = swr_scan_i32_to_i64(S, S->vcount, S->voff, N, nullptr))) return rc;
   // the total, and the local rows' share (the H matrix capacity)
   long long *vt = (long long *)(S->pin_done + SWR_PIN_VERLET);
-  HIP_CHECK(hipMemcpyAsync(vt, S->voff + N, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
-  HIP_CHECK(hipMemcpyAsync(vt + 1, S->voff + S->n, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
+  SwrPublish pub;
+  pub.src[0] = (const int *)(S->voff + N); pub.dst[0] = (int *)vt; pub.words[0] = 2;
+  pub.src[1] = (const int *)(S->voff + S->n); pub.dst[1] = (int *)(vt + 1); pub.words[1] = 2;
+  if ((rc = swr_publish(S, pub))) return rc;
   HIP_CHECK(hipStreamSynchronize(S->stream));
   const long long total = vt[0];
   if (total > S->vcap) {

@@ -476,6 +476,21 @@ k_publish(SwrPublish P) {
 }
 }  // namespace
 
+namespace {
+__global__ void k_qeq_clear(int n, double *__restrict__ s_hist, double *__restrict__ t_hist, double *__restrict__ st) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 5 * n) s_hist[i] = t_hist[i] = 0.0;
+  if (i < 2 * n) st[i] = 0.0;
+}
+}  // namespace
+
+int swr_qeq_clear(swr_system *S) {
+  hipLaunchKernelGGL(k_qeq_clear, dim3(div_up(5LL * S->ncap, 256)), dim3(256), 0, S->stream, S->ncap, S->s_hist,
+                     S->t_hist, (double *)S->st);
+  HIP_CHECK(hipGetLastError());
+  return SWR_OK;
+}
+
 int swr_publish(swr_system *S, const SwrPublish &P) {
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(256), 0, S->stream, P);
   HIP_CHECK(hipGetLastError());

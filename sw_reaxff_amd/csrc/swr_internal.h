@@ -257,6 +257,7 @@ struct swr_system {
   int hbond_cap = 0;
   int *hbslot = nullptr;           // far slots of the estimate pass's hydrogen bonds, at their rows' Verlet offsets
   size_t cap_hbslot = 0;
+  bool just_packed = false;        // Reset need not pack the atoms for its estimate
   bool lists_estimated = false;    // the Reset just done ran the estimate: far list and candidates are current
   swr_hbond_t *hbonds = nullptr;
   bool capacities_set = false;
@@ -482,6 +483,7 @@ struct SwrQGate {
 int swr_qeq_calc_q(swr_system *S, SwrQGate gate);
 // Copies bytes of host memory that the caller may change at once to dst, by way
 // of the system's own pinned memory `which` (grown, never shrunk).
+int swr_qeq_clear(swr_system *S);   // histories and solutions to zero
 int swr_upload(swr_system *S, int which, void *dst, const void *src, size_t bytes);
 // The two halves of it, for a source that is written into the pinned memory.
 int swr_stage_ready(swr_system *S, int which, size_t bytes);
