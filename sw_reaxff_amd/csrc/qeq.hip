@@ -405,6 +405,7 @@ int swr_qeq_layout(swr_system *S) {
   S->nsys = nsys;
   S->ntiles = ntiles;
   S->cg_small = small_rule(S->sys_row, S->mixed);
+  S->cg_tiny = S->cg_small && tiny_rule(S->sys_row);
   S->h_sys_iters.assign(2 * nsys, 0);
   S->layout_dirty = false;
   S->layout_gen++;

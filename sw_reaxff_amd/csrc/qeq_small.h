@@ -16,6 +16,8 @@
 // a dot into 1e-8 of the charges.)
 #pragma once
 
+#include <type_traits>
+
 #include "qeq_cg.h"
 
 namespace swr_cg {
@@ -130,9 +132,21 @@ __device__ __forceinline__ void small_store(CgScalars *o, const CgScalars &c) {
 // values.  One barrier covers the LDS vector and the scalars.  A step in
 // which neither solve goes on to another A step only adds alpha p to x: no
 // product.
-template <int PH, int SH>
-__global__ void __launch_bounds__(SpmvShape<SH>::NT)
-k_cg_small(SmallArgs A) {
+//
+// Returns whether the system goes on (PH_A1, PH_K).
+template <int ROWS, int NDOT>
+struct SmallLds {
+  double2 xl[ROWS];
+  double2 ql[SWR_PANEL_ROWS];
+  double prod[NDOT][SWR_PANEL_ROWS];   // each row's products
+  double sc[6];                        // alpha_x, beta, alpha_a of s and t
+  int sflag;                           // active_b, active_a of s and t
+};
+constexpr bool small_multiplies(int PH) { return PH != PH_A1; }
+constexpr int small_dots_out(int PH) { return PH == PH_S3 ? 6 : PH == PH_A1 || PH == PH_K ? 4 : 0; }
+
+template <int PH, int SH, class Lds>
+__device__ __forceinline__ bool small_step_body(const SmallArgs &A, const int p, Lds &S) {
   constexpr int NT = SpmvShape<SH>::NT, G = SpmvShape<SH>::G;
   constexpr int U = 2;                                  // (a row's sum does not depend on it)
   constexpr int NW = NT / SWR_WAVE;
@@ -142,24 +156,19 @@ k_cg_small(SmallArgs A) {
   constexpr bool DOTS = PH == PH_S3 || PH == PH_A1 || PH == PH_K;
   constexpr int NDIN = PH == PH_A1 ? 6 : 4;             // dots of the step before
   constexpr int NDOUT = PH == PH_S3 ? 6 : 4;
-  __shared__ double2 xl[MUL ? SMALL_ROWS : 1];
-  __shared__ double2 ql[MUL ? SWR_PANEL_ROWS : 1];
-  __shared__ double prod[DOTS ? NDOUT : 1][SWR_PANEL_ROWS];   // each row's products
-  __shared__ double sc[6];    // alpha_x, beta, alpha_a of s and t
-  __shared__ int sflag;       // active_b, active_a of s and t
-  const int p = blockIdx.x;
+  auto &xl = S.xl;
+  auto &ql = S.ql;
+  auto &prod = S.prod;
+  auto &sc = S.sc;
+  int &sflag = S.sflag;
   const SmallPanel pn = A.panel[p];
   const int r0 = pn.r0, r1 = pn.r1;
   const double2 zero = make_double2(0.0, 0.0);
-  if (PH == PH_S1 && p == 0) {
-    for (int k = threadIdx.x; k < 2 * A.nsys; k += NT) A.iters_out[k] = 1;   // (kept by a system without rows)
-    if (threadIdx.x == 0) *A.done_count = 0;
-  }
   if (PH == PH_K) {   // a system that finished before: its scalars move on to the other buffer
     const CgScalars *c = A.cin + 2 * pn.sys;
     if ((c[0].active_a | c[0].active_b | c[1].active_a | c[1].active_b) == 0) {
       if (p == pn.p0 && threadIdx.x < 2) A.cout[2 * pn.sys + threadIdx.x] = c[threadIdx.x];
-      return;
+      return false;
     }
   }
 
@@ -281,7 +290,7 @@ k_cg_small(SmallArgs A) {
     b1 = f & 2;
     a0 = f & 4;
     a1 = f & 8;
-    if (f == 0) return;   // both solves finished
+    if (f == 0) return false;   // both solves finished
     if (PH == PH_K) multiply = a0 || a1;
   }
   const double ax0 = sc[0], be0 = sc[1], aa0 = sc[2], ax1 = sc[3], be1 = sc[4], aa1 = sc[5];
@@ -393,13 +402,79 @@ k_cg_small(SmallArgs A) {
       }
     }
   }
-  if (!DOTS) return;
+  if (!DOTS) return true;
   // ---- the panel's partial dots, each by one wave over the rows
   lds_barrier();
   for (int k = wave_in_block(); k < NDOUT; k += NW) {
     const double v = wave_sum(prod[k][lane_id()]);
     if (lane_id() == 0) A.part_out[(size_t)k * A.pstride + p] = v;
   }
+  return true;
+}
+
+// Before a solve: no system has finished; a system without rows keeps the
+// counts.
+__device__ __forceinline__ void small_begin(const SmallArgs &A) {
+  for (int k = threadIdx.x; k < 2 * A.nsys; k += blockDim.x) A.iters_out[k] = 1;
+  if (threadIdx.x == 0) *A.done_count = 0;
+}
+
+template <int PH, int SH>
+__global__ void __launch_bounds__(SpmvShape<SH>::NT)
+k_cg_small(SmallArgs A) {
+  __shared__ SmallLds<small_multiplies(PH) ? SMALL_ROWS : 1, small_dots_out(PH) ? small_dots_out(PH) : 1> S;
+  if (PH == PH_S1 && blockIdx.x == 0) small_begin(A);
+  small_step_body<PH, SH>(A, blockIdx.x, S);
+}
+
+// ---------------------------------------------------------------- tiny systems
+// When every system has at most TINY_PANELS panels, one workgroup runs its
+// system's whole solve in one launch: the steps above in turn, a barrier
+// between steps.  A launch per iteration is 6.5 us of latency for 2 us of
+// work, fifteen to twenty times over (charges of 60 atoms 216 us, of 64 such
+// systems 265; this 153 and 171, 512 of them 343 either way).  The same
+// functions in the same order: the same bits.  With two panels a workgroup
+// would take them in turn that the launches spread over the chip: 120 atoms
+// 323 us against 280.
+constexpr int TINY_PANELS = 1;
+constexpr int TINY_ROWS = TINY_PANELS * SWR_PANEL_ROWS;
+
+__global__ void __launch_bounds__(256) k_cg_tiny_begin(SmallArgs A) { small_begin(A); }
+
+// Scalars and dots of step k: step k reads those of step k - 1 and writes the
+// other buffers.
+__host__ __device__ inline void small_buffers(SmallArgs &A, CgScalars *cgs, double *partials, int ph, int step) {
+  const size_t half = 2 * (size_t)A.nsys, odd = (size_t)SMALL_PART_ODD * A.pstride;
+  const bool k_odd = ph == PH_K && (step & 1);
+  A.cin = cgs + (ph == PH_K && !k_odd ? half : 0);
+  A.cout = cgs + (k_odd ? half : 0);
+  A.part_in = partials + (k_odd ? odd : 0);
+  A.part_out = partials + (ph == PH_S3 || k_odd ? 0 : odd);
+  A.par_in = (step - 1) & 1;
+}
+
+template <int SH>
+__global__ void __launch_bounds__(SpmvShape<SH>::NT)
+k_cg_tiny(SmallArgs A, CgScalars *cgs, double *partials, const int *__restrict__ sys_panel) {
+  __shared__ SmallLds<TINY_ROWS, 6> S;
+  const int p0 = sys_panel[blockIdx.x], p1 = sys_panel[blockIdx.x + 1];
+  if (p0 >= p1) return;
+  auto phase = [&](auto phc, int step) {
+    constexpr int PH = decltype(phc)::value;
+    small_buffers(A, cgs, partials, PH, step);
+    bool on = true;
+    for (int p = p0; p < p1; p++) {
+      on = small_step_body<PH, SH>(A, p, S);
+      __syncthreads();   // the next step reads what this one stored
+    }
+    return on;
+  };
+  phase(std::integral_constant<int, PH_S1>(), 0);
+  phase(std::integral_constant<int, PH_S2>(), 0);
+  phase(std::integral_constant<int, PH_S3>(), 0);
+  if (!phase(std::integral_constant<int, PH_A1>(), 0)) return;
+  for (int k = 1; k <= A.imax; k++)
+    if (!phase(std::integral_constant<int, PH_K>(), k)) return;
 }
 
 // The vectors in CG scratch of CGV_COUNT slots of cap entries.
@@ -426,22 +501,28 @@ inline int small_step(swr_system *S, const CgRun<double, double> &R, const Small
   A.val = R.val;
   A.panel = (const SmallPanel *)S->small_panel;
   A.V = V;
-  // step k reads the scalars and dots of step k-1 and writes the other buffers
-  const size_t half = 2 * (size_t)R.L.nsys, odd = (size_t)SMALL_PART_ODD * R.pstride;
-  const bool k_odd = ph == PH_K && (step & 1);
-  A.cin = R.cgs + (ph == PH_K && !k_odd ? half : 0);
-  A.cout = R.cgs + (k_odd ? half : 0);
-  A.part_in = R.partials + (k_odd ? odd : 0);
-  A.part_out = R.partials + (ph == PH_S3 || k_odd ? 0 : odd);
   A.pstride = R.pstride;
   A.nsys = R.L.nsys;
+  small_buffers(A, R.cgs, R.partials, ph, step);
   A.imax = R.imax;
   A.tol = R.tol;
   A.iters_out = R.iters_out;
   A.done_count = R.L.done_count;
   A.status = S->status;
-  A.par_in = (step - 1) & 1;
   const int kt = ph == PH_K ? R.kt_iter : R.kt_setup;
+  if (S->cg_tiny) {   // the first step is the whole solve
+    if (ph != PH_S1) return SWR_OK;
+    swr_kt_begin(S, kt);
+    hipLaunchKernelGGL(k_cg_tiny_begin, dim3(1), dim3(256), 0, S->stream, A);
+    spmv_dispatch(S->spmv_shape[0], [&](auto shc) {
+      constexpr int SH = decltype(shc)::value;
+      hipLaunchKernelGGL(k_cg_tiny<SH>, dim3((unsigned)S->sys_row.size() - 1), dim3(SpmvShape<SH>::NT), 0, S->stream, A,
+                         R.cgs, R.partials, (const int *)S->sys_panel);
+    });
+    swr_kt_end(S, kt);
+    HIP_CHECK(hipGetLastError());
+    return SWR_OK;
+  }
   swr_kt_begin(S, kt);
   spmv_dispatch(S->spmv_shape[0], [&](auto shc) {
     constexpr int SH = decltype(shc)::value;
@@ -459,6 +540,13 @@ inline int small_step(swr_system *S, const CgRun<double, double> &R, const Small
   swr_kt_end(S, kt);
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
+}
+
+// Whether every system has at most TINY_PANELS panels (and the rule below holds).
+inline bool tiny_rule(const std::vector<int> &sys_row) {
+  for (size_t k = 0; k + 1 < sys_row.size(); k++)
+    if (sys_row[k + 1] - sys_row[k] > TINY_ROWS) return false;
+  return true;
 }
 
 // Whether the rule above holds for S's systems.

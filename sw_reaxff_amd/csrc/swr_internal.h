@@ -361,6 +361,7 @@ struct swr_system {
   // ---- batch of independent systems (one unless swr_set_batch)
   std::vector<int> sys_row;        // nsys + 1 local-row offsets (host)
   int nsys = 1, ntiles = 0;
+  bool cg_tiny = false;            // and one launch for all of it (one workgroup a system)
   bool cg_small = false;           // the FP64 solve takes one launch per iteration (qeq_small.h)
   bool layout_dirty = true;
   int *atoms_in = nullptr;         // an upload of swr_set_atoms, before k_unpack_atoms spreads it

@@ -105,12 +105,50 @@ def test_gpu_cg_sizes_against_oracle(gpu_lib, oracle_lib, ffield, m):
 
 
 @pytest.mark.gpu
-def test_gpu_small_cg_with_an_empty_system(gpu_lib, ffield):
-    """A batch may hold systems without rows: nothing waits for them."""
+def test_gpu_tiny_cg_takes_the_small_solves_bits(gpu_lib, ffield):
+    """Systems of 3 to 64 rows, solved in one launch; with the last two declared
+    one system of 120 rows the batch takes a launch per iteration: the others'
+    charges and iteration counts are the same bits, in a first solve and from its
+    history."""
     import ctypes as C
 
     from sw_reaxff_amd import _lib
-    s = waters(30, seed=3)
+    from sw_reaxff_amd.batch import Batch
+    w = waters(22, seed=8)
+    cut = systems.System(x=w.x[:64], v=w.v[:64], type=w.type[:64], tag=w.tag[:64], elements=w.elements, lo=w.lo,
+                         hi=w.hi, periodic=False)
+    parts = [waters(1, seed=1), waters(7, seed=2), systems.cluster(20, seed=1), waters(21, seed=3), cut,
+             waters(20, seed=4), waters(20, seed=5)]
+    assert [s.n for s in parts] == [3, 21, 21, 63, 64, 60, 60]
+    got = []
+    for merge in (False, True):
+        bt = Batch(ffield, tol=1e-6)
+        P = bt.load(parts)
+        off = np.ascontiguousarray(np.delete(P.row_off, -2) if merge else P.row_off, dtype=np.int32)
+        h = bt.sys
+        _lib.check(h.L.swr_set_batch(h.h, off.size - 1, off.ctypes.data_as(C.POINTER(C.c_int))), "swr_set_batch")
+        h.build_neighbors(10.0)
+        n = int(P.row_off[5])
+        for _ in range(3):
+            h.call("qeq_init_matvec")
+            h.qeq_cg()
+            h.call("calculate_q")
+            h.sync()
+            got.append((merge, h.get("q")[:n], h.get("sys_iters").reshape(-1, 2)[:5].copy()))
+    for a, b in zip(got[:3], got[3:]):
+        assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+    assert got[0][2].max() > 10
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [20, 30])
+def test_gpu_small_cg_with_an_empty_system(gpu_lib, ffield, m):
+    """A batch may hold systems without rows: nothing waits for them (60 rows:
+    one launch for the solve; 90: one per iteration)."""
+    import ctypes as C
+
+    from sw_reaxff_amd import _lib
+    s = waters(m, seed=3)
     got = []
     for off in ([0, s.n], [0, 0, s.n, s.n]):
         h = _lib.System(ffield, s.elements, tol=1e-6)
