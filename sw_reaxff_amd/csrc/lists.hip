@@ -888,17 +888,18 @@ __global__ void __launch_bounds__(SWR_WAVE) k_validate_end(DevStatus *st, int *_
 // higher neighbours (k_mark_up; in LDS too up to BFS_LDS ghosts): exact when
 // it ends.
 //
-// More (k_bond_mark): a workgroup relaxes MARK_T consecutive ghosts to their
-// local fixed point in LDS (each thread keeps its ghost's bonds to lower atoms
-// in registers), reading the marks of the others MARK_ROUNDS times a launch as
-// the other workgroups' updates land (relaxed atomics).  chg[launch] is set
-// when the launch changed a mark; a launch in which none changed has reached
-// the fixed point, and a launch after it does nothing.  Each launch clears the
-// flag of the next (a stale chg[0] only makes the host look one launch
-// further).
+// More (k_bond_mark): each ghost lowers its mark from its lower neighbours',
+// whose ids it keeps in registers, MARK_SWEEPS times a launch as the others'
+// updates land (relaxed atomics): a hop is one gather.  chg[launch] is set when
+// the launch changed a mark; a launch in which none changed has reached the
+// fixed point, and a launch after it does nothing.  Each launch clears the flag
+// of the next (a stale chg[0] only makes the host look one launch further).
 //
-// Relaxing in global memory alone, 1.6 us a hop in 4 to 7 launches, took 49 us
-// on a 64-water box, 76 on 648 waters, 94 on 2,667 and 100 on 32,000.
+// Walking the bond list for every hop, 1.6 us each, took 49 us on a 64-water
+// box, 76 on 648 waters, 94 on 2,667 and 106 on 32,000 (149 after 200 steps of
+// MD); with the ids in registers 32,000 take 59 (87).  Relaxing 1024 ghosts at
+// a time to their local fixed point in LDS: 85, but 260 after 200 steps, when
+// the chains cross its blocks more often.  Six ids and 8 sweeps: 65 (110).
 constexpr int MARK_BFS = 32512;  // (a ghost's position and two codes in 15 bits)
 constexpr int BFS_LDS = 12288;
 constexpr int BFS_T = 1024;
@@ -982,88 +983,51 @@ k_mark_bfs(int n, int N, const int *__restrict__ bond_index, const int *__restri
   }
 }
 
-constexpr int MARK_T = 1024;
-constexpr int MARK_NB = 6;       // bonds to lower atoms kept in registers
-constexpr int MARK_ROUNDS = 2;   // reads of the outside marks per launch
-constexpr int MARK_SUB = 4;      // passes over the block's bonds between barriers
+constexpr int MARK_T = 256;
+constexpr int MARK_NB = 8;       // bonds to lower atoms kept in registers
+constexpr int MARK_SWEEPS = 12;   // per launch
 
 __global__ void __launch_bounds__(MARK_T)
 k_bond_mark(int n, int N, int launch, const int *__restrict__ bond_index, const int *__restrict__ bond_end,
             const int *__restrict__ bond_nbr, int *__restrict__ mark, int *__restrict__ chg) {
-  __shared__ int m[MARK_T];
-  volatile int *vm = m;
   const bool done = launch > 0 && __hip_atomic_load(&chg[launch - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
   if (blockIdx.x == 0 && threadIdx.x == 0 && launch + 1 < MARK_MAX_LAUNCH)
     __hip_atomic_store(&chg[launch + 1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (done) return;
-  const int t = threadIdx.x, g0 = n + blockIdx.x * MARK_T, g = g0 + t;
-  const bool live = g < N;
-  const int p0 = live ? bond_index[g] : 0, p1 = live ? bond_end[g] : 0;
-  const int first = live ? __hip_atomic_load(&mark[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-  // bonds to lower atoms inside the block (LDS positions) and outside (ids);
-  // unused ones are the ghost itself, which never lowers it, so that the
-  // passes below read all of them at once
-  int in[MARK_NB], out[MARK_NB];
+  const int g = n + blockIdx.x * MARK_T + threadIdx.x;
+  if (g >= N) return;
+  const int p1 = bond_end[g];
+  int p = bond_index[g];
+  int cur = __hip_atomic_load(&mark[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int first = cur;
+  // the first bonds to lower atoms; the others are walked from p on (rare).
+  // Unused places are the ghost itself, which never lowers it, so that a
+  // sweep reads all of them at once
+  int lower[MARK_NB];
 #pragma unroll
-  for (int k = 0; k < MARK_NB; k++) {
-    in[k] = t;
-    out[k] = live ? g : n;
-  }
-  int nin = 0, nout = 0;
-  for (int p = p0; p < p1; p++) {
+  for (int k = 0; k < MARK_NB; k++) lower[k] = g;
+  for (int cnt = 0; p < p1 && cnt < MARK_NB; p++) {
     const int j = bond_nbr[p];
     if (j >= g) continue;
-    const bool inside = j >= g0;
 #pragma unroll
-    for (int k = 0; k < MARK_NB; k++) {
-      if (inside && nin == k) in[k] = j - g0;
-      if (!inside && nout == k) out[k] = j;
-    }
-    nin += inside;
-    nout += !inside;
+    for (int k = 0; k < MARK_NB; k++)
+      if (cnt == k) lower[k] = j;
+    cnt++;
   }
-  const bool more = nin > MARK_NB || nout > MARK_NB;   // (rare: the rest walked in the list)
-  int cur = first, told = first;
-  vm[t] = cur;
-  __syncthreads();
-  for (int round = 0; round < MARK_ROUNDS; round++) {
+  for (int sweep = 0; sweep < MARK_SWEEPS; sweep++) {
     int v[MARK_NB];
 #pragma unroll
-    for (int k = 0; k < MARK_NB; k++) v[k] = __hip_atomic_load(&mark[out[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < MARK_NB; k++)
+      v[k] = __hip_atomic_load(&mark[lower[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int best = cur;
 #pragma unroll
     for (int k = 0; k < MARK_NB; k++) best = min(best, v[k] + 1);
-    if (more)
-      for (int p = p0; p < p1; p++) {
-        const int j = bond_nbr[p];
-        if (j < g0) best = min(best, __hip_atomic_load(&mark[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
-      }
-    bool lower = live && best < cur;
-    if (lower) vm[t] = cur = best;
-    // the block's own chains: MARK_SUB passes between barriers, each reading
-    // what the other waves hold by then; passes in which no mark fell have
-    // settled them (every other set lowers a mark, so it ends)
-    while (__syncthreads_or(lower)) {
-      lower = false;
-      for (int sub = 0; sub < MARK_SUB; sub++) {
-#pragma unroll
-        for (int k = 0; k < MARK_NB; k++) v[k] = vm[in[k]];
-        best = cur;
-#pragma unroll
-        for (int k = 0; k < MARK_NB; k++) best = min(best, v[k] + 1);
-        if (more)
-          for (int p = p0; p < p1; p++) {
-            const int j = bond_nbr[p];
-            if (j >= g0 && j < g) best = min(best, vm[j - g0] + 1);
-          }
-        if (live && best < cur) {
-          vm[t] = cur = best;
-          lower = true;
-        }
-      }
+    for (int q = p; q < p1; q++) {
+      const int j = bond_nbr[q];
+      if (j < g) best = min(best, __hip_atomic_load(&mark[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
     }
-    if (cur < told) {
-      told = cur;
+    if (best < cur) {
+      cur = best;
       __hip_atomic_store(&mark[g], cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }

@@ -192,7 +192,7 @@ def test_gpu_bond_marks_of_crowded_ghosts(gpu_lib, ffield, m, a):
         most = max(most, int((j > i).sum()), int((j < i).sum()))
         if j.size:
             mark[i] = min(mark[i], (mark[j] + 1).min())
-    assert most > 6 and (mark[n:] < 1000).any()
+    assert most > 8 and (mark[n:] < 1000).any()
     assert {8: N - n <= 12288, 10: 12288 < N - n <= 32512, 21: N - n > 32512}[m]
     assert np.array_equal(h.get("bond_mark")[:N], mark)
 
