@@ -439,6 +439,7 @@ int swr_set_atoms(swr_system *S, int n, int N, const int *tag, const int *type, 
   if ((rc = swr_nbr_ensure_atoms(S, std::max(N, 1))) || (rc = ensure_local(S, std::max(n, 1)))) return rc;
   if (n != S->n) {
     S->qeq_initialized = 0;
+    S->H_rows = 0;
     S->sys_row.clear();  // a new atom set is one system until swr_set_batch
   }
   S->layout_dirty = true;
@@ -627,6 +628,7 @@ int swr_qeq_init_matvec(swr_system *S) {
   // (qeq.hip): the last row ends by (voff[n] + 4 n + 3) & ~3
   need = (need + 4LL * S->n + 3) & ~3LL;
   int rc;
+  S->H_rows = 0;   // until this build is queued
   if (need > S->Hcap) {
     long long cap = (long long)(need * 1.15) + 1024;
     if ((rc = swr_alloc(&S->H_jlist, cap)) || (rc = swr_alloc(&S->H_val, cap))) return rc;

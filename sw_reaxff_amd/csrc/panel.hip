@@ -255,6 +255,25 @@ int swr_panel_build(swr_system *S) {
   return S->cg_small ? SWR_OK : swr_panel_lists(S);
 }
 
+int swr_H_check(const swr_system *S) {
+  if (S->n > 0 && S->H_rows == S->n) return SWR_OK;
+  swr_set_error_msg("QEq: no H of the current atoms (call swr_qeq_init_matvec first)");
+  return SWR_ERR_STATE;
+}
+
+int swr_panel_ready(swr_system *S) {
+  int rc;
+  if ((rc = swr_H_check(S)) || (rc = swr_qeq_layout(S))) return rc;
+  if (swr_panel_current(S) && (S->cg_small || S->panel_lists)) return SWR_OK;
+  return swr_panel_build(S);
+}
+
+int swr_panel_gather(swr_system *S) {
+  hipLaunchKernelGGL(k_panels_off, dim3(div_up(S->npanel, 256)), dim3(256), 0, S->stream, S->npanel, S->pcnt);
+  HIP_CHECK(hipGetLastError());
+  return SWR_OK;
+}
+
 int swr_panel_lists(swr_system *S) {
   if (S->panel_lists || S->npanel <= 0) return SWR_OK;
   const int np = S->npanel;

@@ -278,7 +278,9 @@ int swr_qeq_build_H(swr_system *S) {
                      S->s_hist, S->t_hist);
   swr_kt_end(S, KT_BUILD_H);
   HIP_CHECK(hipGetLastError());
-  return swr_panel_build(S);
+  if (int rc = swr_panel_build(S)) return rc;
+  S->H_rows = n;
+  return SWR_OK;
 }
 
 int swr_qeq_spmv(swr_system *S, const double *xv, double *b) {
@@ -428,10 +430,9 @@ CgLayout swr_qeq_cg_layout(swr_system *S) {
 // in shape sh on the current H and vectors (the setup-phase instance, which
 // multiplies d0 into q and always runs; both are scratch between solves).
 int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
-  int rc = swr_qeq_layout(S);
-  if (rc) return rc;
+  int rc;
   if (!S->H_val || S->n <= 0) return SWR_ERR_STATE;
-  if ((rc = swr_panel_lists(S))) return rc;
+  if ((rc = swr_panel_ready(S)) || (rc = swr_panel_lists(S))) return rc;
   CgVecsT<double> V = make_vecs(S);
   const int n = S->n;
   const CgScalars *cgs = S->cgs;
@@ -500,7 +501,7 @@ int swr_publish(swr_system *S, const SwrPublish &P) {
 
 int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
   const int first_batch = last_iters > 0 ? last_iters + 1 : CG_COLD_BATCH;
-  int rc = swr_qeq_layout(S);
+  int rc = swr_panel_ready(S);
   if (rc) return rc;
   CgRun<double, double> R{};
   R.V = make_vecs(S);
@@ -706,6 +707,7 @@ int swr_qeq_cg_noalloc_run(swr_system *S, const double *b, double *x, int *iters
     return SWR_ERR_ARG;
   }
   if (!b || !x) return SWR_ERR_ARG;
+  if (int rc = swr_H_check(S)) return rc;
   unsigned char *base;
   {
     std::lock_guard<std::mutex> g(na_mu);
@@ -761,13 +763,18 @@ int swr_qeq_cg_noalloc_run(swr_system *S, const double *b, double *x, int *iters
   int rc;
   bool finished = false;
   auto nothing = [] { return (int)SWR_OK; };
-  if (S->cg_small) {   // (its columns have no panel lists)
+  if (S->cg_small && swr_panel_current(S)) {   // (its columns have no panel lists)
     R.pstride = SMALL_ROWS / SWR_PANEL_ROWS;
     const SmallVecs W = small_vecs(R, vb, NA_MAX_ROWS);
     rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return small_step(S, R, W, ph, k); }, nothing, &finished);
   } else {
-    rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); }, nothing,
-                  &finished);
+    // panels of another partition (swr_set_batch since the H build) hold the
+    // same rows in some order, which is all that the general solve needs; lists
+    // that were left out would take an allocation
+    rc = S->panel_lists ? SWR_OK : swr_panel_gather(S);
+    if (!rc)
+      rc = cg_solve(S, R, its0 + 2, 1, [&](int ph, int k) { return launch_cg(S, R, ph, (k - 1) & 1, 0); }, nothing,
+                    &finished);
   }
   S->ktime = ktime;
   if (rc) return rc;

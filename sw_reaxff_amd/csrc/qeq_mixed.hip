@@ -488,7 +488,7 @@ int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_don
     swr_set_error_msg("mixed-precision QEq needs the FP32 H (fix qeq/reax ... mixed at setup)");
     return SWR_ERR_STATE;
   }
-  if ((rc = swr_qeq_layout(S)) || (rc = ensure_mixw(S))) return rc;
+  if ((rc = swr_panel_ready(S)) || (rc = ensure_mixw(S))) return rc;
   static_assert(sizeof(MixCtl) <= MS_OFF, "the batch counters must fit their slot");
   const int n = S->n;
   const int nsys = S->nsys;
@@ -624,6 +624,8 @@ int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_don
 // vectors are scratch between solves).
 int swr_qeq_time_mixed(swr_system *S, int which, int sh, int reps, float *ms) {
   if (!S->mixed || !S->mixw || !S->H_val32 || S->n <= 0) return SWR_ERR_STATE;
+  int rc;
+  if ((rc = swr_panel_ready(S)) || (rc = ensure_mixw(S))) return rc;
   const int n = S->n, nsys = S->nsys;
   const bool batch = nsys > 1;
   const int nblk = S->npanel;

@@ -343,6 +343,7 @@ struct swr_system {
   int *small_panel = nullptr; // qeq_small.h: eight ints per panel (its rows, its system's rows and panels)
   bool panel_lists = false;   // pcol, pcnt and jloc hold the lists of the current H
   long long nbr_gen = 0, layout_gen = 0, prow_nbr_gen = -1, prow_layout_gen = -1;
+  int H_rows = 0;             // local atoms H was built for (0: no H, or of another number of atoms than now)
   int panel_shape = -1;   // tuning family "panels": 0 (default) lists on, 1 off
   int *H_firstnbr = nullptr, *H_numnbrs = nullptr, *H_jlist = nullptr;
   double *H_val = nullptr;
@@ -512,6 +513,14 @@ int swr_radix_sort_i32(swr_system *S, const int *keys, const int *vals_in, int n
 // SpMV panels (panel.hip): row order + panel ranges when stale, then the
 // column lists and local indices of the current H
 int swr_panel_build(swr_system *S);
+// Before a solve: H is of the current atoms, and its panels of the current
+// partition (swr_set_batch may come after the H build).
+int swr_panel_ready(swr_system *S);
+inline bool swr_panel_current(const swr_system *S) {
+  return S->prow_n == S->n && S->prow_layout_gen == S->layout_gen;
+}
+int swr_H_check(const swr_system *S);      // SWR_ERR_STATE unless H is of the current atoms
+int swr_panel_gather(swr_system *S);       // the panels without lists: their rows gather
 // the column lists of the current H where swr_panel_build left them out
 // (small systems, whose solve needs none)
 int swr_panel_lists(swr_system *S);

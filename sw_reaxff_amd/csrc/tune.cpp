@@ -139,8 +139,9 @@ int swr_autotune(swr_system *S, int reps) {
   bool far_done = false;
   for (int fam = 0; fam < kNFam; fam++) {
     if (!kFamilies[fam].timed) continue;
-    const bool ok = fam == 0 ? S->H_val != nullptr
-                  : fam <= 2 ? (S->mixed && S->mixw != nullptr && S->H_val32 != nullptr)
+    const bool h_ok = S->n > 0 && S->H_rows == S->n;
+    const bool ok = fam == 0 ? h_ok && S->H_val != nullptr
+                  : fam <= 2 ? (h_ok && S->mixed && S->mixw != nullptr && S->H_val32 != nullptr)
                              : (S->far != nullptr && S->bonds != nullptr);
     if (!ok) continue;
     rep << ", ";
