@@ -440,6 +440,7 @@ int swr_set_atoms(swr_system *S, int n, int N, const int *tag, const int *type, 
   if (n != S->n) {
     S->qeq_initialized = 0;
     S->H_rows = 0;
+    S->panel_lists = false;
     S->sys_row.clear();  // a new atom set is one system until swr_set_batch
   }
   S->layout_dirty = true;
@@ -909,7 +910,11 @@ bool lookup(swr_system *S, const std::string &k, View &v) {
   if (k == "H_val") return set(S->H_val, 8 * S->Hcap);
   if (k == "H_val32") return set(S->H_val32, S->H_val32 ? 4 * S->Hcap : 0);
   if (k == "Hdia_inv") return set(S->Hdia_inv, 8 * n);
-  if (k == "panel_count" || k == "panel_columns" || k == "H_jloc") (void)swr_panel_lists(S);
+  if ((k == "panel_count" || k == "panel_columns" || k == "H_jloc") && !S->panel_lists) {
+    // small systems' solves leave the lists out: built here from the H there is
+    if (S->n <= 0 || S->H_rows != S->n) return set(nullptr, 0);
+    if (swr_panel_lists(S)) return false;
+  }
   if (k == "panel_rows") return set(S->prow, S->prow ? 4 * (int64_t)S->prow_n : 0);
   if (k == "panel_begin") return set(S->pbeg, S->pbeg ? 4 * ((int64_t)S->npanel + 1) : 0);
   if (k == "panel_count") return set(S->pcnt, S->pcnt ? 4 * (int64_t)S->npanel : 0);

@@ -141,3 +141,27 @@ def test_gpu_solve_needs_the_h_of_its_atoms(gpu_lib, ffield):
     h.call("qeq_init_matvec")
     got = solved(h)
     assert got[0] == want[0] and np.array_equal(got[4], want[4])
+
+
+def test_gpu_panel_lists_are_read_of_the_current_h_only(gpu_lib, ffield):
+    """A small system's column lists are made when they are asked for; between
+    swr_set_atoms with another number of atoms and the next H there are none
+    (more rows than the arrays held, and fewer)."""
+    names = ("panel_count", "panel_columns", "H_jloc")
+    P = batch.pack([waters(30, seed=1)])
+    h = loaded(gpu_lib, ffield, P, [1])
+    for m in (300, 12):
+        Q = batch.pack([waters(m, seed=m)])
+        h.set_atoms(Q.n, Q.x, Q.type, Q.tag, owner=Q.owner, img=Q.img)
+        assert all(h.get(k).size == 0 for k in names)
+        assert not any(h.L.swr_device_ptr(h.h, k.encode()) for k in names)
+        h.build_neighbors(batch.CUTGHOST)
+        h.call("qeq_init_matvec")
+        f, nn, jl, loc = h.get("H_firstnbr"), h.get("H_numnbrs"), h.get("H_jlist"), h.get("H_jloc")
+        pb, cnt, col = h.get("panel_begin"), h.get("panel_count"), h.get("panel_columns")
+        rows = h.get("panel_rows")
+        assert cnt.size == -(-Q.n // 64) and pb[-1] == Q.n
+        for p in range(cnt.size):
+            for i in rows[pb[p]:pb[p + 1]]:
+                e = slice(f[i], f[i] + nn[i])
+                assert np.array_equal(col[p * gpu_lib.PANEL_MAXC + loc[e]], jl[e])
