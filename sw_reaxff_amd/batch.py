@@ -60,8 +60,16 @@ def _buffer(bufs, name, shape, dtype):
     return b[:shape[0]]
 
 
+def _per_atom(batch, sizes):
+    """Whether every system's type and tag are arrays of one entry an atom."""
+    try:
+        return all(s.type.shape == (m,) == s.tag.shape for s, m in zip(batch, sizes))
+    except AttributeError:
+        return False
+
+
 def _map_types(batch, elements, out):
-    """out = every atom's 1-based position in `elements`."""
+    """out = every atom's 1-based position in `elements` (types of shape (n,))."""
     kinds, which = {}, []
     for s in batch:
         which.append(kinds.setdefault(tuple(s.elements), len(kinds)))
@@ -83,9 +91,13 @@ def pack(batch: list[systems.System], elements=ELEMENTS, cutghost: float = CUTGH
     arrays; the returned arrays are then views into them."""
     L = _lib.lib()
     K = len(batch)
-    nat = np.array([s.n for s in batch], dtype=np.int32)
+    sizes = [s.n for s in batch]
+    nat = np.array(sizes, dtype=np.int32)
     n = int(nat.sum())
-    if K == 1:
+    # arrays of one entry an atom are joined whole; anything else is assigned
+    # system by system, with numpy's broadcasting and its errors
+    plain = _per_atom(batch, sizes)
+    if K == 1 and plain:
         s = batch[0]
         x = np.ascontiguousarray(s.x, dtype=np.float64)
         tag = np.ascontiguousarray(s.tag, dtype=np.int32)
@@ -96,8 +108,16 @@ def pack(batch: list[systems.System], elements=ELEMENTS, cutghost: float = CUTGH
         tag = _buffer(bufs, "tag_in", (n,), np.int32)
         if n:
             np.concatenate([s.x for s in batch], out=x, casting="unsafe")
+        if n and plain:
             np.concatenate([s.tag for s in batch], out=tag, casting="unsafe")
             _map_types(batch, elements, typ)
+        elif n:
+            a = 0
+            for s in batch:
+                tmap = np.array([elements.index(e) + 1 for e in s.elements], dtype=np.int32)
+                typ[a:a + s.n] = tmap[s.type - 1]
+                tag[a:a + s.n] = s.tag
+                a += s.n
     lo = np.ascontiguousarray([s.lo for s in batch], dtype=np.float64)
     hi = np.ascontiguousarray([s.hi for s in batch], dtype=np.float64)
     per = np.array([1 if s.periodic else 0 for s in batch], dtype=np.int32)

@@ -292,3 +292,27 @@ def test_batch_pack_rejects_bad_input(built_lib):
                           hi.ctypes.data, per0.ctypes.data, C.c_double(10.0), 0, None, None, None, None, None,
                           None, None, None, C.byref(N))
     assert rc == 0 and N.value == 3
+
+
+@pytest.mark.parametrize("field", ["type", "tag"])
+@pytest.mark.parametrize("alone", [True, False])
+def test_batch_pack_checks_each_systems_arrays(built_lib, field, alone):
+    """A type or tag array that is not one entry an atom: an error, also when
+    another system's surplus makes up for what is missing; one entry stands
+    for all of the system's atoms."""
+    import dataclasses
+
+    from sw_reaxff_amd import batch as B
+    a, b = systems.cluster(5, seed=1), systems.cluster(6, seed=2)
+    v, w = getattr(a, field), getattr(b, field)
+    more = np.append(w, w[:1]).astype(np.int32)
+    with_ = lambda s, arr: dataclasses.replace(s, **{field: arr})   # noqa: E731
+    for bad in (v[:-1], v[:0], np.append(v, v[:1]).astype(np.int32)):
+        parts = [with_(a, bad)] + ([] if alone else [with_(b, more) if len(bad) == len(v) - 1 else b])
+        with pytest.raises(ValueError):
+            B.pack(parts, bufs={})
+    parts = [with_(a, v[:1])] + ([] if alone else [b])
+    full = [with_(a, np.repeat(v[:1], a.n))] + ([] if alone else [b])
+    P, Q = B.pack(parts, bufs={}), B.pack(full, bufs={})
+    for f in ("x", "type", "tag", "owner"):
+        assert np.array_equal(getattr(P, f), getattr(Q, f)), f
