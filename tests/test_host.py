@@ -316,3 +316,22 @@ def test_batch_pack_checks_each_systems_arrays(built_lib, field, alone):
     P, Q = B.pack(parts, bufs={}), B.pack(full, bufs={})
     for f in ("x", "type", "tag", "owner"):
         assert np.array_equal(getattr(P, f), getattr(Q, f)), f
+
+
+def test_batch_pack_on_several_threads(built_lib):
+    """From 32,768 atoms a thread on the systems are packed side by side: the
+    arrays equal the numpy restatement, of periodic and isolated systems, alike
+    and unlike in size, into fresh and into reused buffers (larger and smaller
+    packs before)."""
+    from sw_reaxff_amd import batch as B
+    from tests import batch_pack_ref as R
+    small = [systems.water_box(64, seed=40 + k) if k % 3 else systems.cluster(30 + k, seed=k) for k in range(24)]
+    large = [systems.water_box(12000, seed=60), systems.cluster(5000, seed=61), systems.water_box(9000, seed=62)]
+    bufs = {}
+    for parts in (small + large + small[::-1], large, large + small):
+        P1 = R.pack(parts, B.ELEMENTS, 10.0)
+        assert P1.n > 32768
+        P2 = B.pack(parts, cutghost=10.0, bufs=bufs)
+        assert P1.n == P2.n
+        for f in ("x", "type", "tag", "owner", "img", "row_off", "ghost_off", "shift"):
+            assert np.array_equal(getattr(P1, f), getattr(P2, f)), f
