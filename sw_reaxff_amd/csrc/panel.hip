@@ -13,10 +13,9 @@
 // columns keeps pcnt = -1 and its rows gather from global memory as before.
 //
 // Small systems (qeq_small.h) keep their rows in atom order instead, and their
-// lists are built only when something else asks for them (the no-allocation
-// solve, the autotuner, a download).  The row order changes only when the bins or the batch partition
-// change (a neighbour-list build or swr_set_batch); the column lists are rebuilt
-// with H every step.  Dense indices follow the hash table's slot order,
+// lists are built only when swr_get asks for them.  The row order changes only
+// when the bins or the batch partition change (a neighbour-list build or
+// swr_set_batch); the column lists are rebuilt with H every step.  Dense indices follow the hash table's slot order,
 // which can differ between runs, but a row's sum runs over its entries in
 // H order whatever the indices are, so the SpMV results do not depend on it.
 #include <vector>

@@ -426,14 +426,40 @@ CgLayout swr_qeq_cg_layout(swr_system *S) {
   return L;
 }
 
+// The FP64 solve in the system's own buffers.
+static CgRun<double, double> fp64_run(swr_system *S) {
+  CgRun<double, double> R{};
+  R.V = make_vecs(S);
+  R.val = S->H_val;
+  R.L = swr_qeq_cg_layout(S);
+  R.cgs = S->cgs;
+  R.iters_out = S->sys_iters;
+  S->h_sys_iters.resize(2 * (size_t)S->nsys);
+  R.iters_host = S->h_sys_iters.data();
+  R.pin_done = S->pin_done;
+  R.pin_iters = S->pin_iters;
+  R.tol = S->ctl.tol;
+  R.imax = S->imax;
+  R.kt_iter = KT_CG_ITER;
+  R.kt_update = KT_CG_UPDATE;
+  R.kt_setup = KT_CG_SETUP;
+  R.kt_scalars = KT_CG_SCALARS;
+  R.partials = S->partials;
+  R.pstride = S->cg_pstride;
+  return R;
+}
+
 // Autotuner hook: the average time of `reps` launches of the FP64 CG's SpMV
 // in shape sh on the current H and vectors (the setup-phase instance, which
-// multiplies d0 into q and always runs; both are scratch between solves).
+// multiplies d0 and always runs; its vectors are scratch between solves), or
+// of the small solve's same step where that one runs (its columns need no lists).
 int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
   int rc;
   if (!S->H_val || S->n <= 0) return SWR_ERR_STATE;
-  if ((rc = swr_panel_ready(S)) || (rc = swr_panel_lists(S))) return rc;
-  CgVecsT<double> V = make_vecs(S);
+  if ((rc = swr_panel_ready(S))) return rc;
+  const CgRun<double, double> R = fp64_run(S);
+  const CgVecsT<double> &V = R.V;
+  const SmallArgs A = small_args(S, R, small_vecs(R, (double2 *)S->cgv, S->ncap), PH_S2, 0);
   const int n = S->n;
   const CgScalars *cgs = S->cgs;
   const int *row_sys = S->row_sys;
@@ -445,7 +471,9 @@ int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
     const dim3 gb(S->npanel), tb(SpmvShape<SH>::NT);
     for (int r = -1; r < reps; r++) {   // one untimed launch first
       if (r == 0) (void)hipEventRecord(e[0], S->stream);
-      if (S->nsys > 1)
+      if (S->cg_small)
+        hipLaunchKernelGGL((k_cg_small<PH_S2, SH>), gb, tb, 0, S->stream, A);
+      else if (S->nsys > 1)
         hipLaunchKernelGGL((k_cg_spmv<PH_S2, true, double, double, SH>), gb, tb, 0, S->stream, n, S->dp, S->type,
                            S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, V, 0, cgs, row_sys, panel_args(S));
       else
@@ -503,24 +531,7 @@ int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
   const int first_batch = last_iters > 0 ? last_iters + 1 : CG_COLD_BATCH;
   int rc = swr_panel_ready(S);
   if (rc) return rc;
-  CgRun<double, double> R{};
-  R.V = make_vecs(S);
-  R.val = S->H_val;
-  R.L = swr_qeq_cg_layout(S);
-  R.cgs = S->cgs;
-  R.iters_out = S->sys_iters;
-  S->h_sys_iters.resize(2 * (size_t)S->nsys);
-  R.iters_host = S->h_sys_iters.data();
-  R.pin_done = S->pin_done;
-  R.pin_iters = S->pin_iters;
-  R.tol = S->ctl.tol;
-  R.imax = S->imax;
-  R.kt_iter = KT_CG_ITER;
-  R.kt_update = KT_CG_UPDATE;
-  R.kt_setup = KT_CG_SETUP;
-  R.kt_scalars = KT_CG_SCALARS;
-  R.partials = S->partials;
-  R.pstride = S->cg_pstride;
+  const CgRun<double, double> R = fp64_run(S);
   int all = S->nsys;
   if (S->cg_small) {   // (a system without rows has no workgroup to finish it)
     all = 0;

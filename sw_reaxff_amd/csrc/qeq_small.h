@@ -490,8 +490,7 @@ inline SmallVecs small_vecs(const CgRun<double, double> &R, double2 *base, size_
   return V;
 }
 
-// The steps of the solve; step 0 is each setup phase, steps 1.. are PH_K.
-inline int small_step(swr_system *S, const CgRun<double, double> &R, const SmallVecs &V, int ph, int step) {
+inline SmallArgs small_args(const swr_system *S, const CgRun<double, double> &R, const SmallVecs &V, int ph, int step) {
   SmallArgs A;
   A.P = S->dp;
   A.type = S->type;
@@ -509,6 +508,12 @@ inline int small_step(swr_system *S, const CgRun<double, double> &R, const Small
   A.iters_out = R.iters_out;
   A.done_count = R.L.done_count;
   A.status = S->status;
+  return A;
+}
+
+// The steps of the solve; step 0 is each setup phase, steps 1.. are PH_K.
+inline int small_step(swr_system *S, const CgRun<double, double> &R, const SmallVecs &V, int ph, int step) {
+  const SmallArgs A = small_args(S, R, V, ph, step);
   const int kt = ph == PH_K ? R.kt_iter : R.kt_setup;
   if (S->cg_tiny) {   // the first step is the whole solve
     if (ph != PH_S1) return SWR_OK;

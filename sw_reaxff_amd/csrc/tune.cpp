@@ -4,7 +4,8 @@
 // depends on the workload (row lengths, system sizes, how many systems a
 // batch holds) more than on anything known at compile time:
 //
-//   spmv_fp64   the FP64 CG's SpMV (k_cg_spmv): T threads per panel of H
+//   spmv_fp64   the FP64 CG's SpMV (k_cg_spmv, or k_cg_small and k_cg_tiny
+//               for small systems): T threads per panel of H
 //               rows, G lanes per row and U groups of 4 entries in flight
 //               per lane (T512G8U4, T512G8U2, T256G8U4, T256G4U4);
 //   spmv_fp32   the mixed-precision inner solve's FP32 SpMV (k_pcg_spmv);

@@ -165,3 +165,27 @@ def test_gpu_panel_lists_are_read_of_the_current_h_only(gpu_lib, ffield):
             for i in rows[pb[p]:pb[p + 1]]:
                 e = slice(f[i], f[i] + nn[i])
                 assert np.array_equal(col[p * gpu_lib.PANEL_MAXC + loc[e]], jl[e])
+
+
+def test_gpu_autotune_times_the_small_solve(gpu_lib, ffield):
+    """For small systems the FP64 family's shapes are those of the one-launch
+    steps, which use no column lists: timing them makes none (13 MB here)."""
+    hip = _hip()
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t)] * 2
+
+    def free():
+        a, b = C.c_size_t(0), C.c_size_t(0)
+        _ok(hip.hipDeviceSynchronize(), "synchronize")
+        _ok(hip.hipMemGetInfo(C.byref(a), C.byref(b)), "hipMemGetInfo")
+        return a.value
+
+    P = batch.pack([waters(1, seed=k) for k in range(960)] + [waters(22, seed=2000)])
+    h = loaded(gpu_lib, ffield, P, [1] * 961)
+    solved(h)
+    lists = 4 * gpu_lib.PANEL_MAXC * 962
+    before = free()
+    rep = h.autotune(reps=2)
+    assert before - free() < lists // 2
+    assert set(rep["spmv_fp64"]["us"]) == {"T512G8U4", "T512G8U2", "T256G8U4", "T256G4U4"}
+    h.get("panel_count")
+    assert before - free() >= lists // 2       # (the probe sees the lists when they are made)
