@@ -528,9 +528,14 @@ int swr_publish(swr_system *S, const SwrPublish &P) {
 }
 
 int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
-  const int first_batch = last_iters > 0 ? last_iters + 1 : CG_COLD_BATCH;
   int rc = swr_panel_ready(S);
   if (rc) return rc;
+  int first_batch = last_iters + 1;
+  if (last_iters <= 0) {
+    int rows = 0;
+    for (int s = 0; s < S->nsys; s++) rows = std::max(rows, S->sys_row[s + 1] - S->sys_row[s]);
+    first_batch = std::min(CG_COLD_BATCH, rows + 2);
+  }
   const CgRun<double, double> R = fp64_run(S);
   int all = S->nsys;
   if (S->cg_small) {   // (a system without rows has no workgroup to finish it)

@@ -659,15 +659,19 @@ int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzer
 // Launches enqueued after a system finished skip its rows.  step(ph, k)
 // enqueues phase ph, k the iteration of PH_K.
 //
-// A solve from zero history has no last count to size its first batch by: 16
-// launches, then 8 at a time (a wait costs ~30 us of idle GPU, a launch
-// that finds nothing to do ~3; cold solves take 14 to 50 iterations).
-constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8;
-
-//
 // A run with pinned memory reads everything back in one small launch, and
 // behind() may queue work that is to follow a finished solve: it then fills
-// the ~25 us the GPU otherwise waits for the host.  *finished: the last check found all systems done.
+// the ~25 us the GPU otherwise waits for the host.  *finished: the last check
+// found all systems done.
+//
+// A solve from zero history has no last count to size its first batch by: 16
+// launches, then 8 at a time (a wait costs ~30 us of idle GPU, an iteration
+// that finds nothing to do 3 to 20 with the number of systems; cold solves
+// take 14 to 50 iterations).  Fewer where the largest system has fewer rows,
+// since r rows take about r iterations: with sixteen launches an evaluation of
+// 4,096 single waters (4 iterations) took 1,290 us, with five 980; of 12,000 of
+// them 2,707 and 2,129.
+constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8;
 template <typename T, typename VT, class Step, class Behind>
 int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Step step, Behind behind,
              bool *finished) {

@@ -402,3 +402,25 @@ def test_gpu_torsions_of_a_large_batch(gpu_lib, ffield):
         assert np.abs(a).max() > 1e-3
         for r in (0, 1, b.shape[1] // per - 1):
             assert np.max(np.abs(b[:, r * per:(r + 1) * per] - a)) <= 1e-8 * np.abs(a).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,K", [(1, 1), (2, 1), (1, 1100), (2, 1100), (4, 1100)])
+def test_gpu_cold_solves_of_few_rows_launch_few_iterations(gpu_lib, ffield, m, K):
+    """r rows take about r iterations, so a first solve of systems of few rows
+    queues rows + 2 of them, not the sixteen of larger ones."""
+    from sw_reaxff_amd.batch import Batch
+    rng = np.random.default_rng(m)
+    s = waters(m, seed=m)
+    parts = [systems.System(x=s.x + rng.normal(scale=0.05, size=s.x.shape), v=s.v, type=s.type, tag=s.tag,
+                            elements=s.elements, lo=s.lo, hi=s.hi, periodic=False) for _ in range(K)]
+    bt = Batch(ffield, tol=1e-6)
+    bt.load(parts)
+    bt.sys.ktimer_enable()
+    bt.evaluate()
+    bt.sync()
+    _, launches = bt.sys.ktimer_read("cg_iter")
+    its = int(bt.iterations().max())
+    assert 2 <= its <= s.n + 1
+    if K > 1:                               # (one launch for the whole solve otherwise)
+        assert its <= launches <= min(16, s.n + 2)
