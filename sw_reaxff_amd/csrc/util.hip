@@ -1,4 +1,4 @@
-// util.hip — exclusive prefix sums (3-phase, deterministic) and small helpers.
+// util.hip — exclusive prefix sums (one, two or four launches by size; deterministic) and small helpers.
 #include "swr_internal.h"
 #include "swr_device.h"
 
@@ -45,15 +45,19 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_sums(const TI *in, int n,
 }
 
 // A tile's exclusive scan, after the sum of everything before it: every
-// workgroup adds up the earlier tiles' sums (SUMS) or, while there are few
-// tiles, their items.  The last one writes the total.
-template <class TI, class TO, bool SUMS>
+// workgroup adds up the earlier tiles' sums or, while there are few tiles,
+// their items; of many tiles the sums were scanned before.  The last one
+// writes the total.
+enum { SCAN_BY_ITEMS, SCAN_BY_SUMS, SCAN_BY_OFFSETS };
+template <class TI, class TO, int BY>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const TI *in, int n, const TO *tile_sums, TO *out,
                                                              TO *total) {
   __shared__ TO lds[SCAN_THREADS / SWR_WAVE];
   const long long base = (long long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
   TO before = 0;
-  if (SUMS) {
+  if (BY == SCAN_BY_OFFSETS) {
+    if (threadIdx.x == 0) before = tile_sums[blockIdx.x];
+  } else if (BY == SCAN_BY_SUMS) {
     for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_THREADS) before += tile_sums[k];
   } else {
     const int first = blockIdx.x * SCAN_TILE;
@@ -81,6 +85,12 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const TI *in, int n
 // Tiles up to which one launch does (16,384 items: the last workgroup reads 60
 // items a thread first, about a launch's time).
 constexpr int SCAN_DIRECT = 16;
+// Tiles up to which every workgroup adds up the sums before its own: that
+// reading grows with the square of the tiles, and from about four million
+// items on two launches over the sums are cheaper (a neighbour build on a grid
+// of 4.2 million bins 123 us either way, of 14 million 178 and 161, of 33
+// million 349 and 229, of 112 million 1,878 and 549).
+constexpr int SCAN_FLAT = 4096;
 
 template <class TI, class TO>
 int scan_impl(swr_system *S, const TI *in, TO *out, int n, TO *total_dev) {
@@ -90,12 +100,13 @@ int scan_impl(swr_system *S, const TI *in, TO *out, int n, TO *total_dev) {
   }
   const int ntiles = div_up(n, SCAN_TILE);
   if (ntiles <= SCAN_DIRECT && (const void *)in != (const void *)out) {
-    hipLaunchKernelGGL((k_scan_apply<TI, TO, false>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n,
+    hipLaunchKernelGGL((k_scan_apply<TI, TO, SCAN_BY_ITEMS>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n,
                        (const TO *)nullptr, out, total_dev);
     HIP_CHECK(hipGetLastError());
     return SWR_OK;
   }
-  const size_t need = sizeof(TO) * (size_t)ntiles;
+  const int ntiles2 = div_up(ntiles, SCAN_TILE);
+  const size_t need = sizeof(TO) * (2 * (size_t)ntiles + ntiles2);
   if (need > S->scan_tmp_bytes) {
     if (S->scan_tmp) (void)hipFree(S->scan_tmp);
     S->scan_tmp = nullptr;
@@ -105,8 +116,18 @@ int scan_impl(swr_system *S, const TI *in, TO *out, int n, TO *total_dev) {
   }
   TO *tiles = (TO *)S->scan_tmp;
   hipLaunchKernelGGL((k_tile_sums<TI, TO>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n, tiles);
-  hipLaunchKernelGGL((k_scan_apply<TI, TO, true>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n,
-                     (const TO *)tiles, out, total_dev);
+  if (ntiles <= SCAN_FLAT) {
+    hipLaunchKernelGGL((k_scan_apply<TI, TO, SCAN_BY_SUMS>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n,
+                       (const TO *)tiles, out, total_dev);
+  } else {
+    TO *offs = tiles + ntiles, *tiles2 = offs + ntiles;
+    hipLaunchKernelGGL((k_tile_sums<TO, TO>), dim3(ntiles2), dim3(SCAN_THREADS), 0, S->stream, (const TO *)tiles, ntiles,
+                       tiles2);
+    hipLaunchKernelGGL((k_scan_apply<TO, TO, SCAN_BY_SUMS>), dim3(ntiles2), dim3(SCAN_THREADS), 0, S->stream,
+                       (const TO *)tiles, ntiles, (const TO *)tiles2, offs, (TO *)nullptr);
+    hipLaunchKernelGGL((k_scan_apply<TI, TO, SCAN_BY_OFFSETS>), dim3(ntiles), dim3(SCAN_THREADS), 0, S->stream, in, n,
+                       (const TO *)offs, out, total_dev);
+  }
   HIP_CHECK(hipGetLastError());
   return SWR_OK;
 }

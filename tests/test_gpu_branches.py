@@ -424,3 +424,32 @@ def test_gpu_cold_solves_of_few_rows_launch_few_iterations(gpu_lib, ffield, m, K
     assert 2 <= its <= s.n + 1
     if K > 1:                               # (one launch for the whole solve otherwise)
         assert its <= launches <= min(16, s.n + 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bins", [(64, 64, 1023), (64, 64, 1024), (220, 220, 220), (1100, 1100, 90)])
+def test_gpu_scans_of_large_sparse_grids(gpu_lib, ffield, bins):
+    """Two clusters in the far corners of a grid: the bins' prefix sums at the
+    edge of the scan's flat form (4,096 tiles of 1,024) and beyond it, where the
+    tiles' sums are scanned themselves.  Each cluster's rows are those it has
+    alone."""
+    from sw_reaxff_amd import _lib
+    s = waters(64, seed=3)
+    span = np.ptp(s.x, axis=0)
+    far = 5.0 * np.array(bins) + 2.5 - span          # bins of 5 A and a bit: exactly this many of them
+    x = np.vstack([s.x, s.x + far])
+    ty, tag = np.concatenate([s.type, s.type]), np.arange(1, 2 * s.n + 1, dtype=np.int32)
+
+    def rows(n, x, ty, tag):
+        h = _lib.System(ffield, s.elements)
+        h.set_atoms(n, x, ty, tag)
+        h.build_neighbors(10.0)
+        h.sync()
+        off, lst = h.get("verlet_offsets"), h.get("verlet_list")
+        assert off[0] == 0 and off[n] == h.scalar("verlet_total")
+        return [np.sort(lst[off[i]:off[i + 1]]) for i in range(n)]
+
+    alone, both = rows(s.n, s.x, s.type, s.tag), rows(2 * s.n, x, ty, tag)
+    assert sum(map(len, alone)) > 1000
+    for i in range(s.n):
+        assert np.array_equal(both[i], alone[i]) and np.array_equal(both[s.n + i], alone[i] + s.n), i
