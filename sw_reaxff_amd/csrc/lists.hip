@@ -900,7 +900,17 @@ __global__ void __launch_bounds__(SWR_WAVE) k_validate_end(DevStatus *st, int *_
 // MD); with the ids in registers 32,000 take 59 (87).  Relaxing 1024 ghosts at
 // a time to their local fixed point in LDS: 85, but 260 after 200 steps, when
 // the chains cross its blocks more often.  Six ids and 8 sweeps: 65 (110).
-constexpr int MARK_BFS = 32512;  // (a ghost's position and two codes in 15 bits)
+//
+// The search is one workgroup's, so its time grows with the bonds of the
+// ghosts it reaches.  A ghost with more than four higher neighbours has its list
+// walked by the four lanes it gets (by one lane a lattice with a dozen bonds an
+// atom took 204 us at 11,600 ghosts, 382 at 23,500 and 522 at 32,300 where
+// walking every list takes 171, 226 and 222; by four 107, 197 and 283).  The line
+// lies where the relaxation is the faster one on that lattice (27,700 ghosts:
+// 244 and 230 us, 32,300: 263 and 188) while on water the search still is
+// (22,900 ghosts: 49 and 58 us, with the call's wait).
+constexpr int MARK_BFS = 28672;
+static_assert(MARK_BFS <= 0x7ffe, "a ghost's position and two codes in 15 bits");
 constexpr int BFS_LDS = 12288;
 constexpr int BFS_T = 1024;
 constexpr int MARK_FAR = 1000;   // mark of a ghost nothing reaches
@@ -970,13 +980,15 @@ k_mark_bfs(int n, int N, const int *__restrict__ bond_index, const int *__restri
     // four lanes per atom of the frontier, one of its entries each
     for (int f = begin + (int)threadIdx.x / 4; f < end; f += BFS_T / 4) {
       const int r = queue[f], k = threadIdx.x % 4;
-      const int h = ups[4 * r + k] & ~UP_NEAR;
-      if (h == UP_LIST) {
-        for (int p = bond_index[n + r]; p < bond_end[n + r]; p++)
+      if (ups[4 * r + 3] == UP_LIST) {
+        const int p1 = bond_end[n + r];
+#pragma unroll 2
+        for (int p = bond_index[n + r] + k; p < p1; p += 4)
           if (bond_nbr[p] - n > r) reach(bond_nbr[p] - n, level);
-      } else if (h != UP_NONE) {
-        reach(h, level);
+        continue;
       }
+      const int h = ups[4 * r + k] & ~UP_NEAR;
+      if (h != UP_NONE) reach(h, level);
     }
     __syncthreads();
     begin = end;

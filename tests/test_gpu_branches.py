@@ -453,3 +453,37 @@ def test_gpu_scans_of_large_sparse_grids(gpu_lib, ffield, bins):
     assert sum(map(len, alone)) > 1000
     for i in range(s.n):
         assert np.array_equal(both[i], alone[i]) and np.array_equal(both[s.n + i], alone[i] + s.n), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [4, 17, 18])
+def test_gpu_bond_marks_around_the_searchs_limit(gpu_lib, ffield, m):
+    """Crowded ghosts whose neighbour lists four lanes walk together: the last
+    lattice the search takes (27,700 ghosts), the first the relaxation does
+    (30,000) and a box smaller than the ghost shell, whose ghosts have many
+    images."""
+    from sw_reaxff_amd import _lib
+    a = 1.7
+    s = lattice(m, a, seed=m)
+    x = np.mod(s.x - 20.0, m * a)
+    xa, owner = systems.borders(x, np.zeros(3), np.full(3, m * a), min(12.0, m * a))
+    h = _lib.System(ffield, s.elements)
+    h.set_atoms(s.n, xa, s.type[owner], s.tag[owner], owner=owner)
+    h.build_neighbors()
+    h.set_capacities(np.full(owner.size, 32), np.full(owner.size, 256))
+    for stage in ("write_reax_atoms_and_pack", "reset", "write_reax_lists_init_forces", "validate_lists", "sort_bonds"):
+        h.call(stage)
+    h.sync()
+    n, N = s.n, owner.size
+    assert {4: N - n < 12288, 17: 24576 < N - n <= 28672, 18: 28672 < N - n <= 32512}[m]
+    bi, be, nbr = h.get("bond_index"), h.get("bond_end"), h.get("bonds")["nbr"]
+    mark = np.where(np.arange(N) < n, 0, 1000)
+    for i in range(n, N):
+        j = nbr[bi[i]:be[i]]
+        if j.size:
+            mark[i] = min(mark[i], (mark[j] + 1).min())
+    assert (mark[n:] < 1000).any()
+    assert np.array_equal(h.get("bond_mark")[:N], mark)
+    h.call("sort_bonds")                     # once more over its own result
+    h.sync()
+    assert np.array_equal(h.get("bond_mark")[:N], mark)
