@@ -249,9 +249,8 @@ int swr_nbr_ensure_atoms(swr_system *S, int Ncap) {
       (rc = swr_alloc(&S->bond_end, nn)) || (rc = swr_alloc(&S->hbond_index, nn)) ||
       (rc = swr_alloc(&S->hbond_end, nn)) || (rc = swr_alloc(&S->bo_dboc, 2 * nn)) ||
       (rc = swr_alloc(&S->dDeltap_self, 3 * nn)) || (rc = swr_alloc(&S->bond_mark, nn)) ||
-      (rc = swr_alloc(&S->bond_mark2, nn)) || (rc = swr_alloc(&S->counts, 2 * nn)) ||
-      (rc = swr_alloc(&S->ws, WS_COUNT * nn)) || (rc = swr_alloc(&S->far_index, nn)) ||
-      (rc = swr_alloc(&S->far_end, nn)) || (rc = swr_alloc(&S->fcd, 4 * nn)))
+      (rc = swr_alloc(&S->counts, 2 * nn)) || (rc = swr_alloc(&S->ws, WS_COUNT * nn)) ||
+      (rc = swr_alloc(&S->far_index, nn)) || (rc = swr_alloc(&S->far_end, nn)) || (rc = swr_alloc(&S->fcd, 4 * nn)))
     return rc;
   HIP_CHECK(hipMemsetAsync(S->counts, 0, 2 * nn * sizeof(int), S->stream));
   S->Ncap = Ncap;
@@ -403,7 +402,7 @@ int swr_destroy(swr_system *S) {
                   S->fcd, S->nb_partials, S->nb_result, S->nb_eatom, S->be_part, S->be_ce, S->be_bufc, S->be_result, S->hb_part,
                   S->hb_result, S->hb_acc, S->va_part, S->va_result, S->va_acc, S->va_cnt, S->va_order, S->va_ctl, S->to_part, S->to_result, S->to_acc,
                   S->to_sacc, S->to_tc, S->to_task, S->to_ctl, S->to_row, S->f, S->gcsr_cnt, S->gcsr_start, S->gcsr_list,
-                  S->bond_mark2, S->counts, S->ws, S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32,
+                  S->counts, S->ws, S->H_firstnbr, S->H_numnbrs, S->H_jlist, S->H_val, S->H_val32,
                   S->Hdia_inv, S->b_s, S->st, S->s_hist, S->t_hist, S->cgv, S->cgs, S->partials, S->next_totals,
                   S->status, S->scan_tmp, S->tmp_i, S->mixw, S->cand, S->cand_count, S->layout_all, S->atoms_in,
                   S->done_count, S->qsum,

@@ -215,108 +215,56 @@ __device__ __forceinline__ BOpTerms bop_terms(const DevParams *__restrict__ P, i
   return t;
 }
 
-// Pass 1: one wave per atom streams its candidates (the Verlet list, or an
-// existing far list when SRC_FAR) 64 at a time.
-//   FAR  : write the far entries (write_reax_lists_c_para, pair_reaxc_sw64.c:276-331)
-//   CAND : record bond candidates' far slots
-//   HB   : 1 count, 2 write hbonds of local H (Init_Forces_noQEq_HB_Full_C,
-//          reaxc_forces_sw64.c:810-862)
-template <bool SRC_FAR, bool FAR, bool CAND, int HB>
+// Pass 1 from a far list that is there (swr_init_forces_noqeq_full): one wave
+// per atom reads its far entries 64 at a time, records the bond candidates'
+// far slots and writes the hydrogen bonds of local H
+// (Init_Forces_noQEq_HB_Full_C, reaxc_forces_sw64.c:810-862).
 __global__ void __launch_bounds__(LT)
-k_far(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__restrict__ atoms,
-      const long long *__restrict__ voff, const int *__restrict__ vlist, swr_far_neighbor_t *__restrict__ far,
-      int *__restrict__ far_index, int *__restrict__ far_end, int *__restrict__ cand, int *__restrict__ cand_count,
-      const int *__restrict__ Hindex, const int *__restrict__ num_hbonds, const int *__restrict__ hbond_index,
-      int *__restrict__ hbond_end, swr_hbond_t *__restrict__ hbonds, int *__restrict__ hb_count, int hbond_cap,
-      DevStatus *st) {
-  __shared__ double2 sfar[(FAR && !SRC_FAR) ? LW : 1][4 * SWR_WAVE];
-  const int w = wave_in_block();
-  const int blk = blockIdx.x;
-  const int i = blk * LW + w;
+k_from_far(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__restrict__ atoms,
+           swr_far_neighbor_t *__restrict__ far, const int *__restrict__ far_index, const int *__restrict__ far_end,
+           int *__restrict__ cand, int *__restrict__ cand_count, const int *__restrict__ Hindex,
+           const int *__restrict__ num_hbonds, const int *__restrict__ hbond_index, int *__restrict__ hbond_end,
+           swr_hbond_t *__restrict__ hbonds, int *__restrict__ hb_count, int hbond_cap, DevStatus *st) {
+  const int i = blockIdx.x * LW + wave_in_block();
   if (i >= N) return;
   const int lane = lane_id();
-  const swr_atom_pack_t ai = atoms[i];
-  const int ei = ai.type;
-  const double nonb_cutsq = P->nonb_cutsq, bond_cut = P->bond_cut, hbond_cut = P->hbond_cut;
-  long long cbeg, cend;
-  if (SRC_FAR) { cbeg = far_index[i]; cend = far_end[i]; }
-  else { cbeg = voff[i]; cend = voff[i + 1]; }
-  const long long far0 = SRC_FAR ? cbeg : voff[i];
-  int nfar = 0, ncand = 0;
-  const bool doH = HB != 0 && (i < n) && ei >= 0 && P->p_hbond[ei] == 1 && hbond_cut > 0;
-  const int H = (doH && HB == 2) ? Hindex[i] : -1;
-  int htop = (doH && HB == 2) ? hbond_end[H] : 0;
+  const int ei = atoms[i].type;
+  const double bond_cut = P->bond_cut, hbond_cut = P->hbond_cut;
+  const long long cbeg = far_index[i], cend = far_end[i];
+  int ncand = 0;
+  const bool doH = (i < n) && ei >= 0 && P->p_hbond[ei] == 1 && hbond_cut > 0;
+  const int H = doH ? Hindex[i] : -1;
+  int htop = doH ? hbond_end[H] : 0;
   // capacity of this H's slots, never past the end of the list
-  const int hlim = (doH && HB == 2) ? min(hbond_index[H] + num_hbonds[i], hbond_cap) : 0;
+  const int hlim = doH ? min(hbond_index[H] + num_hbonds[i], hbond_cap) : 0;
   const double *rbo = P->rbo + (ei >= 0 ? ei : 0) * SWR_MAX_ELEM;
   int *mycand = cand + (size_t)i * MCAND;
-
-  int jnext = 0;
-  if (!SRC_FAR && cbeg + lane < cend) jnext = vlist[cbeg + lane];
   for (long long base = cbeg; base < cend; base += SWR_WAVE) {
-    const long long k = base + lane;
-    const bool valid = k < cend;
-    int j = 0, tj = -1, tagj = 0;
-    double dx = 0, dy = 0, dz = 0, d = 0, qj = 0;
-    bool infar = false;
-    long long slot = 0;
-    if (SRC_FAR) {
-      if (valid) {
-        const double2 *e = reinterpret_cast<const double2 *>(far + k);
-        const int4 h0 = *reinterpret_cast<const int4 *>(far + k);
-        const double2 e1 = e[1], e3 = e[3];
-        const double2 e2 = e[2];
-        j = h0.x; tj = h0.y; d = e1.y; dx = e2.y; dy = e3.x; dz = e3.y;
-        infar = true;
-        slot = k;
-      }
-    } else {
-      j = jnext;
-      if (k + SWR_WAVE < cend) jnext = vlist[k + SWR_WAVE];
-      if (valid) {
-        const swr_atom_pack_t aj = atoms[j];
-        dx = aj.x[0] - ai.x[0]; dy = aj.x[1] - ai.x[1]; dz = aj.x[2] - ai.x[2];
-        const double dsq = dx * dx + dy * dy + dz * dz;
-        infar = dsq <= nonb_cutsq;
-        if (infar) {
-          d = sqrt(dsq);
-          tj = aj.type; tagj = aj.orig_id; qj = aj.q;
-        }
-      }
-      const unsigned long long m = __ballot(infar);
-      const int r = ballot_rank(m);
-      slot = far0 + nfar + r;
-      if (FAR) {
-        // Compact the wave's entries in LDS, then write them as contiguous
-        // 16-byte pieces (lane t writes piece t, t+64, ...): full-line
-        // stores instead of one 64-byte entry per lane.
-        double2 *sw = sfar[w];
-        if (infar) stage_far(sw, r, j, tj, tagj, d, qj, dx, dy, dz);
-        wave_lds_sync();
-        double2 *dst = reinterpret_cast<double2 *>(far + far0 + nfar);
-        const int pieces = 4 * __popcll(m);
-        for (int t = lane; t < pieces; t += SWR_WAVE) store_nt(dst + t, sw[staged_piece(t)]);
-        wave_lds_sync();
-      }
-      nfar += __popcll(m);
+    const long long slot = base + lane;
+    const bool valid = slot < cend;
+    int j = 0, tj = -1;
+    double d = 0;
+    if (valid) {
+      const int4 h0 = *reinterpret_cast<const int4 *>(far + slot);
+      j = h0.x;
+      tj = h0.y;
+      d = far[slot].d;
     }
-    if (CAND) {
-      const bool iscand = infar && ei >= 0 && tj >= 0 && d <= bond_cut && d <= rbo[tj];
-      const unsigned long long cm = __ballot(iscand);
-      if (iscand) {
-        const int c = ncand + ballot_rank(cm);
-        if (c < MCAND) mycand[c] = (int)slot;
-      }
-      ncand += __popcll(cm);
+    const bool iscand = valid && ei >= 0 && tj >= 0 && d <= bond_cut && d <= rbo[tj];
+    const unsigned long long cm = __ballot(iscand);
+    if (iscand) {
+      const int c = ncand + ballot_rank(cm);
+      if (c < MCAND) mycand[c] = (int)slot;
     }
+    ncand += __popcll(cm);
     if (doH) {
       bool ish = false;
-      if (infar && d <= hbond_cut) {
-        const int tjj = SRC_FAR ? atoms[j].type : tj;
+      if (valid && d <= hbond_cut) {
+        const int tjj = atoms[j].type;
         ish = tjj >= 0 && P->p_hbond[tjj] == 2;
       }
       const unsigned long long hm = __ballot(ish);
-      if (HB == 2 && ish) {
+      if (ish) {
         const int pos = htop + ballot_rank(hm);
         if (pos < hlim) {
           swr_hbond_t hb;
@@ -330,30 +278,20 @@ k_far(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__re
     }
   }
   if (lane == 0) {
-    if (!SRC_FAR) {
-      far_index[i] = (int)far0;
-      far_end[i] = (int)(far0 + nfar);
-    }
-    if (CAND) {
-      cand_count[i] = ncand;
-      if (ncand > MCAND) atomicOr(&st->flags, SWR_F_BOND_LDS);
-    }
+    cand_count[i] = ncand;
+    if (ncand > MCAND) atomicOr(&st->flags, SWR_F_BOND_LDS);
     if (doH) {
-      if (HB == 1) {
-        hb_count[i] = htop;
-      } else {
-        if (htop > hlim) {
-          atomicOr(&st->flags, SWR_F_HBOND_CAP);
-          atomicMax(&st->need_hbond_cap, htop - hbond_index[H]);
-        }
-        hbond_end[H] = htop > hlim ? hlim : htop;
-        hb_count[i] = htop - hbond_index[H];
+      if (htop > hlim) {
+        atomicOr(&st->flags, SWR_F_HBOND_CAP);
+        atomicMax(&st->need_hbond_cap, htop - hbond_index[H]);
       }
+      hbond_end[H] = htop > hlim ? hlim : htop;
+      hb_count[i] = htop - hbond_index[H];
     }
   }
 }
 
-// Pass 1 for a Verlet-list source, split between two kinds of waves.
+// Pass 1 from the Verlet list, split between two kinds of waves.
 //
 // A wave's vector-memory counter (vmcnt) counts loads and stores together
 // and retires them in issue order, so a wave that writes its far entries
@@ -364,8 +302,10 @@ k_far(int n, int N, const DevParams *__restrict__ P, const swr_atom_pack_t *__re
 // entries (plus hbond and bond-candidate records) in LDS, while FWR
 // "writer" waves, which never load from global memory, stream the previous
 // phase's staged entries out as contiguous 16-byte nontemporal stores.  One
-// LDS barrier per phase; double-buffered staging.  Entry order and content
-// are those of k_far (a far list is its Verlet row filtered in order).
+// LDS barrier per phase; double-buffered staging.  A far list is its Verlet
+// row filtered in order (write_reax_lists_c_para, pair_reaxc_sw64.c:276-331).
+// CAND: the bond candidates' far slots too; HB: the hydrogen bonds of local H
+// too, 2 into their list (as k_from_far), 3 their far slots for later.
 // The split (FG gatherers, FWR writers per block) is a template parameter;
 // the autotuner picks among the FarShape variants below.
 template <int FG, int FWR>
@@ -1147,7 +1087,6 @@ int swr_lists_run(swr_system *S, int mode) {
     if (rc) return rc;
   }
   const int N = S->N;
-  const int nblk = div_up(N, LW);
   double *ws = S->ws;
   int rc = SWR_OK;
   if (mode != 0 && (size_t)N * MCAND > S->cand_cap) {
@@ -1155,10 +1094,6 @@ int swr_lists_run(swr_system *S, int mode) {
     S->cand_cap = (size_t)S->Ncap * MCAND;
   }
   int *hb_count = S->counts + S->Ncap;
-#define FAR_ARGS(k)                                                                                              \
-  hipLaunchKernelGGL(k, dim3(nblk), dim3(LT), 0, S->stream, S->n, N, S->dp, S->packed, S->voff, S->vlist, S->far, \
-                     S->far_index, S->far_end, S->cand, S->cand_count, S->Hindex, S->num_hbonds, S->hbond_index,  \
-                     S->hbond_end, S->hbonds, hb_count, S->hbond_cap, S->status)
 #define BOND_ARGS(k)                                                                                              \
   hipLaunchKernelGGL(k, dim3(div_up(N, (SWR_WAVE / BL) * LW)), dim3(LT), 0, S->stream, S->n, N, S->dp, S->packed,     \
                      S->far, S->cand,                                                                              \
@@ -1173,7 +1108,9 @@ int swr_lists_run(swr_system *S, int mode) {
   }
   swr_kt_begin(S, KT_FAR);
   if (mode == 2) {
-    FAR_ARGS((k_far<true, false, true, 2>));
+    hipLaunchKernelGGL(k_from_far, dim3(div_up(N, LW)), dim3(LT), 0, S->stream, S->n, N, S->dp, S->packed, S->far,
+                       S->far_index, S->far_end, S->cand, S->cand_count, S->Hindex, S->num_hbonds, S->hbond_index,
+                       S->hbond_end, S->hbonds, hb_count, S->hbond_cap, S->status);
   } else if (mode == 4) {
     hipLaunchKernelGGL(k_hb_place, dim3(div_up((long long)N * HP_L, LT)), dim3(LT), 0, S->stream, S->n, N, S->Hindex,
                        hb_count, S->num_hbonds, S->voff, S->hbslot, S->far, S->hbond_index, S->hbond_end, S->hbonds,
@@ -1198,7 +1135,6 @@ int swr_lists_run(swr_system *S, int mode) {
     else BOND_ARGS((k_bonds<false>));
     swr_kt_end(S, KT_BONDS);
   }
-#undef FAR_ARGS
 #undef FARWS_ARGS
 #undef BOND_ARGS
   HIP_CHECK(hipGetLastError());

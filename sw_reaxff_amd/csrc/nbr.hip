@@ -724,7 +724,7 @@ int swr_nbr_build(swr_system *S, int local_only) {
                      S->bp_pos, S->bp_id, S->stencil_rows, S->nrows, S->nbin[0], S->nbin[1], S->nbin[2], cutsq,
                      S->vcount, (const long long *)nullptr, (int *)nullptr, nrow);
   swr_kt_end(S, KT_VERLET);
-  if ((rc = swr_scan_i32_to_i64(S, S->vcount, S->voff, N, nullptr))) return rc;
+  if ((rc = swr_scan_i32_to_i64(S, S->vcount, S->voff, N))) return rc;
   // the total, and the local rows' share (the H matrix capacity)
   long long *vt = (long long *)(S->pin_done + SWR_PIN_VERLET);
   SwrPublish pub;

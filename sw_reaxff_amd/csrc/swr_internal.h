@@ -320,7 +320,7 @@ struct swr_system {
   size_t be_stride = 0;            // row stride of be_part/be_ce (the local atom count of the last pass)
   double *bo_dboc = nullptr;       // [N][2]
   double *dDeltap_self = nullptr;  // [N][3]
-  int *bond_mark = nullptr, *bond_mark2 = nullptr;
+  int *bond_mark = nullptr;
   int *counts = nullptr;           // [2][Ncap]: bonds found per atom, hbonds found per H
   int mark_launch_hint = 0;        // bond_mark launches that changed a mark last time
   int *cand = nullptr;             // [Ncap][64]: far slots of bond candidates
@@ -429,7 +429,7 @@ enum {
 enum { CGV_R = 0, CGV_U, CGV_W, CGV_Z, CGV_SS, CGV_V, CGV_P, CGV_D0, CGV_D1, CGV_M, CGV_Q, CGV_COUNT };
 
 // ---- helpers implemented in the .hip files
-int swr_scan_i32_to_i64(swr_system *S, const int *in, long long *out, int n, long long *total_host);
+int swr_scan_i32_to_i64(swr_system *S, const int *in, long long *out, int n);
 int swr_scan_i32(swr_system *S, const int *in, int *out, int n, int *total_dev);
 int swr_ensure_tmp(swr_system *S, size_t bytes);
 

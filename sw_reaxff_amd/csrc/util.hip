@@ -147,15 +147,9 @@ extern "C" const char *swr_last_error(void) {
 }
 
 // Exclusive scan of n ints into int64 offsets; out has n+1 entries
-// (out[n] = total).  If total_host is given, synchronises and returns it.
-int swr_scan_i32_to_i64(swr_system *S, const int *in, long long *out, int n, long long *total_host) {
-  int rc = scan_impl<int, long long>(S, in, out, n, out + n);
-  if (rc) return rc;
-  if (total_host) {
-    HIP_CHECK(hipMemcpyAsync(total_host, out + n, sizeof(long long), hipMemcpyDeviceToHost, S->stream));
-    HIP_CHECK(hipStreamSynchronize(S->stream));
-  }
-  return SWR_OK;
+// (out[n] = total).
+int swr_scan_i32_to_i64(swr_system *S, const int *in, long long *out, int n) {
+  return scan_impl<int, long long>(S, in, out, n, out + n);
 }
 
 // Exclusive scan of n ints into ints; total written to *total_dev (device).
