@@ -86,3 +86,59 @@ def test_mixed_spmv_uses_fp32_values(gpu_lib, ffield):
         want[i] += np.dot(v32[sl].astype(np.float64), x[j[sl]])
     got = h.spmv(x)
     assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
+
+
+def _carbon(m=12, a=1.2, seed=1):
+    """Carbon atoms on a tight shaken lattice: an H so ill-conditioned that inner
+    solves end at their 50 iterations."""
+    from sw_reaxff_amd import systems
+    rng = np.random.default_rng(seed)
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3) * a
+    x = g + rng.normal(scale=0.05, size=g.shape)
+    return systems.System(x=x, v=np.zeros_like(x), type=np.ones(len(x), np.int32),
+                          tag=np.arange(1, len(x) + 1, dtype=np.int32), elements=["C"], lo=x.min(0) - 12.0,
+                          hi=x.max(0) + 12.0, periodic=False)
+
+
+@pytest.mark.parametrize("tol,outer", [(1e-6, None), (1e-30, 20)])
+@pytest.mark.parametrize("batched", [False, True])
+def test_mixed_limits_of_the_inner_and_outer_solves(gpu_lib, ffield, tol, outer, batched):
+    """Inner solves that stop at their 50 iterations, and a tolerance that no
+    pass meets, so the refinement stops after its 20th residual (a warning flag,
+    not an error): the charges are the converged ones, and those queued behind
+    the solve are bit for bit those of a call of their own.  Alone, and in a batch
+    with systems that are done long before."""
+    from sw_reaxff_amd import batch
+    parts = [_carbon()]
+    if batched:
+        w = water_c0(seed=24)
+        small = type(w)(x=w.x[:300], v=w.v[:300], type=w.type[:300], tag=w.tag[:300], elements=w.elements, lo=w.lo,
+                        hi=w.hi, periodic=False)
+        parts = [small, parts[0], small]
+    P = batch.pack(parts)
+
+    def system(**kw):
+        import ctypes as C
+        h = gpu_lib.System(ffield, batch.ELEMENTS, **kw)
+        h.set_atoms(P.n, P.x, P.type, P.tag, owner=P.owner, img=P.img)
+        gpu_lib.check(h.L.swr_set_batch(h.h, len(parts), P.row_off.ctypes.data_as(C.POINTER(C.c_int))), "swr_set_batch")
+        h.build_neighbors(batch.CUTGHOST)
+        return h
+
+    ref = system(tol=1e-10, qeq_imax=1000)
+    ref.call("qeq_pre_force", None, None)
+    ref.sync()
+    queued, staged = system(tol=tol, qeq_mixed=1), system(tol=tol, qeq_mixed=1)
+    queued.call("qeq_pre_force", None, None)
+    staged.call("qeq_init_matvec")
+    staged.qeq_cg()
+    staged.call("calculate_q")
+    assert np.array_equal(queued.get("q"), staged.get("q"))
+    assert np.array_equal(queued.get("sys_iters"), staged.get("sys_iters"))
+    passes = queued.scalar("mixed_outer")
+    its = queued.get("sys_iters").reshape(-1, 2)[1 if batched else 0]
+    assert bool(queued.scalar("flags") & (1 << 8)) == (outer is not None)
+    if outer is not None:
+        assert passes == outer
+        assert its[0] - passes > 49 * (passes - 1)      # of `passes - 1` inner solves one took 50
+    assert np.max(np.abs(queued.get("q")[:P.n] - ref.get("q")[:P.n])) <= Q_MIXED_ATOL
