@@ -592,9 +592,9 @@ __device__ __forceinline__ void hb_triple(const DevHb &hbp, double BOij, const d
 // 2^43), coff elements after it.  A term below 2^10 in magnitude goes to the
 // fine word whole; a larger one is split exactly into a multiple of 2^-20
 // (coarse word) and a remainder of at most 2^-21 (fine word).  Every term
-// thus keeps the 2^-40 resolution (at most 2^-41 rounding per add), the fine
-// word holds at most 2^10 per add (8192 adds before it could wrap), and the
-// pair holds sums up to 2^43.  Both words are integers, so the sums do not
+// thus keeps the 2^-40 resolution (at most 2^-41 rounding per add), a term adds
+// at most 2^10 to the fine word (8192 terms before it could wrap; k_hb adds the
+// terms of a workgroup at once), and the pair holds sums up to 2^43.  Both words are integers, so the sums do not
 // depend on the order the adds arrive in.  A non-finite term, a term beyond
 // ~3.8e12 (2^62 coarse units), or an add that wraps a word (detected from the
 // value atomicAdd returns) raises SWR_F_FIXED_RANGE, which the next swr_sync
@@ -1113,19 +1113,25 @@ __global__ void __launch_bounds__(BT) k_va_scatter(int n, VaArgs A) {
 // Waves of one-wave workgroups a listed pass starts at most; each wave takes
 // its next set of groups that many on (the first ones hold the largest items).
 constexpr int WL_MAX_WAVES = 4096;
-// Shortest group while a list has few items, as lanes in all: below it the
-// pass is bound by each item's chain of loads and transcendentals, not by
-// lanes.
-__device__ __forceinline__ int wl_gmin(int ntask) { return ntask <= 4096 ? 16 : ntask <= 16384 ? 4 : 1; }
+// Shortest group, by the items of the list: with few of them the pass is bound
+// by each item's chain of loads and transcendentals, not by lanes.  Whole passes
+// (us) with 16, 4 and 1 lanes at least; one rule for both (angles cross at about
+// 9,000 and 78,000 items, torsions at 5,000 and 120,000):
+//   valence, water      3,900 items  34  38  49     10,200  60  52  66    36,000 108  72  74
+//                      60,000       167 111 122     78,000 209 132 132    96,000 250 149 146
+//   valence, clusters   2,600        45  54  76     12,100  80  84 115    62,700 241 196 210
+//   torsion, water      3,100        50  54  73      7,200  72  62  81    59,900 321 273 285
+//   torsion, clusters   3,600        63  76 127      8,900  97  94 141   127,600 611 477 475
+__device__ __forceinline__ int wl_gmin(int ntask) { return ntask <= 4096 ? 16 : ntask <= 65536 ? 4 : 1; }
 
 // One group of lanes per listed centre j (largest angle count first): the
 // group's lanes test j's bond pairs and each evaluates one passing pair a
 // round.  What bounds the pass is the latency of one pair's transcendentals
 // (at 1-2 waves a SIMD), so a centre's pairs side by side instead of in turn
 // take the longest centre off the critical path.  Per round the pairs' terms
-// go to LDS and each slot and total is summed by one lane in pair order.  One thread
-// per centre took 52 us on a 64-water box and 150 us on the 32,000-water one;
-// this takes 17 and 115 (512 clusters: 1.05 and 1.11 ms, all lanes busy).
+// go to LDS and each slot and total is summed by one lane in pair order.  One
+// thread per centre took 52 us on a 64-water box, 150 us on the 32,000-water one
+// and 1.05 ms on 512 clusters; this takes 17 us, 94 us and 0.80 ms.
 //
 // SETS: parameter sets per angle type that the round's terms have room for; two
 // (15 KB instead of 29) let eight waves a CU be resident, and the registers are
@@ -1631,11 +1637,17 @@ __global__ void __launch_bounds__(BT) k_to_scatter(int n, ToArgs A) {
 // j's, k's and the bond's over all, each by one lane in order, so the large
 // cotangent terms of a nearly linear angle cancel in FP64 first.  One lane
 // per bond took 87 us on a 64-water box, 133 us on the 32,000-water one and
-// 2.38 ms on 512 clusters; this takes 16, 66 us and 1.31 ms.
+// 2.38 ms on 512 clusters; this takes 15, 65 us and 1.02 ms.
 //
 // WAVES: waves per SIMD the registers are held to.  Two (ten of 266 spilled)
-// pay once a list keeps every SIMD busy with quadruples: 512 clusters 1333 ->
-// 1016 us; 64 clusters 183 -> 188, 96,000 water atoms 64 -> 70, 1,944 17 -> 19.
+// pay once a list keeps every SIMD busy with quadruples (TORSION_TWO_WAVES).
+// From this many atoms on.  The host knows the atoms, not the list's length, but
+// the line is low enough for both kinds of system: the torsion pass with one and
+// with two waves takes 75 and 77 us on 24,000 water atoms (6,600 bonds listed),
+// 134 and 126 on 48,000 (24,700), 182 and 175 on 96,000, 1,294 and 1,263 on
+// 768,000; on clusters of 23,000 atoms (30,700 bonds) 163 and 142, of 40,000 240
+// and 205, of 319,000 1,598 and 1,330.  1,944 atoms: 17 and 19 (the kernel).
+constexpr int TORSION_TWO_WAVES = 32768;
 template <int WAVES>
 __global__ void __launch_bounds__(SWR_WAVE) __attribute__((amdgpu_waves_per_eu(WAVES))) k_torsion(ToArgs A) {
   // the round's quadruples: the bond's and i's terms
@@ -2009,8 +2021,10 @@ int swr_hydrogen_bonds_run(swr_system *S) {
   A.coff = 3 * (size_t)N;
   A.flags = &S->status->flags;
   // atoms per workgroup: few while that fills the chip, more share their
-  // partners' sums
-  const int per = n <= 8192 ? 8 : n <= 32768 ? 16 : HB_ATOMS;
+  // partners' sums.  With 8, 16 and 64 of them (us): 6,000 water atoms 39, 40,
+  // 65; 7,400 of four clusters 39, 36, 56; 8,000 51, 46, 65; 18,000 75, 74, 82;
+  // 24,000 99, 92, 89; 32,000 of thirty clusters 96, 86, 82; 96,000 340, 321, 302
+  const int per = n <= 7168 ? 8 : n <= 24576 ? 16 : HB_ATOMS;
   swr_kt_begin(S, KT_HBONDS);
   if (n > 0) hipLaunchKernelGGL(k_hb, dim3(div_up(n, per)), dim3(BT), 0, S->stream, n, per, A);
   hipLaunchKernelGGL(k_hb_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, S->hb_acc, S->fcd,
@@ -2141,7 +2155,7 @@ int swr_torsion_angles_run(swr_system *S) {
     hipLaunchKernelGGL(k_to_count, dim3(div_up((long long)n * TO_CNT_LANES, BT)), dim3(BT), 0, S->stream, n, A);
     hipLaunchKernelGGL(k_to_scatter, dim3(div_up(n, BT)), dim3(BT), 0, S->stream, n, A);
     const int waves = (int)std::min<long long>(WL_MAX_WAVES, 8LL * n);
-    if (n >= 131072) hipLaunchKernelGGL(k_torsion<2>, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
+    if (n >= TORSION_TWO_WAVES) hipLaunchKernelGGL(k_torsion<2>, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
     else hipLaunchKernelGGL(k_torsion<1>, dim3(waves), dim3(SWR_WAVE), 0, S->stream, A);
   }
   hipLaunchKernelGGL(k_to_fold, dim3(1 + div_up(N, BT)), dim3(BT), 0, S->stream, n, N, A);

@@ -487,3 +487,24 @@ def test_gpu_bond_marks_around_the_searchs_limit(gpu_lib, ffield, m):
     h.call("sort_bonds")                     # once more over its own result
     h.sync()
     assert np.array_equal(h.get("bond_mark")[:N], mark)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [2389, 2390, 4000, 8192, 8193])
+def test_gpu_bonded_groups_around_their_lines(gpu_lib, oracle_lib, ffield, m):
+    """Water boxes on both sides of the lines between workgroups of 8, 16 and 64
+    atoms in the hydrogen-bond pass (7,168 and 24,576 atoms), in the range of four
+    lanes an angle or torsion at least."""
+    s = systems.water_box(m, seed=m)
+    h = harness(s, ffield, tol=1e-10)
+    _gpu_bonded_vs_oracle(gpu_lib, oracle_lib, ffield, h, s.elements, s.type, s.tag)
+    for check in (_gpu_vs_oracle, _gpu_tor_vs_oracle):
+        check(oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
+
+
+@pytest.mark.gpu
+def test_gpu_torsions_at_two_waves(gpu_lib, oracle_lib, ffield):
+    """The first box whose torsions are listed to two waves a SIMD (32,769 atoms)."""
+    s = systems.water_box(10923, seed=9)
+    for check in (_gpu_vs_oracle, _gpu_tor_vs_oracle):
+        check(oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
