@@ -330,8 +330,6 @@ int swr_upload(swr_system *S, int which, void *dst, const void *src, size_t byte
   return swr_stage_send(S, which, dst, bytes);
 }
 
-// Row/tile layout of the (batch of) systems and the buffers sized by it.
-// Rebuilt when the atoms or the batch partition changed.
 int swr_pin_iters_reserve(swr_system *S, int nsys) {
   const int need = 2 * std::max(nsys, 1);
   if (need <= S->pin_iters_cap) return SWR_OK;
@@ -352,6 +350,8 @@ int swr_pin_iters_reserve(swr_system *S, int nsys) {
   return SWR_OK;
 }
 
+// Row/tile layout of the (batch of) systems and the buffers sized by it.
+// Rebuilt when the atoms or the batch partition changed.
 int swr_qeq_layout(swr_system *S) {
   if (!S->layout_dirty) return SWR_OK;
   const int n = S->n;
@@ -492,21 +492,16 @@ int swr_qeq_time_spmv(swr_system *S, int sh, int reps, float *ms) {
   return SWR_OK;
 }
 
-// Runs the FP64 solves of every system to convergence; last_iters: the most
-// iterations of the previous solve (0: from zero history), which size the
-// first batch of iteration launches (one more than it took).
+namespace {
 // Copies up to three runs of words into pinned host memory (one launch; a
 // copy each took ~3 us and a ~5 us gap).
-namespace {
 __global__ void __launch_bounds__(256)
 k_publish(SwrPublish P) {
   for (int r = 0; r < 3; r++)
     for (int k = threadIdx.x; k < P.words[r]; k += 256) P.dst[r][k] = P.src[r][k];
   __threadfence_system();
 }
-}  // namespace
 
-namespace {
 __global__ void k_qeq_clear(int n, double *__restrict__ s_hist, double *__restrict__ t_hist, double *__restrict__ st) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 5 * n) s_hist[i] = t_hist[i] = 0.0;
@@ -527,6 +522,9 @@ int swr_publish(swr_system *S, const SwrPublish &P) {
   return SWR_OK;
 }
 
+// Runs the FP64 solves of every system to convergence; last_iters: the most
+// iterations of the previous solve (0: from zero history), which size the
+// first batch of iteration launches (one more than it took).
 int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
   int rc = swr_panel_ready(S);
   if (rc) return rc;
