@@ -35,6 +35,7 @@
 #include "qeq_cg.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstddef>
 
@@ -46,6 +47,9 @@ constexpr int MAX_OUTER = 20;
 constexpr double OUTER_TOL_FACTOR = 0.001;  // outer target = tol * this
 constexpr double INNER_TOL_MIN = 3e-4;
 constexpr int INNER_IMAX = 50;
+// Inner iterations of a solve's first pass that are queued before the host looks
+// whether the first residual left anything to do: enough to cover the look.
+constexpr int MIX_LOOK = 4;
 // A pass after one whose residual norms were all at most this (relative to
 // |b|) forms its residual incrementally, r -= eta d + H32 d, from the FP32
 // values and the last inner correction d: its rounding, ~1e-6 |H d| with
@@ -285,8 +289,13 @@ k_pcg_init(CgLayout L, const float2 *__restrict__ rhs, const double *__restrict_
 template <int NT>
 __global__ void __launch_bounds__(NT)
 k_pcg_init_scalars(const double *__restrict__ partials, int pstride, CgLayout L,
-                   const CgScalars *__restrict__ inner_all, PcgState *__restrict__ pst, MixCtl *__restrict__ ctl) {
+                   const CgScalars *__restrict__ inner_all, PcgState *__restrict__ pst, MixCtl *__restrict__ ctl,
+                   int *host_first) {
   const int sys = blockIdx.x;
+  if (sys == 0 && threadIdx.x == 0 && host_first) {   // (pinned: the host looks at it while the inner solve runs)
+    *host_first = ctl->first_ndone;
+    __threadfence_system();
+  }
   double tot[4];
   reduce_partials<4, NT>(partials, pstride, L.sys_tile[sys], L.sys_tile[sys + 1], tot);
   if (threadIdx.x != 0) return;
@@ -479,6 +488,15 @@ int ensure_mixw(swr_system *S) {
   return SWR_OK;
 }
 
+// What k_pcg_init_scalars stores in p (-1 before), or -1 should it not come
+// within 20 ms.  (An event would cost the stream a barrier of ~3 us.)
+int mix_look(const volatile int *p) {
+  const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+  int v;
+  while ((v = *p) < 0 && std::chrono::steady_clock::now() < end) {}
+  return v;
+}
+
 }  // namespace
 
 int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_done) {
@@ -550,24 +568,31 @@ int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_don
   residual(1, 0);
   // A pass: the inner FP32 PCG from d = 0, x += d, the next residual.  The
   // first residual hardly ever meets the test, so its inner solve is queued
-  // without a look at it (every launch skips systems that are done).  The
+  // without a look at it (every launch skips systems that are done); the look
+  // comes when MIX_LOOK iterations are queued, while the GPU has those to do.  The
   // iterations go in batches sized from the last solve, each followed by the
   // rest of the pass behind a gate, so a pass usually takes one wait.
   int outer = 1;
   for (;; outer++) {
+    int *host_first = nullptr;
+    if (outer == 1) {
+      host_first = S->pin_done + SWR_PIN_FIRST;
+      *(volatile int *)host_first = -1;
+    }
     swr_kt_begin(S, KT_MIXED_INNER);
     hipLaunchKernelGGL(k_pcg_init, dim3(L.ntiles), dim3(UT), 0, S->stream, L, rhs, S->Hdia_inv, dv, rv, zv, pv,
                        S->partials, ps, ctl);
     if (batch)
       hipLaunchKernelGGL(k_pcg_init_scalars<BT>, dim3(nsys), dim3(BT), 0, S->stream, S->partials, ps, L, inner, pst,
-                         ctl);
+                         ctl, host_first);
     else
       hipLaunchKernelGGL(k_pcg_init_scalars<RT>, dim3(nsys), dim3(RT), 0, S->stream, S->partials, ps, L, inner, pst,
-                         ctl);
+                         ctl, host_first);
     int it = 0;
     int nb = std::max(2, S->mixed_last_inner + 1);
     for (;;) {
       for (int k = 0; k < nb && it < INNER_IMAX; k++, it++) {
+        if (host_first && it == MIX_LOOK && mix_look(host_first) >= nsys) break;
         PcgState *cur = pst + (it & 1) * 2 * nsys, *nxt = pst + ((it + 1) & 1) * 2 * nsys;
         spmv_dispatch(S->spmv_shape[1], [&](auto shc) {
           constexpr int SH = decltype(shc)::value;

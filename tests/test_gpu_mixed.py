@@ -142,3 +142,35 @@ def test_mixed_limits_of_the_inner_and_outer_solves(gpu_lib, ffield, tol, outer,
         assert passes == outer
         assert its[0] - passes > 49 * (passes - 1)      # of `passes - 1` inner solves one took 50
     assert np.max(np.abs(queued.get("q")[:P.n] - ref.get("q")[:P.n])) <= Q_MIXED_ATOL
+
+
+@pytest.mark.parametrize("kind", ["one", "batch", "some"])
+def test_mixed_solve_that_starts_converged(gpu_lib, ffield, kind):
+    """Unmoved atoms with their solution as history (after a cold solve that sizes
+    the first inner batch): the first residual meets the test, so the solve ends
+    there with one product per right-hand side and the histories' charges.  Of a
+    batch with one system from zero history the others stay as they are."""
+    from sw_reaxff_amd import batch, systems
+    parts = [systems.water_box(216, seed=3)] if kind == "one" else [systems.cluster(60 + 9 * k, seed=k) for k in range(7)]
+    exact, bt = (batch.Batch(ffield, mixed=True, tol=t) for t in (1e-9, 1e-6))
+    exact.load(parts)
+    exact.evaluate()
+    exact.sync()
+    hist = [exact.save_history(k, fill=True) for k in range(len(parts))]
+    exact.sync()
+    if kind == "some":
+        hist[3] = None
+    bt.load(parts)
+    bt.evaluate()
+    bt.sync()
+    cold = bt.iterations().copy()
+    assert cold.min() > 10
+    bt.load(parts, hist=hist)
+    bt.evaluate()
+    bt.sync()
+    got = bt.iterations()
+    for k in range(len(parts)):
+        assert tuple(got[k]) == ((1, 1) if hist[k] is not None else tuple(cold[k])), k
+    assert (bt.sys.scalar("mixed_outer") == 1) == (kind != "some")
+    for q, want in zip(bt.charges(), exact.charges()):
+        assert np.max(np.abs(q - want)) <= Q_MIXED_ATOL
