@@ -438,6 +438,7 @@ static CgRun<double, double> fp64_run(swr_system *S) {
   R.iters_host = S->h_sys_iters.data();
   R.pin_done = S->pin_done;
   R.pin_iters = S->pin_iters;
+  R.pin_look = nullptr;
   R.tol = S->ctl.tol;
   R.imax = S->imax;
   R.kt_iter = KT_CG_ITER;
@@ -534,7 +535,8 @@ int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done) {
     for (int s = 0; s < S->nsys; s++) rows = std::max(rows, S->sys_row[s + 1] - S->sys_row[s]);
     first_batch = std::min(CG_COLD_BATCH, rows + 2);
   }
-  const CgRun<double, double> R = fp64_run(S);
+  CgRun<double, double> R = fp64_run(S);
+  if (last_iters <= 0 && !S->cg_small) R.pin_look = S->pin_done + SWR_PIN_LOOK;
   int all = S->nsys;
   if (S->cg_small) {   // (a system without rows has no workgroup to finish it)
     all = 0;

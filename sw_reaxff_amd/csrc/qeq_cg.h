@@ -18,6 +18,7 @@
 // sqrt(u.r)/|b| <= tol (or i = imax) and is frozen while the other runs.
 #pragma once
 
+#include <chrono>
 #include <cstring>
 #include <type_traits>
 
@@ -518,8 +519,12 @@ k_cg_upd(CgVecsT<T> V, int par_in, const CgScalars *__restrict__ cgs, CgLayout L
 template <int PH>
 __global__ void __launch_bounds__(RT)
 k_cg_scalars(const double *__restrict__ partials, int pstride, CgScalars *__restrict__ cgs, CgLayout L, int imax,
-             double tol, DevStatus *st, int *__restrict__ iters_out) {
+             double tol, DevStatus *st, int *__restrict__ iters_out, int *pin_look) {
   const int sys = blockIdx.x;
+  if (PH == PH_A1 && pin_look && sys == 0 && threadIdx.x == 0) {   // systems that the setup found done
+    *pin_look = *L.done_count;
+    __threadfence_system();
+  }
   CgScalars c0 = cgs[2 * sys], c1 = cgs[2 * sys + 1];
   const bool b0 = PH == PH_K && c0.active_b != 0, b1 = PH == PH_K && c1.active_b != 0;
   const bool a0 = PH == PH_S3 || c0.active_a != 0, a1 = PH == PH_S3 || c1.active_a != 0;
@@ -569,12 +574,23 @@ struct CgRun {
   int *iters_host;    // when set: the host copy, refreshed at every done check
   int *pin_done;      // when set: pinned host int and iteration counts the
   int *pin_iters;     // done checks copy into (then iters_host from pin_iters)
+  int *pin_look;      // when set: pinned host int for the systems done at setup
   double tol;         // > 0: set at setup; <= 0: preset in cgs[].tol
   int imax;           // iteration limit (the reference's imax = 200 for the FP64 solve)
   int kt_iter, kt_update, kt_setup, kt_scalars;
   double *partials;   // per-workgroup partial dots, [8][pstride]
   int pstride;
 };
+
+// What a queued kernel stores in pinned p (below 0 before), or p's value should
+// it not come within 20 ms: the host looks at a result while the GPU has later
+// launches to do.  (An event would cost the stream a barrier of ~3 us.)
+inline int swr_look(const volatile int *p) {
+  const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+  int v;
+  while ((v = *p) < 0 && std::chrono::steady_clock::now() < end) {}
+  return v;
+}
 
 // Queues behind()'s work, then waits for what was queued before it.
 template <class Behind>
@@ -596,7 +612,7 @@ int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzer
 #define SP_ARGS n, S->dp, S->type, S->H_firstnbr, S->H_numnbrs, S->H_jlist, R.val, R.V, par_in, R.cgs, R.L.row_sys, \
                 panel_args(S)
 #define UP_ARGS R.V, par_in, R.cgs, R.L, R.partials, ps, xzero
-#define SC_ARGS R.partials, ps, R.cgs, R.L, R.imax, R.tol, S->status, R.iters_out
+#define SC_ARGS R.partials, ps, R.cgs, R.L, R.imax, R.tol, S->status, R.iters_out, R.pin_look
   swr_kt_begin(S, kt);
   spmv_dispatch(S->spmv_shape[0], [&](auto shc) {
     constexpr int SH = decltype(shc)::value;
@@ -671,17 +687,22 @@ int launch_cg(swr_system *S, const CgRun<T, VT> &R, int ph, int par_in, int xzer
 // since r rows take about r iterations: with sixteen launches an evaluation of
 // 4,096 single waters (4 iterations) took 1,290 us, with five 980; of 12,000 of
 // them 2,707 and 2,129.
-constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8;
+// Unmoved atoms with their solution as history are done at setup: with pin_look
+// the host looks after CG_LOOK iterations are queued.
+constexpr int CG_COLD_BATCH = 16, CG_NEXT_BATCH = 8, CG_LOOK = 4;
 template <typename T, typename VT, class Step, class Behind>
 int cg_solve(swr_system *S, const CgRun<T, VT> &R, int first_batch, int all, Step step, Behind behind,
              bool *finished) {
   int rc;
+  if (R.pin_look) *(volatile int *)R.pin_look = -1;
   if ((rc = step(PH_S1, 0)) || (rc = step(PH_S2, 0)) || (rc = step(PH_S3, 0)) || (rc = step(PH_A1, 0))) return rc;
   int k = 1;
   int batch = first_batch > 2 ? first_batch : 2;
   while (k < R.imax + 1) {
-    for (int b = 0; b < batch && k < R.imax + 1; b++, k++)
+    for (int b = 0; b < batch && k < R.imax + 1; b++, k++) {
+      if (k == 1 + CG_LOOK && R.pin_look && swr_look(R.pin_look) >= all) break;
       if ((rc = step(PH_K, k))) return rc;
+    }
     // one round trip: done count, status block and iteration counts (into
     // pinned memory when the run has it)
     int done = 0;

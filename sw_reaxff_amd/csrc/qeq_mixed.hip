@@ -35,7 +35,6 @@
 #include "qeq_cg.h"
 
 #include <algorithm>
-#include <chrono>
 #include <cmath>
 #include <cstddef>
 
@@ -488,15 +487,6 @@ int ensure_mixw(swr_system *S) {
   return SWR_OK;
 }
 
-// What k_pcg_init_scalars stores in p (-1 before), or -1 should it not come
-// within 20 ms.  (An event would cost the stream a barrier of ~3 us.)
-int mix_look(const volatile int *p) {
-  const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
-  int v;
-  while ((v = *p) < 0 && std::chrono::steady_clock::now() < end) {}
-  return v;
-}
-
 }  // namespace
 
 int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_done) {
@@ -576,7 +566,7 @@ int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_don
   for (;; outer++) {
     int *host_first = nullptr;
     if (outer == 1) {
-      host_first = S->pin_done + SWR_PIN_FIRST;
+      host_first = S->pin_done + SWR_PIN_LOOK;
       *(volatile int *)host_first = -1;
     }
     swr_kt_begin(S, KT_MIXED_INNER);
@@ -592,7 +582,7 @@ int swr_qeq_mixed_solve(swr_system *S, bool then_q, bool *read_back, bool *q_don
     int nb = std::max(2, S->mixed_last_inner + 1);
     for (;;) {
       for (int k = 0; k < nb && it < INNER_IMAX; k++, it++) {
-        if (host_first && it == MIX_LOOK && mix_look(host_first) >= nsys) break;
+        if (host_first && it == MIX_LOOK && swr_look(host_first) >= nsys) break;
         PcgState *cur = pst + (it & 1) * 2 * nsys, *nxt = pst + ((it + 1) & 1) * 2 * nsys;
         spmv_dispatch(S->spmv_shape[1], [&](auto shc) {
           constexpr int SH = decltype(shc)::value;

@@ -472,7 +472,7 @@ int swr_qeq_cg_run(swr_system *S, int last_iters, bool then_q, bool *q_done);
 #define SWR_PIN_MIX 4096
 #define SWR_PIN_VERLET 4    // in pin_done: two 64-bit Verlet totals
 #define SWR_PIN_BORDERS 8   // in pin_done: six atom counts of the border passes
-#define SWR_PIN_FIRST 14    // in pin_done: systems done on a mixed solve's first residual
+#define SWR_PIN_LOOK 14    // in pin_done: systems done at a solve's setup
 // Grows the pinned iteration-count buffer to nsys systems (synchronises the
 // stream before replacing it).
 int swr_pin_iters_reserve(swr_system *S, int nsys);

@@ -508,3 +508,37 @@ def test_gpu_torsions_at_two_waves(gpu_lib, oracle_lib, ffield):
     s = systems.water_box(10923, seed=9)
     for check in (_gpu_vs_oracle, _gpu_tor_vs_oracle):
         check(oracle_lib, ffield, harness(s, ffield, tol=1e-10), s.elements, s.type, s.tag)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[1400], [1100, 30, 1200], [1100, 1200]])
+def test_gpu_solves_done_at_setup_queue_few_iterations(gpu_lib, ffield, sizes):
+    """Unmoved atoms with their solution as history: the general solve is done at
+    its setup, and the host sees it after a few queued iterations instead of the
+    sixteen of a first solve; with one system from zero history the batch goes on."""
+    from sw_reaxff_amd.batch import Batch
+    parts = [waters(m, seed=m) for m in sizes]
+    exact, bt = Batch(ffield, tol=1e-9), Batch(ffield, tol=1e-6)
+    exact.load(parts)
+    exact.evaluate()
+    exact.sync()
+    hist = [exact.save_history(k, fill=True) for k in range(len(parts))]
+    exact.sync()
+    bt.sys.ktimer_enable()
+
+    def solve(h):
+        bt.load(parts, hist=h)
+        bt.sys.ktimer_read("cg_iter", True)
+        bt.evaluate()
+        bt.sync()
+        return bt.sys.ktimer_read("cg_iter")[1], bt.iterations().copy(), [q.copy() for q in bt.charges()]
+
+    launches, its, q = solve(hist)
+    assert its.max() == 1 and launches <= 6
+    assert all(np.max(np.abs(a - b)) <= 1e-7 for a, b in zip(q, exact.charges()))
+    cold_launches, cold_its, cold_q = solve(None)
+    assert cold_its.min() > 10 and cold_launches >= cold_its.max() - 1     # (the setup counts as one)
+    if len(parts) > 1:
+        launches, its, q = solve([None] + hist[1:])
+        assert tuple(its[0]) == tuple(cold_its[0]) and its[1:].max() == 1
+        assert np.array_equal(q[0], cold_q[0])
